@@ -80,6 +80,8 @@ SIGNATURES = {
     "sy_decode_attention_qkv": (_c_int, [_c_void_p, _c_void_p, _c_void_p, _c_float, _c_float, _c_void_p, _c_void_p, _c_int,
                                          _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int,
                                          _c_void_p, _c_void_p, _c_void_p, _c_void_p]),
+    "sy_prefill_attention": (_c_int, [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int,
+                                      _c_int, _c_int, _c_void_p, _c_void_p]),
     "sy_decode_attention": (_c_int, [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int,
                                      _c_int, _c_int, _c_void_p, _c_void_p]),
 }
@@ -692,6 +694,24 @@ class Ext:
                    slot.data_ptr(), B, rows // B, int(heads), int(kv_heads), D, kcache.shape[2], q.data_ptr(),
                    kcache.data_ptr(), vcache.data_ptr(), _stream())
         return q
+
+    def prefill_attention(self, q, kcache, vcache, real, first, heads):
+        """q [B*T, heads D] at cache positions first .. first + T - 1 of their sequences, against kcache
+        / vcache [B, kv_heads, capacity, D]: each query sees the positions up to its own that `real`
+        [B, capacity] (bool) marks, or its own value if there is none -> [B*T, heads D]."""
+        for t, name in ((q, "q"), (kcache, "kcache"), (vcache, "vcache")):
+            _check(t, name, torch.float16)
+        _check(real, "real", torch.bool)
+        if kcache.dim() != 4 or vcache.shape != kcache.shape:
+            raise RuntimeError("prefill_attention: caches must be [B, kv_heads, capacity, head_dim]")
+        B, kv_heads, capacity, D = kcache.shape
+        rows = q.shape[0]
+        if B == 0 or rows == 0 or rows % B or tuple(q.shape) != (rows, heads * D) or tuple(real.shape) != (B, capacity):
+            raise RuntimeError("prefill_attention: shapes of q / caches / real do not match")
+        out = torch.empty_like(q)
+        self._call(self.lib.sy_prefill_attention, q.data_ptr(), kcache.data_ptr(), vcache.data_ptr(), real.data_ptr(),
+                   int(first), B, rows // B, int(heads), kv_heads, D, capacity, out.data_ptr(), _stream())
+        return out
 
     def decode_attention(self, q, kcache, vcache, real, slot, heads):
         """q [B, heads D] against kcache / vcache [B, kv_heads, capacity, D], keys 0..slot that

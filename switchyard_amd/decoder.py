@@ -14,6 +14,7 @@ stream) and a prompt goes through `prefill_fused` (the same row kernels around P
 attention call); fp32 and the CPU use the PyTorch operators (`forward`, `step_static`).
 """
 
+import functools
 from dataclasses import dataclass
 
 import torch
@@ -138,11 +139,16 @@ class Span:
             slot_real = cache.real[:, :self.end]
         else:
             slot_real = self.real
+        self._slot_real = slot_real
+
+    @functools.cached_property
+    def visible(self):
+        dev = self._slot_real.device
         query_slot = torch.arange(self.first, self.end, device=dev)[:, None]
         slot = torch.arange(self.end, device=dev)[None, :]
-        sees = (slot <= query_slot)[None] & slot_real[:, None, :]
+        sees = (slot <= query_slot)[None] & self._slot_real[:, None, :]
         alone = ~sees.any(-1, keepdim=True)
-        self.visible = (sees | (alone & (slot == query_slot)[None]))[:, None]   # broadcast over heads
+        return (sees | (alone & (slot == query_slot)[None]))[:, None]   # broadcast over heads
 
     def commit(self, cache):
         """The span now belongs to the cache."""
@@ -250,7 +256,8 @@ class Decoder:
         and the cache write are one launch each over all B*T rows (in PyTorch they are some
         seventy element-wise launches per layer, each a pass over the activations), the three
         input projections are one GEMM, and the lm_head runs on B rows instead of B*T.
-        Attention itself is PyTorch's fused scaled-dot-product call under the same mask."""
+        Attention is one launch too, with the mask's rule instead of a mask tensor, straight from
+        and into the layouts of its neighbours."""
         from . import kernels
 
         s, W, E = self.s, self.w, kernels.ext()
@@ -265,10 +272,8 @@ class Decoder:
             after = W["layers"][i + 1]["attn_norm"] if i + 1 < s.layers else W["final_norm"]
             q = E.qk_norm_rope_cache(kernels.dense(xn, wqkv[i]), L["q_norm"], L["k_norm"], s.rms_eps, s.clip_qkv, self.cos,
                                      self.sin, flat_positions, slot, s.heads, s.kv_heads, s.head_dim, cache.k[i], cache.v[i])
-            a = F.scaled_dot_product_attention(q.view(B, T, s.heads, s.head_dim).transpose(1, 2),
-                                               cache.k[i, :, :, :span.end], cache.v[i, :, :, :span.end],
-                                               attn_mask=span.visible, enable_gqa=s.kv_heads != s.heads)
-            o = kernels.dense(a.transpose(1, 2).reshape(B * T, s.heads * s.head_dim), L["wo"])
+            a = E.prefill_attention(q, cache.k[i], cache.v[i], cache.real, span.first, s.heads)
+            o = kernels.dense(a, L["wo"])
             x, h = E.add_rmsnorm(x, o, L["mlp_norm"], s.rms_eps, x_out=x)
             if self._own_moe and s.top_k <= 64:
                 y, pos_of, idx = kernels.experts_rows(h, None, L["gate_up"], L["down"], s.top_k, s.norm_topk_prob,

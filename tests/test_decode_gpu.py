@@ -197,6 +197,39 @@ def test_qk_norm_rope_cache(B, heads, kv_heads, hd, clip):
     assert torch.equal(kc[:, :, keep], kc0[:, :, keep]) and torch.equal(vc[:, :, keep], vc0[:, :, keep])
 
 
+@pytest.mark.parametrize("B,T,first,heads,kv_heads,hd", [
+    (2, 1, 0, 4, 4, 128), (1, 1, 64, 1, 1, 64),                     # one query; one behind a whole tile of keys
+    (2, 31, 0, 4, 2, 64), (2, 33, 0, 4, 4, 128), (1, 64, 0, 2, 2, 128), (1, 65, 63, 2, 1, 64),   # edges of the tiles
+    (3, 127, 5, 8, 8, 128), (2, 129, 200, 16, 4, 64),               # behind a filled cache
+    (8, 300, 0, 16, 16, 128),                                       # 128 queries per workgroup (many pairs)
+    (1, 437, 0, 16, 16, 128), (2, 1100, 1000, 16, 2, 64)])
+@pytest.mark.parametrize("holes", [False, True])
+def test_prefill_attention(B, T, first, heads, kv_heads, hd, holes):
+    g = torch.Generator().manual_seed(21)
+    cap = first + T + 7
+    q = rnd(B * T, heads * hd, seed=22, std=1.5)
+    kc, vc = rnd(B, kv_heads, cap, hd, seed=23), rnd(B, kv_heads, cap, hd, seed=24)
+    # left padding of different lengths (whole tiles and query blocks of it), and any pattern of holes
+    pad = torch.randint(0, first + T, (B,), generator=g)
+    pad[0] = 0
+    real = torch.arange(cap)[None] >= pad[:, None]
+    if holes:
+        real &= torch.rand(B, cap, generator=g) > 0.3
+    real = real.cuda()
+    out = kernels.ext().prefill_attention(q, kc, vc, real, first, heads)
+    slot, at = torch.arange(first + T, device="cuda")[None], torch.arange(first, first + T, device="cuda")[:, None]
+    sees = (slot <= at)[None] & real[:, None, :first + T]
+    sees |= ~sees.any(-1, keepdim=True) & (slot == at)[None]     # a query that sees nothing takes its own value
+    ref = [t.float().cpu() for t in (q.view(B, T, heads, hd).transpose(1, 2), kc[:, :, :first + T], vc[:, :, :first + T])]
+    ref[1:] = [t.repeat_interleave(heads // kv_heads, 1) for t in ref[1:]]
+    p = (ref[0] @ ref[1].transpose(-1, -2).contiguous() / math.sqrt(hd)).masked_fill(~sees.cpu()[:, None], -math.inf).softmax(-1)
+    want, spread = p @ ref[2], p @ ref[2].abs()
+    got = out.view(B, T, heads, hd).transpose(1, 2).float().cpu()
+    # each probability is rounded to f16 once (half an ulp of itself), and so is the result; the rest is fp32
+    bound = ULP / 2 * (spread + want.abs()) * 1.05 + 1e-4
+    assert ((got - want).abs() <= bound).all(), ((got - want).abs() - bound).max()
+
+
 @pytest.mark.parametrize("B,heads,kv_heads,hd,cap,slot_at", [
     (8, 16, 16, 128, 640, 600),    # OLMoE at batch 8: 16 wavefronts per (sequence, head)
     (64, 16, 16, 128, 200, 199),   # many pairs: 4 wavefronts each; the last slot of the cache
