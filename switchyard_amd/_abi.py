@@ -31,7 +31,7 @@ class SyMoeLayer(ctypes.Structure):
                 ("scratch_bytes", _c_size_t)]
 
 
-# name -> (restype, argtypes); mirrors include/switchyard_moe.h and include/switchyard_decode.h
+# name -> (restype, argtypes); mirrors include/switchyard_moe.h, include/switchyard_decode.h and csrc/passes.h
 SIGNATURES = {
     "sy_version": (_c_int, []),
     "sy_last_error": (ctypes.c_char_p, []),

@@ -33,7 +33,7 @@
 #include <type_traits>
 
 #include "common.h"
-#include "../../include/switchyard_decode.h"
+#include "passes.h"
 
 namespace {
 

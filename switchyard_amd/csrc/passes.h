@@ -1,0 +1,23 @@
+/* Entry points that the library offers its own Python host code (switchyard_amd/decoder.py) beside
+ * the two public headers: pieces of whole passes of the decoder. Conventions as in
+ * include/switchyard_moe.h: device pointers, sizes, a hipStream_t; SY_OK or an SY_ERR_* code with a
+ * message in sy_last_error(); nothing is allocated and nothing waits. */
+#pragma once
+
+#include "../../include/switchyard_moe.h"
+
+extern "C" {
+
+/* T queries per sequence against the KV cache (a prompt, or further tokens behind what the cache
+ * holds); replaces the scores / mask / softmax / value product of _attention()
+ * (switchyard/model.py:78-84) for T >= 1.
+ * q f16 [B*T, heads*D]: query t of sequence b sits at cache position first + t; kcache, vcache
+ * f16 [B, kv_heads, capacity, D] hold the positions 0 .. first + T - 1; real uint8 [B, capacity]
+ * marks real tokens. A query sees the real positions up to its own; one that would see none (left
+ * padding) takes its own value -> out f16 [B*T, heads*D] (fp32 inside, probabilities rounded to
+ * f16 for the value product). Query head h reads kv head h / (heads / kv_heads).
+ * Limits: D is 64 or 128, first + T <= capacity. B == 0 is a no-op. */
+SY_API int sy_prefill_attention(const void* q, const void* kcache, const void* vcache, const uint8_t* real, int first,
+                                int B, int T, int heads, int kv_heads, int D, int capacity, void* out, void* stream);
+
+}  // extern "C"
