@@ -80,6 +80,9 @@ SIGNATURES = {
     "sy_decode_attention_qkv": (_c_int, [_c_void_p, _c_void_p, _c_void_p, _c_float, _c_float, _c_void_p, _c_void_p, _c_int,
                                          _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int,
                                          _c_void_p, _c_void_p, _c_void_p, _c_void_p]),
+    "sy_padding_twins": (_c_int, [_c_void_p, _c_void_p, _c_int, _c_int, _c_void_p, _c_void_p]),
+    "sy_moe_add_rmsnorm": (_c_int, [ctypes.POINTER(SyMoeLayer), _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_float,
+                                    _c_void_p, _c_void_p, _c_void_p]),
     "sy_prefill_attention": (_c_int, [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int,
                                       _c_int, _c_int, _c_void_p, _c_void_p]),
     "sy_decode_attention": (_c_int, [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int,
@@ -431,6 +434,49 @@ class Ext:
         desc = SyMoeLayer(N, E, k, norm, H, I, int(mfma_tiles), 0, router.data_ptr(), gate_up.data_ptr(), down.data_ptr(),
                           plan[2].data_ptr(), plan[2].numel())
         return desc, plan
+
+    def padding_twins(self, tokens, real):
+        """tokens int64 and real bool, both [B, T], of prompts that start a cache -> int32 [B*T]: for each
+        row one that holds the same values in every layer (itself, or for left padding the first
+        row of such padding in the batch that has the same token)."""
+        _check(tokens, "tokens", torch.int64)
+        _check(real, "real", torch.bool)
+        if tokens.dim() != 2 or real.shape != tokens.shape:
+            raise RuntimeError("padding_twins: tokens and real must be [B, T]")
+        twin = torch.empty(tokens.numel(), dtype=torch.int32, device=tokens.device)
+        self._call(self.lib.sy_padding_twins, tokens.data_ptr(), real.data_ptr(), *tokens.shape, twin.data_ptr(), _stream())
+        return twin
+
+    def moe_layer_scratch(self, N, E, k, H, I, device):
+        """Scratch for the moe_add_rmsnorm calls of one pass (they run in order on one stream)."""
+        return torch.empty(max(self.lib.sy_moe_layer_scratch_bytes(N, E, k, H, I), 256), dtype=torch.uint8, device=device)
+
+    def moe_add_rmsnorm(self, h, router, gate_up, down, k, norm, x, weight, eps, scratch, twin=None, x_out=None):
+        """The MoE layer of h [N, H], the residual add and the next norm in one call: returns
+        (x + moe_layer(h), its RMS norm times weight). `twin` (padding_twins) names rows of h that are
+        the same, whose experts are then run once. A prompt's path: N > 64, router_route_ok."""
+        for t, name in ((h, "h"), (router, "router"), (gate_up, "gate_up"), (down, "down"), (x, "x"), (weight, "weight")):
+            _check(t, name, torch.float16)
+        N, H = h.shape
+        E, I = router.shape[0], down.shape[2]
+        if tuple(router.shape) != (E, H) or tuple(gate_up.shape) != (E, 2 * I, H) or tuple(down.shape) != (E, H, I):
+            raise RuntimeError("moe_add_rmsnorm: shapes of h / router / gate_up / down do not match")
+        if x.shape != h.shape or weight.numel() != H:
+            raise RuntimeError("moe_add_rmsnorm: x [N, H], weight [H]")
+        if twin is not None:
+            _check(twin, "twin", torch.int32)
+            if twin.numel() != N:
+                raise RuntimeError("moe_add_rmsnorm: twin [N]")
+        x_out = torch.empty_like(x) if x_out is None else x_out
+        _check(x_out, "x_out", torch.float16)
+        if x_out.shape != x.shape:
+            raise RuntimeError("moe_add_rmsnorm: x_out has another shape than x")
+        h_out = torch.empty_like(h)
+        layer = SyMoeLayer(N, E, int(k), int(bool(norm)), H, I, 1, 0, router.data_ptr(), gate_up.data_ptr(), down.data_ptr(),
+                           scratch.data_ptr(), scratch.numel())
+        self._call(self.lib.sy_moe_add_rmsnorm, layer, h.data_ptr(), twin.data_ptr() if twin is not None else None,
+                   x.data_ptr(), weight.data_ptr(), float(eps), x_out.data_ptr(), h_out.data_ptr(), _stream())
+        return x_out, h_out
 
     def experts_routed(self, h, idx, w, gate_up, down, mfma_tiles=False):
         """experts() of the reference in one call of the library: h [N, H], idx int32 [N, k],

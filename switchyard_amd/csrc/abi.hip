@@ -4,6 +4,7 @@
 
 #include "common.h"
 #include "../../include/switchyard_decode.h"
+#include "passes.h"
 
 namespace {
 thread_local char g_error[512] = "";
@@ -70,7 +71,8 @@ extern "C" SY_API int sy_moe_experts(const void* h, const void* router, void* lo
     // sort's first pass where the sort runs over many workgroups
     SY_REQUIRE(!one_launch_front, "moe_experts: one_launch_front with a router is for at most 64 tokens");
     const bool counted = sy_router_route_counts(N, k) && sort_workspace && sort_workspace_bytes >= sy_sort_workspace_bytes(N, k, E);
-    rc = sy_router_route_counting(h, router, N, H, E, k, norm, logits, idx, w, counted ? sort_workspace : nullptr, stream);
+    rc = sy_router_route_counting(h, router, N, H, E, k, norm, logits, idx, w, counted ? sort_workspace : nullptr, nullptr,
+                                  stream);
     if (rc) return rc;
     rc = counted ? sy_sort_assign_counted(idx, w, N, k, E, counts, offsets, token, wsorted, pos_of, sort_workspace, stream)
                  : sy_sort_by_expert(idx, w, 2, N, k, E, counts, offsets, token, wsorted, pos_of, sort_workspace,
@@ -155,6 +157,42 @@ extern "C" SY_API int sy_moe_layer(const SyMoeLayer* L, const void* h, void* out
                         (int32_t*)(b + s.idx), b + s.w, (int32_t*)(b + s.counts), (int32_t*)(b + s.offsets),
                         (int32_t*)(b + s.token), b + s.wsorted, (int32_t*)(b + s.pos_of), b + s.act, b + s.y, out,
                         s.sort_bytes ? b + s.sort_ws : nullptr, s.sort_bytes, stream);
+}
+
+// moe_layer() and what follows it in a prompt's pass, the residual add and the next norm, in one
+// call: the router GEMM, route and (from 2048 choices on) the sort's first pass in one launch, the
+// sort, the two projections, and combine + add + norm in one launch.
+extern "C" SY_API int sy_moe_add_rmsnorm(const SyMoeLayer* L, const void* h, const int32_t* twin, const void* x,
+                                         const void* weight, float eps, void* x_out, void* h_out, void* stream) {
+  SY_REQUIRE(L, "moe_add_rmsnorm: null layer");
+  SY_REQUIRE(L->N >= 0 && L->E >= 1 && L->k >= 1 && L->H >= 8 && L->I >= 8, "moe_add_rmsnorm: N = %d, E = %d, k = %d, H = %d, I = %d",
+             L->N, L->E, L->k, L->H, L->I);
+  if (L->N == 0) return SY_OK;
+  SY_REQUIRE(L->router && L->gate_up && L->down && h && x && weight && h_out, "moe_add_rmsnorm: null pointer");
+  const int N = L->N, E = L->E, k = L->k, H = L->H, I = L->I, M = N * k;
+  SY_REQUIRE(sy_router_route_shape_ok(N, H, E, k), "moe_add_rmsnorm: H a multiple of 512, at most 128 experts and top-8 "
+             "(got N = %d, H = %d, E = %d, k = %d)", N, H, E, k);
+  const LayerScratch s = layer_scratch(N, E, k, H, I);
+  SY_REQUIRE(L->scratch && L->scratch_bytes >= s.end && ((uintptr_t)L->scratch & 255) == 0,
+             "moe_add_rmsnorm: scratch of %zu bytes, 256-byte aligned, needed (%zu given)", s.end, L->scratch_bytes);
+  char* b = (char*)L->scratch;
+  int32_t *idx = (int32_t*)(b + s.idx), *counts = (int32_t*)(b + s.counts), *offsets = (int32_t*)(b + s.offsets);
+  int32_t *token = (int32_t*)(b + s.token), *pos_of = (int32_t*)(b + s.pos_of);
+  void *w = b + s.w, *wsorted = b + s.wsorted, *act = b + s.act, *y = b + s.y, *ws = b + s.sort_ws;
+  const bool counted = sy_router_route_counts(N, k);
+  int rc = sy_router_route_counting(h, L->router, N, H, E, k, L->norm, b + s.logits, idx, w, counted ? ws : nullptr, twin, stream);
+  if (rc) return rc;
+  rc = counted ? sy_sort_assign_counted(idx, w, N, k, E, counts, offsets, token, wsorted, pos_of, ws, stream)
+               : sy_sort_by_expert(idx, w, 2, N, k, E, counts, offsets, token, wsorted, pos_of, ws, s.sort_bytes, stream);
+  if (rc) return rc;
+  // the same choice as in sy_experts_sorted: the 256-row tile leaves the router weights to the combine
+  const bool combine_scales = sy_gemm_rows_per_tile(M, E, I) == 256;
+  rc = sy_grouped_gemm(h, token, L->gate_up, offsets, E, M, I, H, 1, nullptr, act, stream);
+  if (rc) return rc;
+  rc = sy_grouped_gemm(act, nullptr, L->down, offsets, E, M, H, I, 0, combine_scales ? nullptr : wsorted, y, stream);
+  if (rc) return rc;
+  return sy_combine_add_rmsnorm_twins(y, pos_of, idx, combine_scales ? w : nullptr, k, twin, x, weight, eps, N, H, x_out, h_out,
+                                      stream);
 }
 
 // experts() of the reference in one call: sort, the two projections, combine, from the routing.

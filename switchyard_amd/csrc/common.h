@@ -29,12 +29,15 @@ int sy_sort_assign_counted(const int32_t* idx, const void* w, int N, int k, int 
                            int32_t* token, void* wsorted, int32_t* pos_of, void* workspace, void* stream);
 // front.hip: router logits + route in one launch; with `hist` also the sort's per-piece histograms
 int sy_router_route_counting(const void* h, const void* router, int N, int H, int E, int k, int norm, void* logits,
-                             int32_t* idx, void* w, void* hist, void* stream);
+                             int32_t* idx, void* w, void* hist, const int32_t* twin, void* stream);
 bool sy_router_route_counts(int N, int k);
 // front.hip: whether that launch takes the shape (H a multiple of 512, at most 128 experts, top-8)
 bool sy_router_route_shape_ok(int N, int H, int E, int k);
 // gemm.hip: rows of the tile that sy_grouped_gemm picks for `rows` sorted rows over E experts (64, 128 or 256)
 int sy_gemm_rows_per_tile(int rows, int E, int K);
+int sy_combine_add_rmsnorm_twins(const void* y, const int32_t* pos_of, const int32_t* idx, const void* w, int k,
+                                 const int32_t* twin, const void* x, const void* weight, float eps, int N, int H,
+                                 void* x_out, void* h_out, void* stream);
 // decode.hip: router GEMM + route for a few rows (one workgroup per row)
 int sy_router_route_rows(const void* h, const void* router, int N, int H, int E, int k, int norm, void* logits, int32_t* idx,
                          void* w, void* stream);

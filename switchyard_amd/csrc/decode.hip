@@ -73,7 +73,7 @@ row_kernel(const half_t* x, const half_t* __restrict__ delta, const half_t* __re
            const int* __restrict__ pos_of, const int* __restrict__ idx, int k, const half_t* __restrict__ weight,
            float eps, const half_t* __restrict__ router, int E, int H, half_t* x_out, half_t* __restrict__ h_out,
            half_t* __restrict__ logits, const int64_t* __restrict__ gather, int src_rows,
-           front_core::Outputs front = front_core::Outputs{}) {  // x_out may be x
+           front_core::Outputs front = front_core::Outputs{}, const int* __restrict__ twin = nullptr) {  // x_out may be x
   extern __shared__ __attribute__((aligned(16))) half_t hs[];  // LOGITS: the normalised row [H]; FRONT: the tail's LDS behind it
   __shared__ float part[16];
   __shared__ int rows[ROW_MAX_K];
@@ -91,8 +91,9 @@ row_kernel(const half_t* x, const half_t* __restrict__ delta, const half_t* __re
   if (COMBINE) {
     // rank the k choices by (expert id, slot); rows[] lists their rows of y in that order
     if (tid < WAVE) {
-      const int mine = tid < k ? idx[(size_t)t * k + tid] : 0x7fffffff;
-      const int src = tid < k ? pos_of[(size_t)t * k + tid] : 0;
+      const int of = twin ? twin[t] : t;   // the token whose expert outputs are this one's (front.hip)
+      const int mine = tid < k ? idx[(size_t)of * k + tid] : 0x7fffffff;
+      const int src = tid < k ? pos_of[(size_t)of * k + tid] : 0;
       int rank = 0;
       for (int j = 0; j < k; ++j) {
         const int other = read_lane(mine, j);
@@ -100,7 +101,7 @@ row_kernel(const half_t* x, const half_t* __restrict__ delta, const half_t* __re
       }
       if (tid < k) {
         rows[rank] = src;
-        wts[rank] = delta ? (float)delta[(size_t)t * k + tid] : 1.f;
+        wts[rank] = delta ? (float)delta[(size_t)of * k + tid] : 1.f;
       }
     }
     __syncthreads();
@@ -814,17 +815,64 @@ extern "C" SY_API int sy_add_rmsnorm_route_sort(const void* x, const void* delta
   return sy_check_launch("add_rmsnorm_route_sort");
 }
 
-extern "C" SY_API int sy_combine_add_rmsnorm(const void* y, const int32_t* pos_of, const int32_t* idx, const void* w, int k,
-                                             const void* x, const void* weight, float eps, int N, int H, void* x_out,
-                                             void* h_out, void* stream) {
+int sy_combine_add_rmsnorm_twins(const void* y, const int32_t* pos_of, const int32_t* idx, const void* w, int k,
+                                 const int32_t* twin, const void* x, const void* weight, float eps, int N, int H,
+                                 void* x_out, void* h_out, void* stream) {
   ROW_LIMITS("combine_add_rmsnorm");
   SY_REQUIRE(k >= 1 && k <= ROW_MAX_K, "combine_add_rmsnorm: 1 <= k <= %d (got %d)", ROW_MAX_K, k);
   if (N == 0) return SY_OK;
   SY_REQUIRE(y && pos_of && idx && x && weight && h_out, "combine_add_rmsnorm: null pointer");
   row_kernel<true, false><<<N, ROW_THREADS, 0, (hipStream_t)stream>>>(
       (const half_t*)x, (const half_t*)w, (const half_t*)y, pos_of, idx, k, (const half_t*)weight, eps, nullptr, 0, H,
-      (half_t*)x_out, (half_t*)h_out, nullptr, nullptr, 0);
+      (half_t*)x_out, (half_t*)h_out, nullptr, nullptr, 0, front_core::Outputs{}, twin);
   return sy_check_launch("combine_add_rmsnorm");
+}
+
+extern "C" SY_API int sy_combine_add_rmsnorm(const void* y, const int32_t* pos_of, const int32_t* idx, const void* w, int k,
+                                             const void* x, const void* weight, float eps, int N, int H, void* x_out,
+                                             void* h_out, void* stream) {
+  return sy_combine_add_rmsnorm_twins(y, pos_of, idx, w, k, nullptr, x, weight, eps, N, H, x_out, h_out, stream);
+}
+
+// One workgroup per sequence of a batch of prompts. A row in front of its sequence's first real token
+// holds the same numbers in every layer as any other such row with the same token: no query but its
+// own sees it, and it sees itself alone, so nothing but its token's embedding ever reaches it. All
+// of them are made twins of the first such row of the batch whose token they share; every
+// other row is its own. What it saves is the experts' work for the padding, which is all on the same
+// eight of them: 8 prompts of 256 to 512 tokens, gate/up 264 -> 217 us a layer, down 154 -> 126.
+__global__ void __launch_bounds__(ROW_THREADS)
+padding_twins_kernel(const int64_t* __restrict__ tokens, const uint8_t* __restrict__ real, int B, int T, int* __restrict__ twin) {
+  __shared__ int s_row, s_first;
+  const int b = blockIdx.x;
+  if (threadIdx.x == 0) {
+    s_row = B;     // the first sequence that starts with padding
+    s_first = T;   // this sequence's first real token
+  }
+  __syncthreads();
+  for (int r = threadIdx.x; r < B; r += ROW_THREADS)
+    if (!real[(size_t)r * T]) {
+      atomicMin(&s_row, r);
+      break;
+    }
+  for (int t = threadIdx.x; t < T; t += ROW_THREADS)
+    if (real[(size_t)b * T + t]) {
+      atomicMin(&s_first, t);
+      break;
+    }
+  __syncthreads();
+  const int first = s_first, row = s_row < B ? s_row * T : 0;
+  for (int t = threadIdx.x; t < T; t += ROW_THREADS) {
+    const int at = b * T + t;
+    twin[at] = t < first && tokens[at] == tokens[row] ? row : at;
+  }
+}
+
+extern "C" SY_API int sy_padding_twins(const int64_t* tokens, const uint8_t* real, int B, int T, int32_t* twin, void* stream) {
+  SY_REQUIRE(B >= 0 && T >= 1 && (long)B * T < (1l << 31), "padding_twins: B = %d, T = %d", B, T);
+  if (B == 0) return SY_OK;
+  SY_REQUIRE(tokens && real && twin, "padding_twins: null pointer");
+  padding_twins_kernel<<<B, ROW_THREADS, 0, (hipStream_t)stream>>>(tokens, real, B, T, twin);
+  return sy_check_launch("padding_twins");
 }
 
 extern "C" SY_API int sy_qk_norm_rope_cache(const void* qkv, const void* q_norm, const void* k_norm, float eps, float clip,

@@ -79,7 +79,10 @@ front_kernel(const half_t* __restrict__ logits, int N, int E, int k, int norm, i
 // route a token each from LDS with the code of route.hip. Everything here is latency, so the
 // workgroup is as wide as the shape allows: 21 us with 4 wavefronts at 4096 tokens. With `hist` the
 // workgroup is one piece of the sort (sort.hip): it owns piece / k tokens, 16 at a time, and
-// leaves the histogram of its choices where the sort's second launch expects it.
+// leaves the histogram of its choices where the sort's second launch expects it. `twin` names for
+// every token one that has the same row (itself, as a rule; for the padding of a batch of prompts
+// one row of that padding): a token that is not its own twin gets -1 for its choices, which the sort
+// passes over, so the experts see the row once and the combine reads the twin's results.
 //
 // Fuses F.linear(h, router) + route() of the reference (switchyard/kernels.py:30-32,
 // switchyard/csrc/moe_kernels.cu:23-89) and count_kernel (:91-104).
@@ -91,7 +94,7 @@ template <int PER_LANE, int RR_WAVES>
 __global__ void __launch_bounds__(RR_WAVES * WAVE)
 router_route_kernel(const half_t* __restrict__ h, const half_t* __restrict__ router, int N, int H, int E, int k, int norm,
                     int nbits, int groups, half_t* __restrict__ logits, int* __restrict__ idx, half_t* __restrict__ w,
-                    int* __restrict__ hist_out) {
+                    int* __restrict__ hist_out, const int* __restrict__ twin) {
   constexpr int EB = 4 * PER_LANE;             // blocks of 16 experts
   constexpr int RR_THREADS = RR_WAVES * WAVE;
   constexpr int EP = 16 * EB;                  // experts, padded
@@ -168,6 +171,7 @@ router_route_kernel(const half_t* __restrict__ h, const half_t* __restrict__ rou
       if (t < N) {
         float my_w;
         route_core::route_token<half_t, PER_LANE>(lg + tok * EP, E, k, norm, my_e, my_w);
+        if (twin && twin[t] != t) my_e = -1;   // another token's rows are this one's too: the sort passes it over
         if (lane < k) {
           idx[(size_t)t * k + lane] = my_e;
           w[(size_t)t * k + lane] = (half_t)my_w;
@@ -236,7 +240,7 @@ __device__ __forceinline__ void buffer_to_lds(int4v_t rsrc, unsigned voffset, un
 __global__ void __launch_bounds__(RS_THREADS)
 router_route_staged_kernel(const half_t* __restrict__ h, const half_t* __restrict__ router, int N, int H, int E, int k,
                            int norm, int nbits, int groups, half_t* __restrict__ logits, int* __restrict__ idx,
-                           half_t* __restrict__ w, int* __restrict__ hist_out) {
+                           half_t* __restrict__ w, int* __restrict__ hist_out, const int* __restrict__ twin) {
   constexpr int EP = 64;
   constexpr unsigned OUT_OF_RANGE = 0x80000000u;
   extern __shared__ __attribute__((aligned(1024))) char lds_raw[];
@@ -321,6 +325,7 @@ router_route_staged_kernel(const half_t* __restrict__ h, const half_t* __restric
       if (t < N) {
         float my_w;
         route_core::route_token<half_t, 1>(lg + tok * EP, E, k, norm, my_e, my_w);
+        if (twin && twin[t] != t) my_e = -1;   // another token's rows are this one's too: the sort passes it over
         if (lane < k) {
           idx[(size_t)t * k + lane] = my_e;
           w[(size_t)t * k + lane] = (half_t)my_w;
@@ -347,7 +352,7 @@ bool router_route_shape_ok(int N, int H, int E, int k) {
 }
 
 int launch_router_route(const void* h, const void* router, int N, int H, int E, int k, int norm, void* logits,
-                        int32_t* idx, void* w, void* hist, hipStream_t st) {
+                        int32_t* idx, void* w, void* hist, const int32_t* twin, hipStream_t st) {
   int nbits = 0;
   while ((1 << nbits) < E) ++nbits;
   const long M = (long)N * k;
@@ -362,7 +367,7 @@ int launch_router_route(const void* h, const void* router, int N, int H, int E, 
     if (hipFuncSetAttribute((const void*)router_route_staged_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
       return sy_fail(SY_ERR_LAUNCH, "router_route: cannot reserve %zu bytes of LDS", lds);
     router_route_staged_kernel<<<grid, RS_THREADS, lds, st>>>((const half_t*)h, (const half_t*)router, N, H, E, k, norm, nbits,
-                                                             groups, (half_t*)logits, idx, (half_t*)w, (int*)hist);
+                                                             groups, (half_t*)logits, idx, (half_t*)w, (int*)hist, twin);
     return sy_check_launch("router_route");
   }
   const int EP = E <= 64 ? 64 : 128;
@@ -370,12 +375,13 @@ int launch_router_route(const void* h, const void* router, int N, int H, int E, 
   const int waves = wide ? 16 : 4;
   const size_t lds = sizeof(float) * waves * RR_TOKENS * EP + sizeof(half_t) * RR_TOKENS * EP +
                      sizeof(int) * ((size_t)groups * RR_TOKENS * k + E);
-  void (*kern)(const half_t*, const half_t*, int, int, int, int, int, int, int, half_t*, int*, half_t*, int*) =
+  void (*kern)(const half_t*, const half_t*, int, int, int, int, int, int, int, half_t*, int*, half_t*, int*,
+               const int*) =
       wide ? router_route_kernel<1, 16> : E <= 64 ? router_route_kernel<1, 4> : router_route_kernel<2, 4>;
   if (lds > 48 * 1024 && hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
     return sy_fail(SY_ERR_LAUNCH, "router_route: cannot reserve %zu bytes of LDS", lds);
   kern<<<grid, waves * WAVE, lds, st>>>((const half_t*)h, (const half_t*)router, N, H, E, k, norm, nbits, groups,
-                                        (half_t*)logits, idx, (half_t*)w, (int*)hist);
+                                        (half_t*)logits, idx, (half_t*)w, (int*)hist, twin);
   return sy_check_launch("router_route");
 }
 
@@ -415,12 +421,12 @@ bool sy_router_route_counts(int N, int k) {
 }
 
 int sy_router_route_counting(const void* h, const void* router, int N, int H, int E, int k, int norm, void* logits,
-                             int32_t* idx, void* w, void* hist, void* stream) {
+                             int32_t* idx, void* w, void* hist, const int32_t* twin, void* stream) {
   SY_REQUIRE(router_route_shape_ok(N, H, E, k),
              "router_route: H a multiple of 512, at most 128 experts and top-8 (got N = %d, H = %d, E = %d, k = %d)", N, H, E, k);
   SY_REQUIRE(h && router && logits && idx && w, "router_route: null pointer");
   SY_REQUIRE(!hist || sy_router_route_counts(N, k), "router_route: no histograms for N = %d, k = %d", N, k);
-  return launch_router_route(h, router, N, H, E, k, norm, logits, idx, w, hist, (hipStream_t)stream);
+  return launch_router_route(h, router, N, H, E, k, norm, logits, idx, w, hist, twin, (hipStream_t)stream);
 }
 
 extern "C" SY_API int sy_router_route(const void* h, const void* router, int N, int H, int E, int k, int norm, void* logits,
@@ -428,5 +434,5 @@ extern "C" SY_API int sy_router_route(const void* h, const void* router, int N, 
   if (N == 0) return SY_OK;
   // a decode step: one workgroup per row (the kernels above take 16 rows to a workgroup)
   if (N <= 64) return sy_router_route_rows(h, router, N, H, E, k, norm, logits, idx, w, stream);
-  return sy_router_route_counting(h, router, N, H, E, k, norm, logits, idx, w, nullptr, stream);
+  return sy_router_route_counting(h, router, N, H, E, k, norm, logits, idx, w, nullptr, nullptr, stream);
 }

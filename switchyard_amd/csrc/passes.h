@@ -20,4 +20,18 @@ extern "C" {
 SY_API int sy_prefill_attention(const void* q, const void* kcache, const void* vcache, const uint8_t* real, int first,
                                 int B, int T, int heads, int kv_heads, int D, int capacity, void* out, void* stream);
 
+/* For the rows of a batch of B prompts of T positions that starts a cache (tokens int64 [B*T], real uint8
+ * [B*T]): twin int32 [B*T] names for each row one whose values are the same in every layer of a decoder with
+ * causal attention over real positions. Rows of left padding (in front of their sequence's first real
+ * token) that hold the token of the batch's first such row are twins of that row, which is its own
+ * twin like every other row. */
+SY_API int sy_padding_twins(const int64_t* tokens, const uint8_t* real, int B, int T, int32_t* twin, void* stream);
+
+/* sy_moe_layer's result for h, added to the residual x, and the RMS norm of the sum: x_out [N, H] =
+ * x + moe_layer(h) (may be x), h_out [N, H]. Expert outputs are computed once per twin: twin int32 [N] or
+ * null; twin[t] is a row with the same values as t and is its own twin. Limits: H a multiple of 512,
+ * at most 128 experts and top-8; the projections run on the MFMA tiles whatever L->mfma_tiles says. */
+SY_API int sy_moe_add_rmsnorm(const SyMoeLayer* L, const void* h, const int32_t* twin, const void* x, const void* weight,
+                              float eps, void* x_out, void* h_out, void* stream);
+
 }  // extern "C"

@@ -266,7 +266,15 @@ class Decoder:
         wqkv = self._stacked_qkv()
         slot = torch.tensor([span.first], dtype=torch.long, device=tokens.device)
         flat_positions = span.positions.reshape(-1).contiguous()
-        x, xn = E.embed_rmsnorm(tokens.reshape(-1).contiguous(), W["embed"], W["layers"][0]["attn_norm"], s.rms_eps)
+        tokens = tokens.contiguous()
+        x, xn = E.embed_rmsnorm(tokens.reshape(-1), W["embed"], W["layers"][0]["attn_norm"], s.rms_eps)
+        # The MoE layer, the residual add and the next norm are one call where the router's kernel takes
+        # the shape; the padding of a batch that starts its cache then goes through the experts once
+        # instead of once per row
+        in_one = self._own_moe and B * T > kernels.OWN_ROUTER_MAX_TOKENS and E.router_route_ok(B * T, s.hidden, s.experts, s.top_k)
+        if in_one:
+            scratch = E.moe_layer_scratch(B * T, s.experts, s.top_k, s.hidden, W["layers"][0]["down"].shape[2], x.device)
+            twin = E.padding_twins(tokens, span.real.contiguous()) if B > 1 and valid is not None and span.first == 0 else None
         for i in range(s.layers):
             L = W["layers"][i]
             after = W["layers"][i + 1]["attn_norm"] if i + 1 < s.layers else W["final_norm"]
@@ -275,7 +283,10 @@ class Decoder:
             a = E.prefill_attention(q, cache.k[i], cache.v[i], cache.real, span.first, s.heads)
             o = kernels.dense(a, L["wo"])
             x, h = E.add_rmsnorm(x, o, L["mlp_norm"], s.rms_eps, x_out=x)
-            if self._own_moe and s.top_k <= 64:
+            if in_one:
+                x, xn = E.moe_add_rmsnorm(h, L["router"], L["gate_up"], L["down"], s.top_k, s.norm_topk_prob, x, after,
+                                          s.rms_eps, scratch, twin, x_out=x)
+            elif self._own_moe and s.top_k <= 64:
                 y, pos_of, idx = kernels.experts_rows(h, None, L["gate_up"], L["down"], s.top_k, s.norm_topk_prob,
                                                       router=L["router"])
                 x, xn = E.combine_add_rmsnorm(y, pos_of, idx, x, after, s.rms_eps, x_out=x)

@@ -309,6 +309,57 @@ def test_decode_attention_without_a_real_key_gives_zeros():
     assert torch.allclose(out[1].view(heads, hd).float(), vc[1, :, 3].float(), atol=1e-3)
 
 
+def twins_reference(tokens, real):
+    """What sy_padding_twins says, from its definition, one row at a time."""
+    B, T = tokens.shape
+    lead = [(b, t) for b in range(B) for t in range(T) if not real[b, :t + 1].any()]
+    twin = torch.arange(B * T, dtype=torch.int32)
+    for b, t in lead:
+        if tokens[b, t] == tokens[lead[0]]:
+            twin[b * T + t] = lead[0][0] * T + lead[0][1]
+    return twin
+
+
+@pytest.mark.parametrize("B,T", [(1, 1), (2, 70), (5, 300), (300, 3), (3, 257)])
+@pytest.mark.parametrize("other_tokens", [False, True])
+def test_padding_twins(B, T, other_tokens):
+    g = torch.Generator().manual_seed(B * T)
+    first = torch.randint(0, T + 1, (B,), generator=g)
+    if B > 2:
+        first[0], first[1], first[2] = 0, T, 0      # no padding; nothing but padding
+    real = (torch.arange(T)[None] >= first[:, None]) & (torch.rand(B, T, generator=g) > 0.2)   # holes behind it
+    tokens = torch.randint(0, 9, (B, T), generator=g)
+    if not other_tokens:
+        tokens *= real
+    got = kernels.ext().padding_twins(tokens.cuda(), real.cuda()).cpu()
+    assert torch.equal(got, twins_reference(tokens, real))
+
+
+@pytest.mark.parametrize("N,pad,E,H,I,k", [
+    (65, 30, 64, 512, 256, 8), (256, 255, 64, 2048, 256, 8),       # one workgroup sorts; all but one row the same
+    (257, 100, 64, 512, 256, 8), (1000, 1, 16, 1024, 128, 4),      # the router's launch counts for the sort
+    (700, 300, 128, 512, 128, 8), (333, 0, 64, 512, 256, 6),       # another router kernel; no padding; a k the sort counts for itself
+    (4096, 900, 64, 2048, 1024, 8)])                               # the 256-row tile, whose combine scales
+def test_moe_layer_with_the_add_and_norm(N, pad, E, H, I, k):
+    """One call against the calls it replaces, bit for bit, without twins and with them."""
+    ext = kernels.ext()
+    h = rnd(N, H, seed=41)
+    rows = torch.randperm(N, generator=torch.Generator().manual_seed(42))[:pad].sort().values.cuda()
+    twin = torch.arange(N, dtype=torch.int32, device="cuda")
+    if pad:
+        h[rows] = h[rows[0]].clone()
+        twin[rows] = rows[0].int().clone()
+    router, gate_up, down = rnd(E, H, seed=43, std=0.05), rnd(E, 2 * I, H, seed=44, std=0.03), rnd(E, H, I, seed=45, std=0.03)
+    x, weight = rnd(N, H, seed=46), 1 + rnd(H, seed=47, std=0.1)
+    y, pos_of, idx = kernels.experts_rows(h, None, gate_up, down, k, True, router=router)
+    want = ext.combine_add_rmsnorm(y, pos_of, idx, x, weight, 1e-5)
+    for t in (None, twin):
+        scratch = ext.moe_layer_scratch(N, E, k, H, I, "cuda")
+        scratch.fill_(0xff)      # whatever an earlier layer left there
+        got = ext.moe_add_rmsnorm(h, router, gate_up, down, k, True, x, weight, 1e-5, scratch, t)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
 @pytest.mark.parametrize("rows,Nout,K", [(1, 6144, 2048), (8, 6144, 2048), (8, 2048, 2048), (16, 2048, 2048), (8, 50304, 2048),
                                         (8, 1000, 512), (3, 1001, 512), (17, 2048, 2048), (64, 6144, 2048),
                                         (64, 50304, 2048), (40, 1000, 512)])
