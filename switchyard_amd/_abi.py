@@ -83,6 +83,10 @@ SIGNATURES = {
     "sy_padding_twins": (_c_int, [_c_void_p, _c_void_p, _c_int, _c_int, _c_void_p, _c_void_p]),
     "sy_moe_add_rmsnorm": (_c_int, [ctypes.POINTER(SyMoeLayer), _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_float,
                                     _c_void_p, _c_void_p, _c_void_p]),
+    "sy_decode_attention_shares": (_c_int, [_c_int, _c_int]),
+    "sy_decode_attention_qkv_split": (_c_int, [_c_void_p, _c_void_p, _c_void_p, _c_float, _c_float, _c_void_p, _c_void_p,
+                                               _c_int, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int,
+                                               _c_int] + [_c_void_p] * 6),
     "sy_prefill_attention": (_c_int, [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int,
                                       _c_int, _c_int, _c_void_p, _c_void_p]),
     "sy_decode_attention": (_c_int, [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int,
@@ -777,10 +781,12 @@ class Ext:
         return out
 
     def decode_attention_qkv(self, qkv, q_norm, k_norm, eps, clip, cos, sin, positions, slot, real, heads, kv_heads,
-                             head_dim, kcache, vcache):
+                             head_dim, kcache, vcache, split=None):
         """qk_norm_rope_cache and decode_attention in one launch: qkv [B, (heads + 2 kv_heads) D]
         -> attention output [B, heads D]; the new key and value are written at `slot`, and
-        real[:, slot] is set (the new token is a real one)."""
+        real[:, slot] is set (the new token is a real one). `split` is (parts, one launch's row of
+        tickets) of attention_split for this batch: a few sequences' keys are then read by more
+        workgroups."""
         for t, name in ((qkv, "qkv"), (q_norm, "q_norm"), (k_norm, "k_norm"), (cos, "cos"), (sin, "sin"),
                         (kcache, "kcache"), (vcache, "vcache")):
             _check(t, name, torch.float16)
@@ -799,8 +805,26 @@ class Ext:
         if positions.numel() != B or slot.numel() != 1 or tuple(real.shape) != (B, capacity):
             raise RuntimeError("decode_attention_qkv: positions [B], slot [1], real [B, capacity]")
         out = torch.empty((B, heads * D), dtype=torch.float16, device=qkv.device)
-        self._call(self.lib.sy_decode_attention_qkv, qkv.data_ptr(), q_norm.data_ptr(), k_norm.data_ptr(), float(eps),
+        parts = tickets = None
+        if split is not None:
+            parts, tickets = split
+            _check(parts, "parts", torch.float32)
+            _check(tickets, "tickets", torch.int32)
+            if parts.numel() < B * heads * 16 * (D + 2) or \
+                    tickets.numel() < B * heads:
+                raise RuntimeError("decode_attention_qkv: parts / tickets are too small for this batch")
+            parts, tickets = parts.data_ptr(), tickets.data_ptr()
+        self._call(self.lib.sy_decode_attention_qkv_split, qkv.data_ptr(), q_norm.data_ptr(), k_norm.data_ptr(), float(eps),
                    float(clip or 0.0), cos.data_ptr(), sin.data_ptr(), cos.shape[0], positions.data_ptr(),
                    slot.data_ptr(), real.data_ptr(), B, int(heads), int(kv_heads), D, capacity, kcache.data_ptr(),
-                   vcache.data_ptr(), out.data_ptr(), _stream())
+                   vcache.data_ptr(), out.data_ptr(), parts, tickets, _stream())
         return out
+
+    def attention_split(self, launches, B, heads, head_dim, device):
+        """What `launches` decode_attention_qkv launches of one stream need to deal a pair's keys to
+        several workgroups: (parts, which they share one after the other; tickets, zero, a row for
+        each), or None where one workgroup per pair fills the chip."""
+        if not self.lib.sy_decode_attention_shares(B, int(heads)):
+            return None
+        return (torch.empty(B * heads * 16 * (int(head_dim) + 2), dtype=torch.float32, device=device),
+                torch.zeros((launches, B * heads), dtype=torch.int32, device=device))

@@ -35,6 +35,7 @@
 #include "common.h"
 #include "front_core.h"
 #include "../../include/switchyard_decode.h"
+#include "passes.h"
 
 namespace {
 
@@ -342,6 +343,7 @@ __device__ __forceinline__ float key_sum(float v) {
 }
 
 constexpr float MASKED = -1.0e30f;   // running maximum before any key was seen
+constexpr int ATT_WAVES = 16;   // wavefronts of a (sequence, head) pair where there are few pairs
 
 // One workgroup per (sequence, query head), NW wavefronts. A load instruction covers KPL =
 // 64 / LPK consecutive keys (LPK = D / 8 lanes per key, 16 bytes per lane: whole 256-byte rows
@@ -406,34 +408,95 @@ struct KeyBatch {
 // The first batch of keys and values is requested before any of that. (Requesting each further
 // batch while the previous one is multiplied costs registers, hence resident wavefronts, and
 // with them bandwidth: 67.5 us against 55.3 us at 64 sequences x 16 heads x 536 keys.)
-// NW wavefronts per workgroup, each with a batch of UNROLL key groups in flight: 16 wavefronts
-// when there are few (sequence, head) pairs, so that the cache is still read by many, 4 when
-// the pairs fill the chip.
-template <int LPK, bool FUSED, int NW, int UNROLL>
+// LW wavefronts per (sequence, head) pair, each with a batch of UNROLL key groups in flight: 16 when
+// there are few pairs, so that the cache is still read by many, 4 when the pairs fill the chip.
+// Batches in front of the sequence's first real key (left padding) are not read: every wavefront looks
+// for that key in the mask itself. At 64 sequences of 288 to 576 keys, 16 heads: 52.6 us a launch with them,
+// 45.6 without.
+// NW < LW: the pair's wavefronts are dealt to LW / NW workgroups, because what one compute unit can
+// have in flight (about 10 KB, a microsecond away) takes a while over a pair's keys and values: 17.2
+// -> 14.6 us for one sequence of 700 keys, 15.5 -> 14.7 for 8 of 256 to 512 (16 workgroups of one
+// wavefront, each with the whole of the norms to do: 16.0 for one sequence).
+// Every workgroup leaves its wavefronts' results in `parts` and draws a number from the pair's
+// ticket; the one that draws the last merges them, as a workgroup of LW wavefronts would have done (the
+// same bits), and sets the ticket back to zero. Nobody waits for anybody. The results travel by
+// agent-scope atomic stores and loads, which go past the XCDs' own L2s, and the store counter is
+// waited for before the draw: a release fence would write back the whole L2 of the XCD each time
+// (22 us a launch at 1024 workgroups).
+template <int LPK, bool FUSED, int NW, int UNROLL, int LW = NW>
 __global__ void __launch_bounds__(NW * WAVE)
 decode_attention_kernel(const half_t* __restrict__ q, const half_t* kcache, const half_t* vcache,
                                         const uint8_t* __restrict__ real, const int64_t* __restrict__ slot_ptr,
                                         int heads, int kv_heads, int capacity, float scale_log2e,
-                                        half_t* __restrict__ out, NewToken nt) {
+                                        half_t* __restrict__ out, NewToken nt, float* __restrict__ parts,
+                                        unsigned* __restrict__ tickets) {
   constexpr int D = LPK * 8, KPL = WAVE / LPK;
+  constexpr int SPLITS = LW / NW;   // workgroups per pair
+  constexpr bool SPLIT = SPLITS > 1;
   extern __shared__ float merge[];  // [NW][D + 2]: accumulators, maximum, sum
   __shared__ float part[32];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int sub = lane / LPK, c = lane % LPK;
-  const int b = blockIdx.x / heads, qh = blockIdx.x % heads;
+  const int pair = blockIdx.x / SPLITS, vwave = blockIdx.x % SPLITS * NW + wave;   // the wavefront's number in its pair
+  const int b = pair / heads, qh = pair % heads;
   const int group = heads / kv_heads, kvh = qh / group;
+  const half8_t zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+  const int qd = heads * D, kvd = kv_heads * D;
+  const bool owner = vwave < NW;   // the workgroup of the pair's first wavefronts takes the new key
+  const half_t* row = nt.qkv + (size_t)b * (qd + 2 * kvd);
+  HeadChunk<LPK> hq, hk;
+  half8_t knew = zero8, vnew = zero8, cc = zero8, ss = zero8;
+  half8_t eq[SPLITS], ek[SPLITS];   // 16-byte chunks of the q row and of the k row, for their norms
+  long pos = FUSED ? (long)nt.positions[b] : 0;
+  auto new_row = [&] {
+#pragma unroll
+    for (int u = 0; u < SPLITS; ++u) {
+      const int i = (u * NW + wave) * WAVE + lane;
+      eq[u] = ek[u] = zero8;
+      if (i < (qd >> 3)) eq[u] = *reinterpret_cast<const half8_t*>(row + i * 8);
+      if (owner && i < (kvd >> 3)) ek[u] = *reinterpret_cast<const half8_t*>(row + qd + i * 8);
+    }
+    hq.load(row + qh * D, nt.q_norm + qh * D, c);
+    hk.load(row + qd + kvh * D, nt.k_norm + kvh * D, c);
+    vnew = *reinterpret_cast<const half8_t*>(row + qd + kvd + kvh * D + c * 8);
+    pos = pos < 0 ? 0 : pos >= nt.max_positions ? nt.max_positions - 1 : pos;
+    cc = *reinterpret_cast<const half8_t*>(nt.cos_t + (size_t)pos * D + c * 8);
+    ss = *reinterpret_cast<const half8_t*>(nt.sin_t + (size_t)pos * D + c * 8);
+  };
+  // Loads return in order, so what stands behind the keys and values is waited for with them: the new
+  // token's row, which does not depend on the slot, goes first (64 sequences 46.8 -> 45.6 us), except
+  // where 16 wavefronts ask at once and the keys are late enough as it is (17.2 against 18.0 at one).
+  constexpr bool ROW_FIRST = NW < ATT_WAVES;
+  if (FUSED && ROW_FIRST) new_row();
   const long slot = (long)*slot_ptr;
   long n = FUSED ? slot : slot + 1;   // cached keys the loop visits
   n = n < 0 ? 0 : n > capacity ? capacity : n;
   const size_t base = ((size_t)b * kv_heads + kvh) * (size_t)capacity * D + c * 8;
   const uint8_t* rl = real + (size_t)b * capacity;
-  const half8_t zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
-  const int groups = ((int)n + KPL - 1) / KPL, stride = NW * UNROLL;
-
+  const int groups = ((int)n + KPL - 1) / KPL;
+  constexpr int STRIDE = LW * UNROLL;   // key groups of one batch of all the pair's wavefronts
+  // the first batch that holds a real key, found 512 positions at a time (few pairs wait for the
+  // look at the mask longer than for the batches it would spare)
+  int from = LW > 4 ? 0 : groups;
+  for (int p0 = LW > 4 ? (int)n : 0; p0 < (int)n; p0 += 8 * WAVE) {
+    uint8_t at[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) at[u] = rl[min(p0 + u * WAVE + lane, (int)n - 1)];
+    int first = 8 * WAVE;
+#pragma unroll
+    for (int u = 7; u >= 0; --u) {
+      const uint64_t seen = __ballot(at[u] != 0);
+      if (seen) first = u * WAVE + __builtin_ctzll(seen);
+    }
+    if (first < 8 * WAVE) {
+      from = (p0 + first) / (STRIDE * KPL) * STRIDE;
+      break;
+    }
+  }
   auto fetch = [&](KeyBatch<UNROLL>& kb, int g0) {
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {
-      const int key = (g0 + u * NW) * KPL + sub;
+      const int key = (g0 + u * LW) * KPL + sub;
       kb.ok[u] = key < n;
       kb.kk[u] = zero8;
       kb.vv[u] = zero8;
@@ -445,42 +508,39 @@ decode_attention_kernel(const half_t* __restrict__ q, const half_t* kcache, cons
     }
   };
   KeyBatch<UNROLL> ka;
-  fetch(ka, wave);   // requested before the prologue, so that the two waits overlap
+  fetch(ka, from + vwave);   // requested before the rest of the prologue, so that the two waits overlap
 
   float qf[8];
-  half8_t knew = zero8, vnew = zero8;
+  if (FUSED && !ROW_FIRST) new_row();
   if (FUSED) {
-    const int qd = heads * D, kvd = kv_heads * D;
-    const half_t* row = nt.qkv + (size_t)b * (qd + 2 * kvd);
-    long pos = (long)nt.positions[b];
-    pos = pos < 0 ? 0 : pos >= nt.max_positions ? nt.max_positions - 1 : pos;
-    HeadChunk<LPK> hq, hk;
-    hq.load(row + qh * D, nt.q_norm + qh * D, c);
-    hk.load(row + qd + kvh * D, nt.k_norm + kvh * D, c);
-    vnew = *reinterpret_cast<const half8_t*>(row + qd + kvd + kvh * D + c * 8);
-    const half8_t cc = *reinterpret_cast<const half8_t*>(nt.cos_t + (size_t)pos * D + c * 8);
-    const half8_t ss = *reinterpret_cast<const half8_t*>(nt.sin_t + (size_t)pos * D + c * 8);
+    // The sums of squares as LW wavefronts would take them, whose sums are then added in order: a
+    // workgroup of fewer takes the others' shares one after the other.
     float sq = 0.f, sk = 0.f;
-    for (int i = threadIdx.x; i < (qd >> 3); i += blockDim.x) {
-      const half8_t v = *reinterpret_cast<const half8_t*>(row + i * 8);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) sq += (float)v[j] * (float)v[j];
-    }
-    for (int i = threadIdx.x; i < (kvd >> 3); i += blockDim.x) {
-      const half8_t v = *reinterpret_cast<const half8_t*>(row + qd + i * 8);
+    for (int u = 0; u < SPLITS; ++u) {
+      const int v = u * NW + wave;
+      float q2 = 0.f, k2 = 0.f;
+      for (int i = v * WAVE + lane; i < (qd >> 3); i += LW * WAVE) {
+        const half8_t e = i < LW * WAVE ? eq[u] : *reinterpret_cast<const half8_t*>(row + i * 8);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) sk += (float)v[j] * (float)v[j];
+        for (int j = 0; j < 8; ++j) q2 += (float)e[j] * (float)e[j];
+      }
+      if (owner)
+        for (int i = v * WAVE + lane; i < (kvd >> 3); i += LW * WAVE) {
+          const half8_t e = i < LW * WAVE ? ek[u] : *reinterpret_cast<const half8_t*>(row + qd + i * 8);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) k2 += (float)e[j] * (float)e[j];
+        }
+      q2 = wave_sum(q2);
+      k2 = wave_sum(k2);
+      if (lane == 0) {
+        part[v] = q2;
+        part[16 + v] = k2;
+      }
     }
     // both sums through one barrier
-    sq = wave_sum(sq);
-    sk = wave_sum(sk);
-    if (lane == 0) {
-      part[wave] = sq;
-      part[16 + wave] = sk;
-    }
     __syncthreads();
-    sq = sk = 0.f;
-    for (int w = 0; w < NW; ++w) {
+    for (int w = 0; w < LW; ++w) {
       sq += part[w];
       sk += part[16 + w];
     }
@@ -491,7 +551,7 @@ decode_attention_kernel(const half_t* __restrict__ q, const half_t* kcache, cons
     knew = hk.finish(rk, nt.clip, cc, ss, c);
 #pragma unroll
     for (int j = 0; j < 8; ++j) vnew[j] = clamp_f16(vnew[j], nt.clip);
-    if (slot >= 0 && slot < capacity && qh % group == 0 && wave == 0 && sub == 0) {
+    if (slot >= 0 && slot < capacity && qh % group == 0 && vwave == 0 && sub == 0) {
       const size_t at = (((size_t)b * kv_heads + kvh) * capacity + slot) * D + c * 8;
       *reinterpret_cast<half8_t*>(nt.kcache_w + at) = knew;
       *reinterpret_cast<half8_t*>(nt.vcache_w + at) = vnew;
@@ -531,12 +591,23 @@ decode_attention_kernel(const half_t* __restrict__ q, const half_t* kcache, cons
       for (int j = 0; j < 8; ++j) acc[j] += p * (float)kb.vv[u][j];
     }
   };
-  for (int g0 = wave; g0 < groups; g0 += stride) {
-    if (g0 != wave) fetch(ka, g0);
-    consume(ka);
+  if (SPLIT) {   // few wavefronts on a compute unit, registers to spare: a batch ahead
+    KeyBatch<UNROLL> kb;
+    for (int g0 = from + vwave; g0 < groups; g0 += 2 * STRIDE) {
+      fetch(kb, g0 + STRIDE);
+      consume(ka);
+      if (g0 + STRIDE >= groups) break;
+      fetch(ka, g0 + 2 * STRIDE);
+      consume(kb);
+    }
+  } else {
+    for (int g0 = from + vwave; g0 < groups; g0 += STRIDE) {
+      if (g0 != from + vwave) fetch(ka, g0);
+      consume(ka);
+    }
   }
 
-  if (FUSED && wave == 0 && slot >= 0 && slot < capacity) {
+  if (FUSED && vwave == 0 && slot >= 0 && slot < capacity) {
     // the new token's own key and value, from registers: one more key for the first key group
     float d = 0.f;
 #pragma unroll
@@ -576,18 +647,50 @@ decode_attention_kernel(const half_t* __restrict__ q, const half_t* kcache, cons
     }
   }
   __syncthreads();
-  // ---- merge the wavefronts: thread d < D finishes output dimension d
-  if (threadIdx.x < D) {
-    float M = MASKED;
-    for (int w = 0; w < NW; ++w) M = fmaxf(M, merge[w * (D + 2) + D]);
-    float num = 0.f, den = 0.f;
-    for (int w = 0; w < NW; ++w) {
-      const float f = __builtin_amdgcn_exp2f(merge[w * (D + 2) + D] - M);
-      num += f * merge[w * (D + 2) + threadIdx.x];
-      den += f * merge[w * (D + 2) + D + 1];
+  // ---- merge the wavefronts: lane i of the first one finishes output dimensions i, i + 64
+  if (wave != 0) return;
+  constexpr int DIMS = D / WAVE;
+  float pm[LW], pl[LW], pa[LW][DIMS];   // every wavefront's maximum, sum and accumulators
+  if (SPLIT) {
+    float* all = parts + (size_t)pair * LW * (D + 2);
+    for (int i = lane; i < NW * (D + 2); i += WAVE)
+      __hip_atomic_store(all + vwave * (D + 2) + i, merge[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // they are where every XCD's atomic loads find them
+    unsigned drawn = 0;
+    if (lane == 0) drawn = __hip_atomic_fetch_add(tickets + pair, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (__builtin_amdgcn_readfirstlane(drawn) != (unsigned)(SPLITS - 1)) return;
+    asm volatile("" ::: "memory");
+    if (lane == 0) __hip_atomic_store(tickets + pair, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    auto get = [&](int i) { return __hip_atomic_load(all + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+#pragma unroll
+    for (int w = 0; w < LW; ++w) {
+      pm[w] = get(w * (D + 2) + D);
+      pl[w] = get(w * (D + 2) + D + 1);
+#pragma unroll
+      for (int i = 0; i < DIMS; ++i) pa[w][i] = get(w * (D + 2) + i * WAVE + lane);
     }
-    out[((size_t)b * heads + qh) * D + threadIdx.x] = (half_t)(den > 0.f ? num / den : 0.f);
+  } else {
+#pragma unroll
+    for (int w = 0; w < LW; ++w) {
+      pm[w] = merge[w * (D + 2) + D];
+      pl[w] = merge[w * (D + 2) + D + 1];
+#pragma unroll
+      for (int i = 0; i < DIMS; ++i) pa[w][i] = merge[w * (D + 2) + i * WAVE + lane];
+    }
   }
+  float M = MASKED, den = 0.f, num[DIMS] = {};
+#pragma unroll
+  for (int w = 0; w < LW; ++w) M = fmaxf(M, pm[w]);
+#pragma unroll
+  for (int w = 0; w < LW; ++w) {
+    const float f = __builtin_amdgcn_exp2f(pm[w] - M);
+    den += f * pl[w];
+#pragma unroll
+    for (int i = 0; i < DIMS; ++i) num[i] += f * pa[w][i];
+  }
+#pragma unroll
+  for (int i = 0; i < DIMS; ++i)
+    out[((size_t)b * heads + qh) * D + i * WAVE + lane] = (half_t)(den > 0.f ? num[i] / den : 0.f);
 }
 
 // One workgroup per sequence: the arg-max of its logits (the lowest index among equal maxima)
@@ -898,6 +1001,10 @@ extern "C" SY_API int sy_qk_norm_rope_cache(const void* qkv, const void* q_norm,
   return sy_check_launch("qk_norm_rope_cache");
 }
 
+// Whether the (sequence, head) pairs are too few to fill the chip with four wavefronts each: they then
+// get 16, in one workgroup or, with room for their results, in four.
+extern "C" SY_API int sy_decode_attention_shares(int B, int heads) { return (long)B * heads < 2l * sy_compute_units(); }
+
 extern "C" SY_API int sy_decode_attention(const void* q, const void* kcache, const void* vcache, const uint8_t* real,
                                           const int64_t* slot, int B, int heads, int kv_heads, int D, int capacity,
                                           void* out, void* stream) {
@@ -907,24 +1014,25 @@ extern "C" SY_API int sy_decode_attention(const void* q, const void* kcache, con
   SY_REQUIRE(capacity >= 1, "decode_attention: capacity = %d", capacity);
   if (B == 0) return SY_OK;
   SY_REQUIRE(q && kcache && vcache && real && slot && out, "decode_attention: null pointer");
-  // few (sequence, head) pairs: 16 wavefronts each, so that the cache is still read by many
   const long pairs = (long)B * heads;
-  const int waves = pairs >= 2l * sy_compute_units() ? 4 : 16;
+  const int waves = sy_decode_attention_shares(B, heads) ? ATT_WAVES : 4;
   const size_t lds = (size_t)waves * (D + 2) * sizeof(float);
   const float scale_log2e = 1.4426950408889634f / sqrtf((float)D);
   auto kern = D == 128 ? (waves == 4 ? decode_attention_kernel<16, false, 4, 4> : decode_attention_kernel<16, false, 16, 4>)
                        : (waves == 4 ? decode_attention_kernel<8, false, 4, 4> : decode_attention_kernel<8, false, 16, 4>);
   kern<<<(unsigned)pairs, waves * WAVE, lds, (hipStream_t)stream>>>((const half_t*)q, (const half_t*)kcache,
                                                                    (const half_t*)vcache, real, slot, heads, kv_heads,
-                                                                   capacity, scale_log2e, (half_t*)out, NewToken{});
+                                                                   capacity, scale_log2e, (half_t*)out, NewToken{}, nullptr,
+                                                                   nullptr);
   return sy_check_launch("decode_attention");
 }
 
-extern "C" SY_API int sy_decode_attention_qkv(const void* qkv, const void* q_norm, const void* k_norm, float eps, float clip,
-                                              const void* cos_table, const void* sin_table, int max_positions,
-                                              const int64_t* positions, const int64_t* slot, uint8_t* real, int B,
-                                              int heads, int kv_heads, int D, int capacity, void* kcache, void* vcache,
-                                              void* out, void* stream) {
+extern "C" SY_API int sy_decode_attention_qkv_split(const void* qkv, const void* q_norm, const void* k_norm, float eps,
+                                                    float clip, const void* cos_table, const void* sin_table,
+                                                    int max_positions, const int64_t* positions, const int64_t* slot,
+                                                    uint8_t* real, int B, int heads, int kv_heads, int D, int capacity,
+                                                    void* kcache, void* vcache, void* out, void* parts, void* tickets,
+                                                    void* stream) {
   SY_REQUIRE(B >= 0 && heads >= 1 && kv_heads >= 1 && heads % kv_heads == 0,
              "decode_attention_qkv: B = %d, heads = %d, kv_heads = %d", B, heads, kv_heads);
   SY_REQUIRE(D == 64 || D == 128, "decode_attention_qkv: head_dim must be 64 or 128 (got %d)", D);
@@ -934,17 +1042,31 @@ extern "C" SY_API int sy_decode_attention_qkv(const void* qkv, const void* q_nor
   SY_REQUIRE(qkv && q_norm && k_norm && cos_table && sin_table && positions && slot && real && kcache && vcache && out,
              "decode_attention_qkv: null pointer");
   const long pairs = (long)B * heads;
-  const int waves = pairs >= 2l * sy_compute_units() ? 4 : 16;
-  const size_t lds = (size_t)waves * (D + 2) * sizeof(float);
-  const float scale_log2e = 1.4426950408889634f / sqrtf((float)D);
   NewToken nt{(const half_t*)qkv, (const half_t*)q_norm, (const half_t*)k_norm, (const half_t*)cos_table,
               (const half_t*)sin_table, positions, (half_t*)kcache, (half_t*)vcache, real, eps, clip, max_positions};
-  auto kern = D == 128 ? (waves == 4 ? decode_attention_kernel<16, true, 4, 4> : decode_attention_kernel<16, true, 16, 4>)
-                       : (waves == 4 ? decode_attention_kernel<8, true, 4, 4> : decode_attention_kernel<8, true, 16, 4>);
-  kern<<<(unsigned)pairs, waves * WAVE, lds, (hipStream_t)stream>>>(nullptr, (const half_t*)kcache, (const half_t*)vcache,
-                                                                   real, slot, heads, kv_heads, capacity, scale_log2e,
-                                                                   (half_t*)out, nt);
+  const float scale_log2e = 1.4426950408889634f / sqrtf((float)D);
+  const bool few = sy_decode_attention_shares(B, heads), split = few && parts && tickets;
+  const int waves = few && !split ? ATT_WAVES : 4, splits = split ? ATT_WAVES / waves : 1;
+  const size_t lds = (size_t)waves * (D + 2) * sizeof(float);
+  auto kern = D == 128 ? (split   ? decode_attention_kernel<16, true, 4, 4, ATT_WAVES>
+                          : few ? decode_attention_kernel<16, true, ATT_WAVES, 4>
+                                : decode_attention_kernel<16, true, 4, 4>)
+                       : (split   ? decode_attention_kernel<8, true, 4, 4, ATT_WAVES>
+                          : few ? decode_attention_kernel<8, true, ATT_WAVES, 4>
+                                : decode_attention_kernel<8, true, 4, 4>);
+  kern<<<(unsigned)(pairs * splits), waves * WAVE, lds, (hipStream_t)stream>>>(
+      nullptr, (const half_t*)kcache, (const half_t*)vcache, real, slot, heads, kv_heads, capacity, scale_log2e, (half_t*)out,
+      nt, (float*)parts, (unsigned*)tickets);
   return sy_check_launch("decode_attention_qkv");
+}
+
+extern "C" SY_API int sy_decode_attention_qkv(const void* qkv, const void* q_norm, const void* k_norm, float eps, float clip,
+                                              const void* cos_table, const void* sin_table, int max_positions,
+                                              const int64_t* positions, const int64_t* slot, uint8_t* real, int B,
+                                              int heads, int kv_heads, int D, int capacity, void* kcache, void* vcache,
+                                              void* out, void* stream) {
+  return sy_decode_attention_qkv_split(qkv, q_norm, k_norm, eps, clip, cos_table, sin_table, max_positions, positions, slot,
+                                       real, B, heads, kv_heads, D, capacity, kcache, vcache, out, nullptr, nullptr, stream);
 }
 
 extern "C" SY_API int sy_greedy_advance(const void* logits, int B, int V, int64_t* tok, int64_t* out, int out_stride,

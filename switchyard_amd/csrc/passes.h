@@ -20,6 +20,17 @@ extern "C" {
 SY_API int sy_prefill_attention(const void* q, const void* kcache, const void* vcache, const uint8_t* real, int first,
                                 int B, int T, int heads, int kv_heads, int D, int capacity, void* out, void* stream);
 
+/* sy_decode_attention_qkv (include/switchyard_decode.h) with the keys of a (sequence, head) pair dealt to
+ * four workgroups where the pairs are few and both buffers are given: parts f32 [B*heads, 16, D + 2] is
+ * scratch of this call; tickets uint32 [B*heads] is zero before the launch and after it, and no two
+ * launches that can run at the same time may share it. `out` has the bits of
+ * sy_decode_attention_qkv's. */
+SY_API int sy_decode_attention_qkv_split(const void* qkv, const void* q_norm, const void* k_norm, float eps, float clip,
+                                         const void* cos_table, const void* sin_table, int max_positions,
+                                         const int64_t* positions, const int64_t* slot, uint8_t* real, int B, int heads,
+                                         int kv_heads, int D, int capacity, void* kcache, void* vcache, void* out,
+                                         void* parts, void* tickets, void* stream);
+
 /* For the rows of a batch of B prompts of T positions that starts a cache (tokens int64 [B*T], real uint8
  * [B*T]): twin int32 [B*T] names for each row one whose values are the same in every layer of a decoder with
  * causal attention over real positions. Rows of left padding (in front of their sequence's first real
@@ -33,5 +44,9 @@ SY_API int sy_padding_twins(const int64_t* tokens, const uint8_t* real, int B, i
  * at most 128 experts and top-8; the projections run on the MFMA tiles whatever L->mfma_tiles says. */
 SY_API int sy_moe_add_rmsnorm(const SyMoeLayer* L, const void* h, const int32_t* twin, const void* x, const void* weight,
                               float eps, void* x_out, void* h_out, void* stream);
+
+/* Whether decode attention's (sequence, head) pairs are few enough for sy_decode_attention_qkv_split to
+ * deal their keys to several workgroups. */
+SY_API int sy_decode_attention_shares(int B, int heads);
 
 }  // extern "C"

@@ -365,12 +365,13 @@ class Decoder:
         wqkv = self._stacked_qkv()
         positions = cache.next_position
         x, xn = E.embed_rmsnorm(tok.reshape(-1), W["embed"], W["layers"][0]["attn_norm"], s.rms_eps)
+        split = E.attention_split(s.layers, x.shape[0], s.heads, s.head_dim, x.device)
         for i in range(s.layers):
             L = W["layers"][i]
             after = W["layers"][i + 1]["attn_norm"] if i + 1 < s.layers else W["final_norm"]
             a = E.decode_attention_qkv(kernels.dense(xn, wqkv[i]), L["q_norm"], L["k_norm"], s.rms_eps, s.clip_qkv,
                                        self.cos, self.sin, positions, slot, cache.real, s.heads, s.kv_heads,
-                                       s.head_dim, cache.k[i], cache.v[i])
+                                       s.head_dim, cache.k[i], cache.v[i], split and (split[0], split[1][i]))
             o = kernels.dense(a, L["wo"])
             if self._own_moe and s.experts <= 1024 and s.top_k <= 64:
                 # the router's logits come out of the norm's launch, and combine goes into the next norm's

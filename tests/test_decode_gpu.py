@@ -299,6 +299,43 @@ def test_attention_with_the_norm_and_rotary_in_its_prologue(B, heads, kv_heads, 
     assert torch.allclose(got.float(), want.float(), rtol=2 * ULP, atol=1e-3)
 
 
+@pytest.mark.parametrize("B,heads,kv_heads,hd,cap,slot_at", [
+    (1, 16, 16, 128, 732, 700), (8, 16, 16, 128, 544, 512), (3, 8, 2, 64, 77, 50),   # 16, 4 and 4 workgroups per pair
+    (2, 4, 4, 128, 9, 0), (1, 16, 16, 64, 40, 5), (1, 4, 1, 128, 70, 63),            # fewer keys than wavefronts
+    (31, 16, 16, 128, 1100, 1030), (1, 2, 2, 128, 4100, 4099), (2, 8, 8, 64, 2000, 1999),   # many batches each
+    (5, 20, 4, 128, 300, 299),                                                       # rows of 2560: a fifth wavefront's sum
+    (2, 4, 4, 64, 10, 10)])                                                          # a slot past the cache
+def test_attention_over_several_workgroups(B, heads, kv_heads, hd, cap, slot_at):
+    """The keys of a pair dealt to several workgroups against one workgroup: the same cache and the
+    same output, bit for bit; the tickets are back at zero, so the buffers serve the next launch;
+    rows of padding up to the slot (no real key but the new one) among them."""
+    ext, max_pos = kernels.ext(), 700
+    g = torch.Generator().manual_seed(31)
+    qkv = rnd(B, (heads + 2 * kv_heads) * hd, seed=32, std=0.7)
+    qn, kn = 1 + rnd(heads * hd, seed=33, std=0.1), 1 + rnd(kv_heads * hd, seed=34, std=0.1)
+    cos, sin = rnd(max_pos, hd, seed=35, std=0.5), rnd(max_pos, hd, seed=36, std=0.5)
+    positions = torch.randint(0, max_pos, (B,), generator=g).cuda()
+    slot = torch.tensor([slot_at], device="cuda")
+    pad = torch.randint(0, slot_at + 1, (B,), generator=g)
+    pad[0], pad[B // 2] = 0, slot_at
+    real = ((torch.arange(cap)[None] >= pad[:, None]) & (torch.rand(B, cap, generator=g) > 0.2)).cuda()
+    kc, vc = rnd(B, kv_heads, cap, hd, seed=37), rnd(B, kv_heads, cap, hd, seed=38)
+    split = ext.attention_split(2, B, heads, hd, "cuda")
+    assert split is not None
+    results = []
+    for share in (None, (split[0], split[1][0]), (split[0], split[1][0]), (split[0], split[1][1])):
+        k, v, r = kc.clone(), vc.clone(), real.clone()
+        out = ext.decode_attention_qkv(qkv, qn, kn, 1e-5, None, cos, sin, positions, slot, r, heads, kv_heads, hd, k, v, share)
+        results.append((out, k, v, r))
+        assert not split[1].any()
+    want = results[0]
+    for got in results[1:]:
+        assert torch.equal(got[1].view(torch.int16), want[1].view(torch.int16)) and torch.equal(got[3], want[3])
+        assert torch.equal(got[2].view(torch.int16), want[2].view(torch.int16))
+        assert torch.equal(got[0], want[0])
+    assert ext.attention_split(2, 4096, heads, hd, "cuda") is None
+
+
 def test_decode_attention_without_a_real_key_gives_zeros():
     B, heads, hd, cap = 2, 4, 64, 16
     q, kc, vc = rnd(B, heads * hd), rnd(B, heads, cap, hd), rnd(B, heads, cap, hd)
