@@ -31,6 +31,22 @@ class SyMoeLayer(ctypes.Structure):
                 ("scratch_bytes", _c_size_t)]
 
 
+class SyDecodeLayer(ctypes.Structure):
+    """A layer of sy_decode_step (csrc/passes.h)."""
+    _fields_ = [(n, ctypes.c_void_p) for n in ("wqkv", "q_norm", "k_norm", "wo", "mlp_norm", "router", "gate_up", "down",
+                                               "next_norm", "kcache", "vcache")]
+
+
+class SyDecodeStep(ctypes.Structure):
+    """What sy_decode_step takes beside its layers (csrc/passes.h)."""
+    _fields_ = ([(n, ctypes.c_int) for n in ("B", "layers", "H", "heads", "kv_heads", "D", "capacity", "E", "I", "k", "norm",
+                                             "vocab", "embed_rows", "max_positions", "gemv_max_rows")]
+                + [("eps", ctypes.c_float), ("clip", ctypes.c_float)]
+                + [(n, ctypes.c_void_p) for n in ("embed", "first_norm", "lm_head", "cos", "sin", "tok", "positions", "slot",
+                                                  "real", "out", "scratch")]
+                + [("scratch_bytes", ctypes.c_size_t)])
+
+
 # name -> (restype, argtypes); mirrors include/switchyard_moe.h, include/switchyard_decode.h and csrc/passes.h
 SIGNATURES = {
     "sy_version": (_c_int, []),
@@ -84,6 +100,8 @@ SIGNATURES = {
     "sy_moe_add_rmsnorm": (_c_int, [ctypes.POINTER(SyMoeLayer), _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_float,
                                     _c_void_p, _c_void_p, _c_void_p]),
     "sy_decode_attention_shares": (_c_int, [_c_int, _c_int]),
+    "sy_decode_step_scratch_bytes": (_c_size_t, [ctypes.POINTER(SyDecodeStep)]),
+    "sy_decode_step": (_c_int, [ctypes.POINTER(SyDecodeStep), ctypes.POINTER(SyDecodeLayer), _c_void_p]),
     "sy_decode_attention_qkv_split": (_c_int, [_c_void_p, _c_void_p, _c_void_p, _c_float, _c_float, _c_void_p, _c_void_p,
                                                _c_int, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int,
                                                _c_int] + [_c_void_p] * 6),
@@ -818,6 +836,56 @@ class Ext:
                    float(clip or 0.0), cos.data_ptr(), sin.data_ptr(), cos.shape[0], positions.data_ptr(),
                    slot.data_ptr(), real.data_ptr(), B, int(heads), int(kv_heads), D, capacity, kcache.data_ptr(),
                    vcache.data_ptr(), out.data_ptr(), parts, tickets, _stream())
+        return out
+
+    STEP_MAX_ROWS = 16   # SY_STEP_MAX_ROWS: up to here every projection of a step is a weight stream
+
+    def decode_step(self, tok, weights, wqkv, cos, sin, positions, slot, real, kcache, vcache, heads, kv_heads, head_dim, k,
+                    norm, eps, clip, gemv_max_rows):
+        """One decode step of the whole model in one call: tok int64 [B] -> logits f16 [B, vocab]. weights:
+        the decoder's dictionary (embed, final_norm, lm_head, layers), wqkv: its stacked projections;
+        kcache, vcache [layers, B, kv_heads, capacity, D]. Every tensor is looked at in every call, and
+        its address is used for this call only."""
+        layers = weights["layers"]
+        (B,), (n, _, _, capacity, D) = tok.shape, kcache.shape
+        (vocab, H), (E, _), I = weights["embed"].shape, layers[0]["router"].shape, layers[0]["down"].shape[2]
+        qd, kvd = heads * D, kv_heads * D
+        f16, i64 = torch.float16, torch.int64
+        want = [(tok, i64, (B,)), (positions, i64, (B,)), (slot, i64, (1,)), (real, torch.bool, (B, capacity)),
+                (kcache, f16, (n, B, kv_heads, capacity, D)), (vcache, f16, (n, B, kv_heads, capacity, D)),
+                (cos, f16, (cos.shape[0], D)), (sin, f16, (cos.shape[0], D)), (weights["embed"], f16, (vocab, H)),
+                (weights["final_norm"], f16, (H,)), (weights["lm_head"], f16, (weights["lm_head"].shape[0], H))]
+        for L, stack in zip(layers, wqkv):
+            want += [(stack, f16, (qd + 2 * kvd, H)), (L["q_norm"], f16, (qd,)), (L["k_norm"], f16, (kvd,)),
+                     (L["wo"], f16, (H, qd)), (L["attn_norm"], f16, (H,)), (L["mlp_norm"], f16, (H,)),
+                     (L["router"], f16, (E, H)), (L["gate_up"], f16, (E, 2 * I, H)), (L["down"], f16, (E, H, I))]
+        device = tok.device
+        for t, dtype, shape in want:
+            if t.dtype != dtype or t.shape != shape or t.device != device or not t.is_contiguous():
+                raise RuntimeError(f"decode_step: a contiguous {dtype} GPU tensor {shape} was expected, got {t.dtype} "
+                                   f"{tuple(t.shape)} on {t.device}")
+        if not tok.is_cuda or D != head_dim or len(layers) != n or len(wqkv) != n:
+            raise RuntimeError("decode_step: tensors on the GPU, one cache per layer, caches of head_dim")
+        rows = (SyDecodeLayer * n)()
+        k0, v0 = kcache.data_ptr(), vcache.data_ptr()
+        per_layer = B * kv_heads * capacity * D * 2
+        for i, (L, stack) in enumerate(zip(layers, wqkv)):
+            after = layers[i + 1]["attn_norm"] if i + 1 < n else weights["final_norm"]
+            rows[i] = SyDecodeLayer(stack.data_ptr(), L["q_norm"].data_ptr(), L["k_norm"].data_ptr(), L["wo"].data_ptr(),
+                                    L["mlp_norm"].data_ptr(), L["router"].data_ptr(), L["gate_up"].data_ptr(),
+                                    L["down"].data_ptr(), after.data_ptr(), k0 + i * per_layer, v0 + i * per_layer)
+        lm_head = weights["lm_head"]
+        out = torch.empty((B, lm_head.shape[0]), dtype=f16, device=device)
+        step = SyDecodeStep(B, n, H, heads, kv_heads, D, capacity, E, I, int(k), int(bool(norm)), lm_head.shape[0], vocab,
+                            cos.shape[0], int(gemv_max_rows), float(eps), float(clip or 0.0), weights["embed"].data_ptr(),
+                            layers[0]["attn_norm"].data_ptr(), lm_head.data_ptr(), cos.data_ptr(), sin.data_ptr(),
+                            tok.data_ptr(), positions.data_ptr(), slot.data_ptr(), real.data_ptr(), out.data_ptr())
+        step.scratch_bytes = self.lib.sy_decode_step_scratch_bytes(step)
+        if not step.scratch_bytes:
+            raise RuntimeError(self.lib.sy_last_error().decode())
+        scratch = torch.empty(step.scratch_bytes, dtype=torch.uint8, device=device)
+        step.scratch = scratch.data_ptr()
+        self._call(self.lib.sy_decode_step, step, rows, _stream())
         return out
 
     def attention_split(self, launches, B, heads, head_dim, device):

@@ -88,6 +88,10 @@ row_kernel(const half_t* x, const half_t* __restrict__ delta, const half_t* __re
     long g = (long)gather[t];
     g = g < 0 ? 0 : g >= src_rows ? src_rows - 1 : g;
     xrow = x + (size_t)g * H;
+    if (t == 0 && front.ticket) {   // the first launch of a step: its counters, and its projections' row range
+      for (int i = tid; i < front.k; i += nthreads) front.ticket[i] = 0;
+      if (tid < 2) front.offsets[tid] = tid ? (int)gridDim.x : 0;
+    }
   }
   if (COMBINE) {
     // rank the k choices by (expert id, slot); rows[] lists their rows of y in that order
@@ -773,16 +777,26 @@ extern "C" SY_API int sy_add_rmsnorm(const void* x, const void* delta, const voi
   return sy_check_launch("add_rmsnorm");
 }
 
-extern "C" SY_API int sy_embed_rmsnorm(const int64_t* tokens, const void* embed, int vocab, const void* weight, float eps,
-                                       int N, int H, void* x_out, void* h_out, void* stream) {
+int sy_embed_rmsnorm_step(const int64_t* tokens, const void* embed, int vocab, const void* weight, float eps, int N, int H,
+                          void* x_out, void* h_out, unsigned* tickets, int ntickets, int32_t* one, void* stream) {
   ROW_LIMITS("embed_rmsnorm");
   SY_REQUIRE(vocab >= 1, "embed_rmsnorm: vocab = %d", vocab);
   if (N == 0) return SY_OK;
   SY_REQUIRE(tokens && embed && weight && x_out && h_out, "embed_rmsnorm: null pointer");
+  front_core::Outputs first{};
+  // (no counters: the offsets' own address stands in, and none of it is cleared)
+  first.ticket = one ? tickets ? tickets : (unsigned*)one : nullptr;
+  first.k = tickets ? ntickets : 0;
+  first.offsets = one;
   row_kernel<false, false><<<N, ROW_THREADS, 0, (hipStream_t)stream>>>(
       (const half_t*)embed, nullptr, nullptr, nullptr, nullptr, 0, (const half_t*)weight, eps, nullptr, 0, H,
-      (half_t*)x_out, (half_t*)h_out, nullptr, tokens, vocab);
+      (half_t*)x_out, (half_t*)h_out, nullptr, tokens, vocab, first);
   return sy_check_launch("embed_rmsnorm");
+}
+
+extern "C" SY_API int sy_embed_rmsnorm(const int64_t* tokens, const void* embed, int vocab, const void* weight, float eps,
+                                       int N, int H, void* x_out, void* h_out, void* stream) {
+  return sy_embed_rmsnorm_step(tokens, embed, vocab, weight, eps, N, H, x_out, h_out, nullptr, 0, nullptr, stream);
 }
 
 extern "C" SY_API int sy_add_rmsnorm_logits(const void* x, const void* delta, const void* weight, float eps,
@@ -897,6 +911,21 @@ int sy_router_route_rows(const void* h, const void* router, int N, int H, int E,
       (const half_t*)h, nullptr, nullptr, nullptr, nullptr, 0, nullptr, 0.f, (const half_t*)router, E, H, nullptr, nullptr,
       (half_t*)logits, nullptr, 0, front);
   return sy_check_launch("router_route");
+}
+
+int sy_add_rmsnorm_route(const void* x, const void* delta, const void* weight, float eps, const void* router, int E, int N,
+                         int H, int k, int norm, void* x_out, void* h_out, void* logits, int32_t* idx, void* w, void* stream) {
+  ROW_LIMITS("add_rmsnorm_route");
+  SY_REQUIRE(E >= 1 && E <= 128 && k >= 1 && k <= front_core::TAIL_MAX_K && k <= E,
+             "add_rmsnorm_route: at most 128 experts and top-8 (got E = %d, k = %d)", E, k);
+  if (N == 0) return SY_OK;
+  SY_REQUIRE(x && weight && h_out && router && logits && idx && w, "add_rmsnorm_route: null pointer");
+  front_core::Outputs front{idx, (half_t*)w, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, k, norm, 0};
+  const size_t lds = (size_t)H * sizeof(half_t) + sizeof(half_t) * ((size_t)(E + 7) / 8 * 8);
+  row_kernel<false, true, FRONT_ROUTE><<<N, 1024, lds, (hipStream_t)stream>>>(
+      (const half_t*)x, (const half_t*)delta, nullptr, nullptr, nullptr, 0, (const half_t*)weight, eps,
+      (const half_t*)router, E, H, (half_t*)x_out, (half_t*)h_out, (half_t*)logits, nullptr, 0, front);
+  return sy_check_launch("add_rmsnorm_route");
 }
 
 extern "C" SY_API int sy_add_rmsnorm_route_sort(const void* x, const void* delta, const void* weight, float eps,

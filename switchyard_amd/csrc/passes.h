@@ -49,4 +49,27 @@ SY_API int sy_moe_add_rmsnorm(const SyMoeLayer* L, const void* h, const int32_t*
  * deal their keys to several workgroups. */
 SY_API int sy_decode_attention_shares(int B, int heads);
 
+/* One decode step of a model of `layers` layers for B <= SY_STEP_MAX_ROWS sequences: tok int64 [B] -> out f16
+ * [B, vocab] (logits), the new keys and values written at *slot and real[:, *slot] set; the counters
+ * stay where they are. All weights f16, nn.Linear layout. The experts run on the weight stream up to
+ * gemv_max_rows sequences and on the MFMA tiles above. Scratch is the caller's
+ * (sy_decode_step_scratch_bytes; 0 for a shape that is not taken), 256-byte aligned, and overwritten.
+ * Limits: those of the launches (at most 128 experts, top-8, H and heads * D at most 4096). */
+#define SY_STEP_MAX_ROWS 16
+typedef struct SyDecodeLayer {
+  const void *wqkv, *q_norm, *k_norm, *wo, *mlp_norm, *router, *gate_up, *down, *next_norm; /* next_norm: of the next layer, or the final one */
+  void *kcache, *vcache; /* [B, kv_heads, capacity, D] */
+} SyDecodeLayer;
+typedef struct SyDecodeStep {
+  int B, layers, H, heads, kv_heads, D, capacity, E, I, k, norm, vocab, embed_rows, max_positions, gemv_max_rows;
+  float eps, clip;
+  const void *embed, *first_norm, *lm_head, *cos, *sin;
+  const int64_t *tok, *positions, *slot;
+  uint8_t* real;
+  void *out, *scratch;
+  size_t scratch_bytes;
+} SyDecodeStep;
+SY_API size_t sy_decode_step_scratch_bytes(const SyDecodeStep* s);
+SY_API int sy_decode_step(const SyDecodeStep* step, const SyDecodeLayer* layers, void* stream);
+
 }  // extern "C"

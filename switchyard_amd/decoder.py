@@ -364,6 +364,20 @@ class Decoder:
         s, W, E = self.s, self.w, kernels.ext()
         wqkv = self._stacked_qkv()
         positions = cache.next_position
+        rows, width = tok.numel(), s.heads * s.head_dim
+        if (self._own_moe and 1 <= rows <= E.STEP_MAX_ROWS and s.layers and s.experts <= 128 and s.top_k <= min(8, s.experts)
+                and max(s.hidden, width, W["layers"][0]["down"].shape[2]) <= 4096 and cache.k.is_contiguous()
+                and cache.v.is_contiguous()):
+            # few rows: every launch of the step from one call of the library (the host's share of a
+            # launch made here is about as long as the launch)
+            logits = E.decode_step(tok.reshape(-1), W, wqkv, self.cos, self.sin, positions.reshape(-1),
+                                   slot.reshape(-1), cache.real, cache.k,
+                                   cache.v, s.heads, s.kv_heads, s.head_dim, s.top_k, s.norm_topk_prob, s.rms_eps, s.clip_qkv,
+                                   kernels.GEMV_MAX_TOKENS)
+            if advance:
+                cache.next_position += 1
+                slot += 1
+            return logits
         x, xn = E.embed_rmsnorm(tok.reshape(-1), W["embed"], W["layers"][0]["attn_norm"], s.rms_eps)
         split = E.attention_split(s.layers, x.shape[0], s.heads, s.head_dim, x.device)
         for i in range(s.layers):

@@ -346,6 +346,30 @@ def test_decode_attention_without_a_real_key_gives_zeros():
     assert torch.allclose(out[1].view(heads, hd).float(), vc[1, :, 3].float(), atol=1e-3)
 
 
+@pytest.mark.parametrize("B,kw", [
+    (1, {}), (8, {}), (9, {}), (16, {}),                       # the gate/up stream sorts; the MFMA tiles
+    (3, dict(heads=4, kv_heads=2, head_dim=128, clip_qkv=0.5)), (12, dict(experts=128, top_k=4)),
+    (2, dict(experts=6, top_k=3, norm_topk_prob=True, heads=2, kv_heads=1, intermediate=160)),
+    (5, dict(layers=1, vocab=1003))])
+def test_a_step_in_one_call_equals_its_launches_one_by_one(B, kw, monkeypatch):
+    s, w, ps = model(7, B, **kw)
+    dec = D.Decoder(s, w)
+    tokens, valid = D.left_padded(ps, "cuda")
+    outs = []
+    for most in (kernels.ext().STEP_MAX_ROWS, 0):
+        monkeypatch.setattr(kernels.ext(), "STEP_MAX_ROWS", most, raising=False)
+        cache = D.KVCache(s, B, tokens.shape[1] + 4, torch.float16, "cuda")
+        tok = dec.prefill_fused(tokens, cache, valid).argmax(-1)[:, None]
+        slot = torch.tensor([cache.filled], device="cuda")
+        logits = []
+        for _ in range(3):
+            logits.append(dec.step_fused(tok, cache, slot))
+            tok = logits[-1].argmax(-1)[:, None]
+        outs.append((*logits, cache.k, cache.v, cache.real, cache.next_position, slot))
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
+
+
 def twins_reference(tokens, real):
     """What sy_padding_twins says, from its definition, one row at a time."""
     B, T = tokens.shape
