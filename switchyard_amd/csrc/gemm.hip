@@ -1,8 +1,7 @@
 // grouped_gemm: the prefill path. Every expert's slice of the sorted rows goes through that
 // expert's weights on fp16 MFMA tiles, all experts in one launch. Three tiles, chosen by the
-// host from the mean rows per expert: 64 or 128 rows (gemm_kernel, below) while the launch is
-// mostly a stream over the weights, 256 rows (gemm_stream_kernel, further down) once it is
-// bound by the MFMAs and by what a compute unit can pull through its L1.
+// host from the mean rows per expert: 64 or 128 rows (gemm_kernel, below) for a few rows per
+// expert, 256 rows (gemm_stream_kernel, further down) from 32 on.
 //
 // gemm_kernel. Tile: 64*MI rows x 256 weight rows (MI = 1 or 2), K in slices of 64, 4 wavefronts, each computing
 // all of the tile's rows x 64 weight rows as (2*MI) x 2 v_mfma_f32_32x32x16_f16 blocks with fp32
@@ -436,7 +435,11 @@ struct StreamTile {
 // average), so their loads are marked non-temporal: 1024 tokens 108.8 -> 104.7 us (gate/up) and
 // 61.7 -> 54.1 (down), 2048 tokens 157.8 -> 154.6 and 90.5 -> 86.0. With two row tiles per
 // column tile (4096 tokens) the second one finds the weights in L2, and the hint costs 3 to 7 %.
-template <bool SWIGLU, bool SCALE, int EPL, bool STREAMED>
+// LOW: few rows per expert (at most 96 on average): a row load whose 8 rows all lie past the tile's end
+// is not issued. A compute unit takes one such load every 25 to 40 cycles, empty or not. The layer, us,
+// without and with: 437 tokens 166 -> 162, with uneven routing (Zipf, exponent 1.1) 190 -> 176; 768
+// tokens 181 -> 175 and 205 -> 191; at 1024 tokens the branches cost what the loads did (191, 194).
+template <bool SWIGLU, bool SCALE, int EPL, bool STREAMED, bool LOW = false>
 __global__ void __launch_bounds__(512, 1)
 gemm_stream_kernel(const half_t* __restrict__ A, const int* __restrict__ a_rows, const half_t* __restrict__ B,
                    const int* __restrict__ offsets, int E, int M, int Nout, int K, const half_t* __restrict__ scale,
@@ -599,6 +602,10 @@ gemm_stream_kernel(const half_t* __restrict__ A, const int* __restrict__ a_rows,
     int at = later ? p - nk + rot_n : p + rot_c;
     at = at >= nk ? at - nk : at;
     const unsigned vc = oa_c[q], vn = oa_n[q];
+    if (LOW) {   // the same in the whole wavefront
+      const int rows_c = cur.row_end - cur.row0, rows_n = nxt.row_end - nxt.row0;
+      if (8 * (WAVES * q + wave) >= __builtin_amdgcn_readfirstlane(later ? rows_n : rows_c)) return;
+    }
     load_to_lds(arsrc, later ? vn : vc, (unsigned)at * (BIG_BK * 2), wave_base + stage * BIG_A_BYTES + q * (WAVES * 1024));
   };
   auto issue_weights = [&](int p, int stage, int q) {
@@ -643,7 +650,9 @@ gemm_stream_kernel(const half_t* __restrict__ A, const int* __restrict__ a_rows,
 #pragma unroll
     for (int q = 0; q < LOADS; ++q) issue_weights(p, p, q);
   }
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * LOADS) : "memory");
+  // slice 0 has landed when only slice 1 is in flight (LOW: its weights; of its rows some were not asked
+  // for. In the loop the youngest loads in flight are always LOADS of weights, whatever rows there are.)
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((LOW ? 1 : 2) * LOADS) : "memory");
   __syncthreads();
   int a_stage = 0, b_stage = 0;  // where the current tile's slice 0 is
 
@@ -890,11 +899,16 @@ int launch_gemm_stream(const half_t* a, const int32_t* a_rows, const half_t* b, 
   const int ncol_tiles = (Nout + cols - 1) / cols;
   const int grid = sy_compute_units() / XCDS * XCDS;
   const bool streamed = (long)rows <= 256l * E;   // one row tile per expert, mostly
-#define SY_STREAM_LAUNCH(SW, SC, ST) \
-  gemm_stream_kernel<SW, SC, EPL, ST><<<grid, 512, 0, st>>>(a, a_rows, b, offsets, E, rows, Nout, K, SC ? s : nullptr, c, ncol_tiles)
-  if (swiglu) { if (streamed) SY_STREAM_LAUNCH(true, false, true); else SY_STREAM_LAUNCH(true, false, false); }
-  else if (s) { if (streamed) SY_STREAM_LAUNCH(false, true, true); else SY_STREAM_LAUNCH(false, true, false); }
-  else { if (streamed) SY_STREAM_LAUNCH(false, false, true); else SY_STREAM_LAUNCH(false, false, false); }
+  const bool low = (long)rows <= 96l * E;         // most of a tile's rows do not exist
+#define SY_STREAM_LAUNCH(SW, SC, ST, LO) \
+  gemm_stream_kernel<SW, SC, EPL, ST, LO><<<grid, 512, 0, st>>>(a, a_rows, b, offsets, E, rows, Nout, K, SC ? s : nullptr, c, ncol_tiles)
+#define SY_STREAM_PICK(SW, SC) \
+  do { if (low) SY_STREAM_LAUNCH(SW, SC, true, true); else if (streamed) SY_STREAM_LAUNCH(SW, SC, true, false); \
+       else SY_STREAM_LAUNCH(SW, SC, false, false); } while (0)
+  if (swiglu) SY_STREAM_PICK(true, false);
+  else if (s) SY_STREAM_PICK(false, true);
+  else SY_STREAM_PICK(false, false);
+#undef SY_STREAM_PICK
 #undef SY_STREAM_LAUNCH
   return sy_check_launch("grouped_gemm");
 }
@@ -922,18 +936,26 @@ int launch_gemm(const half_t* a, const int32_t* a_rows, const half_t* b, const i
 
 }  // namespace
 
-// Rows per tile: 64 while the typical expert fits in one such tile (the launch is then a stream
-// over the weights and the smaller tile halves the padded MFMA work), 128 up to that many, else
-// 256. Under near-uniform routing an expert's rows scatter around the mean by about its square
-// root. Measured on 64 experts, 2048 x 1024: the 256-row tile wins from about 128 rows per
-// expert on. Its loads run three slices ahead, into the next tile, so it wants four slices of
-// K; its tile table is one or two experts per lane.
+// Rows per tile: 256 from 32 rows per expert on; below that 64 while the typical busiest expert (under
+// near-uniform routing an expert's rows scatter around the mean by about its square root) fits in
+// one such tile, else 128.
+//
+// What decides is the tail. The small tiles run two workgroups a compute unit, one tile each, and
+// evenly routed tokens make exactly one round of them: 64 experts x 8 column tiles. Routing is not
+// even behind a trained router, and the row tiles of popular experts then make a second round that
+// is nearly empty. The 256-row tile has one row tile for almost any expert, and deals its list to
+// resident workgroups by height. The layer, us, small tiles -> 256-row tile, with a Zipf bias (exponent
+// 1.1) / evenly routed: 257 tokens 184 -> 147 / 151 -> 154, 333 tokens 190 -> 153 / 153 -> 156, 437 tokens
+// 225 -> 175 / 158 -> 160, 600 tokens 244 -> 183 / 169 -> 169, 768 tokens 265 -> 191 / 179 -> 174; but 160 tokens
+// 146 -> 141 / 143 -> 147, and 96 tokens 130 -> 136 / 140 -> 143. Its loads run three slices ahead, into the
+// next tile, so it wants four slices of K; its tile table is one or two experts per lane.
 int sy_gemm_rows_per_tile(int rows, int E, int K) {
   const int mean = (rows + E - 1) / E;
+  const bool stream_ok = K % BIG_BK == 0 && K / BIG_BK >= 4 && E <= 2 * WAVE;
+  if (stream_ok && mean >= 32) return 256;
   int typical = mean;
   while ((typical - mean) * (typical - mean) < 4 * mean) ++typical;
-  const bool stream_ok = K % BIG_BK == 0 && K / BIG_BK >= 4 && E <= 2 * WAVE;
-  return typical <= 64 ? 64 : (typical <= 128 || !stream_ok) ? 128 : 256;
+  return typical <= 64 ? 64 : 128;
 }
 
 extern "C" SY_API int sy_grouped_gemm(const void* A, const int32_t* a_rows, const void* B, const int32_t* offsets, int E,

@@ -285,6 +285,40 @@ def test_grouped_gemm_every_tile_kind(K, counts, K_, Nout, swiglu):
     assert torch.allclose(got, want, rtol=2.0 ** -9, atol=1e-2)
 
 
+@pytest.mark.parametrize("swiglu", [True, False])
+@pytest.mark.parametrize("counts,K_,Nout", [
+    ([0, 1, 7, 8, 9, 31, 32, 33, 64, 65, 250, 256, 0, 100], 256, 264),      # 61 rows per expert, edges of the loads of 8 rows
+    ([700] + [3] * 15, 512, 136),                                           # one popular expert with three row tiles
+    ([1, 0, 300, 0, 2, 257, 5, 0] * 9, 256, 128),                           # 72 experts: two per lane of the tile table
+    ([96] * 16, 320, 200)])                                                 # the most rows that still leave loads out
+def test_grouped_gemm_stream_tile_with_few_rows_per_expert(K, counts, K_, Nout, swiglu):
+    """The 256-row tile where row loads past a tile's end are not issued: what LDS holds in their place
+    (NaN, left by a launch over NaN rows) must reach no output."""
+    E, rows = len(counts), sum(counts)
+    assert 32 * E <= rows <= 96 * E
+    g = torch.Generator().manual_seed(rows)
+    src = torch.randn(rows // 2 + 3, K_, generator=g).half()
+    a_rows = torch.randint(0, src.shape[0], (rows,), generator=g).int()
+    B = (torch.randn(E, Nout * (2 if swiglu else 1), K_, generator=g) * K_ ** -0.5).half()
+    scale = None if swiglu else torch.rand(rows, generator=g).half()
+    offsets = torch.zeros(E + 1, dtype=torch.int32)
+    offsets[1:] = torch.cumsum(torch.tensor(counts), 0)
+    nan = torch.full((256 * 512, K_), float("nan"), dtype=torch.float16, device=DEV)
+    K.ext().grouped_gemm(nan, None, B[:1].to(DEV), torch.tensor([0, len(nan)], dtype=torch.int32, device=DEV), None, 0, len(nan),
+                         swiglu, None)
+    got = K.ext().grouped_gemm(src.to(DEV), a_rows.to(DEV), B.to(DEV), offsets.to(DEV), None, 0, rows, swiglu,
+                               None if scale is None else scale.to(DEV)).float().cpu()
+    A = src[a_rows.long()]
+    want = torch.empty(rows, Nout)
+    for e in range(E):
+        s, t = int(offsets[e]), int(offsets[e + 1])
+        r = F.linear(A[s:t].float(), B[e].float())
+        want[s:t] = F.silu(r[:, :Nout].half().float()).half().float() * r[:, Nout:].half().float() if swiglu \
+            else r.half().float() * scale[s:t, None].float()
+    # one rounding to f16 of differently ordered fp32 sums, as in the test above
+    assert torch.allclose(got, want, rtol=2.0 ** -9, atol=1e-2)
+
+
 def test_grouped_gemm_stream_tile_with_operands_at_odd_addresses(K):
     """The 256-row tile reads row numbers and scales in runs through the scalar cache, from the
     4-byte word at or below where they start and moved up where a run would pass the end: the
