@@ -99,6 +99,7 @@ SIGNATURES = {
     "sy_padding_twins": (_c_int, [_c_void_p, _c_void_p, _c_int, _c_int, _c_void_p, _c_void_p]),
     "sy_moe_add_rmsnorm": (_c_int, [ctypes.POINTER(SyMoeLayer), _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_float,
                                     _c_void_p, _c_void_p, _c_void_p]),
+    "sy_dense_rows": (_c_int, [_c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_void_p, _c_void_p]),
     "sy_decode_attention_shares": (_c_int, [_c_int, _c_int]),
     "sy_decode_step_scratch_bytes": (_c_size_t, [ctypes.POINTER(SyDecodeStep)]),
     "sy_decode_step": (_c_int, [ctypes.POINTER(SyDecodeStep), ctypes.POINTER(SyDecodeLayer), _c_void_p]),
@@ -836,6 +837,17 @@ class Ext:
                    float(clip or 0.0), cos.data_ptr(), sin.data_ptr(), cos.shape[0], positions.data_ptr(),
                    slot.data_ptr(), real.data_ptr(), B, int(heads), int(kv_heads), D, capacity, kcache.data_ptr(),
                    vcache.data_ptr(), out.data_ptr(), parts, tickets, _stream())
+        return out
+
+    def dense_rows(self, x, weight):
+        """x [rows, K] @ weight [Nout, K]^T, the weights read once per 16 rows (K a multiple of 8 up to 4096)."""
+        _check(x, "x", torch.float16)
+        _check(weight, "weight", torch.float16)
+        if x.dim() != 2 or weight.dim() != 2 or x.shape[1] != weight.shape[1]:
+            raise RuntimeError("dense_rows: x [rows, K], weight [Nout, K]")
+        out = torch.empty((x.shape[0], weight.shape[0]), dtype=torch.float16, device=x.device)
+        self._call(self.lib.sy_dense_rows, x.data_ptr(), weight.data_ptr(), x.shape[0], weight.shape[0], x.shape[1],
+                   out.data_ptr(), _stream())
         return out
 
     STEP_MAX_ROWS = 16   # SY_STEP_MAX_ROWS: up to here every projection of a step is a weight stream

@@ -88,10 +88,8 @@ row_kernel(const half_t* x, const half_t* __restrict__ delta, const half_t* __re
     long g = (long)gather[t];
     g = g < 0 ? 0 : g >= src_rows ? src_rows - 1 : g;
     xrow = x + (size_t)g * H;
-    if (t == 0 && front.ticket) {   // the first launch of a step: its counters, and its projections' row range
+    if (t == 0 && front.ticket)   // the first launch of a step clears its counters
       for (int i = tid; i < front.k; i += nthreads) front.ticket[i] = 0;
-      if (tid < 2) front.offsets[tid] = tid ? (int)gridDim.x : 0;
-    }
   }
   if (COMBINE) {
     // rank the k choices by (expert id, slot); rows[] lists their rows of y in that order
@@ -778,16 +776,14 @@ extern "C" SY_API int sy_add_rmsnorm(const void* x, const void* delta, const voi
 }
 
 int sy_embed_rmsnorm_step(const int64_t* tokens, const void* embed, int vocab, const void* weight, float eps, int N, int H,
-                          void* x_out, void* h_out, unsigned* tickets, int ntickets, int32_t* one, void* stream) {
+                          void* x_out, void* h_out, unsigned* tickets, int ntickets, void* stream) {
   ROW_LIMITS("embed_rmsnorm");
   SY_REQUIRE(vocab >= 1, "embed_rmsnorm: vocab = %d", vocab);
   if (N == 0) return SY_OK;
   SY_REQUIRE(tokens && embed && weight && x_out && h_out, "embed_rmsnorm: null pointer");
   front_core::Outputs first{};
-  // (no counters: the offsets' own address stands in, and none of it is cleared)
-  first.ticket = one ? tickets ? tickets : (unsigned*)one : nullptr;
-  first.k = tickets ? ntickets : 0;
-  first.offsets = one;
+  first.ticket = tickets;
+  first.k = ntickets;
   row_kernel<false, false><<<N, ROW_THREADS, 0, (hipStream_t)stream>>>(
       (const half_t*)embed, nullptr, nullptr, nullptr, nullptr, 0, (const half_t*)weight, eps, nullptr, 0, H,
       (half_t*)x_out, (half_t*)h_out, nullptr, tokens, vocab, first);
@@ -796,7 +792,7 @@ int sy_embed_rmsnorm_step(const int64_t* tokens, const void* embed, int vocab, c
 
 extern "C" SY_API int sy_embed_rmsnorm(const int64_t* tokens, const void* embed, int vocab, const void* weight, float eps,
                                        int N, int H, void* x_out, void* h_out, void* stream) {
-  return sy_embed_rmsnorm_step(tokens, embed, vocab, weight, eps, N, H, x_out, h_out, nullptr, 0, nullptr, stream);
+  return sy_embed_rmsnorm_step(tokens, embed, vocab, weight, eps, N, H, x_out, h_out, nullptr, 0, stream);
 }
 
 extern "C" SY_API int sy_add_rmsnorm_logits(const void* x, const void* delta, const void* weight, float eps,

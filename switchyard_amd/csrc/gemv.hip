@@ -77,8 +77,12 @@ struct Pass {
 
 // One wavefront streams units [unit0, unit0 + nunits) of one expert against NQ staged quads.
 // EXACT: K is a multiple of a chunk (512) and Nout of a unit (4), so nothing needs masking.
-template <bool SWIGLU, bool SCALE, bool EXACT, int CH, int NQ>
-__device__ __forceinline__ void run_pass(const Pass& p) {
+// `behind_first` runs once, in every wavefront, when the first chunk has been asked for.
+struct Nothing {
+  __device__ void operator()() const {}
+};
+template <bool SWIGLU, bool SCALE, bool EXACT, int CH, int NQ, typename Behind = Nothing>
+__device__ __forceinline__ void run_pass(const Pass& p, Behind behind_first = Behind{}) {
   const int lane = threadIdx.x & 63, blk = lane >> 2, sub = lane & 3;
   const int klane = blk * 8;
   constexpr int PARTS = SWIGLU ? 2 : 1;  // a unit is streamed as its gate rows, then its up rows
@@ -180,9 +184,10 @@ __device__ __forceinline__ void run_pass(const Pass& p) {
 
   // chunk q+1 is in flight while chunk q is multiplied
   const int total = p.nunits * PARTS * p.nchunks;
-  if (total <= 0) return;
   Chunk<CH> c0, c1;
-  issue(c0);
+  if (total > 0) issue(c0);
+  behind_first();
+  if (total <= 0) return;
   int q = 0;
   for (; q + 3 <= total; q += 2) {
     issue(c1);
@@ -222,7 +227,12 @@ __host__ __device__ constexpr size_t sort_here_ints(int E) {
 // weight stream of tens of microseconds that costs each workgroup a few hundred cycles where
 // its scan of `offsets` stood, and the launch before it need not gather every token's choices
 // in one place.
-template <bool SWIGLU, bool SCALE, bool EXACT, int CH, bool SORT = false>
+//
+// DENSE: one matrix and `sort.M` rows of A in their own order (the projections around the MoE layer):
+// there is no list of experts to build, so a launch begins with its loads. The rows (up to 8 of
+// at most 2048) are asked for first, then the first weights, and the rows go to LDS behind those.
+// DENSE_NOTE
+template <bool SWIGLU, bool SCALE, bool EXACT, int CH, bool SORT = false, bool DENSE = false>
 __global__ void __launch_bounds__(GEMV_THREADS)
 gemv_kernel(const half_t* __restrict__ A, const int* __restrict__ a_rows, const half_t* __restrict__ B,
             const int* __restrict__ offsets, int E, int Nout, int K, const half_t* __restrict__ scale,
@@ -235,6 +245,64 @@ gemv_kernel(const half_t* __restrict__ A, const int* __restrict__ a_rows, const 
   const int RS = K + ROW_PAD;
   int* used = reinterpret_cast<int*>(xs + (size_t)row_cap * RS);  // [E] ids of experts with rows, [E] = how many
   const half8_t zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+  if constexpr (DENSE) {
+    const int rows = sort.M, units = (Nout + UNIT_COLS - 1) / UNIT_COLS;
+    const int lo = (int)((long)units * blockIdx.x / gridDim.x), count = (int)((long)units * (blockIdx.x + 1) / gridDim.x) - lo;
+    Pass p;
+    p.xs = xs;
+    p.rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(B), 0, (int)((size_t)Nout * K * 2), 0x00020000);
+    p.scale = scale;
+    p.C = C;
+    p.Nout = Nout;
+    p.K = K;
+    p.RS = RS;
+    p.nchunks = ((K + STEP_K - 1) / STEP_K + CH - 1) / CH;
+    p.unit0 = lo + (int)((long)count * wave / GEMV_WAVES);
+    p.nunits = lo + (int)((long)count * (wave + 1) / GEMV_WAVES) - p.unit0;
+    constexpr int EARLY_ROWS = 2, EARLY_CHUNKS = 4;   // per wavefront; chunks of 64 x 16 bytes
+    for (int r0 = 0; r0 < rows; r0 += row_cap) {
+      const int nr = min(row_cap, rows - r0), nq = (nr + QUAD - 1) / QUAD;
+      p.r0 = r0;
+      p.nr = nr;
+      const bool early = nq * QUAD <= EARLY_ROWS * GEMV_WAVES && K <= EARLY_CHUNKS * WAVE * 8;
+      half8_t x[EARLY_ROWS][EARLY_CHUNKS];
+      if (early) {
+#pragma unroll
+        for (int i = 0; i < EARLY_ROWS; ++i)
+#pragma unroll
+          for (int j = 0; j < EARLY_CHUNKS; ++j) {
+            const int r = wave + GEMV_WAVES * i, kk = (lane + WAVE * j) * 8;
+            x[i][j] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+            if (r < nr && kk < K) x[i][j] = *reinterpret_cast<const half8_t*>(A + (size_t)(r0 + r) * K + kk);
+          }
+      }
+      auto stage = [&] {
+        if (r0) __syncthreads();   // the rows of the pass before have been read
+        if (early) {
+#pragma unroll
+          for (int i = 0; i < EARLY_ROWS; ++i)
+#pragma unroll
+            for (int j = 0; j < EARLY_CHUNKS; ++j) {
+              const int r = wave + GEMV_WAVES * i, kk = (lane + WAVE * j) * 8;
+              if (r < nq * QUAD && kk < K) *reinterpret_cast<half8_t*>(xs + r * RS + kk) = x[i][j];
+            }
+        } else {
+          for (int r = wave; r < nq * QUAD; r += GEMV_WAVES)
+            for (int kk = lane * 8; kk < K; kk += WAVE * 8)
+              *reinterpret_cast<half8_t*>(xs + r * RS + kk) =
+                  r < nr ? *reinterpret_cast<const half8_t*>(A + (size_t)(r0 + r) * K + kk) : half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+        }
+        __syncthreads();
+      };
+      switch (nq) {
+        case 1: run_pass<SWIGLU, SCALE, EXACT, CH, 1>(p, stage); break;
+        case 2: run_pass<SWIGLU, SCALE, EXACT, CH, 2>(p, stage); break;
+        case 3: run_pass<SWIGLU, SCALE, EXACT, CH, 3>(p, stage); break;
+        default: run_pass<SWIGLU, SCALE, EXACT, CH, 4>(p, stage); break;
+      }
+    }
+    return;
+  }
   // SORT: the sort's results in LDS, behind the list of used experts
   int* s_counts = used + E + 1;
   int* s_offsets = s_counts + E;
@@ -333,18 +401,20 @@ gemv_kernel(const half_t* __restrict__ A, const int* __restrict__ a_rows, const 
 
 int launch_gemv(const void* A, const int32_t* a_rows, const void* B, const int32_t* offsets, int E, int rows,
                 int max_rows_hint, int Nout, int K, int swiglu, const void* scale, void* C, hipStream_t stream,
-                const SortHere* sort = nullptr) {
+                const SortHere* sort = nullptr, bool dense = false) {
   // rows staged per pass: no expert has more rows than there are rows in all; a caller that
   // knows a tighter bound (the number of tokens) saves LDS and gains occupancy
   const int bound = max_rows_hint > 0 && max_rows_hint < rows ? max_rows_hint : rows;
   int row_cap = (bound + QUAD - 1) / QUAD * QUAD;
   row_cap = row_cap > MAX_QUADS * QUAD ? MAX_QUADS * QUAD : row_cap;
   const size_t lds = (size_t)row_cap * (K + ROW_PAD) * sizeof(half_t) + (size_t)(E + 1) * sizeof(int) +
-                     (sort ? sort_here_ints(E) * sizeof(int) : 0);
+                     (sort && !dense ? sort_here_ints(E) * sizeof(int) : 0);
   // Loads in flight per wavefront: a chunk of 4 KB, or of 8 KB where a unit is long enough to be
   // cut into such chunks (gate and up rows of 2048 at 8 tokens: 56.6 us against 57.5; for rows of
   // 1024 the longer chunk is one per unit and loses: 34.8 us against 30.6).
-  const bool long_chunks = swiglu && K % (CH_LONG * STEP_K) == 0 && K >= 2 * CH_LONG * STEP_K;
+  // The dense projections' rows of 2048 are one unit to a wavefront or a few: two long chunks have
+  // the whole unit in flight.
+  const bool long_chunks = (swiglu || dense) && K % (CH_LONG * STEP_K) == 0 && K >= 2 * CH_LONG * STEP_K;
   const bool exact = K % (CH_SHORT * STEP_K) == 0 && Nout % UNIT_COLS == 0;
   // persistent: a fixed number of workgroups per CU, but no more than there are units. Two per
   // CU stream best when a unit is 32 KB of weights (gate and up rows of 2048: 57.8 us against
@@ -355,7 +425,8 @@ int launch_gemv(const void* A, const int32_t* a_rows, const void* B, const int32
   if (!exact && per_cu > 3) per_cu = 3;                       // the masked variants need more registers
   const long fit = (160 * 1024) / (long)(lds ? lds : 1);      // by LDS
   per_cu = per_cu > fit ? (fit > 0 ? fit : 1) : per_cu;
-  const long max_units = (long)(E < rows ? E : rows) * ((Nout + UNIT_COLS - 1) / UNIT_COLS);
+  long max_units = (long)(E < rows ? E : rows) * ((Nout + UNIT_COLS - 1) / UNIT_COLS);
+  if (dense) max_units = (max_units + GEMV_WAVES - 1) / GEMV_WAVES;   // a unit for every wavefront
   long grid = (long)sy_compute_units() * per_cu;
   grid = grid > max_units ? max_units : grid;
   const half_t* a = (const half_t*)A;
@@ -363,7 +434,9 @@ int launch_gemv(const void* A, const int32_t* a_rows, const void* B, const int32
   const half_t* s = (const half_t*)scale;
   half_t* c = (half_t*)C;
   void (*kern)(const half_t*, const int*, const half_t*, const int*, int, int, int, const half_t*, half_t*, int, SortHere);
-  if (sort && long_chunks && exact) kern = gemv_kernel<true, false, true, CH_LONG, true>;
+  if (dense && long_chunks && exact) kern = gemv_kernel<false, false, true, CH_LONG, false, true>;
+  else if (dense) kern = exact ? gemv_kernel<false, false, true, CH_SHORT, false, true> : gemv_kernel<false, false, false, CH_SHORT, false, true>;
+  else if (sort && long_chunks && exact) kern = gemv_kernel<true, false, true, CH_LONG, true>;
   else if (sort) kern = exact ? gemv_kernel<true, false, true, CH_SHORT, true> : gemv_kernel<true, false, false, CH_SHORT, true>;
   else if (swiglu && long_chunks && exact) kern = gemv_kernel<true, false, true, CH_LONG>;
   else if (swiglu) kern = exact ? gemv_kernel<true, false, true, CH_SHORT> : gemv_kernel<true, false, false, CH_SHORT>;
@@ -640,6 +713,17 @@ int sy_gemv_down_combine(const void* act, const void* down, const int32_t* offse
 // Whether sy_grouped_gemv_sorting takes this shape: one choice per lane of a wavefront.
 bool sy_gemv_sorts(int N, int k, int E, int H) {
   return N >= 1 && k >= 1 && (long)N * k <= SORT_HERE_MAX && E >= 1 && E <= 128 && k <= E && H >= 8 && H % 8 == 0 && H <= 4096;
+}
+
+extern "C" SY_API int sy_dense_rows(const void* x, const void* weight, int rows, int Nout, int K, void* out, void* stream) {
+  SY_REQUIRE(rows >= 0 && Nout >= 1, "dense_rows: rows = %d, Nout = %d", rows, Nout);
+  SY_REQUIRE(K >= 8 && K % 8 == 0 && K <= 4096, "dense_rows: K must be a multiple of 8 up to 4096 (got %d)", K);
+  SY_REQUIRE((long)Nout * K * 2 < (1l << 31), "dense_rows: the matrix must stay under 2 GiB");
+  if (rows == 0) return SY_OK;
+  SY_REQUIRE(x && weight && out, "dense_rows: null pointer");
+  SortHere all{};
+  all.M = rows;
+  return launch_gemv(x, nullptr, weight, nullptr, 1, rows, rows, Nout, K, 0, nullptr, out, (hipStream_t)stream, &all, true);
 }
 
 extern "C" SY_API int sy_grouped_gemv(const void* A, const int32_t* a_rows, const void* B, const int32_t* offsets,

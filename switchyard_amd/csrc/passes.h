@@ -45,6 +45,10 @@ SY_API int sy_padding_twins(const int64_t* tokens, const uint8_t* real, int B, i
 SY_API int sy_moe_add_rmsnorm(const SyMoeLayer* L, const void* h, const int32_t* twin, const void* x, const void* weight,
                               float eps, void* x_out, void* h_out, void* stream);
 
+/* x f16 [rows, K] @ weight f16 [Nout, K]^T -> out f16 [rows, Nout] as one weight stream per 16 rows: the bits
+ * of sy_grouped_gemv with one expert that owns every row. K a multiple of 8 up to 4096. */
+SY_API int sy_dense_rows(const void* x, const void* weight, int rows, int Nout, int K, void* out, void* stream);
+
 /* Whether decode attention's (sequence, head) pairs are few enough for sy_decode_attention_qkv_split to
  * deal their keys to several workgroups. */
 SY_API int sy_decode_attention_shares(int B, int heads);

@@ -6,8 +6,7 @@
 // 13 us (the checks, the allocation of its outputs, the marshalling): 1467 us to enqueue a step, now
 // 527, and one sequence's step behind 700 positions takes 1134 us where it took 1299.
 //
-// What the launches are, per layer: q/k/v projection (a weight stream with one expert that owns every
-// row), attention with the q/k norm, the rotary embedding and the cache write in its prologue, output
+// What the launches are, per layer: q/k/v projection (a weight stream), attention with the q/k norm, the rotary embedding and the cache write in its prologue, output
 // projection, residual add + norm + router logits + route (+ sort), gate/up, down, and combine +
 // residual add + the next norm. Up to 64 choices (8 tokens of top-8) the front only routes and
 // the gate/up stream sorts for itself, as in sy_moe_layer.
@@ -18,7 +17,7 @@
 namespace {
 
 struct StepScratch {
-  size_t x, xn, qkv, a, o, h, logits, idx, w, counts, offsets, token, wsorted, pos_of, act, y, parts, tickets, one, end;
+  size_t x, xn, qkv, a, o, h, logits, idx, w, counts, offsets, token, wsorted, pos_of, act, y, parts, tickets, end;
 };
 
 StepScratch step_scratch(const SyDecodeStep& s) {
@@ -49,7 +48,6 @@ StepScratch step_scratch(const SyDecodeStep& s) {
   const bool shares = sy_decode_attention_shares(s.B, s.heads);
   r.parts = take(shares ? B * s.heads * 16 * (s.D + 2) * 4 : 0);
   r.tickets = take(shares ? B * s.heads * 4 : 0);
-  r.one = take(2 * 4);
   r.end = at;
   return r;
 }
@@ -82,23 +80,23 @@ extern "C" SY_API int sy_decode_step(const SyDecodeStep* step, const SyDecodeLay
   void *x = b + at.x, *xn = b + at.xn, *qkv = b + at.qkv, *a = b + at.a, *o = b + at.o, *h = b + at.h, *logits = b + at.logits;
   void *w = b + at.w, *wsorted = b + at.wsorted, *act = b + at.act, *y = b + at.y;
   int32_t *idx = (int32_t*)(b + at.idx), *counts = (int32_t*)(b + at.counts), *offsets = (int32_t*)(b + at.offsets);
-  int32_t *token = (int32_t*)(b + at.token), *pos_of = (int32_t*)(b + at.pos_of), *one = (int32_t*)(b + at.one);
+  int32_t *token = (int32_t*)(b + at.token), *pos_of = (int32_t*)(b + at.pos_of);
   const bool shares = sy_decode_attention_shares(s.B, s.heads);
   void *parts = shares ? b + at.parts : nullptr, *tickets = shares ? b + at.tickets : nullptr;
   const int B = s.B, H = s.H, I = s.I, E = s.E, k = s.k, M = B * k, qd = s.heads * s.D, kvd = s.kv_heads * s.D;
   const bool stream_experts = B <= s.gemv_max_rows, sorts = stream_experts && sy_gemv_sorts(B, k, E, H);
 
   int rc = sy_embed_rmsnorm_step(s.tok, s.embed, s.embed_rows, s.first_norm, s.eps, B, H, x, xn, (unsigned*)tickets,
-                                 shares ? B * s.heads : 0, one, stream);
+                                 shares ? B * s.heads : 0, stream);
   for (int i = 0; i < s.layers && !rc; ++i) {
     const SyDecodeLayer& L = layers[i];
     // one projection after another; the first that fails ends the step
-    rc = sy_grouped_gemv(xn, nullptr, L.wqkv, one, 1, B, B, qd + 2 * kvd, H, 0, nullptr, qkv, stream);
+    rc = sy_dense_rows(xn, L.wqkv, B, qd + 2 * kvd, H, qkv, stream);
     if (!rc)
       rc = sy_decode_attention_qkv_split(qkv, L.q_norm, L.k_norm, s.eps, s.clip, s.cos, s.sin, s.max_positions, s.positions,
                                          s.slot, s.real, B, s.heads, s.kv_heads, s.D, s.capacity, L.kcache, L.vcache, a, parts,
                                          tickets, stream);
-    if (!rc) rc = sy_grouped_gemv(a, nullptr, L.wo, one, 1, B, B, H, qd, 0, nullptr, o, stream);
+    if (!rc) rc = sy_dense_rows(a, L.wo, B, H, qd, o, stream);
     if (rc) break;
     if (sorts) {
       rc = sy_add_rmsnorm_route(x, o, L.mlp_norm, s.eps, L.router, E, B, H, k, s.norm, x, h, logits, idx, w, stream);
@@ -118,6 +116,6 @@ extern "C" SY_API int sy_decode_step(const SyDecodeStep* step, const SyDecodeLay
     if (!rc)
       rc = sy_combine_add_rmsnorm(y, pos_of, idx, stream_experts ? w : nullptr, k, x, L.next_norm, s.eps, B, H, x, xn, stream);
   }
-  if (!rc) rc = sy_grouped_gemv(xn, nullptr, s.lm_head, one, 1, B, B, s.vocab, H, 0, nullptr, s.out, stream);
+  if (!rc) rc = sy_dense_rows(xn, s.lm_head, B, s.vocab, H, s.out, stream);
   return rc;
 }

@@ -129,9 +129,6 @@ def experts(h, idx, w, gate_up, down, mode="auto"):
     return E.combine(y, pos_of, idx, N)
 
 
-_ONE_EXPERT = {}
-
-
 def dense(x, weight):
     """x [rows, K] @ weight [Nout, K]^T for the projections around the MoE layer at decode
     (q/k/v, output, lm_head), which are weight streams like the experts are. Up to 16 rows the
@@ -143,10 +140,7 @@ def dense(x, weight):
     rows = x.shape[0]
     if rows > 16 or weight.shape[1] > 4096 or weight.shape[1] % 8:
         return F.linear(x, weight)
-    key = (rows, x.device)
-    if key not in _ONE_EXPERT:
-        _ONE_EXPERT[key] = torch.tensor([0, rows], dtype=torch.int32, device=x.device)
-    return ext().grouped_gemv(x, None, weight[None], _ONE_EXPERT[key], rows, False, None, rows)
+    return ext().dense_rows(x, weight)
 
 
 # Up to this many tokens route and sort run as one launch of one workgroup (a decode step is

@@ -434,6 +434,17 @@ def test_dense_projection(rows, Nout, K):
     assert torch.allclose(got.float(), want, rtol=2 * ULP, atol=2e-3)
 
 
+@pytest.mark.parametrize("rows", [1, 3, 4, 5, 8, 9, 16, 17, 33])
+@pytest.mark.parametrize("Nout,K", [(6144, 2048), (2048, 1024), (1001, 2048), (7, 512), (130, 520), (36, 4096), (64, 8),
+                                    (4100, 3072)])
+def test_dense_rows_equal_the_weight_stream_of_one_expert(rows, Nout, K):
+    """Rows staged early and late, chunks of both lengths, ragged edges, several passes over 16 rows."""
+    x, w = rnd(rows, K, seed=51), rnd(Nout, K, seed=52, std=0.03)
+    offsets = torch.tensor([0, rows], dtype=torch.int32, device="cuda")
+    want = kernels.ext().grouped_gemv(x, None, w[None], offsets, rows, False, None, rows)
+    assert torch.equal(kernels.ext().dense_rows(x, w), want)
+
+
 def model(seed, batch, **kw):
     s = D.Shape(**{**dict(vocab=1000, hidden=512, intermediate=256, layers=3, heads=8, kv_heads=8, head_dim=64, experts=64,
                           top_k=8), **kw})
