@@ -1,7 +1,7 @@
 // grouped_gemm: the prefill path. Every expert's slice of the sorted rows goes through that
 // expert's weights on fp16 MFMA tiles, all experts in one launch. Three tiles, chosen by the
 // host from the mean rows per expert: 64 or 128 rows (gemm_kernel, below) for a few rows per
-// expert, 256 rows (gemm_stream_kernel, further down) from 32 on.
+// expert, 256 rows (gemm_stream_kernel, further down) above 32.
 //
 // gemm_kernel. Tile: 64*MI rows x 256 weight rows (MI = 1 or 2), K in slices of 64, 4 wavefronts, each computing
 // all of the tile's rows x 64 weight rows as (2*MI) x 2 v_mfma_f32_32x32x16_f16 blocks with fp32
@@ -936,7 +936,7 @@ int launch_gemm(const half_t* a, const int32_t* a_rows, const half_t* b, const i
 
 }  // namespace
 
-// Rows per tile: 256 from 32 rows per expert on; below that 64 while the typical busiest expert (under
+// Rows per tile: 256 above 32 rows per expert; up to that 64 while the typical busiest expert (under
 // near-uniform routing an expert's rows scatter around the mean by about its square root) fits in
 // one such tile, else 128.
 //
@@ -952,7 +952,7 @@ int launch_gemm(const half_t* a, const int32_t* a_rows, const half_t* b, const i
 int sy_gemm_rows_per_tile(int rows, int E, int K) {
   const int mean = (rows + E - 1) / E;
   const bool stream_ok = K % BIG_BK == 0 && K / BIG_BK >= 4 && E <= 2 * WAVE;
-  if (stream_ok && mean >= 32) return 256;
+  if (stream_ok && rows > 32l * E) return 256;
   int typical = mean;
   while ((typical - mean) * (typical - mean) < 4 * mean) ++typical;
   return typical <= 64 ? 64 : 128;
