@@ -23,15 +23,24 @@
 // padding) are skipped whole, and only tiles that touch the diagonal or hold padding pay for
 // masking.
 //
+// Precision. The first product's sums, the softmax and the output stay in fp32. For the second product
+// probabilities are rounded to f16, relative to the maximum of the keys up to the end of their step: against
+// that exact maximum the largest probability is 1 and has no rounding error. (A maximum rounded up to a
+// whole power of two, with rescaling put off until it grew by 2^8, was faster - 13.8, 22.8 and 68 us
+// at the sizes below - and had 9 to 37 % more error against 64 bits.) A step's length matters in the same
+// way, less: 32 keys have 0.3 to 0.8 % more error than 16, 64 again 0.3 to 0.6 % more, and each takes 5 to 11 %
+// less time. launch_steps below picks the longest that is no less precise than PyTorch's fused call, which
+// this kernel replaces. With fewer key heads than query heads what it replaces held the probabilities in
+// 32 bits, and so does WIDE: the sum of two f16 numbers, each with a product of its own, 2^14 times as
+// large as above so that the second one stays normal. One prompt of 437 tokens, 16 heads over 4: 16.7 us.
+//
 // Measured (16 heads of 128, us a launch; before: PyTorch's fused call with a mask tensor, beside which
 // the mask's conversion, a workspace fill and a transposed copy were launches of their own): one
-// prompt of 437 tokens 14 (43 before), 8 of 512 22 (64), 3 of 2000 68 (643). At 3 x 2000 that is 720
+// prompt of 437 tokens 15.8 (43 before), 8 of 512 24.6 (64), 3 of 2000 67.5 (643). At 3 x 2000 that is 730
 // Tflop/s of the causal half; matrix pipes, LDS reads and the exponentials each need about a third
-// of the time, and what is lost is their overlap. 128 queries per workgroup at every size: 64 were
-// never faster (437 tokens 14.6 against 14.2, 8 x 512 27.2 against 22.2, 3 x 2000 105 against 68) and
-// 256 only at 16 x 128 (9.0 against 10.0; 3 x 2000 72 against 68).
-#include <type_traits>
-
+// of the time, and what is lost is their overlap. 128 queries per workgroup at every size: with the
+// power-of-two rule 64 were never faster (437 tokens 14.6 against 14.2, 8 x 512 27.2 against 22.2, 3 x
+// 2000 105 against 68) and 256 only at 16 x 128 (9.0 against 10.0; 3 x 2000 72 against 68).
 #include "common.h"
 #include "passes.h"
 
@@ -41,11 +50,6 @@ constexpr int ATT_KEYS = 64;           // keys per tile
 constexpr int ATT_QROWS = 32;          // queries per wavefront
 constexpr int ATT_WAVES = 4;           // wavefronts per workgroup, of one head of one sequence
 constexpr float ATT_NONE = -1.0e30f;   // running maximum before any key was seen
-// The running maximum is a whole power of two, so what a probability is rounded to in f16 does not
-// depend on the tiles it is met in and rescaling is exact; and the output is rescaled only when the
-// maximum has grown by more than this many powers of two: until then the probabilities are at most
-// 2^8 and fit f16.
-constexpr float ATT_SLACK = 8.f;
 
 typedef int att_int4 __attribute__((ext_vector_type(4)));
 typedef short att_short4 __attribute__((__vector_size__(8)));
@@ -81,11 +85,8 @@ __device__ __forceinline__ float other_half(float v) {
   return (threadIdx.x & 32) ? __uint_as_float(r[0]) : __uint_as_float(r[1]);
 }
 
-// SHORT: at most one tile
-// of keys, where time is latency and the softmax goes by 16 keys with the maximum itself: the steps
-// that PyTorch's fused attention takes at these sizes, so a short prompt keeps its bits (0.1 % of the
-// values differ in the last one; 9 % would with the rule below, and one bit can decide a router's tie).
-template <int D, bool SHORT>
+// STEP: keys per step of the running softmax (16, 32 or 64). WIDE: probabilities of 22 bits instead of 11.
+template <int D, int STEP, bool WIDE>
 __global__ void __launch_bounds__(ATT_WAVES * WAVE, 2)
 prefill_attention_kernel(const half_t* __restrict__ q, const half_t* __restrict__ kcache, const half_t* __restrict__ vcache,
                          const uint8_t* __restrict__ real, int first, int T, int pairs, int heads, int kv_heads, int capacity,
@@ -215,16 +216,16 @@ prefill_attention_kernel(const half_t* __restrict__ q, const half_t* __restrict_
           }
       }
       // one step of the running softmax over registers r0 .. r1 - 1 of blocks k0 .. k1 - 1
-      half8_t p[2][2];
-      auto softmax = [&](auto exact, int k0, int k1, int r0, int r1) {
+      half8_t p[2][2], rest[2][2];
+      auto softmax = [&](int k0, int k1, int r0, int r1) {
         float mx = -INFINITY;
 #pragma unroll
         for (int kb = k0; kb < k1; ++kb)
 #pragma unroll
           for (int r = r0; r < r1; ++r) mx = fmaxf(mx, s[kb][r]);
         mx = fmaxf(mx, other_half(mx)) * scale_log2e;
-        if (__any(mx > m + (decltype(exact)::value ? 0.f : ATT_SLACK))) {
-          const float mn = fmaxf(m, decltype(exact)::value ? mx : __builtin_ceilf(mx));
+        if (__any(mx > m)) {
+          const float mn = fmaxf(m, mx);
           const float alpha = __builtin_amdgcn_exp2f(m - mn);
           m = mn;
           l *= alpha;
@@ -237,9 +238,11 @@ prefill_attention_kernel(const half_t* __restrict__ q, const half_t* __restrict_
         for (int kb = k0; kb < k1; ++kb)
 #pragma unroll
           for (int r = r0; r < r1; ++r) {
-            const float e = __builtin_amdgcn_exp2f(s[kb][r] * scale_log2e - m);
+            const float e = __builtin_amdgcn_exp2f(s[kb][r] * scale_log2e - (m - (WIDE ? 14.f : 0.f)));
             l += e;
-            p[kb][r >> 3][r & 7] = (half_t)e;
+            const half_t rounded = (half_t)e;
+            p[kb][r >> 3][r & 7] = rounded;
+            if (WIDE) rest[kb][r >> 3][r & 7] = (half_t)(e - (float)rounded);
           }
       };
       const unsigned vt = lds_base + (unsigned)(2 * stage + 1) * TILE_BYTES;
@@ -252,22 +255,18 @@ prefill_attention_kernel(const half_t* __restrict__ q, const half_t* __restrict_
           const half4_t hi = __builtin_bit_cast(half4_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(size_t)(at + vread8[d])));
           const half8_t vf = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
           o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, p[kb][st], o[d], 0, 0, 0);
+          if (WIDE) o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, rest[kb][st], o[d], 0, 0, 0);
         }
       };
-      if constexpr (SHORT) {
+      if (STEP == 64) softmax(0, 2, 0, 16);
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
+      for (int kb = 0; kb < 2; ++kb) {
+        if (STEP == 32) softmax(kb, kb + 1, 0, 16);
 #pragma unroll
-          for (int st = 0; st < 2; ++st) {
-            softmax(std::true_type{}, kb, kb + 1, 8 * st, 8 * st + 8);
-            values(kb, st);
-          }
-      } else {
-        softmax(std::false_type{}, 0, 2, 0, 16);
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-          for (int st = 0; st < 2; ++st) values(kb, st);
+        for (int st = 0; st < 2; ++st) {
+          if (STEP == 16) softmax(kb, kb + 1, 8 * st, 8 * st + 8);
+          values(kb, st);
+        }
       }
     }
     tile = after;
@@ -305,18 +304,36 @@ prefill_attention_kernel(const half_t* __restrict__ q, const half_t* __restrict_
     }
 }
 
-template <int D, bool SHORT>
+template <int D, int STEP, bool WIDE>
 int launch_prefill_attention(const half_t* q, const half_t* kc, const half_t* vc, const uint8_t* real, int first, int B, int T,
                              int heads, int kv_heads, int capacity, half_t* out, hipStream_t st) {
   const int pairs = B * heads, rows = ATT_WAVES * ATT_QROWS, nblocks = (T + rows - 1) / rows;
   const size_t lds = (size_t)4 * ATT_KEYS * D * 2 + sizeof(uint64_t) * (size_t)((first + T + ATT_KEYS - 1) / ATT_KEYS);
   SY_REQUIRE(lds <= 160 * 1024, "prefill_attention: %d positions are too many", first + T);
-  const auto kern = prefill_attention_kernel<D, SHORT>;
+  const auto kern = prefill_attention_kernel<D, STEP, WIDE>;
   if (lds > 48 * 1024 && hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
     return sy_fail(SY_ERR_LAUNCH, "prefill_attention: cannot reserve %zu bytes of LDS", lds);
   kern<<<(unsigned)(pairs * nblocks), ATT_WAVES * WAVE, lds, st>>>(q, kc, vc, real, first, T, pairs, heads, kv_heads, capacity,
                                                           1.4426950408889634f / sqrtf((float)D), out);
   return sy_check_launch("prefill_attention");
+}
+
+// PyTorch's fused call (its results were compared with each step's, over queries and positions from 1 to
+// 3000 on this card) takes 16 keys at a time up to 256 positions and, for 33 to 64 queries, up to 1024; 32 at
+// 257 to 1024 queries and as many positions, and for heads of 64 up to 2048 queries; 64 or more otherwise.
+template <int D>
+int launch_steps(const half_t* q, const half_t* kc, const half_t* vc, const uint8_t* real, int first, int B, int T, int heads,
+                 int kv_heads, int capacity, half_t* out, hipStream_t st) {
+  const int positions = first + T;
+#define SY_PREFILL(STEP_, WIDE_) \
+  launch_prefill_attention<D, STEP_, WIDE_>(q, kc, vc, real, first, B, T, heads, kv_heads, capacity, out, st)
+  if (kv_heads != heads) return SY_PREFILL(64, true);
+  if (positions <= 256 || (T <= 64 && positions <= 1024)) return SY_PREFILL(16, false);
+  if constexpr (D == 128) {
+    if (positions > 1024) return SY_PREFILL(64, false);
+  }
+  return SY_PREFILL(32, false);
+#undef SY_PREFILL
 }
 
 }  // namespace
@@ -335,9 +352,6 @@ extern "C" SY_API int sy_prefill_attention(const void* q, const void* kcache, co
   const half_t *qh = (const half_t*)q, *kc = (const half_t*)kcache, *vc = (const half_t*)vcache;
   half_t* o = (half_t*)out;
   hipStream_t st = (hipStream_t)stream;
-#define SY_PREFILL(D_, SHORT_) \
-  launch_prefill_attention<D_, SHORT_>(qh, kc, vc, real, first, B, T, heads, kv_heads, capacity, o, st)
-  if (first + T <= ATT_KEYS) return D == 128 ? SY_PREFILL(128, true) : SY_PREFILL(64, true);
-  return D == 128 ? SY_PREFILL(128, false) : SY_PREFILL(64, false);
-#undef SY_PREFILL
+  return D == 128 ? launch_steps<128>(qh, kc, vc, real, first, B, T, heads, kv_heads, capacity, o, st)
+                  : launch_steps<64>(qh, kc, vc, real, first, B, T, heads, kv_heads, capacity, o, st);
 }

@@ -230,6 +230,68 @@ def test_prefill_attention(B, T, first, heads, kv_heads, hd, holes):
     assert ((got - want).abs() <= bound).all(), ((got - want).abs() - bound).max()
 
 
+def seen_by(real, first, T):
+    """[B, T, first + T]: which positions a query at first + t sees (its own, if it would see none)."""
+    slot, at = torch.arange(first + T)[None], torch.arange(first, first + T)[:, None]
+    sees = (slot <= at)[None] & real[:, None, :first + T]
+    return sees | ~sees.any(-1, keepdim=True) & (slot == at)[None]
+
+
+def running_softmax(scores, v, step):
+    """softmax(scores) @ v as prefill_attention defines it, in 64 bits but for the probabilities: `step`
+    keys at a time, each probability rounded to f16 relative to the maximum so far."""
+    m, l, o = torch.full(scores.shape[:-1] + (1,), -1e30, dtype=torch.float64), 0.0, 0.0
+    for k0 in range(0, scores.shape[-1], step):
+        s = scores[..., k0:k0 + step]
+        new = torch.maximum(m, s.amax(-1, keepdim=True))
+        e = torch.exp2(s - new)
+        l = l * torch.exp2(m - new) + e.sum(-1, keepdim=True)
+        o = o * torch.exp2(m - new) + e.half().double() @ v[..., k0:k0 + step, :]
+        m = new
+    return o / l
+
+
+@pytest.mark.parametrize("T,first,hd,step", [(40, 0, 128, 16), (256, 0, 64, 16), (60, 196, 128, 16), (64, 960, 64, 16),
+                                             (257, 0, 128, 32), (65, 192, 128, 32), (65, 959, 64, 32), (1024, 0, 128, 32),
+                                             (1025, 0, 64, 32), (64, 961, 64, 32), (1025, 0, 128, 64), (64, 961, 128, 64)])
+@pytest.mark.parametrize("std", [1.0, 4.0])
+def test_prefill_attention_rounds_relative_to_the_exact_maximum(T, first, hd, step, std):
+    """The precision of the fused call that the kernel replaces: against the exact running maximum of
+    the stated steps a row's largest probability is 1 and has no rounding error."""
+    B, heads, n = 2, 2, first + T
+    q, kc, vc = rnd(B * T, heads * hd, seed=61, std=std), rnd(B, heads, n + 3, hd, seed=62), rnd(B, heads, n + 3, hd, seed=63)
+    real = torch.arange(n + 3)[None] >= torch.tensor([[0], [n // 3]])
+    got = kernels.ext().prefill_attention(q, kc, vc, real.cuda(), first, heads).view(B, T, heads, hd).transpose(1, 2).cpu()
+    qd, kd, vd = (t.double().cpu() for t in (q.view(B, T, heads, hd).transpose(1, 2), kc[:, :, :n], vc[:, :, :n]))
+    s = (qd @ kd.transpose(-1, -2) * (math.log2(math.e) / math.sqrt(hd))).masked_fill(~seen_by(real, first, T)[:, None], -math.inf)
+    want, exact = running_softmax(s, vd, step), (s * math.log(2)).softmax(-1) @ vd
+    # What differs is fp32 against 64 bits. An exponent off by 2^-20 at most moves up to 2^-20 / 2^-11 = 1 / 512 of
+    # the probabilities across a rounding to f16, each by 2^-11 of itself. A result is a sum of n such terms
+    # of either sign, so n / 512 of them move it by about 2^-11 / sqrt(512) of itself: 1 / 23 of the distance
+    # between two f16 numbers, hence at most one result in 23 is rounded the other way. (A maximum rounded up to
+    # a power of two changes 35 to 50 % of the results.)
+    assert (got != want.half()).double().mean() < 1 / 23
+    assert (got.double() - exact).norm() < 1.002 * (want.half().double() - exact).norm()
+
+
+@pytest.mark.parametrize("T,first,hd,kv_heads", [(40, 0, 128, 1), (300, 0, 64, 2), (100, 1000, 128, 2), (1500, 0, 128, 1)])
+@pytest.mark.parametrize("std", [1.0, 4.0])
+def test_prefill_attention_of_shared_key_heads_keeps_32_bits(T, first, hd, kv_heads, std):
+    """Nothing but the result is rounded: all but a few results are the exact ones' f16 numbers."""
+    B, heads, n = 2, 4, first + T
+    q = rnd(B * T, heads * hd, seed=64, std=std)
+    kc, vc = rnd(B, kv_heads, n + 3, hd, seed=65), rnd(B, kv_heads, n + 3, hd, seed=66)
+    real = torch.arange(n + 3)[None] >= torch.tensor([[0], [n // 3]])
+    got = kernels.ext().prefill_attention(q, kc, vc, real.cuda(), first, heads).view(B, T, heads, hd).transpose(1, 2).cpu()
+    qd = q.double().cpu().view(B, T, heads, hd).transpose(1, 2)
+    kd, vd = (t[:, :, :n].double().cpu().repeat_interleave(heads // kv_heads, 1) for t in (kc, vc))
+    s = (qd @ kd.transpose(-1, -2) / math.sqrt(hd)).masked_fill(~seen_by(real, first, T)[:, None], -math.inf)
+    exact = s.softmax(-1) @ vd
+    # an error of 2^-18 of a result's terms (scores of up to 30 in fp32: 2^-19; probabilities of 22 bits) against
+    # a rounding that moves in steps of 2^-10 or 2^-11 of the result: at most 1 result in 128 is rounded the other way
+    assert (got != exact.half()).double().mean() < 1 / 128
+
+
 @pytest.mark.parametrize("B,heads,kv_heads,hd,cap,slot_at", [
     (8, 16, 16, 128, 640, 600),    # OLMoE at batch 8: 16 wavefronts per (sequence, head)
     (64, 16, 16, 128, 200, 199),   # many pairs: 4 wavefronts each; the last slot of the cache
