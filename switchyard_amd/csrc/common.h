@@ -35,9 +35,9 @@ bool sy_router_route_counts(int N, int k);
 bool sy_router_route_shape_ok(int N, int H, int E, int k);
 // gemm.hip: rows of the tile that sy_grouped_gemm picks for `rows` sorted rows over E experts (64, 128 or 256)
 int sy_gemm_rows_per_tile(int rows, int E, int K);
-// decode.hip: sy_embed_rmsnorm at the head of a step, which also clears its counters
+// decode.hip: sy_embed_rmsnorm at the head of a step, which also sets nclear counters to zero
 int sy_embed_rmsnorm_step(const int64_t* tokens, const void* embed, int vocab, const void* weight, float eps, int N, int H,
-                          void* x_out, void* h_out, unsigned* tickets, int ntickets, void* stream);
+                          void* x_out, void* h_out, unsigned* clear, int nclear, void* stream);
 // decode.hip: sy_add_rmsnorm_route_sort without the sort, for the launch that sorts for itself
 int sy_add_rmsnorm_route(const void* x, const void* delta, const void* weight, float eps, const void* router, int E, int N,
                          int H, int k, int norm, void* x_out, void* h_out, void* logits, int32_t* idx, void* w, void* stream);

@@ -67,14 +67,21 @@ constexpr int ROW_MAX_K = 64;  // choices per token the combining variant ranks 
 // With FRONT (and LOGITS) the workgroup then routes its token from the logits in LDS; with FRONT
 // == FRONT_SORT the last workgroup of the launch to get there also sorts every token's choices
 // (front_core.h): the layer's router GEMM, route and sort in one launch.
+// FROM says where a row's inputs are, and each answer is an instance of its own, so that the rows of a
+// layer pay for neither of the others (as run-time questions they cost every instance 23 to 37
+// instructions, and the logits one a wavefront of occupancy): EMBEDDED looks row t up in x by gather[t], and
+// its first workgroup sets the `nclear` counters at `clear` to zero for the launches behind it; TWINNED
+// (with COMBINE) takes the expert outputs of token twin[t] (front.hip).
 constexpr int FRONT_ROUTE = 1, FRONT_SORT = 2;
-template <bool COMBINE, bool LOGITS, int FRONT = 0>
+constexpr int OWN_ROWS = 0, EMBEDDED = 1, TWINNED = 2;
+template <bool COMBINE, bool LOGITS, int FRONT = 0, int FROM = OWN_ROWS>
 __global__ void __launch_bounds__(LOGITS ? 1024 : ROW_THREADS)
 row_kernel(const half_t* x, const half_t* __restrict__ delta, const half_t* __restrict__ y,
            const int* __restrict__ pos_of, const int* __restrict__ idx, int k, const half_t* __restrict__ weight,
            float eps, const half_t* __restrict__ router, int E, int H, half_t* x_out, half_t* __restrict__ h_out,
            half_t* __restrict__ logits, const int64_t* __restrict__ gather, int src_rows,
-           front_core::Outputs front = front_core::Outputs{}, const int* __restrict__ twin = nullptr) {  // x_out may be x
+           front_core::Outputs front = front_core::Outputs{}, const int* __restrict__ twin = nullptr,
+           unsigned* __restrict__ clear = nullptr, int nclear = 0) {  // x_out may be x
   extern __shared__ __attribute__((aligned(16))) half_t hs[];  // LOGITS: the normalised row [H]; FRONT: the tail's LDS behind it
   __shared__ float part[16];
   __shared__ int rows[ROW_MAX_K];
@@ -82,19 +89,18 @@ row_kernel(const half_t* x, const half_t* __restrict__ delta, const half_t* __re
   const int t = blockIdx.x, tid = threadIdx.x, nthreads = blockDim.x;
   const size_t row = (size_t)t * H;
   const int chunks = H >> 3;
-  // the input row: row t of x, or (an embedding lookup) the row of x that gather[t] names
   const half_t* xrow = x + row;
-  if (gather) {
+  if (FROM == EMBEDDED) {
     long g = (long)gather[t];
     g = g < 0 ? 0 : g >= src_rows ? src_rows - 1 : g;
     xrow = x + (size_t)g * H;
-    if (t == 0 && front.ticket)   // the first launch of a step clears its counters
-      for (int i = tid; i < front.k; i += nthreads) front.ticket[i] = 0;
+    if (t == 0)
+      for (int i = tid; i < nclear; i += nthreads) clear[i] = 0;
   }
   if (COMBINE) {
     // rank the k choices by (expert id, slot); rows[] lists their rows of y in that order
     if (tid < WAVE) {
-      const int of = twin ? twin[t] : t;   // the token whose expert outputs are this one's (front.hip)
+      const int of = FROM == TWINNED ? twin[t] : t;
       const int mine = tid < k ? idx[(size_t)of * k + tid] : 0x7fffffff;
       const int src = tid < k ? pos_of[(size_t)of * k + tid] : 0;
       int rank = 0;
@@ -776,17 +782,14 @@ extern "C" SY_API int sy_add_rmsnorm(const void* x, const void* delta, const voi
 }
 
 int sy_embed_rmsnorm_step(const int64_t* tokens, const void* embed, int vocab, const void* weight, float eps, int N, int H,
-                          void* x_out, void* h_out, unsigned* tickets, int ntickets, void* stream) {
+                          void* x_out, void* h_out, unsigned* clear, int nclear, void* stream) {
   ROW_LIMITS("embed_rmsnorm");
   SY_REQUIRE(vocab >= 1, "embed_rmsnorm: vocab = %d", vocab);
   if (N == 0) return SY_OK;
-  SY_REQUIRE(tokens && embed && weight && x_out && h_out, "embed_rmsnorm: null pointer");
-  front_core::Outputs first{};
-  first.ticket = tickets;
-  first.k = ntickets;
-  row_kernel<false, false><<<N, ROW_THREADS, 0, (hipStream_t)stream>>>(
+  SY_REQUIRE(tokens && embed && weight && x_out && h_out && (clear || !nclear), "embed_rmsnorm: null pointer");
+  row_kernel<false, false, 0, EMBEDDED><<<N, ROW_THREADS, 0, (hipStream_t)stream>>>(
       (const half_t*)embed, nullptr, nullptr, nullptr, nullptr, 0, (const half_t*)weight, eps, nullptr, 0, H,
-      (half_t*)x_out, (half_t*)h_out, nullptr, tokens, vocab, first);
+      (half_t*)x_out, (half_t*)h_out, nullptr, tokens, vocab, front_core::Outputs{}, nullptr, clear, nclear);
   return sy_check_launch("embed_rmsnorm");
 }
 
@@ -950,9 +953,10 @@ int sy_combine_add_rmsnorm_twins(const void* y, const int32_t* pos_of, const int
   SY_REQUIRE(k >= 1 && k <= ROW_MAX_K, "combine_add_rmsnorm: 1 <= k <= %d (got %d)", ROW_MAX_K, k);
   if (N == 0) return SY_OK;
   SY_REQUIRE(y && pos_of && idx && x && weight && h_out, "combine_add_rmsnorm: null pointer");
-  row_kernel<true, false><<<N, ROW_THREADS, 0, (hipStream_t)stream>>>(
+  auto kern = twin ? row_kernel<true, false, 0, TWINNED> : row_kernel<true, false>;
+  kern<<<N, ROW_THREADS, 0, (hipStream_t)stream>>>(
       (const half_t*)x, (const half_t*)w, (const half_t*)y, pos_of, idx, k, (const half_t*)weight, eps, nullptr, 0, H,
-      (half_t*)x_out, (half_t*)h_out, nullptr, nullptr, 0, front_core::Outputs{}, twin);
+      (half_t*)x_out, (half_t*)h_out, nullptr, nullptr, 0, front_core::Outputs{}, twin, nullptr, 0);
   return sy_check_launch("combine_add_rmsnorm");
 }
 

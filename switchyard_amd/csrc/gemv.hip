@@ -29,6 +29,8 @@
 //
 // Replaces grouped_gemv_kernel / grouped_gemv of the reference
 // (switchyard/csrc/moe_kernels.cu:301-415); epilogue rounding points as :373-378.
+#include <type_traits>
+
 #include "sort_core.h"
 
 namespace {
@@ -77,7 +79,9 @@ struct Pass {
 
 // One wavefront streams units [unit0, unit0 + nunits) of one expert against NQ staged quads.
 // EXACT: K is a multiple of a chunk (512) and Nout of a unit (4), so nothing needs masking.
-// `behind_first` runs once, in every wavefront, when the first chunk has been asked for.
+// `behind_first` runs once, in every wavefront, when the first chunk has been asked for. Where there is
+// none, nothing stands between the check and the first load: the guarded load and the late return cost
+// every instance instructions and the gate/up ones two registers.
 struct Nothing {
   __device__ void operator()() const {}
 };
@@ -185,9 +189,14 @@ __device__ __forceinline__ void run_pass(const Pass& p, Behind behind_first = Be
   // chunk q+1 is in flight while chunk q is multiplied
   const int total = p.nunits * PARTS * p.nchunks;
   Chunk<CH> c0, c1;
-  if (total > 0) issue(c0);
-  behind_first();
-  if (total <= 0) return;
+  if constexpr (std::is_same<Behind, Nothing>::value) {
+    if (total <= 0) return;
+    issue(c0);
+  } else {
+    if (total > 0) issue(c0);
+    behind_first();
+    if (total <= 0) return;
+  }
   int q = 0;
   for (; q + 3 <= total; q += 2) {
     issue(c1);
