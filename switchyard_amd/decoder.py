@@ -274,7 +274,8 @@ class Decoder:
         in_one = self._own_moe and B * T > kernels.OWN_ROUTER_MAX_TOKENS and E.router_route_ok(B * T, s.hidden, s.experts, s.top_k)
         if in_one:
             scratch = E.moe_layer_scratch(B * T, s.experts, s.top_k, s.hidden, W["layers"][0]["down"].shape[2], x.device)
-            twin = E.padding_twins(tokens, span.real.contiguous()) if B > 1 and valid is not None and span.first == 0 else None
+            # (the cache's mask: bool and a row per sequence, whatever `valid` was)
+            twin = E.padding_twins(tokens, cache.real[:, :T].contiguous()) if B > 1 and valid is not None and span.first == 0 else None
         for i in range(s.layers):
             L = W["layers"][i]
             after = W["layers"][i + 1]["attn_norm"] if i + 1 < s.layers else W["final_norm"]

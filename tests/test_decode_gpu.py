@@ -598,6 +598,23 @@ def test_prefill_on_the_kernels_gives_the_cache_and_last_logits_of_the_torch_pre
     assert int((per_seq > 2e-2).sum()) <= max(1, B // 20) and per_seq.max().item() < 0.3, per_seq
 
 
+@pytest.mark.parametrize("dtype", [torch.int64, torch.uint8, torch.int32])
+@pytest.mark.parametrize("rows", [3, 1])
+def test_prefill_takes_a_mask_of_whole_numbers_and_one_for_all_rows(dtype, rows):
+    """A tokenizer's mask of zeros and ones, and one row for the whole batch, mean what a bool mask of
+    every row means (more than 64 tokens, where the padding goes through the experts once)."""
+    s, w, ps = model(7, 3)
+    dec = D.Decoder(s, w)
+    tokens = torch.randint(3, s.vocab, (3, 40), generator=torch.Generator().manual_seed(2)).cuda()
+    valid = torch.arange(40, device="cuda")[None] >= torch.tensor([[9], [0], [25]], device="cuda")[:rows]
+    outs = []
+    for v in (valid.expand(3, 40).contiguous(), valid.to(dtype)):
+        cache = D.KVCache(s, 3, 44, torch.float16, "cuda")
+        outs.append((dec.prefill_fused(tokens, cache, v), cache.k, cache.v, cache.real, cache.next_position))
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
+
+
 def test_generation_on_the_decode_kernels_picks_the_torch_models_tokens_up_to_ties():
     """Greedy decoding through `step_fused`; every picked token is the PyTorch-attention
     model's top-1 for the same prefix, or within the logits tolerance of it."""
