@@ -276,8 +276,12 @@ prefill_attention_kernel(const half_t* __restrict__ q, const half_t* __restrict_
   // ---- the lane holds columns 32 d + 8 g + 4 half + 0..3 of its query; after swapping with the lane 32
   // further on it holds 8 consecutive ones (group g of the lower half's two, g + 1 of the upper's)
   l += other_half(l);
-  const bool alone = l == 0.f;   // saw no key: the query takes its own value (a padding query; a real one sees itself)
-  const float inv = alone ? 0.f : 1.f / l;
+  // A query that saw no key takes its own value (a padding query; a real one sees itself). A sum of zero alone
+  // does not say so: scores of minus infinity leave it too, and their softmax is NaN.
+  bool alone = l == 0.f;
+  for (int i = 0, last = slot / ATT_KEYS; alone && i <= last; ++i)
+    alone = (i < last ? masks[i] : masks[i] & ((2ull << (slot - last * ATT_KEYS)) - 1)) == 0;
+  const float inv = 1.f / l;
   if (!wave_live) return;
   half_t* orow = out + ((size_t)b * T + tq) * ((size_t)heads * D) + (size_t)h * D;
   const half_t* own = vcache + cache_at + (size_t)slot * D;

@@ -292,6 +292,33 @@ def test_prefill_attention_of_shared_key_heads_keeps_32_bits(T, first, hd, kv_he
     assert (got != exact.half()).double().mean() < 1 / 128
 
 
+@pytest.mark.parametrize("T,first,hd,kv_heads", [(40, 0, 128, 4), (300, 0, 64, 4), (70, 1000, 128, 2), (1100, 0, 128, 4)])
+@pytest.mark.parametrize("bad", [math.inf, -math.inf, math.nan])
+def test_prefill_attention_keeps_what_is_not_finite(T, first, hd, kv_heads, bad):
+    """Queries that see an infinite or undefined score get what the softmax in 64 bits gives: NaN where the
+    largest score is infinite, the sum is undefined or every score is minus infinity, finite values
+    where only some scores are minus infinity; padding queries keep their own value."""
+    B, heads, n = 2, 4, first + T
+    q, kc, vc = rnd(B * T, heads * hd, seed=67).abs(), rnd(B, kv_heads, n + 3, hd, seed=68), rnd(B, kv_heads, n + 3, hd, seed=69)
+    pad = torch.tensor([0, n // 3])
+    real = torch.arange(n + 3)[None] >= pad[:, None]
+    kc[0, 0, 0, 3] = bad                  # the first key of all, alone for the query beside it
+    kc[1, -1, n // 3, 5] = bad            # the first real key behind the padding
+    kc[0, -1, n - 2, 1] = bad
+    got = kernels.ext().prefill_attention(q, kc, vc, real.cuda(), first, heads).view(B, T, heads, hd).transpose(1, 2).cpu()
+    qd = q.double().cpu().view(B, T, heads, hd).transpose(1, 2)
+    kd, vd = (t[:, :, :n].double().cpu().repeat_interleave(heads // kv_heads, 1) for t in (kc, vc))
+    s = (qd @ kd.transpose(-1, -2) / math.sqrt(hd)).masked_fill(~seen_by(real, first, T)[:, None], -math.inf)
+    want = s.softmax(-1) @ vd
+    assert torch.equal(got.isnan(), want.isnan())
+    # (behind a filled cache every query sees other keys too, whose scores are finite)
+    assert bool(want.isnan().any()) == (bad != -math.inf or first == 0) and bool(want.isfinite().any())
+    # finite results: half an ulp for each probability and for the result, as where every score is finite
+    spread = s.softmax(-1) @ vd.abs()
+    ok = want.isfinite()
+    assert ((got.double() - want).abs() <= ULP / 2 * (spread + want.abs()) * 1.05 + 1e-4)[ok].all()
+
+
 @pytest.mark.parametrize("B,heads,kv_heads,hd,cap,slot_at", [
     (8, 16, 16, 128, 640, 600),    # OLMoE at batch 8: 16 wavefronts per (sequence, head)
     (64, 16, 16, 128, 200, 199),   # many pairs: 4 wavefronts each; the last slot of the cache
