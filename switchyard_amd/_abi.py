@@ -855,9 +855,9 @@ class Ext:
     def decode_step(self, tok, weights, wqkv, cos, sin, positions, slot, real, kcache, vcache, heads, kv_heads, head_dim, k,
                     norm, eps, clip, gemv_max_rows):
         """One decode step of the whole model in one call: tok int64 [B] -> logits f16 [B, vocab]. weights:
-        the decoder's dictionary (embed, final_norm, lm_head, layers), wqkv: its stacked projections;
-        kcache, vcache [layers, B, kv_heads, capacity, D]. Every tensor is looked at in every call, and
-        its address is used for this call only."""
+        the decoder's dictionary (embed, final_norm, lm_head, layers, whose experts have one shape in
+        every layer), wqkv: its stacked projections; kcache, vcache [layers, B, kv_heads, capacity, D].
+        Every tensor is looked at in every call, and its address is used for this call only."""
         layers = weights["layers"]
         (B,), (n, _, _, capacity, D) = tok.shape, kcache.shape
         (vocab, H), (E, _), I = weights["embed"].shape, layers[0]["router"].shape, layers[0]["down"].shape[2]
@@ -866,12 +866,14 @@ class Ext:
         want = [(tok, i64, (B,)), (positions, i64, (B,)), (slot, i64, (1,)), (real, torch.bool, (B, capacity)),
                 (kcache, f16, (n, B, kv_heads, capacity, D)), (vcache, f16, (n, B, kv_heads, capacity, D)),
                 (cos, f16, (cos.shape[0], D)), (sin, f16, (cos.shape[0], D)), (weights["embed"], f16, (vocab, H)),
-                (weights["final_norm"], f16, (H,)), (weights["lm_head"], f16, (weights["lm_head"].shape[0], H))]
+                (weights["lm_head"], f16, (weights["lm_head"].shape[0], H))]
+        vectors = [(weights["final_norm"], H)]      # of any shape with that many entries
         for L, stack in zip(layers, wqkv):
-            want += [(stack, f16, (qd + 2 * kvd, H)), (L["q_norm"], f16, (qd,)), (L["k_norm"], f16, (kvd,)),
-                     (L["wo"], f16, (H, qd)), (L["attn_norm"], f16, (H,)), (L["mlp_norm"], f16, (H,)),
-                     (L["router"], f16, (E, H)), (L["gate_up"], f16, (E, 2 * I, H)), (L["down"], f16, (E, H, I))]
+            want += [(stack, f16, (qd + 2 * kvd, H)), (L["wo"], f16, (H, qd)), (L["router"], f16, (E, H)),
+                     (L["gate_up"], f16, (E, 2 * I, H)), (L["down"], f16, (E, H, I))]
+            vectors += [(L["q_norm"], qd), (L["k_norm"], kvd), (L["attn_norm"], H), (L["mlp_norm"], H)]
         device = tok.device
+        want += [(t, f16, t.shape if t.numel() == entries else (entries,)) for t, entries in vectors]
         for t, dtype, shape in want:
             if t.dtype != dtype or t.shape != shape or t.device != device or not t.is_contiguous():
                 raise RuntimeError(f"decode_step: a contiguous {dtype} GPU tensor {shape} was expected, got {t.dtype} "

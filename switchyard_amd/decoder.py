@@ -270,10 +270,12 @@ class Decoder:
         x, xn = E.embed_rmsnorm(tokens.reshape(-1), W["embed"], W["layers"][0]["attn_norm"], s.rms_eps)
         # The MoE layer, the residual add and the next norm are one call where the router's kernel takes
         # the shape; the padding of a batch that starts its cache then goes through the experts once
-        # instead of once per row
-        in_one = self._own_moe and B * T > kernels.OWN_ROUTER_MAX_TOKENS and E.router_route_ok(B * T, s.hidden, s.experts, s.top_k)
+        # instead of once per row. The layers share scratch for the largest of them
+        experts = max(L["router"].shape[0] for L in W["layers"])
+        in_one = self._own_moe and B * T > kernels.OWN_ROUTER_MAX_TOKENS and E.router_route_ok(B * T, s.hidden, experts, s.top_k)
         if in_one:
-            scratch = E.moe_layer_scratch(B * T, s.experts, s.top_k, s.hidden, W["layers"][0]["down"].shape[2], x.device)
+            widest = max(L["down"].shape[2] for L in W["layers"])
+            scratch = E.moe_layer_scratch(B * T, experts, s.top_k, s.hidden, widest, x.device)
             # (the cache's mask: bool and a row per sequence, whatever `valid` was)
             twin = E.padding_twins(tokens, cache.real[:, :T].contiguous()) if B > 1 and valid is not None and span.first == 0 else None
         for i in range(s.layers):
@@ -368,7 +370,7 @@ class Decoder:
         rows, width = tok.numel(), s.heads * s.head_dim
         if (self._own_moe and 1 <= rows <= E.STEP_MAX_ROWS and s.layers and s.experts <= 128 and s.top_k <= min(8, s.experts)
                 and max(s.hidden, width, W["layers"][0]["down"].shape[2]) <= 4096 and cache.k.is_contiguous()
-                and cache.v.is_contiguous()):
+                and cache.v.is_contiguous() and len({(L["router"].shape, L["down"].shape) for L in W["layers"]}) == 1):
             # few rows: every launch of the step from one call of the library (the host's share of a
             # launch made here is about as long as the launch)
             logits = E.decode_step(tok.reshape(-1), W, wqkv, self.cos, self.sin, positions.reshape(-1),

@@ -459,6 +459,49 @@ def test_a_step_in_one_call_equals_its_launches_one_by_one(B, kw, monkeypatch):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("B", [3, 12])
+def test_layers_of_different_sizes_and_norms_of_any_shape(B, monkeypatch):
+    """A model whose layers differ in the number and the width of their experts (pruned ones), with norms that
+    are no vectors: prompt and step as by the calls for each part."""
+    s, w, ps = model(7, B)
+    big = D.random_weights(D.Shape(**{**s.__dict__, "experts": 96, "intermediate": 384}), device="cuda", seed=8, std=0.05)["layers"]
+    w["layers"][1].update({n: big[1][n] for n in ("router", "gate_up", "down")})
+    for L in w["layers"]:
+        L.update({n: L[n][None] for n in ("attn_norm", "mlp_norm")}, q_norm=L["q_norm"].view(8, -1), k_norm=L["k_norm"].view(8, -1))
+    w["final_norm"] = w["final_norm"][None]
+    dec = D.Decoder(s, w)
+    tokens, valid = D.left_padded([p + list(range(3, 20)) for p in ps], "cuda")      # more than 64 tokens
+    outs = []
+    for apart in (False, True):
+        if apart:
+            monkeypatch.setattr(kernels.ext(), "STEP_MAX_ROWS", 0, raising=False)
+            monkeypatch.setattr(kernels, "OWN_ROUTER_MAX_TOKENS", 1 << 30)
+        cache = D.KVCache(s, B, tokens.shape[1] + 2, torch.float16, "cuda")
+        first = dec.prefill_fused(tokens, cache, valid)
+        slot = torch.tensor([cache.filled], device="cuda")
+        outs.append((first, dec.step_fused(first.argmax(-1)[:, None], cache, slot), cache.k, cache.v))
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
+
+
+def test_a_step_in_one_call_takes_norms_of_any_shape():
+    s, w, ps = model(7, 4)
+    outs = []
+    for shaped in (False, True):
+        if shaped:
+            for L in w["layers"]:
+                L.update({n: L[n][None] for n in ("attn_norm", "mlp_norm")}, q_norm=L["q_norm"].view(8, -1), k_norm=L["k_norm"].view(8, -1))
+            w["final_norm"] = w["final_norm"][None]
+        dec = D.Decoder(s, w)
+        tokens, valid = D.left_padded(ps, "cuda")
+        cache = D.KVCache(s, 4, tokens.shape[1] + 2, torch.float16, "cuda")
+        first = dec.prefill_fused(tokens, cache, valid)
+        slot = torch.tensor([cache.filled], device="cuda")
+        outs.append((first, dec.step_fused(first.argmax(-1)[:, None], cache, slot), cache.k, cache.v))
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
+
+
 def twins_reference(tokens, real):
     """What sy_padding_twins says, from its definition, one row at a time."""
     B, T = tokens.shape
