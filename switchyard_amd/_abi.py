@@ -108,6 +108,7 @@ SIGNATURES = {
                                                _c_int] + [_c_void_p] * 6),
     "sy_prefill_attention": (_c_int, [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int,
                                       _c_int, _c_int, _c_void_p, _c_void_p]),
+    "sy_prefill_attention_takes": (_c_int, [_c_int, _c_int, _c_int]),
     "sy_decode_attention": (_c_int, [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int,
                                      _c_int, _c_int, _c_void_p, _c_void_p]),
 }
@@ -763,6 +764,10 @@ class Ext:
                    slot.data_ptr(), B, rows // B, int(heads), int(kv_heads), D, kcache.shape[2], q.data_ptr(),
                    kcache.data_ptr(), vcache.data_ptr(), _stream())
         return q
+
+    def prefill_attention_ok(self, positions, capacity, head_dim):
+        """Whether prefill_attention takes this many positions of a cache of this capacity."""
+        return bool(self.lib.sy_prefill_attention_takes(int(positions), int(capacity), int(head_dim)))
 
     def prefill_attention(self, q, kcache, vcache, real, first, heads):
         """q [B*T, heads D] at cache positions first .. first + T - 1 of their sequences, against kcache

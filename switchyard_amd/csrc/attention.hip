@@ -308,12 +308,16 @@ prefill_attention_kernel(const half_t* __restrict__ q, const half_t* __restrict_
     }
 }
 
+// LDS of a launch over `positions` positions: two stages of keys and values, and a mask per tile
+size_t att_lds_bytes(int positions, int D) {
+  return (size_t)4 * ATT_KEYS * D * 2 + sizeof(uint64_t) * (((size_t)positions + ATT_KEYS - 1) / ATT_KEYS);
+}
+
 template <int D, int STEP, bool WIDE>
 int launch_prefill_attention(const half_t* q, const half_t* kc, const half_t* vc, const uint8_t* real, int first, int B, int T,
                              int heads, int kv_heads, int capacity, half_t* out, hipStream_t st) {
   const int pairs = B * heads, rows = ATT_WAVES * ATT_QROWS, nblocks = (T + rows - 1) / rows;
-  const size_t lds = (size_t)4 * ATT_KEYS * D * 2 + sizeof(uint64_t) * (size_t)((first + T + ATT_KEYS - 1) / ATT_KEYS);
-  SY_REQUIRE(lds <= 160 * 1024, "prefill_attention: %d positions are too many", first + T);
+  const size_t lds = att_lds_bytes(first + T, D);
   const auto kern = prefill_attention_kernel<D, STEP, WIDE>;
   if (lds > 48 * 1024 && hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
     return sy_fail(SY_ERR_LAUNCH, "prefill_attention: cannot reserve %zu bytes of LDS", lds);
@@ -342,6 +346,11 @@ int launch_steps(const half_t* q, const half_t* kc, const half_t* vc, const uint
 
 }  // namespace
 
+extern "C" SY_API int sy_prefill_attention_takes(int positions, int capacity, int D) {
+  return (D == 64 || D == 128) && positions >= 1 && positions <= capacity && (long)capacity * D * 2 < (1l << 31) &&
+         att_lds_bytes(positions, D) <= 160 * 1024;
+}
+
 extern "C" SY_API int sy_prefill_attention(const void* q, const void* kcache, const void* vcache, const uint8_t* real, int first,
                                            int B, int T, int heads, int kv_heads, int D, int capacity, void* out, void* stream) {
   SY_REQUIRE(B >= 0 && T >= 1 && heads >= 1 && kv_heads >= 1 && heads % kv_heads == 0,
@@ -349,7 +358,8 @@ extern "C" SY_API int sy_prefill_attention(const void* q, const void* kcache, co
   SY_REQUIRE(D == 64 || D == 128, "prefill_attention: head_dim must be 64 or 128 (got %d)", D);
   SY_REQUIRE(first >= 0 && capacity >= 1 && (long)first + T <= capacity, "prefill_attention: positions %d .. %ld of %d", first,
              (long)first + T - 1, capacity);
-  SY_REQUIRE((long)capacity * D * 2 < (1l << 31), "prefill_attention: a head's cache must stay under 2 GiB");
+  SY_REQUIRE(sy_prefill_attention_takes(first + T, capacity, D), "prefill_attention: %d positions of %d are too many", first + T,
+             capacity);
   if (B == 0) return SY_OK;
   SY_REQUIRE((long)B * heads * ((T + 127) / 128) < (1l << 31), "prefill_attention: too many queries (B = %d, heads = %d, T = %d)", B, heads, T);
   SY_REQUIRE(q && kcache && vcache && real && out, "prefill_attention: null pointer");

@@ -16,9 +16,13 @@ extern "C" {
  * marks real tokens. A query sees the real positions up to its own; one that would see none (left
  * padding) takes its own value -> out f16 [B*T, heads*D] (fp32 inside, probabilities rounded to
  * f16 for the value product). Query head h reads kv head h / (heads / kv_heads).
- * Limits: D is 64 or 128, first + T <= capacity. B == 0 is a no-op. */
+ * Limits: D is 64 or 128, first + T <= capacity, sy_prefill_attention_takes(). B == 0 is a no-op. */
 SY_API int sy_prefill_attention(const void* q, const void* kcache, const void* vcache, const uint8_t* real, int first,
                                 int B, int T, int heads, int kv_heads, int D, int capacity, void* out, void* stream);
+
+/* Whether sy_prefill_attention takes this many positions (the tiles' masks are held in LDS: 786 432 positions
+ * of 128, 1 048 576 of 64) of a cache of this capacity (a head's part under 2 GiB). */
+SY_API int sy_prefill_attention_takes(int positions, int capacity, int D);
 
 /* sy_decode_attention_qkv (include/switchyard_decode.h) with the keys of a (sequence, head) pair dealt to
  * four workgroups where the pairs are few and both buffers are given: parts f32 [B*heads, 16, D + 2] is

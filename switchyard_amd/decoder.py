@@ -278,12 +278,19 @@ class Decoder:
             scratch = E.moe_layer_scratch(B * T, experts, s.top_k, s.hidden, widest, x.device)
             # (the cache's mask: bool and a row per sequence, whatever `valid` was)
             twin = E.padding_twins(tokens, cache.real[:, :T].contiguous()) if B > 1 and valid is not None and span.first == 0 else None
+        own_attention = E.prefill_attention_ok(span.end, cache.k.shape[3], s.head_dim)   # some 780 000 positions
         for i in range(s.layers):
             L = W["layers"][i]
             after = W["layers"][i + 1]["attn_norm"] if i + 1 < s.layers else W["final_norm"]
             q = E.qk_norm_rope_cache(kernels.dense(xn, wqkv[i]), L["q_norm"], L["k_norm"], s.rms_eps, s.clip_qkv, self.cos,
                                      self.sin, flat_positions, slot, s.heads, s.kv_heads, s.head_dim, cache.k[i], cache.v[i])
-            a = E.prefill_attention(q, cache.k[i], cache.v[i], cache.real, span.first, s.heads)
+            if own_attention:
+                a = E.prefill_attention(q, cache.k[i], cache.v[i], cache.real, span.first, s.heads)
+            else:
+                a = F.scaled_dot_product_attention(q.view(B, T, s.heads, s.head_dim).transpose(1, 2),
+                                                   cache.k[i, :, :, :span.end], cache.v[i, :, :, :span.end],
+                                                   attn_mask=span.visible, enable_gqa=s.kv_heads != s.heads)
+                a = a.transpose(1, 2).reshape(B * T, s.heads * s.head_dim)
             o = kernels.dense(a, L["wo"])
             x, h = E.add_rmsnorm(x, o, L["mlp_norm"], s.rms_eps, x_out=x)
             if in_one:

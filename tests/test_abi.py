@@ -120,6 +120,18 @@ def test_argument_errors_are_reported_without_a_device(lib):
     assert lib.sy_sort_by_expert_static(None, None, 3, 4, 8, 64, None, None, None, None, None, None) == 1
 
 
+def test_the_prompts_attention_says_which_lengths_it_takes(lib):
+    takes = lib.sy_prefill_attention_takes
+    assert takes(1, 1, 128) and takes(4096, 4096, 64)
+    assert takes(786432, 786433, 128) and not takes(786433, 786433, 128)
+    assert takes(1048576, 1 << 23, 64) and not takes(1048577, 1 << 23, 64)
+    assert takes(5, (1 << 23) - 1, 128) and not takes(5, 1 << 23, 128)       # a head's cache of 2 GiB
+    assert not takes(0, 5, 128) and not takes(6, 5, 128) and not takes(5, 5, 96)
+    p = ctypes.c_void_p(256)     # refused before anything is launched
+    assert lib.sy_prefill_attention(p, p, p, p, 786400, 1, 33, 1, 1, 128, 800000, p, None) == 1
+    assert "too many" in lib.sy_last_error().decode()
+
+
 def test_empty_inputs_are_no_ops(lib):
     assert lib.sy_route(None, 0, 0, 64, 8, 0, None, None, None) == 0
     assert lib.sy_grouped_gemv(None, None, None, None, 64, 0, 0, 1024, 2048, 1, None, None, None) == 0

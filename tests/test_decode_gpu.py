@@ -502,6 +502,25 @@ def test_a_step_in_one_call_takes_norms_of_any_shape():
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("kw", [{}, {"kv_heads": 2}])
+def test_prefill_beyond_the_own_attentions_lengths(kw, monkeypatch):
+    """Where the prompt's attention does not take the length, PyTorch's call takes its place: the same
+    cache and logits to fp16 roundings (no router's tie here: the experts are few and all taken)."""
+    s, w, ps = model(7, 5, experts=4, top_k=4, **kw)
+    dec = D.Decoder(s, w)
+    tokens, valid = D.left_padded(ps, "cuda")
+    outs = []
+    for own in (True, False):
+        if not own:
+            monkeypatch.setattr(kernels.ext(), "prefill_attention_ok", lambda *a: False, raising=False)
+            monkeypatch.setattr(kernels.ext(), "prefill_attention", None, raising=False)
+        cache = D.KVCache(s, 5, tokens.shape[1] + 5, torch.float16, "cuda")
+        first = dec.prefill_fused(tokens, cache, valid)
+        outs.append((first, dec.prefill_fused(tokens[:, :3], cache), cache.k * cache.real[None, :, None, :, None], cache.real))
+    for a, b in zip(*outs):
+        assert (a.float() - b.float()).abs().max() <= 2e-2
+
+
 def twins_reference(tokens, real):
     """What sy_padding_twins says, from its definition, one row at a time."""
     B, T = tokens.shape
