@@ -201,7 +201,7 @@ def test_qk_norm_rope_cache(B, heads, kv_heads, hd, clip):
     (2, 1, 0, 4, 4, 128), (1, 1, 64, 1, 1, 64),                     # one query; one behind a whole tile of keys
     (2, 31, 0, 4, 2, 64), (2, 33, 0, 4, 4, 128), (1, 64, 0, 2, 2, 128), (1, 65, 63, 2, 1, 64),   # edges of the tiles
     (3, 127, 5, 8, 8, 128), (2, 129, 200, 16, 4, 64),               # behind a filled cache
-    (8, 300, 0, 16, 16, 128),                                       # 128 queries per workgroup (many pairs)
+    (8, 300, 0, 16, 16, 128),                                       # many pairs, three workgroups of 128 queries each
     (1, 437, 0, 16, 16, 128), (2, 1100, 1000, 16, 2, 64)])
 @pytest.mark.parametrize("holes", [False, True])
 def test_prefill_attention(B, T, first, heads, kv_heads, hd, holes):
@@ -290,6 +290,39 @@ def test_prefill_attention_of_shared_key_heads_keeps_32_bits(T, first, hd, kv_he
     # an error of 2^-18 of a result's terms (scores of up to 30 in fp32: 2^-19; probabilities of 22 bits) against
     # a rounding that moves in steps of 2^-10 or 2^-11 of the result: at most 1 result in 128 is rounded the other way
     assert (got != exact.half()).double().mean() < 1 / 128
+
+
+@pytest.mark.parametrize("T,first,hd,kv_heads", [(200, 0, 128, 4), (300, 0, 64, 4), (300, 0, 128, 2), (300, 900, 64, 2),
+                                                 (40, 1400, 128, 4), (1100, 0, 128, 4)])
+@pytest.mark.parametrize("grow", [7.5, 8.5, 30.0])
+def test_prefill_attention_of_growing_scores(T, first, hd, kv_heads, grow):
+    """Scores of half of the queries that grow by `grow` powers of two from one block of 64 keys to the next (up
+    to six times, then they stay), those of the other half that do not grow, mixed in every wavefront: the
+    output and the sum so far are rescaled by anything from 2^-7.5 to 2^-30 for some lanes and by 1 for others."""
+    B, heads, n = 2, 4, first + T
+    start = max(0, first // 64 - 2) * 64                     # the growth begins two blocks in front of the queries
+    level = ((torch.arange(n + 3) - start).clamp(min=0) // 64).clamp(max=6).float()
+    q = rnd(B * T, heads * hd, seed=71).cpu().view(B, T, heads, hd)
+    kc, vc = rnd(B, kv_heads, n + 3, hd, seed=72).cpu(), rnd(B, kv_heads, n + 3, hd, seed=73)
+    # dimensions 0 .. 7 carry the growth: 8 times the same product, zero for every second query
+    to_score = math.log2(math.e) / math.sqrt(hd)             # of the sum, in powers of two
+    q[..., :8] = 4.0 * (torch.arange(T) % 2).half()[None, :, None, None]
+    kc[..., :8] = (level * grow / (8 * 4.0 * to_score)).half()[None, None, :, None]
+    real = torch.arange(n + 3)[None] >= torch.tensor([[0], [n // 3]])
+    got = kernels.ext().prefill_attention(q.reshape(B * T, -1).contiguous().cuda(), kc.cuda(), vc, real.cuda(), first, heads)
+    got = got.view(B, T, heads, hd).transpose(1, 2).cpu()
+    qd = q.double().transpose(1, 2)
+    kd, vd = (t[:, :, :n].double().cpu().repeat_interleave(heads // kv_heads, 1) for t in (kc, vc))
+    s = (qd @ kd.transpose(-1, -2) / math.sqrt(hd)).masked_fill(~seen_by(real, first, T)[:, None], -math.inf)
+    # the maximum of each block of 64 keys against that of all blocks before it, in powers of two
+    blocks = F.pad(s, (0, -n % 64), value=-math.inf).unflatten(-1, (-1, 64)).amax(-1) * math.log2(math.e)
+    rise = (blocks[..., 1:] - blocks.cummax(-1).values[..., :-1])[torch.isfinite(blocks[..., :-1]) & torch.isfinite(blocks[..., 1:])]
+    assert (rise > grow - 4).double().mean() > 0.03 and (rise < 1).double().mean() > 0.2
+    exact, spread = s.softmax(-1) @ vd, s.softmax(-1) @ vd.abs()
+    # each probability is rounded to f16 once (half an ulp of itself, or of 2^-14 of the largest, of which n keys may
+    # be that small), and so is the result; scores of up to 200 in fp32 are off by 2^-16, their probabilities as much
+    bound = (ULP / 2 * (spread + exact.abs()) * 1.05 + n * 2.0 ** -25 * vd.abs().amax() + 2.0 ** -15 * spread + 1e-6)
+    assert ((got.double() - exact).abs() <= bound).all(), ((got.double() - exact).abs() - bound).max()
 
 
 @pytest.mark.parametrize("T,first,hd,kv_heads", [(40, 0, 128, 4), (300, 0, 64, 4), (70, 1000, 128, 2), (1100, 0, 128, 4)])
@@ -389,36 +422,38 @@ def test_attention_with_the_norm_and_rotary_in_its_prologue(B, heads, kv_heads, 
 
 
 @pytest.mark.parametrize("B,heads,kv_heads,hd,cap,slot_at", [
-    (1, 16, 16, 128, 732, 700), (8, 16, 16, 128, 544, 512), (3, 8, 2, 64, 77, 50),   # 16, 4 and 4 workgroups per pair
+    (1, 16, 16, 128, 732, 700), (8, 16, 16, 128, 544, 512), (3, 8, 2, 64, 77, 50),   # four workgroups per pair
     (2, 4, 4, 128, 9, 0), (1, 16, 16, 64, 40, 5), (1, 4, 1, 128, 70, 63),            # fewer keys than wavefronts
     (31, 16, 16, 128, 1100, 1030), (1, 2, 2, 128, 4100, 4099), (2, 8, 8, 64, 2000, 1999),   # many batches each
     (5, 20, 4, 128, 300, 299),                                                       # rows of 2560: a fifth wavefront's sum
     (2, 4, 4, 64, 10, 10)])                                                          # a slot past the cache
 def test_attention_over_several_workgroups(B, heads, kv_heads, hd, cap, slot_at):
     """The keys of a pair dealt to several workgroups against one workgroup: the same cache and the
-    same output, bit for bit; the tickets are back at zero, so the buffers serve the next launch;
-    rows of padding up to the slot (no real key but the new one) among them."""
+    same output, bit for bit; the tickets are back at zero, so the buffers serve the next launch, which
+    has other inputs, so that what an earlier one left there would show; rows of padding up to the
+    slot (no real key but the new one) among them."""
     ext, max_pos = kernels.ext(), 700
     g = torch.Generator().manual_seed(31)
-    qkv = rnd(B, (heads + 2 * kv_heads) * hd, seed=32, std=0.7)
     qn, kn = 1 + rnd(heads * hd, seed=33, std=0.1), 1 + rnd(kv_heads * hd, seed=34, std=0.1)
     cos, sin = rnd(max_pos, hd, seed=35, std=0.5), rnd(max_pos, hd, seed=36, std=0.5)
-    positions = torch.randint(0, max_pos, (B,), generator=g).cuda()
-    slot = torch.tensor([slot_at], device="cuda")
-    pad = torch.randint(0, slot_at + 1, (B,), generator=g)
-    pad[0], pad[B // 2] = 0, slot_at
-    real = ((torch.arange(cap)[None] >= pad[:, None]) & (torch.rand(B, cap, generator=g) > 0.2)).cuda()
-    kc, vc = rnd(B, kv_heads, cap, hd, seed=37), rnd(B, kv_heads, cap, hd, seed=38)
     split = ext.attention_split(2, B, heads, hd, "cuda")
     assert split is not None
-    results = []
-    for share in (None, (split[0], split[1][0]), (split[0], split[1][0]), (split[0], split[1][1])):
-        k, v, r = kc.clone(), vc.clone(), real.clone()
-        out = ext.decode_attention_qkv(qkv, qn, kn, 1e-5, None, cos, sin, positions, slot, r, heads, kv_heads, hd, k, v, share)
-        results.append((out, k, v, r))
-        assert not split[1].any()
-    want = results[0]
-    for got in results[1:]:
+    split[0].fill_(math.nan)
+    for launch, at in enumerate((slot_at, slot_at * 3 // 4, slot_at)):
+        qkv = rnd(B, (heads + 2 * kv_heads) * hd, seed=32 + 10 * launch, std=0.7)
+        kc, vc = rnd(B, kv_heads, cap, hd, seed=37 + 10 * launch), rnd(B, kv_heads, cap, hd, seed=38 + 10 * launch)
+        positions = torch.randint(0, max_pos, (B,), generator=g).cuda()
+        slot = torch.tensor([at], device="cuda")
+        pad = torch.randint(0, at + 1, (B,), generator=g)
+        pad[(B // 2 + launch) % B], pad[launch % B] = at, 0      # (one sequence: its keys are all real but for holes)
+        real = ((torch.arange(cap)[None] >= pad[:, None]) & (torch.rand(B, cap, generator=g) > 0.2)).cuda()
+        results = []
+        for share in (None, (split[0], split[1][launch // 2])):      # the row of tickets of the launch before, then another
+            k, v, r = kc.clone(), vc.clone(), real.clone()
+            out = ext.decode_attention_qkv(qkv, qn, kn, 1e-5, None, cos, sin, positions, slot, r, heads, kv_heads, hd, k, v, share)
+            results.append((out, k, v, r))
+            assert not split[1].any()
+        want, got = results
         assert torch.equal(got[1].view(torch.int16), want[1].view(torch.int16)) and torch.equal(got[3], want[3])
         assert torch.equal(got[2].view(torch.int16), want[2].view(torch.int16))
         assert torch.equal(got[0], want[0])
