@@ -421,10 +421,10 @@ struct KeyBatch {
 // Batches in front of the sequence's first real key (left padding) are not read: every wavefront looks
 // for that key in the mask itself. At 64 sequences of 288 to 576 keys, 16 heads: 52.6 us a launch with them,
 // 45.6 without.
-// NW < LW: the pair's wavefronts are dealt to LW / NW workgroups, because what one compute unit can
-// have in flight (about 10 KB, a microsecond away) takes a while over a pair's keys and values: 17.2
-// -> 14.6 us for one sequence of 700 keys, 15.5 -> 14.7 for 8 of 256 to 512 (16 workgroups of one
-// wavefront, each with the whole of the norms to do: 16.0 for one sequence).
+// NW < LW: the pair's wavefronts are dealt to LW / NW workgroups, so that a pair's keys and values (358 KB
+// at 700 keys of 128) come through four compute units and not one: 17.2 -> 14.6 us for one sequence of
+// 700 keys, 15.5 -> 14.7 for 8 of 256 to 512 (16 workgroups of one wavefront, each with the whole of
+// the norms to do: 16.0 for one sequence).
 // Every workgroup leaves its wavefronts' results in `parts` and draws a number from the pair's
 // ticket; the one that draws the last merges them, as a workgroup of LW wavefronts would have done (the
 // same bits), and sets the ticket back to zero. Nobody waits for anybody. The results travel by

@@ -1,7 +1,8 @@
 // grouped_gemm: the prefill path. Every expert's slice of the sorted rows goes through that
 // expert's weights on fp16 MFMA tiles, all experts in one launch. Three tiles, chosen by the
-// host from the mean rows per expert: 64 or 128 rows (gemm_kernel, below) for a few rows per
-// expert, 256 rows (gemm_stream_kernel, further down) above 32.
+// host from the mean rows per expert: 64 rows (gemm_kernel, below) up to 32 rows per expert, 256
+// rows (gemm_stream_kernel, further down) above. 128 rows (gemm_kernel) are for shapes that the
+// 256-row tile does not take.
 //
 // gemm_kernel. Tile: 64*MI rows x 256 weight rows (MI = 1 or 2), K in slices of 64, 4 wavefronts, each computing
 // all of the tile's rows x 64 weight rows as (2*MI) x 2 v_mfma_f32_32x32x16_f16 blocks with fp32
@@ -936,19 +937,23 @@ int launch_gemm(const half_t* a, const int32_t* a_rows, const half_t* b, const i
 
 }  // namespace
 
-// Rows per tile: 256 above 32 rows per expert; up to that 64 while the typical busiest expert (under
-// near-uniform routing an expert's rows scatter around the mean by about its square root) fits in
-// one such tile, else 128.
+// Rows per tile. Where the 256-row tile takes the shape: 256 above 32 rows per expert, 64 up to that. Its
+// loads run three slices ahead, into the next tile, so it wants K in whole slices and four of them;
+// its tile table is one or two experts per lane, 128 in all. Other shapes: 64 while the typical
+// busiest expert (under near-uniform routing an expert's rows scatter around the mean by about its
+// square root) fits in one such tile, else 128.
 //
 // What decides is the tail. The small tiles run two workgroups a compute unit, one tile each, and
 // evenly routed tokens make exactly one round of them: 64 experts x 8 column tiles. Routing is not
 // even behind a trained router, and the row tiles of popular experts then make a second round that
 // is nearly empty. The 256-row tile has one row tile for almost any expert, and deals its list to
 // resident workgroups by height. The layer, us, small tiles -> 256-row tile, with a Zipf bias (exponent
-// 1.1) / evenly routed: 257 tokens 184 -> 147 / 151 -> 154, 333 tokens 190 -> 153 / 153 -> 156, 437 tokens
-// 225 -> 175 / 158 -> 160, 600 tokens 244 -> 183 / 169 -> 169, 768 tokens 265 -> 191 / 179 -> 174; but 160 tokens
-// 146 -> 141 / 143 -> 147, and 96 tokens 130 -> 136 / 140 -> 143. Its loads run three slices ahead, into the
-// next tile, so it wants four slices of K; its tile table is one or two experts per lane.
+// 1.1) / evenly routed: 257 tokens 182 -> 147 / 149 -> 153, 333 tokens 193 -> 152 / 153 -> 156, 437 tokens
+// 218 -> 178 / 158 -> 161, 600 tokens 228 -> 185 / 168 -> 170, 768 tokens 265 -> 191 / 179 -> 174; but 160 tokens
+// 146 -> 141 / 143 -> 147, and 96 tokens 130 -> 136 / 140 -> 143. So even routing pays 1.5 to 2.7 % at 257 to
+// 600 tokens, in both projections alike, for 20 % where it is uneven; only the device knows which it is.
+// `rows` counts every choice, also those of padding that the sort passes over: a batch of prompts that
+// is mostly padding takes the larger tile from fewer real rows on.
 int sy_gemm_rows_per_tile(int rows, int E, int K) {
   const int mean = (rows + E - 1) / E;
   const bool stream_ok = K % BIG_BK == 0 && K / BIG_BK >= 4 && E <= 2 * WAVE;

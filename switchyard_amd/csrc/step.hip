@@ -2,14 +2,14 @@
 // layer by layer (switchyard_amd/decoder.py), enqueued here back to back. There is no kernel in this
 // file.
 //
-// Why: a step of one sequence is 115 launches of 3 to 16 us, and from Python each costs the host about
+// Why: a step of one sequence is 114 launches of 3 to 16 us, and from Python each costs the host about
 // 13 us (the checks, the allocation of its outputs, the marshalling): 1467 us to enqueue a step, now
 // 527, and one sequence's step behind 700 positions takes 1134 us where it took 1299.
 //
-// What the launches are, per layer: q/k/v projection (a weight stream), attention with the q/k norm, the rotary embedding and the cache write in its prologue, output
-// projection, residual add + norm + router logits + route (+ sort), gate/up, down, and combine +
-// residual add + the next norm. Up to 64 choices (8 tokens of top-8) the front only routes and
-// the gate/up stream sorts for itself, as in sy_moe_layer.
+// What the launches are, per layer: q/k/v projection (a weight stream), attention with the q/k norm, the
+// rotary embedding and the cache write in its prologue, output projection, residual add + norm + router
+// logits + route (+ sort), gate/up, down, and combine + residual add + the next norm. Up to 64 choices
+// (8 tokens of top-8) the front only routes and the gate/up stream sorts for itself, as in sy_moe_layer.
 #include "common.h"
 #include "../../include/switchyard_decode.h"
 #include "passes.h"

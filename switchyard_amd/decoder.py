@@ -1,9 +1,9 @@
 """An OLMoE decoder around the MoE layer: the caller of the hot path.
 
 Counterpart of the reference's switchyard/model.py (the `self.moe(i, h)` hook at :39-42,135)
-and of the tensor layout its weights.py defines (:36-69). Attention stays in PyTorch; every
-mixture-of-experts layer goes through `moe(layer_index, h[B*T, H]) -> [B*T, H]`, which by
-default is `kernels.moe_layer` on the layer's router / gate_up / down tensors.
+and of the tensor layout its weights.py defines (:36-69). Every mixture-of-experts layer goes
+through `moe(layer_index, h[B*T, H]) -> [B*T, H]`, which by default is `kernels.moe_layer` on the
+layer's router / gate_up / down tensors.
 
 Built for decode on one GPU: the KV cache is allocated once for the whole generation, rotary
 tables are precomputed, and the greedy loop keeps its tokens on the device, so a decode step
@@ -182,9 +182,8 @@ class KVCache:
 
 class Decoder:
     def __init__(self, shape, weights, moe=None, max_positions=4096, attention="auto"):
-        """attention: "kernels" (the library's kernels for the decode step and around the prompt's
-        attention), "torch" (PyTorch operators throughout), or "auto": kernels where they apply
-        (GPU, fp16, head_dim 64 or 128)."""
+        """attention: "kernels" (the library's kernels for the decode step and for prompts), "torch"
+        (PyTorch operators throughout), or "auto": kernels where they apply (GPU, fp16, head_dim 64 or 128)."""
         self.s, self.w = shape, weights
         self.moe = moe or self.kernel_moe
         self._own_moe = moe is None     # the step may then fold the layer's ends into its neighbours

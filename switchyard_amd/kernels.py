@@ -132,8 +132,8 @@ def experts(h, idx, w, gate_up, down, mode="auto"):
 def dense(x, weight):
     """x [rows, K] @ weight [Nout, K]^T for the projections around the MoE layer at decode
     (q/k/v, output, lm_head), which are weight streams like the experts are. Up to 16 rows the
-    weight-stream kernel runs with a single expert that owns every row (one pass over the
-    matrix; measured in a replayed graph at 8 rows: 9.7 us for [6144, 2048], 6.8 us for
+    weight-stream kernel runs in its form for one matrix and rows in their own order (one pass over
+    the matrix; measured in a replayed graph at 8 rows: 9.7 us for [6144, 2048], 6.8 us for
     [2048, 2048], 36.9 us for [50304, 2048], against 12.4, 8.8 and 52.9 us for the library
     GEMM). Above that a plain GEMM is the library's job (12.5 us at 64 rows where the kernel's
     four passes take 33.6 us)."""
