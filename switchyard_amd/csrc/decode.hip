@@ -32,6 +32,7 @@
 // the scores to fp16 first), which is the more exact of the two.
 #include <mutex>
 
+#include "combine_core.h"
 #include "common.h"
 #include "front_core.h"
 #include "../../include/switchyard_decode.h"
@@ -53,6 +54,18 @@ __device__ __forceinline__ float block_sum(float v, float* lds, int slot_base) {
   return total;
 }
 
+// The same where the values are those of the workgroup's first four wavefronts (the others' are zero): one
+// read of four sums, not a loop over them.
+__device__ __forceinline__ float block_sum_of_four(float v, float* lds) {
+  v = wave_sum(v);
+  const int wave = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0 && wave < 4) lds[wave] = v;
+  __syncthreads();
+  const float4_t p = *reinterpret_cast<const float4_t*>(lds);
+  return p[0] + p[1] + p[2] + p[3];
+}
+
+constexpr int FEW_ROWS = 64;   // up to these the row kernels are built for a short chain of waits, not for many wavefronts
 constexpr int ROW_MAX_K = 64;  // choices per token the combining variant ranks in one wavefront
 
 // One workgroup per token (row). The residual `delta` is either a tensor, or (COMBINE) the
@@ -72,9 +85,13 @@ constexpr int ROW_MAX_K = 64;  // choices per token the combining variant ranks 
 // instructions, and the logits one a wavefront of occupancy): EMBEDDED looks row t up in x by gather[t], and
 // its first workgroup sets the `nclear` counters at `clear` to zero for the launches behind it; TWINNED
 // (with COMBINE) takes the expert outputs of token twin[t] (front.hip).
+// FEW (with COMBINE): a launch of few rows is a chain of waits. The norm's weights and the row are asked for
+// first, and a token's choices are ranked without LDS and their rows of y asked for together (combine_core.h):
+// one row 5.2 -> 4.4 us a launch, 8 rows 5.6 -> 5.0. It takes 26 more registers, and with many rows it is
+// the wavefronts in flight that count: 437 rows 6.7 -> 7.3, 4096 rows 31.9 -> 33.2.
 constexpr int FRONT_ROUTE = 1, FRONT_SORT = 2;
 constexpr int OWN_ROWS = 0, EMBEDDED = 1, TWINNED = 2;
-template <bool COMBINE, bool LOGITS, int FRONT = 0, int FROM = OWN_ROWS>
+template <bool COMBINE, bool LOGITS, int FRONT = 0, int FROM = OWN_ROWS, bool FEW = false>
 __global__ void __launch_bounds__(LOGITS ? 1024 : ROW_THREADS)
 row_kernel(const half_t* x, const half_t* __restrict__ delta, const half_t* __restrict__ y,
            const int* __restrict__ pos_of, const int* __restrict__ idx, int k, const half_t* __restrict__ weight,
@@ -83,12 +100,25 @@ row_kernel(const half_t* x, const half_t* __restrict__ delta, const half_t* __re
            front_core::Outputs front = front_core::Outputs{}, const int* __restrict__ twin = nullptr,
            unsigned* __restrict__ clear = nullptr, int nclear = 0) {  // x_out may be x
   extern __shared__ __attribute__((aligned(16))) half_t hs[];  // LOGITS: the normalised row [H]; FRONT: the tail's LDS behind it
-  __shared__ float part[16];
+  __shared__ __attribute__((aligned(16))) float part[16];
   __shared__ int rows[ROW_MAX_K];
   __shared__ float wts[ROW_MAX_K];   // COMBINE: the router weight of each row, 1 where y is already scaled
   const int t = blockIdx.x, tid = threadIdx.x, nthreads = blockDim.x;
   const size_t row = (size_t)t * H;
   const int chunks = H >> 3;
+  half8_t v[MAX_CHUNKS], wn[MAX_CHUNKS];
+  combine_core::Choices own;
+  if (FEW) {
+#pragma unroll
+    for (int i = 0; i < MAX_CHUNKS; ++i) {
+      const int c = tid + i * nthreads;
+      if (c < chunks) {
+        wn[i] = *reinterpret_cast<const half8_t*>(weight + c * 8);
+        v[i] = *reinterpret_cast<const half8_t*>(x + row + c * 8);
+      }
+    }
+    own = combine_core::ranked(idx, pos_of, delta, (size_t)t * k, k);
+  }
   const half_t* xrow = x + row;
   if (FROM == EMBEDDED) {
     long g = (long)gather[t];
@@ -97,7 +127,7 @@ row_kernel(const half_t* x, const half_t* __restrict__ delta, const half_t* __re
     if (t == 0)
       for (int i = tid; i < nclear; i += nthreads) clear[i] = 0;
   }
-  if (COMBINE) {
+  if (COMBINE && !FEW) {
     // rank the k choices by (expert id, slot); rows[] lists their rows of y in that order
     if (tid < WAVE) {
       const int of = FROM == TWINNED ? twin[t] : t;
@@ -115,21 +145,29 @@ row_kernel(const half_t* x, const half_t* __restrict__ delta, const half_t* __re
     }
     __syncthreads();
   }
-  half8_t v[MAX_CHUNKS];
   float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < MAX_CHUNKS; ++i) {
     const int c = tid + i * nthreads;
     if (c < chunks) {
-      v[i] = *reinterpret_cast<const half8_t*>(xrow + c * 8);
+      if (!FEW) v[i] = *reinterpret_cast<const half8_t*>(xrow + c * 8);
       if (COMBINE) {
         float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        for (int j = 0; j < k; ++j) {
-          const half8_t e = __builtin_nontemporal_load(reinterpret_cast<const half8_t*>(y + (size_t)rows[j] * H + c * 8));   // read once
-          const float wt = wts[j];
-          // the rounding of the down projection's scaled epilogue (times 1 it changes nothing)
+        auto fetch = [&](int r) { return __builtin_nontemporal_load(reinterpret_cast<const half8_t*>(y + (size_t)r * H + c * 8)); };   // read once
+        // the rounding of the down projection's scaled epilogue (times 1 it changes nothing)
+        auto add = [&](half8_t e, float wt) {
 #pragma unroll
           for (int q = 0; q < 8; ++q) acc[q] += (float)(half_t)((float)e[q] * wt);
+        };
+        if (FEW) {
+          half8_t e[combine_core::AT_ONCE];
+#pragma unroll
+          for (int j = 0; j < combine_core::AT_ONCE; ++j) e[j] = fetch(own.row[j]);
+#pragma unroll
+          for (int j = 0; j < combine_core::AT_ONCE; ++j)
+            if (j < k) add(e[j], own.weight[j]);
+        } else {
+          for (int j = 0; j < k; ++j) add(fetch(rows[j]), wts[j]);
         }
 #pragma unroll
         for (int q = 0; q < 8; ++q) v[i][q] = (half_t)((float)v[i][q] + (float)(half_t)acc[q]);
@@ -150,12 +188,12 @@ row_kernel(const half_t* x, const half_t* __restrict__ delta, const half_t* __re
       if (c < chunks) *reinterpret_cast<half8_t*>(hs + c * 8) = v[i];
     }
   } else {
-    const float rs = rsqrtf(block_sum(ss, part, 0) / (float)H + eps);
+    const float rs = rsqrtf((FEW ? block_sum_of_four(ss, part) : block_sum(ss, part, 0)) / (float)H + eps);
 #pragma unroll
     for (int i = 0; i < MAX_CHUNKS; ++i) {
       const int c = tid + i * nthreads;
       if (c < chunks) {
-        const half8_t w = *reinterpret_cast<const half8_t*>(weight + c * 8);
+        const half8_t w = FEW ? wn[i] : *reinterpret_cast<const half8_t*>(weight + c * 8);
         half8_t h;
 #pragma unroll
         for (int j = 0; j < 8; ++j) h[j] = (half_t)((float)w[j] * (float)(half_t)((float)v[i][j] * rs));
@@ -953,7 +991,8 @@ int sy_combine_add_rmsnorm_twins(const void* y, const int32_t* pos_of, const int
   SY_REQUIRE(k >= 1 && k <= ROW_MAX_K, "combine_add_rmsnorm: 1 <= k <= %d (got %d)", ROW_MAX_K, k);
   if (N == 0) return SY_OK;
   SY_REQUIRE(y && pos_of && idx && x && weight && h_out, "combine_add_rmsnorm: null pointer");
-  auto kern = twin ? row_kernel<true, false, 0, TWINNED> : row_kernel<true, false>;
+  auto kern = twin ? row_kernel<true, false, 0, TWINNED>
+              : N <= FEW_ROWS && k <= combine_core::AT_ONCE ? row_kernel<true, false, 0, OWN_ROWS, true> : row_kernel<true, false>;
   kern<<<N, ROW_THREADS, 0, (hipStream_t)stream>>>(
       (const half_t*)x, (const half_t*)w, (const half_t*)y, pos_of, idx, k, (const half_t*)weight, eps, nullptr, 0, H,
       (half_t*)x_out, (half_t*)h_out, nullptr, nullptr, 0, front_core::Outputs{}, twin, nullptr, 0);

@@ -105,6 +105,23 @@ def test_combine_add_rmsnorm(N, H, E, k):
     assert xo3 is x3 and torch.equal(x3, xo) and torch.equal(h3, h)
 
 
+@pytest.mark.parametrize("N", [1, 64, 65])   # 64: the last of the launches for few rows
+@pytest.mark.parametrize("H,k", [(8, 1), (2048, 3), (2056, 8), (8192, 8), (512, 9)])   # 9: more choices than are ranked in registers
+def test_combine_add_rmsnorm_of_few_rows(N, H, k):
+    """The rows in any order of ids, ids that repeat inside a token among them: the bits of the two launches."""
+    E = 16
+    g = torch.Generator().manual_seed(N + H + k)
+    idx = torch.randint(E, (N, k), generator=g, dtype=torch.int32).cuda()
+    wts = torch.rand(N, k, generator=g).half().cuda()
+    ext = kernels.ext()
+    _, _, _, wsorted, pos_of = ext.sort_by_expert(idx, wts, E)
+    y, x, w = rnd(N * k, H, seed=6), rnd(N, H, seed=7), 1 + rnd(H, seed=8, std=0.1)
+    scaled = (y.float() * wsorted.float()[:, None]).half()
+    want = ext.add_rmsnorm(x, ext.combine(scaled, pos_of, idx, N), w, 1e-5)
+    got = ext.combine_add_rmsnorm(y, pos_of, idx, x, w, 1e-5, w=wts)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
 @pytest.mark.parametrize("N,H,vocab", [(8, 2048, 50304), (64, 2048, 50304), (3, 64, 10), (1, 520, 77)])
 def test_embed_rmsnorm(N, H, vocab):
     """The embedding rows bit for bit, their norm as add_rmsnorm gives it; ids outside the table are clamped."""
