@@ -71,6 +71,7 @@ struct Chunk {
 
 struct Pass {
   const half_t* xs;             // staged rows
+  const int* rows;              // GATHERED: which staged row each of the pass's rows is
   __amdgpu_buffer_rsrc_t rsrc;  // the expert's weight matrix
   const half_t* scale;
   half_t* C;
@@ -85,7 +86,9 @@ struct Pass {
 struct Nothing {
   __device__ void operator()() const {}
 };
-template <bool SWIGLU, bool SCALE, bool EXACT, int CH, int NQ, typename Behind = Nothing>
+// GATHERED: the pass's rows are anywhere among the staged ones (rows past the last read the last one's: the
+// columns of the MFMA do not mix).
+template <bool SWIGLU, bool SCALE, bool EXACT, int CH, int NQ, bool GATHERED = false, typename Behind = Nothing>
 __device__ __forceinline__ void run_pass(const Pass& p, Behind behind_first = Behind{}) {
   const int lane = threadIdx.x & 63, blk = lane >> 2, sub = lane & 3;
   const int klane = blk * 8;
@@ -129,7 +132,12 @@ __device__ __forceinline__ void run_pass(const Pass& p, Behind behind_first = Be
   float4_t acc[NQ], gate[NQ];
 #pragma unroll
   for (int q = 0; q < NQ; ++q) acc[q] = gate[q] = float4_t{0.f, 0.f, 0.f, 0.f};
-  const half_t* xlane = p.xs + sub * p.RS + klane;  // row `sub` of quad 0 at this lane's K offset
+  const half_t* xlane[NQ];   // row `sub` of each quad at this lane's K offset
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    const int r = q * QUAD + sub;
+    xlane[q] = p.xs + (GATHERED ? p.rows[min(r, p.nr - 1)] : r) * p.RS + klane;
+  }
 
   auto compute = [&](const Chunk<CH>& c) {
 #pragma unroll
@@ -138,7 +146,7 @@ __device__ __forceinline__ void run_pass(const Pass& p, Behind behind_first = Be
       const int kk = (at - (at >= nsteps ? nsteps : 0)) * STEP_K;
 #pragma unroll
       for (int q = 0; q < NQ; ++q) {
-        half8_t x = *reinterpret_cast<const half8_t*>(xlane + q * QUAD * p.RS + kk);
+        half8_t x = *reinterpret_cast<const half8_t*>(xlane[q] + kk);
         if (!EXACT && kk + klane >= p.K) x = zero8;  // the weights are 0 there; keep stale LDS out
         acc[q] = __builtin_amdgcn_mfma_f32_4x4x4f16(lo4(c.w[s]), lo4(x), acc[q], 0, 0, 0);
         acc[q] = __builtin_amdgcn_mfma_f32_4x4x4f16(hi4(c.w[s]), hi4(x), acc[q], 0, 0, 0);
@@ -227,7 +235,7 @@ struct SortHere {
 };
 constexpr int SORT_HERE_MAX = WAVE;   // choices that one wavefront sorts with one per lane
 __host__ __device__ constexpr size_t sort_here_ints(int E) {
-  return (size_t)E + (E + 1) + 2 * SORT_HERE_MAX + SORT_HERE_MAX / 2 + (2 * E + 1);
+  return (size_t)E + 2 * SORT_HERE_MAX + SORT_HERE_MAX / 2 + (2 * E + 1);
 }
 
 // With SORT the launch has no sorted rows to start from, only the routing: every workgroup
@@ -237,136 +245,177 @@ __host__ __device__ constexpr size_t sort_here_ints(int E) {
 // its scan of `offsets` stood, and the launch before it need not gather every token's choices
 // in one place.
 //
+// ALL (with SORT, up to 8 tokens of 2048): every token's row is asked for at once, with the routing, and the
+// stream picks its rows among them by token. No row waits for the sort, which is the better part of a
+// microsecond in front of the stream, and no workgroup stages rows again for its next expert: one token in a
+// decode step 15.9 -> 14.3 us, 8 tokens 56.9 -> 55.6. (Rows behind the first weights, as a DENSE launch has
+// them, cost the down projection's sixteen wavefronts to a compute unit more than the wait: 9.8 -> 12.0 and
+// 30.3 -> 33.4.)
+//
 // DENSE: one matrix and `sort.M` rows of A in their own order (the projections around the MoE layer):
-// there is no list of experts to build, so a launch begins with its loads. The rows (up to 8 of
-// at most 2048) are asked for first, then the first weights, and the rows go to LDS behind those.
+// there is no list of experts to build, so a launch begins with its loads: the rows, then the first weights,
+// and the rows go to LDS behind those.
 // One row, q/k/v and output projection on average: 8.2 us a launch as a grouped call, 7.1 so.
-template <bool SWIGLU, bool SCALE, bool EXACT, int CH, bool SORT = false, bool DENSE = false>
+constexpr int EARLY_ROWS = 2, EARLY_CHUNKS = 4;   // rows that a wavefront asks for ahead, in chunks of 64 x 16 bytes
+constexpr int ALL_ROWS = 8;                       // tokens of an ALL launch, a chunk of 16 bytes of each per thread
+
+template <bool SWIGLU, bool SCALE, bool EXACT, int CH, bool SORT = false, bool DENSE = false, bool ALL = false>
 __global__ void __launch_bounds__(GEMV_THREADS)
 gemv_kernel(const half_t* __restrict__ A, const int* __restrict__ a_rows, const half_t* __restrict__ B,
             const int* __restrict__ offsets, int E, int Nout, int K, const half_t* __restrict__ scale,
             half_t* __restrict__ C, int row_cap, SortHere sort = SortHere{}) {
-  extern __shared__ __attribute__((aligned(16))) half_t xs[];  // [row_cap][K + ROW_PAD], then the used experts
+  extern __shared__ __attribute__((aligned(16))) half_t xs[];  // [row_cap][K + ROW_PAD], then the experts' lists
   // the wavefront's number is the same in all its lanes, and said so: every unit, K offset and
   // buffer descriptor below derives from it, and what the compiler cannot prove uniform it wraps
   // in a loop over the lanes' values, around every load of the stream
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  constexpr int waves = GEMV_WAVES;
   const int RS = K + ROW_PAD;
-  int* used = reinterpret_cast<int*>(xs + (size_t)row_cap * RS);  // [E] ids of experts with rows, [E] = how many
-  const half8_t zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
-  if constexpr (DENSE) {
-    const int rows = sort.M, units = (Nout + UNIT_COLS - 1) / UNIT_COLS;
-    const int lo = (int)((long)units * blockIdx.x / gridDim.x), count = (int)((long)units * (blockIdx.x + 1) / gridDim.x) - lo;
-    Pass p;
-    p.xs = xs;
-    p.rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(B), 0, (int)((size_t)Nout * K * 2), 0x00020000);
-    p.scale = scale;
-    p.C = C;
-    p.Nout = Nout;
-    p.K = K;
-    p.RS = RS;
-    p.nchunks = ((K + STEP_K - 1) / STEP_K + CH - 1) / CH;
-    p.unit0 = lo + (int)((long)count * wave / GEMV_WAVES);
-    p.nunits = lo + (int)((long)count * (wave + 1) / GEMV_WAVES) - p.unit0;
-    constexpr int EARLY_ROWS = 2, EARLY_CHUNKS = 4;   // per wavefront; chunks of 64 x 16 bytes
-    for (int r0 = 0; r0 < rows; r0 += row_cap) {
-      const int nr = min(row_cap, rows - r0), nq = (nr + QUAD - 1) / QUAD;
-      p.r0 = r0;
-      p.nr = nr;
-      const bool early = nq * QUAD <= EARLY_ROWS * GEMV_WAVES && K <= EARLY_CHUNKS * WAVE * 8;
-      half8_t x[EARLY_ROWS][EARLY_CHUNKS];
+  Pass p;
+  p.xs = xs;
+  p.rows = nullptr;
+  p.scale = scale;
+  p.C = C;
+  p.Nout = Nout;
+  p.K = K;
+  p.RS = RS;
+  p.nchunks = ((K + STEP_K - 1) / STEP_K + CH - 1) / CH;
+  bool staged = false;
+  // rows r0 .. r0 + nr - 1 (row i is row_of(i) of A) against the units of `p`; missing rows of the last quad are zero
+  auto pass_rows = [&](int r0, int nr, auto row_of) {
+    const int nq = (nr + QUAD - 1) / QUAD;
+    p.r0 = r0;
+    p.nr = nr;
+    const half8_t zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+    // DENSE: the rows are asked for first, then the first weights, and the rows go to LDS behind those
+    const bool early = DENSE && nq * QUAD <= EARLY_ROWS * waves && K <= EARLY_CHUNKS * WAVE * 8;
+    half8_t x[EARLY_ROWS][EARLY_CHUNKS];
+    if (early) {
+#pragma unroll
+      for (int i = 0; i < EARLY_ROWS; ++i)
+#pragma unroll
+        for (int j = 0; j < EARLY_CHUNKS; ++j) {
+          const int r = wave + waves * i, kk = (lane + WAVE * j) * 8;
+          x[i][j] = zero8;
+          if (r < nr && kk < K) x[i][j] = *reinterpret_cast<const half8_t*>(A + (size_t)row_of(r0 + r) * K + kk);
+        }
+    }
+    auto stage = [&] {
+      if (staged) __syncthreads();   // the rows of the pass before have been read
+      staged = true;
       if (early) {
 #pragma unroll
         for (int i = 0; i < EARLY_ROWS; ++i)
 #pragma unroll
           for (int j = 0; j < EARLY_CHUNKS; ++j) {
-            const int r = wave + GEMV_WAVES * i, kk = (lane + WAVE * j) * 8;
-            x[i][j] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
-            if (r < nr && kk < K) x[i][j] = *reinterpret_cast<const half8_t*>(A + (size_t)(r0 + r) * K + kk);
+            const int r = wave + waves * i, kk = (lane + WAVE * j) * 8;
+            if (r < nq * QUAD && kk < K) *reinterpret_cast<half8_t*>(xs + r * RS + kk) = x[i][j];
           }
-      }
-      auto stage = [&] {
-        if (r0) __syncthreads();   // the rows of the pass before have been read
-        if (early) {
-#pragma unroll
-          for (int i = 0; i < EARLY_ROWS; ++i)
-#pragma unroll
-            for (int j = 0; j < EARLY_CHUNKS; ++j) {
-              const int r = wave + GEMV_WAVES * i, kk = (lane + WAVE * j) * 8;
-              if (r < nq * QUAD && kk < K) *reinterpret_cast<half8_t*>(xs + r * RS + kk) = x[i][j];
-            }
-        } else {
-          for (int r = wave; r < nq * QUAD; r += GEMV_WAVES)
-            for (int kk = lane * 8; kk < K; kk += WAVE * 8)
-              *reinterpret_cast<half8_t*>(xs + r * RS + kk) =
-                  r < nr ? *reinterpret_cast<const half8_t*>(A + (size_t)(r0 + r) * K + kk) : half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+      } else {
+        for (int r = wave; r < nq * QUAD; r += waves) {
+          const half_t* src = r < nr ? A + (size_t)row_of(r0 + r) * K : nullptr;
+          for (int kk = lane * 8; kk < K; kk += WAVE * 8)
+            *reinterpret_cast<half8_t*>(xs + r * RS + kk) = src ? *reinterpret_cast<const half8_t*>(src + kk) : zero8;
         }
-        __syncthreads();
-      };
-      switch (nq) {
-        case 1: run_pass<SWIGLU, SCALE, EXACT, CH, 1>(p, stage); break;
-        case 2: run_pass<SWIGLU, SCALE, EXACT, CH, 2>(p, stage); break;
-        case 3: run_pass<SWIGLU, SCALE, EXACT, CH, 3>(p, stage); break;
-        default: run_pass<SWIGLU, SCALE, EXACT, CH, 4>(p, stage); break;
       }
+      __syncthreads();
+    };
+    auto run = [&](auto quads) {
+      constexpr int NQ = decltype(quads)::value;
+      if constexpr (DENSE) {
+        run_pass<SWIGLU, SCALE, EXACT, CH, NQ>(p, stage);
+      } else {
+        stage();
+        run_pass<SWIGLU, SCALE, EXACT, CH, NQ>(p);
+      }
+    };
+    switch (nq) {
+      case 1: run(std::integral_constant<int, 1>{}); break;
+      case 2: run(std::integral_constant<int, 2>{}); break;
+      case 3: run(std::integral_constant<int, 3>{}); break;
+      default: run(std::integral_constant<int, 4>{}); break;
     }
+  };
+
+  if constexpr (DENSE) {
+    const int rows = sort.M, units = (Nout + UNIT_COLS - 1) / UNIT_COLS;
+    const int lo = (int)((long)units * blockIdx.x / gridDim.x), count = (int)((long)units * (blockIdx.x + 1) / gridDim.x) - lo;
+    p.rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(B), 0, (int)((size_t)Nout * K * 2), 0x00020000);
+    p.unit0 = lo + count * wave / waves;
+    p.nunits = lo + count * (wave + 1) / waves - p.unit0;
+    for (int r0 = 0; r0 < rows; r0 += row_cap) pass_rows(r0, min(row_cap, rows - r0), [](int r) { return r; });
     return;
   }
-  // SORT: the sort's results in LDS, behind the list of used experts
-  int* s_counts = used + E + 1;
-  int* s_offsets = s_counts + E;
-  int* s_token = s_offsets + E + 1;
+
+  int* used = reinterpret_cast<int*>(xs + (size_t)row_cap * RS);  // [E] ids of experts with rows, [E] = how many
+  int* s_offsets = used + E + 1;                                  // [E + 1]
+  // SORT: the sort's other results in LDS, behind
+  int* s_counts = s_offsets + E + 1;
+  int* s_token = s_counts + E;
   int* s_pos = s_token + SORT_HERE_MAX;
   uint16_t* s_wsorted = reinterpret_cast<uint16_t*>(s_pos + SORT_HERE_MAX);
-  if (SORT) {
-    if (wave == 0)
-      sort_core::sort_one_wave<uint16_t>(sort.idx, reinterpret_cast<const uint16_t*>(sort.w), sort.M, sort.k, E, sort.nbits,
-                                         s_counts, s_offsets, s_token, s_wsorted, s_pos,
-                                         reinterpret_cast<int*>(s_wsorted + SORT_HERE_MAX));
-    __syncthreads();
-    if (blockIdx.x == 0) {
-      for (int i = threadIdx.x; i <= E; i += GEMV_THREADS) {
-        sort.offsets[i] = s_offsets[i];
-        if (i < E) sort.counts[i] = s_counts[i];
-      }
-      for (int i = threadIdx.x; i < sort.M; i += GEMV_THREADS) {
-        sort.token[i] = s_token[i];
-        sort.pos_of[i] = s_pos[i];
-        reinterpret_cast<uint16_t*>(sort.wsorted)[i] = s_wsorted[i];
-      }
-    }
+  int key = -1;
+  uint16_t weight = 0;
+  if (SORT && wave == 0 && lane < sort.M) {
+    key = sort.idx[lane];
+    weight = reinterpret_cast<const uint16_t*>(sort.w)[lane];
   }
-
-  // ---- the experts that received rows, in order (one wavefront, 64 experts per step)
+  const int tokens = ALL ? sort.M / sort.k : 0;
+  half8_t all[ALL ? ALL_ROWS : 1];
+  if (ALL) {
+#pragma unroll
+    for (int r = 0; r < ALL_ROWS; ++r)
+      if (r < tokens && (int)threadIdx.x * 8 < K) all[r] = *reinterpret_cast<const half8_t*>(A + (size_t)r * K + threadIdx.x * 8);
+  }
   if (wave == 0) {
+    if (SORT) {
+      sort_core::sort_one_wave_loaded<uint16_t>(key, weight, sort.M, sort.k, E, sort.nbits, s_counts, s_offsets, s_token, s_wsorted,
+                                                s_pos, reinterpret_cast<int*>(s_wsorted + SORT_HERE_MAX));
+      __builtin_amdgcn_wave_barrier();
+    }
+    // ---- the experts that received rows, in order (one wavefront, 64 experts per step)
     int n = 0;
     for (int e0 = 0; e0 < E; e0 += WAVE) {
       const int e = e0 + lane;
-      const bool has = e < E && (SORT ? s_offsets[e + 1] > s_offsets[e] : offsets[e + 1] > offsets[e]);
-      const uint64_t m = __ballot(has);
-      if (has) used[n + __popcll(m & lanemask_lt())] = e;
+      int first = 0, last = 0;
+      if (e < E) {
+        first = SORT ? s_offsets[e] : offsets[e];
+        last = SORT ? s_offsets[e + 1] : offsets[e + 1];
+        if (!SORT) {
+          s_offsets[e] = first;
+          if (e == E - 1) s_offsets[E] = last;
+        }
+      }
+      const uint64_t m = __ballot(last > first);
+      if (last > first) used[n + __popcll(m & lanemask_lt())] = e;
       n += __popcll(m);
     }
     if (lane == 0) used[E] = n;
   }
+  if (ALL) {
+#pragma unroll
+    for (int r = 0; r < ALL_ROWS; ++r)
+      if (r < tokens && (int)threadIdx.x * 8 < K) *reinterpret_cast<half8_t*>(xs + r * RS + threadIdx.x * 8) = all[r];
+  }
   __syncthreads();
+  if (SORT && blockIdx.x == 0) {
+    for (int i = threadIdx.x; i <= E; i += GEMV_THREADS) {
+      sort.offsets[i] = s_offsets[i];
+      if (i < E) sort.counts[i] = s_counts[i];
+    }
+    for (int i = threadIdx.x; i < sort.M; i += GEMV_THREADS) {
+      sort.token[i] = s_token[i];
+      sort.pos_of[i] = s_pos[i];
+      reinterpret_cast<uint16_t*>(sort.wsorted)[i] = s_wsorted[i];
+    }
+  }
   const int nused = used[E];
   const int units_per_expert = (Nout + UNIT_COLS - 1) / UNIT_COLS;
 
   // ---- this workgroup's equal share of all units, a contiguous range [lo, hi)
   const long total_units = (long)nused * units_per_expert;
   const int lo = (int)(total_units * blockIdx.x / gridDim.x), hi = (int)(total_units * (blockIdx.x + 1) / gridDim.x);
-
-  Pass p;
-  p.xs = xs;
-  p.Nout = Nout;
-  p.K = K;
-  p.RS = RS;
-  p.scale = scale;
-  p.C = C;
-  p.nchunks = ((K + STEP_K - 1) / STEP_K + CH - 1) / CH;
   const int Nfull = SWIGLU ? 2 * Nout : Nout;
-  bool staged = false;
 
   for (int at = lo; at < hi;) {
     // the part of the range that falls into one expert
@@ -375,8 +424,8 @@ gemv_kernel(const half_t* __restrict__ A, const int* __restrict__ a_rows, const 
     // the same in every lane, and said so: the weights' buffer descriptor is built from it, and a
     // descriptor that the compiler cannot prove uniform costs every load a loop over its lanes
     const int e = __builtin_amdgcn_readfirstlane(used[u]);
-    const int start = __builtin_amdgcn_readfirstlane(SORT ? s_offsets[e] : offsets[e]);
-    const int end = __builtin_amdgcn_readfirstlane(SORT ? s_offsets[e + 1] : offsets[e + 1]);
+    const int start = __builtin_amdgcn_readfirstlane(s_offsets[e]);
+    const int end = __builtin_amdgcn_readfirstlane(s_offsets[e + 1]);
     p.rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(B + (size_t)e * Nfull * K), 0,
                                                (int)((size_t)Nfull * K * 2), 0x00020000);
     // wavefront w takes a contiguous quarter of the units
@@ -385,23 +434,16 @@ gemv_kernel(const half_t* __restrict__ A, const int* __restrict__ a_rows, const 
 
     for (int r0 = start; r0 < end; r0 += row_cap) {
       const int nr = min(row_cap, end - r0);
-      const int nq = (nr + QUAD - 1) / QUAD;
-      // ---- stage the pass's rows: wavefront w copies rows w, w+4, ...; missing rows of the last quad are zero
-      if (staged) __syncthreads();
-      for (int r = wave; r < nq * QUAD; r += GEMV_WAVES) {
-        const half_t* src = r < nr ? A + (size_t)(SORT ? s_token[r0 + r] : a_rows ? a_rows[r0 + r] : r0 + r) * K : nullptr;
-        for (int kk = lane * 8; kk < K; kk += WAVE * 8)
-          *reinterpret_cast<half8_t*>(xs + r * RS + kk) = src ? *reinterpret_cast<const half8_t*>(src + kk) : zero8;
-      }
-      __syncthreads();
-      staged = true;
-      p.r0 = r0;
-      p.nr = nr;
-      switch (nq) {
-        case 1: run_pass<SWIGLU, SCALE, EXACT, CH, 1>(p); break;
-        case 2: run_pass<SWIGLU, SCALE, EXACT, CH, 2>(p); break;
-        case 3: run_pass<SWIGLU, SCALE, EXACT, CH, 3>(p); break;
-        default: run_pass<SWIGLU, SCALE, EXACT, CH, 4>(p); break;
+      if constexpr (ALL) {
+        p.r0 = r0;
+        p.nr = nr;
+        p.rows = s_token + r0;
+        if (nr <= QUAD) run_pass<SWIGLU, SCALE, EXACT, CH, 1, true>(p);
+        else run_pass<SWIGLU, SCALE, EXACT, CH, 2, true>(p);
+      } else if constexpr (SORT) {
+        pass_rows(r0, nr, [&](int r) { return s_token[r]; });
+      } else {
+        pass_rows(r0, nr, [&](int r) { return a_rows ? a_rows[r] : r; });
       }
     }
     at += count;
@@ -416,7 +458,7 @@ int launch_gemv(const void* A, const int32_t* a_rows, const void* B, const int32
   const int bound = max_rows_hint > 0 && max_rows_hint < rows ? max_rows_hint : rows;
   int row_cap = (bound + QUAD - 1) / QUAD * QUAD;
   row_cap = row_cap > MAX_QUADS * QUAD ? MAX_QUADS * QUAD : row_cap;
-  const size_t lds = (size_t)row_cap * (K + ROW_PAD) * sizeof(half_t) + (size_t)(E + 1) * sizeof(int) +
+  const size_t lds = (size_t)row_cap * (K + ROW_PAD) * sizeof(half_t) + (size_t)2 * (E + 1) * sizeof(int) +
                      (sort && !dense ? sort_here_ints(E) * sizeof(int) : 0);
   // Loads in flight per wavefront: a chunk of 4 KB, or of 8 KB where a unit is long enough to be
   // cut into such chunks (gate and up rows of 2048 at 8 tokens: 56.6 us against 57.5; for rows of
@@ -445,6 +487,9 @@ int launch_gemv(const void* A, const int32_t* a_rows, const void* B, const int32
   void (*kern)(const half_t*, const int*, const half_t*, const int*, int, int, int, const half_t*, half_t*, int, SortHere);
   if (dense && long_chunks && exact) kern = gemv_kernel<false, false, true, CH_LONG, false, true>;
   else if (dense) kern = exact ? gemv_kernel<false, false, true, CH_SHORT, false, true> : gemv_kernel<false, false, false, CH_SHORT, false, true>;
+  // (more than 8 tokens have at most 64 choices only where k < 8; one row of LDS per token)
+  else if (sort && long_chunks && exact && rows / sort->k <= ALL_ROWS && rows / sort->k <= row_cap && K <= GEMV_THREADS * 8)
+    kern = gemv_kernel<true, false, true, CH_LONG, true, false, true>;
   else if (sort && long_chunks && exact) kern = gemv_kernel<true, false, true, CH_LONG, true>;
   else if (sort) kern = exact ? gemv_kernel<true, false, true, CH_SHORT, true> : gemv_kernel<true, false, false, CH_SHORT, true>;
   else if (swiglu && long_chunks && exact) kern = gemv_kernel<true, false, true, CH_LONG>;

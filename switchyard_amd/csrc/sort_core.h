@@ -165,18 +165,18 @@ __device__ __forceinline__ void sort_small_block(const int* idx, const W* w, int
 }
 
 // The whole sort by one wavefront when there are at most 64 choices (a decode step of 8 tokens):
-// one choice per lane, no workgroup barrier. `lds` holds 2 * E + 1 ints; E <= 128.
+// one choice per lane, no workgroup barrier; lane i < M gives choice i's expert and weight. `lds` holds
+// 2 * E + 1 ints; E <= 128.
 template <typename W>
-__device__ __forceinline__ void sort_one_wave(const int* idx, const W* w, int M, int k, int E, int nbits,
-                                              int* __restrict__ counts, int* __restrict__ offsets,
-                                              int* __restrict__ token, W* __restrict__ wsorted,
-                                              int* __restrict__ pos_of, int* lds) {
+__device__ __forceinline__ void sort_one_wave_loaded(int key, W weight, int M, int k, int E, int nbits,
+                                                     int* __restrict__ counts, int* __restrict__ offsets,
+                                                     int* __restrict__ token, W* __restrict__ wsorted,
+                                                     int* __restrict__ pos_of, int* lds) {
   int* total = lds;      // [E]
   int* offs = lds + E;   // [E + 1]
   const int lane = threadIdx.x & 63;
   for (int x = lane; x < E; x += WAVE) total[x] = 0;
-  int key = lane < M ? idx[lane] : -1;
-  const bool valid = (unsigned)key < (unsigned)E;
+  const bool valid = lane < M && (unsigned)key < (unsigned)E;
   key = valid ? key : 0;
   const uint64_t m = match_lanes(key, valid, nbits);
   const int rank = __popcll(m & lanemask_lt()), cnt = __popcll(m);
@@ -204,9 +204,19 @@ __device__ __forceinline__ void sort_one_wave(const int* idx, const W* w, int M,
   if (valid) {
     const int row = offs[key] + rank;
     token[row] = lane / k;
-    wsorted[row] = w[lane];
+    wsorted[row] = weight;
     pos_of[lane] = row;
   }
+}
+
+template <typename W>
+__device__ __forceinline__ void sort_one_wave(const int* idx, const W* w, int M, int k, int E, int nbits,
+                                              int* __restrict__ counts, int* __restrict__ offsets,
+                                              int* __restrict__ token, W* __restrict__ wsorted,
+                                              int* __restrict__ pos_of, int* lds) {
+  const int lane = threadIdx.x & 63;
+  sort_one_wave_loaded<W>(lane < M ? idx[lane] : -1, lane < M ? w[lane] : W(0), M, k, E, nbits, counts, offsets, token, wsorted,
+                          pos_of, lds);
 }
 
 }  // namespace sort_core

@@ -122,6 +122,22 @@ def test_combine_add_rmsnorm_of_few_rows(N, H, k):
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
 
 
+@pytest.mark.parametrize("N,k", [(1, 8), (2, 8), (5, 8), (8, 8), (8, 1), (3, 5), (9, 7), (16, 4), (64, 1)])   # up to 8 tokens: staged once
+@pytest.mark.parametrize("H,I", [(2048, 36), (2048, 1000), (1024, 36), (2056, 4)])
+def test_gate_up_that_sorts_for_itself(N, k, H, I):
+    """Against sort and projection of their own, bit for bit; ids that repeat inside a token are rows of their own."""
+    E = 16
+    g = torch.Generator().manual_seed(N * 100 + k)
+    idx = torch.randint(E, (N, k), generator=g, dtype=torch.int32).cuda()
+    wts = torch.rand(N, k, generator=g).half().cuda()
+    h, gate_up = rnd(N, H, seed=61), rnd(E, 2 * I, H, seed=62, std=0.03)
+    ext = kernels.ext()
+    counts, offsets, token, wsorted, pos_of = want = ext.sort_by_expert(idx, wts, E)
+    got = ext.grouped_gemv_sorting(h, idx, wts, gate_up)
+    for a, b in zip(got, (*want, ext.grouped_gemv(h, token, gate_up, offsets, N * k, True, None))):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("N,H,vocab", [(8, 2048, 50304), (64, 2048, 50304), (3, 64, 10), (1, 520, 77)])
 def test_embed_rmsnorm(N, H, vocab):
     """The embedding rows bit for bit, their norm as add_rmsnorm gives it; ids outside the table are clamped."""
