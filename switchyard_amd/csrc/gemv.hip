@@ -258,9 +258,10 @@ __host__ __device__ constexpr size_t sort_here_ints(int E) {
 // One row, q/k/v and output projection on average: 8.2 us a launch as a grouped call, 7.1 so.
 constexpr int EARLY_ROWS = 2, EARLY_CHUNKS = 4;   // rows that a wavefront asks for ahead, in chunks of 64 x 16 bytes
 constexpr int ALL_ROWS = 8;                       // tokens of an ALL launch, a chunk of 16 bytes of each per thread
+constexpr int DENSE_MAX_WAVES = 8;
 
 template <bool SWIGLU, bool SCALE, bool EXACT, int CH, bool SORT = false, bool DENSE = false, bool ALL = false>
-__global__ void __launch_bounds__(GEMV_THREADS)
+__global__ void __launch_bounds__(DENSE ? DENSE_MAX_WAVES * WAVE : GEMV_THREADS)
 gemv_kernel(const half_t* __restrict__ A, const int* __restrict__ a_rows, const half_t* __restrict__ B,
             const int* __restrict__ offsets, int E, int Nout, int K, const half_t* __restrict__ scale,
             half_t* __restrict__ C, int row_cap, SortHere sort = SortHere{}) {
@@ -269,7 +270,7 @@ gemv_kernel(const half_t* __restrict__ A, const int* __restrict__ a_rows, const 
   // buffer descriptor below derives from it, and what the compiler cannot prove uniform it wraps
   // in a loop over the lanes' values, around every load of the stream
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  constexpr int waves = GEMV_WAVES;
+  const int waves = DENSE ? (int)(blockDim.x >> 6) : GEMV_WAVES;
   const int RS = K + ROW_PAD;
   Pass p;
   p.xs = xs;
@@ -450,6 +451,34 @@ gemv_kernel(const half_t* __restrict__ A, const int* __restrict__ a_rows, const 
   }
 }
 
+// Workgroups per compute unit and wavefronts per workgroup of a DENSE launch, for `units` units per compute
+// unit. The wavefronts of a compute unit take its units in rounds and the last round should be full: the
+// number of wavefronts, up to 12 (more only take registers from the loads in flight), with the fewest places
+// left empty, the most wavefronts where that is equal. 6 units (q/k/v of 2048, 6144 columns on 256 compute units) are 6
+// wavefronts in one workgroup, 2 (output projection) are 2, and 49 (50 304 columns) are 10 in two, where 4
+// wavefronts to a workgroup and a unit to a wavefront left 128 compute units with half the work of the others
+// or none: q/k/v and output projection on average 8.1 -> 6.9 us a launch with one row, 8.6 -> 7.5 with 8. A single workgroup gets as many wavefronts as ask for its rows in one go, with or
+// without units of their own.
+void dense_shape(long units, int rows, long fit, long& per_cu, int& waves) {
+  long best = 1, spare = units + 12;
+  for (long n = 1; n <= 12; ++n) {
+    const long left = (units + n - 1) / n * n - units;
+    if (n > units && n > 1) break;
+    // fewer wavefronts than 8 only where they are a round by themselves
+    if (n < 8 && n < units) continue;
+    if (left <= spare) {
+      best = n;
+      spare = left;
+    }
+  }
+  per_cu = (best + DENSE_MAX_WAVES - 1) / DENSE_MAX_WAVES;
+  per_cu = per_cu > fit ? (fit > 0 ? fit : 1) : per_cu;
+  waves = (int)((best + per_cu - 1) / per_cu);
+  const int ask = (rows + EARLY_ROWS - 1) / EARLY_ROWS;
+  if (per_cu == 1 && waves < ask) waves = ask;
+  waves = waves > DENSE_MAX_WAVES ? DENSE_MAX_WAVES : waves;
+}
+
 int launch_gemv(const void* A, const int32_t* a_rows, const void* B, const int32_t* offsets, int E, int rows,
                 int max_rows_hint, int Nout, int K, int swiglu, const void* scale, void* C, hipStream_t stream,
                 const SortHere* sort = nullptr, bool dense = false) {
@@ -477,9 +506,15 @@ int launch_gemv(const void* A, const int32_t* a_rows, const void* B, const int32
   const long fit = (160 * 1024) / (long)(lds ? lds : 1);      // by LDS
   per_cu = per_cu > fit ? (fit > 0 ? fit : 1) : per_cu;
   long max_units = (long)(E < rows ? E : rows) * ((Nout + UNIT_COLS - 1) / UNIT_COLS);
-  if (dense) max_units = (max_units + GEMV_WAVES - 1) / GEMV_WAVES;   // a unit for every wavefront
   long grid = (long)sy_compute_units() * per_cu;
   grid = grid > max_units ? max_units : grid;
+  int waves = GEMV_WAVES;
+  if (dense) {
+    const long cus = sy_compute_units();
+    dense_shape((max_units + cus - 1) / cus, row_cap, fit, per_cu, waves);
+    grid = cus * per_cu;
+    grid = grid > max_units ? max_units : grid;
+  }
   const half_t* a = (const half_t*)A;
   const half_t* b = (const half_t*)B;
   const half_t* s = (const half_t*)scale;
@@ -499,7 +534,7 @@ int launch_gemv(const void* A, const int32_t* a_rows, const void* B, const int32
   hipError_t attr = hipSuccess;
   if (lds > 48 * 1024) attr = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (attr != hipSuccess) return sy_fail(SY_ERR_LAUNCH, "grouped_gemv: cannot reserve %zu bytes of LDS", lds);
-  kern<<<(unsigned)grid, GEMV_THREADS, lds, stream>>>(a, a_rows, b, offsets, E, Nout, K, swiglu ? nullptr : s, c, row_cap,
+  kern<<<(unsigned)grid, (unsigned)waves * WAVE, lds, stream>>>(a, a_rows, b, offsets, E, Nout, K, swiglu ? nullptr : s, c, row_cap,
                                                       sort ? *sort : SortHere{});
   return sy_check_launch("grouped_gemv");
 }
