@@ -99,6 +99,8 @@ SIGNATURES = {
     "sy_padding_twins": (_c_int, [_c_void_p, _c_void_p, _c_int, _c_int, _c_void_p, _c_void_p]),
     "sy_moe_add_rmsnorm": (_c_int, [ctypes.POINTER(SyMoeLayer), _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_float,
                                     _c_void_p, _c_void_p, _c_void_p]),
+    "sy_dense_tiles": (_c_int, [_c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_void_p, _c_void_p]),
+    "sy_dense_tiles_takes": (_c_int, [_c_int, _c_int, _c_int]),
     "sy_dense_rows": (_c_int, [_c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_void_p, _c_void_p]),
     "sy_decode_attention_shares": (_c_int, [_c_int, _c_int]),
     "sy_decode_step_scratch_bytes": (_c_size_t, [ctypes.POINTER(SyDecodeStep)]),
@@ -852,6 +854,21 @@ class Ext:
             raise RuntimeError("dense_rows: x [rows, K], weight [Nout, K]")
         out = torch.empty((x.shape[0], weight.shape[0]), dtype=torch.float16, device=x.device)
         self._call(self.lib.sy_dense_rows, x.data_ptr(), weight.data_ptr(), x.shape[0], weight.shape[0], x.shape[1],
+                   out.data_ptr(), _stream())
+        return out
+
+    def dense_tiles_ok(self, rows, Nout, K):
+        """Whether dense_tiles takes this shape: a few dozen rows, no more tiles than compute units."""
+        return bool(self.lib.sy_dense_tiles_takes(int(rows), int(Nout), int(K)))
+
+    def dense_tiles(self, x, weight):
+        """x [rows, K] @ weight [Nout, K]^T on small MFMA tiles (dense_tiles_ok says which shapes)."""
+        _check(x, "x", torch.float16)
+        _check(weight, "weight", torch.float16)
+        if x.dim() != 2 or weight.dim() != 2 or x.shape[1] != weight.shape[1]:
+            raise RuntimeError("dense_tiles: x [rows, K], weight [Nout, K]")
+        out = torch.empty((x.shape[0], weight.shape[0]), dtype=torch.float16, device=x.device)
+        self._call(self.lib.sy_dense_tiles, x.data_ptr(), weight.data_ptr(), x.shape[0], weight.shape[0], x.shape[1],
                    out.data_ptr(), _stream())
         return out
 

@@ -53,6 +53,12 @@ SY_API int sy_moe_add_rmsnorm(const SyMoeLayer* L, const void* h, const int32_t*
  * of sy_grouped_gemv with one expert that owns every row. K a multiple of 8 up to 4096. */
 SY_API int sy_dense_rows(const void* x, const void* weight, int rows, int Nout, int K, void* out, void* stream);
 
+/* x f16 [rows, K] @ weight f16 [Nout, K]^T -> out f16 [rows, Nout] on small MFMA tiles, for a few dozen rows: K a
+ * multiple of 128, each operand under 2 GiB, no more tiles than compute units (sy_dense_tiles_takes). 16-byte
+ * aligned rows. */
+SY_API int sy_dense_tiles(const void* x, const void* weight, int rows, int Nout, int K, void* out, void* stream);
+SY_API int sy_dense_tiles_takes(int rows, int Nout, int K);
+
 /* Whether decode attention's (sequence, head) pairs are few enough for sy_decode_attention_qkv_split to
  * deal their keys to several workgroups. */
 SY_API int sy_decode_attention_shares(int B, int heads);

@@ -281,7 +281,7 @@ class Decoder:
         for i in range(s.layers):
             L = W["layers"][i]
             after = W["layers"][i + 1]["attn_norm"] if i + 1 < s.layers else W["final_norm"]
-            q = E.qk_norm_rope_cache(kernels.dense(xn, wqkv[i]), L["q_norm"], L["k_norm"], s.rms_eps, s.clip_qkv, self.cos,
+            q = E.qk_norm_rope_cache(kernels.project(xn, wqkv[i]), L["q_norm"], L["k_norm"], s.rms_eps, s.clip_qkv, self.cos,
                                      self.sin, flat_positions, slot, s.heads, s.kv_heads, s.head_dim, cache.k[i], cache.v[i])
             if own_attention:
                 a = E.prefill_attention(q, cache.k[i], cache.v[i], cache.real, span.first, s.heads)
@@ -290,7 +290,7 @@ class Decoder:
                                                    cache.k[i, :, :, :span.end], cache.v[i, :, :, :span.end],
                                                    attn_mask=span.visible, enable_gqa=s.kv_heads != s.heads)
                 a = a.transpose(1, 2).reshape(B * T, s.heads * s.head_dim)
-            o = kernels.dense(a, L["wo"])
+            o = kernels.project(a, L["wo"])
             x, h = E.add_rmsnorm(x, o, L["mlp_norm"], s.rms_eps, x_out=x)
             if in_one:
                 x, xn = E.moe_add_rmsnorm(h, L["router"], L["gate_up"], L["down"], s.top_k, s.norm_topk_prob, x, after,
@@ -392,10 +392,10 @@ class Decoder:
         for i in range(s.layers):
             L = W["layers"][i]
             after = W["layers"][i + 1]["attn_norm"] if i + 1 < s.layers else W["final_norm"]
-            a = E.decode_attention_qkv(kernels.dense(xn, wqkv[i]), L["q_norm"], L["k_norm"], s.rms_eps, s.clip_qkv,
+            a = E.decode_attention_qkv(kernels.project(xn, wqkv[i]), L["q_norm"], L["k_norm"], s.rms_eps, s.clip_qkv,
                                        self.cos, self.sin, positions, slot, cache.real, s.heads, s.kv_heads,
                                        s.head_dim, cache.k[i], cache.v[i], split and (split[0], split[1][i]))
-            o = kernels.dense(a, L["wo"])
+            o = kernels.project(a, L["wo"])
             if self._own_moe and s.experts <= 1024 and s.top_k <= 64:
                 # the router's logits come out of the norm's launch, and combine goes into the next norm's
                 if x.shape[0] <= 256 and s.experts <= 128 and s.top_k <= min(8, s.experts):

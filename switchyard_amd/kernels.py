@@ -143,6 +143,15 @@ def dense(x, weight):
     return ext().dense_rows(x, weight)
 
 
+def project(x, weight):
+    """`dense` inside the decoder's fused passes (f16 on the GPU, no gradients): where there are a few dozen
+    rows and the library's own tiles take the shape, they do (64 rows, [2048, 2048]: 6.9 us against 11.0)."""
+    if (x.shape[0] > 16 and weight.is_contiguous() and weight.dtype == torch.float16 and weight.data_ptr() % 16 == 0
+            and ext().dense_tiles_ok(x.shape[0], *weight.shape)):
+        return ext().dense_tiles(x, weight)
+    return dense(x, weight)
+
+
 # Up to this many tokens route and sort run as one launch of one workgroup (a decode step is
 # launch- and latency-bound in front of its two projections). Measured in a replayed graph, one
 # launch against route + sort_by_expert: 8 tokens 3.7 against 6.5 us, 16 tokens 6.5 against 6.6,

@@ -664,6 +664,32 @@ def test_dense_rows_equal_the_weight_stream_of_one_expert(rows, Nout, K):
     assert torch.equal(kernels.ext().dense_rows(x, w), want)
 
 
+@pytest.mark.parametrize("rows,Nout,K", [(1, 16, 128), (17, 6144, 2048), (32, 6144, 2048), (33, 6144, 2048), (64, 6144, 2048), (17, 2048, 2048),
+                                        (33, 2048, 2048), (64, 2048, 2048), (65, 2048, 2048), (128, 2048, 2048), (129, 2048, 2048),
+                                        (256, 2048, 2048), (48, 2041, 128), (50, 3001, 384), (31, 100, 4096), (64, 6145, 640)])
+def test_dense_tiles(rows, Nout, K):
+    """Every tile, at the last and first rows of each, ragged columns, a ring longer than K: an in-order sum of
+    fp32 products, one rounding. fp32 sums in another order differ by K rounding errors of 2^-24 at most, which
+    is far below half an fp16 ulp of a result of the size of the terms' sum."""
+    ext = kernels.ext()
+    assert ext.dense_tiles_ok(rows, Nout, K)
+    x, w = rnd(rows, K, seed=71), rnd(Nout, K, seed=72, std=0.03)
+    got = ext.dense_tiles(x, w).double()
+    want = x.double() @ w.double().T
+    size = x.double().abs() @ w.double().abs().T
+    assert ((got - want).abs() <= want.abs() * 2.0 ** -11 + size * K * 2.0 ** -24 + 2.0 ** -24).all()
+
+
+def test_dense_tiles_limits():
+    ext = kernels.ext()
+    assert not ext.dense_tiles_ok(65, 6144, 2048) and not ext.dense_tiles_ok(17, 50304, 2048)   # more tiles than compute units
+    assert not ext.dense_tiles_ok(32, 64, 192) and not ext.dense_tiles_ok(0, 64, 128)
+    with pytest.raises(RuntimeError):
+        ext.dense_tiles(rnd(65, 2048, seed=1), rnd(6144, 2048, seed=2))
+    x, w = rnd(40, 256, seed=3), rnd(64, 512, seed=4)[:, ::2]
+    assert torch.equal(kernels.project(x, w), F.linear(x, w))   # weights that are not contiguous go to the library
+
+
 def model(seed, batch, **kw):
     s = D.Shape(**{**dict(vocab=1000, hidden=512, intermediate=256, layers=3, heads=8, kv_heads=8, head_dim=64, experts=64,
                           top_k=8), **kw})
