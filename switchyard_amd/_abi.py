@@ -47,6 +47,20 @@ class SyDecodeStep(ctypes.Structure):
                 + [("scratch_bytes", ctypes.c_size_t)])
 
 
+class SyPrompt(ctypes.Structure):
+    """A prompt's pass (csrc/passes.h)."""
+    _fields_ = ([(n, ctypes.c_int) for n in ("B", "T", "first", "capacity", "H", "heads", "kv_heads", "D", "k", "norm", "max_positions")]
+                + [("eps", ctypes.c_float), ("clip", ctypes.c_float)]
+                + [(n, ctypes.c_void_p) for n in ("cos", "sin", "positions", "real", "place", "map", "count", "scratch")]
+                + [("scratch_bytes", ctypes.c_size_t)])
+
+
+class SyPromptLayer(ctypes.Structure):
+    """A layer of a prompt's pass (csrc/passes.h)."""
+    _fields_ = [("E", ctypes.c_int), ("I", ctypes.c_int)] + [(n, ctypes.c_void_p) for n in (
+        "q_norm", "k_norm", "mlp_norm", "router", "gate_up", "down", "next_norm", "kcache", "vcache")]
+
+
 # name -> (restype, argtypes); mirrors include/switchyard_moe.h, include/switchyard_decode.h and csrc/passes.h
 SIGNATURES = {
     "sy_version": (_c_int, []),
@@ -99,6 +113,14 @@ SIGNATURES = {
     "sy_padding_twins": (_c_int, [_c_void_p, _c_void_p, _c_int, _c_int, _c_void_p, _c_void_p]),
     "sy_moe_add_rmsnorm": (_c_int, [ctypes.POINTER(SyMoeLayer), _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_float,
                                     _c_void_p, _c_void_p, _c_void_p]),
+    "sy_dense_gemm": (_c_int, [_c_void_p, _c_void_p, _c_int, _c_void_p, _c_int, _c_int, _c_void_p, _c_void_p]),
+    "sy_prompt_span": (_c_int, [_c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
+                                _c_void_p, _c_void_p]),
+    "sy_prompt_embed": (_c_int, [ctypes.POINTER(SyPrompt), _c_void_p, _c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p]),
+    "sy_prompt_attention": (_c_int, [ctypes.POINTER(SyPrompt), ctypes.POINTER(SyPromptLayer), _c_void_p, _c_void_p, _c_void_p,
+                                     _c_void_p]),
+    "sy_prompt_moe": (_c_int, [ctypes.POINTER(SyPrompt), ctypes.POINTER(SyPromptLayer), _c_void_p, _c_void_p, _c_void_p, _c_void_p,
+                               _c_void_p]),
     "sy_dense_tiles": (_c_int, [_c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_void_p, _c_void_p]),
     "sy_dense_tiles_takes": (_c_int, [_c_int, _c_int, _c_int]),
     "sy_dense_rows": (_c_int, [_c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_void_p, _c_void_p]),
@@ -872,6 +894,50 @@ class Ext:
                    out.data_ptr(), _stream())
         return out
 
+    def dense_gemm(self, x, weight, count=None):
+        """x [rows, K] @ weight [Nout, K]^T on the 256-row MFMA tile (K a multiple of 64 from 256 on); with count, an
+        int32 on the device, only the first count rows are computed."""
+        _check(x, "x", torch.float16)
+        _check(weight, "weight", torch.float16)
+        if x.dim() != 2 or weight.dim() != 2 or x.shape[1] != weight.shape[1]:
+            raise RuntimeError("dense_gemm: x [rows, K], weight [Nout, K]")
+        if count is not None:
+            _check(count, "count", torch.int32)
+        out = torch.empty((x.shape[0], weight.shape[0]), dtype=torch.float16, device=x.device)
+        self._call(self.lib.sy_dense_gemm, x.data_ptr(), weight.data_ptr(), x.shape[0],
+                   count.data_ptr() if count is not None else None, weight.shape[0], x.shape[1], out.data_ptr(), _stream())
+        return out
+
+    def prompt_span(self, tokens, real, first, cache_real, seen, pack=False):
+        """What a prompt's pass needs to know about its batch (csrc/prompt.hip): tokens int64 [B, T] at cache
+        positions first .. of cache_real [B, capacity] (bool, written there), real bool [B, T] or None, seen
+        int64 [B] -> (positions int64 [B*T], the positions behind them [B], rows). rows is None or, with
+        pack, (place [B*T], map [B*T], last [B], count [1]), int32: the rows that exist, where a batch's padding
+        with one token is one row."""
+        _check(tokens, "tokens", torch.int64)
+        _check(cache_real, "cache_real", torch.bool)
+        _check(seen, "seen", torch.int64)
+        B, T = tokens.shape
+        if real is not None:
+            _check(real, "real", torch.bool)
+        if cache_real.dim() != 2 or cache_real.shape[0] != B or seen.numel() != B or (real is not None and real.shape != tokens.shape):
+            raise RuntimeError("prompt_span: tokens and real [B, T], cache_real [B, capacity], seen [B]")
+        if pack and real is None:
+            raise RuntimeError("prompt_span: rows are packed by their mask")
+        positions = torch.empty(B * T, dtype=torch.int64, device=tokens.device)
+        after = torch.empty_like(seen)
+        rows = torch.empty(2 * B * T + 3 * B + 1, dtype=torch.int32, device=tokens.device) if pack else None
+        self._call(self.lib.sy_prompt_span, tokens.data_ptr(), real.data_ptr() if real is not None else None, B, T, int(first),
+                   cache_real.shape[1], seen.data_ptr(), cache_real.data_ptr(), positions.data_ptr(), after.data_ptr(),
+                   rows.data_ptr() if pack else None, _stream())
+        if not pack:
+            return positions, after, None
+        n = B * T
+        return positions, after, (rows[:n], rows[n:2 * n], rows[2 * n:2 * n + B], rows[2 * n + B:2 * n + B + 1])
+
+    def prompt_pass(self, *args, **kw):
+        return PromptPass(self, *args, **kw)
+
     STEP_MAX_ROWS = 16   # SY_STEP_MAX_ROWS: up to here every projection of a step is a weight stream
 
     def decode_step(self, tok, weights, wqkv, cos, sin, positions, slot, real, kcache, vcache, heads, kv_heads, head_dim, k,
@@ -932,3 +998,75 @@ class Ext:
             return None
         return (torch.empty(B * heads * 16 * (int(head_dim) + 2), dtype=torch.float32, device=device),
                 torch.zeros((launches, B * heads), dtype=torch.int32, device=device))
+
+
+class PromptPass:
+    """The launches of a prompt's pass that belong to its rows, two host calls a layer (csrc/prompt.hip); the projections
+    between them are the caller's. It holds every tensor whose address it uses. `rows`: prompt_span's, or None. A
+    layer's tensors are looked at when it is reached: the GPU is at work on the one before by then."""
+
+    def __init__(self, ext, layers, final_norm, tokens, positions, first, real, rows, kcache, vcache, cos, sin, heads, kv_heads,
+                 head_dim, k, norm, eps, clip):
+        f16 = torch.float16
+        B, T = tokens.shape
+        n, _, _, capacity, D = kcache.shape
+        H, qd, kvd = final_norm.numel(), heads * head_dim, kv_heads * head_dim
+        N, self.device = B * T, tokens.device
+        self._check([(kcache, f16, (n, B, kv_heads, capacity, D)), (vcache, f16, (n, B, kv_heads, capacity, D)),
+                     (real, torch.bool, (B, capacity)), (positions, torch.int64, (N,)), (cos, f16, (cos.shape[0], D)),
+                     (sin, f16, (cos.shape[0], D))])
+        if not tokens.is_cuda or D != head_dim or len(layers) != n:
+            raise RuntimeError("prompt_pass: tensors on the GPU, one cache per layer, caches of head_dim")
+        self.ext, self.lib, self.tokens, self.layers, self.final_norm = ext, ext.lib, tokens, layers, final_norm
+        self.H, self.qd, self.kvd = H, qd, kvd
+        bytes_ = max(self.lib.sy_moe_layer_scratch_bytes(N, E, k, H, I) for E, I in {(L["router"].shape[0], L["down"].shape[2]) for L in layers})
+        self.scratch = torch.empty(max(bytes_, 256), dtype=torch.uint8, device=self.device)
+        self.hold = (kcache, vcache, positions, real, rows, cos, sin)
+        self.x, self.xn, self.h = (torch.empty((N, H), dtype=f16, device=self.device) for _ in range(3))
+        self.q, self.a = (torch.empty((N, qd), dtype=f16, device=self.device) for _ in range(2))
+        place, map_, _, count = rows if rows is not None else (None,) * 4
+        ptr = lambda t: t.data_ptr() if t is not None else None
+        self.desc = SyPrompt(B, T, int(first), capacity, H, heads, kv_heads, D, int(k), int(bool(norm)), cos.shape[0], float(eps),
+                             float(clip or 0.0), cos.data_ptr(), sin.data_ptr(), positions.data_ptr(), real.data_ptr(), ptr(place),
+                             ptr(map_), ptr(count), self.scratch.data_ptr(), self.scratch.numel())
+        self.caches = (kcache.data_ptr(), vcache.data_ptr(), B * kv_heads * capacity * D * 2)
+        self.stream = _stream()
+
+    def _check(self, want):
+        for t, dtype, shape in want:
+            if t.dtype != dtype or t.shape != shape or t.device != self.device or not t.is_contiguous():
+                raise RuntimeError(f"prompt_pass: a contiguous {dtype} GPU tensor {tuple(shape)} was expected, got {t.dtype} "
+                                   f"{tuple(t.shape)} on {t.device}")
+
+    def _vector(self, t, entries):   # a norm, of any shape with that many entries
+        return t, torch.float16, t.shape if t.numel() == entries else (entries,)
+
+    def embed(self, table, weight):
+        """x = the tokens' embedding rows; returns their norm."""
+        self._check([(table, torch.float16, (table.shape[0], self.H)), self._vector(weight, self.H)])
+        self.ext._call(self.lib.sy_prompt_embed, self.desc, self.tokens.data_ptr(), table.data_ptr(), table.shape[0],
+                       weight.data_ptr(), self.x.data_ptr(), self.xn.data_ptr(), self.stream)
+        return self.xn
+
+    def attention(self, i, qkv):
+        """Layer i's q/k norm, rotary embedding, cache write and attention of qkv -> [rows, heads D]."""
+        L, f16, H = self.layers[i], torch.float16, self.H
+        E, I = L["router"].shape[0], L["down"].shape[2]
+        after = self.layers[i + 1]["attn_norm"] if i + 1 < len(self.layers) else self.final_norm
+        self._check([(qkv, f16, (self.x.shape[0], self.qd + 2 * self.kvd)), (L["router"], f16, (E, H)), (L["gate_up"], f16, (E, 2 * I, H)),
+                     (L["down"], f16, (E, H, I)), self._vector(L["q_norm"], self.qd), self._vector(L["k_norm"], self.kvd),
+                     self._vector(L["mlp_norm"], H), self._vector(after, H)])
+        k0, v0, each = self.caches
+        self.layer = SyPromptLayer(E, I, L["q_norm"].data_ptr(), L["k_norm"].data_ptr(), L["mlp_norm"].data_ptr(),
+                                   L["router"].data_ptr(), L["gate_up"].data_ptr(), L["down"].data_ptr(), after.data_ptr(),
+                                   k0 + i * each, v0 + i * each)
+        self.ext._call(self.lib.sy_prompt_attention, self.desc, self.layer, qkv.data_ptr(), self.q.data_ptr(), self.a.data_ptr(),
+                       self.stream)
+        return self.a
+
+    def moe(self, o):
+        """Adds o and the MoE layer (of the layer whose attention was the last) to the rows; returns the next norm of them."""
+        self._check([(o, torch.float16, self.x.shape)])
+        self.ext._call(self.lib.sy_prompt_moe, self.desc, self.layer, o.data_ptr(), self.x.data_ptr(), self.h.data_ptr(),
+                       self.xn.data_ptr(), self.stream)
+        return self.xn

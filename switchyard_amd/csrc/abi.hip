@@ -72,7 +72,7 @@ extern "C" SY_API int sy_moe_experts(const void* h, const void* router, void* lo
     SY_REQUIRE(!one_launch_front, "moe_experts: one_launch_front with a router is for at most 64 tokens");
     const bool counted = sy_router_route_counts(N, k) && sort_workspace && sort_workspace_bytes >= sy_sort_workspace_bytes(N, k, E);
     rc = sy_router_route_counting(h, router, N, H, E, k, norm, logits, idx, w, counted ? sort_workspace : nullptr, nullptr,
-                                  stream);
+                                  nullptr, stream);
     if (rc) return rc;
     rc = counted ? sy_sort_assign_counted(idx, w, N, k, E, counts, offsets, token, wsorted, pos_of, sort_workspace, stream)
                  : sy_sort_by_expert(idx, w, 2, N, k, E, counts, offsets, token, wsorted, pos_of, sort_workspace,
@@ -164,6 +164,11 @@ extern "C" SY_API int sy_moe_layer(const SyMoeLayer* L, const void* h, void* out
 // sort, the two projections, and combine + add + norm in one launch.
 extern "C" SY_API int sy_moe_add_rmsnorm(const SyMoeLayer* L, const void* h, const int32_t* twin, const void* x,
                                          const void* weight, float eps, void* x_out, void* h_out, void* stream) {
+  return sy_moe_add_rmsnorm_rows(L, h, twin, nullptr, x, weight, eps, x_out, h_out, stream);
+}
+
+int sy_moe_add_rmsnorm_rows(const SyMoeLayer* L, const void* h, const int32_t* twin, const int32_t* count, const void* x,
+                            const void* weight, float eps, void* x_out, void* h_out, void* stream) {
   SY_REQUIRE(L, "moe_add_rmsnorm: null layer");
   SY_REQUIRE(L->N >= 0 && L->E >= 1 && L->k >= 1 && L->H >= 8 && L->I >= 8, "moe_add_rmsnorm: N = %d, E = %d, k = %d, H = %d, I = %d",
              L->N, L->E, L->k, L->H, L->I);
@@ -180,7 +185,8 @@ extern "C" SY_API int sy_moe_add_rmsnorm(const SyMoeLayer* L, const void* h, con
   int32_t *token = (int32_t*)(b + s.token), *pos_of = (int32_t*)(b + s.pos_of);
   void *w = b + s.w, *wsorted = b + s.wsorted, *act = b + s.act, *y = b + s.y, *ws = b + s.sort_ws;
   const bool counted = sy_router_route_counts(N, k);
-  int rc = sy_router_route_counting(h, L->router, N, H, E, k, L->norm, b + s.logits, idx, w, counted ? ws : nullptr, twin, stream);
+  int rc = sy_router_route_counting(h, L->router, N, H, E, k, L->norm, b + s.logits, idx, w, counted ? ws : nullptr, twin, count,
+                                    stream);
   if (rc) return rc;
   rc = counted ? sy_sort_assign_counted(idx, w, N, k, E, counts, offsets, token, wsorted, pos_of, ws, stream)
                : sy_sort_by_expert(idx, w, 2, N, k, E, counts, offsets, token, wsorted, pos_of, ws, s.sort_bytes, stream);
@@ -191,8 +197,8 @@ extern "C" SY_API int sy_moe_add_rmsnorm(const SyMoeLayer* L, const void* h, con
   if (rc) return rc;
   rc = sy_grouped_gemm(act, nullptr, L->down, offsets, E, M, H, I, 0, combine_scales ? nullptr : wsorted, y, stream);
   if (rc) return rc;
-  return sy_combine_add_rmsnorm_twins(y, pos_of, idx, combine_scales ? w : nullptr, k, twin, x, weight, eps, N, H, x_out, h_out,
-                                      stream);
+  return sy_combine_add_rmsnorm_twins(y, pos_of, idx, combine_scales ? w : nullptr, k, twin, count, x, weight, eps, N, H, x_out,
+                                      h_out, stream);
 }
 
 // experts() of the reference in one call: sort, the two projections, combine, from the routing.

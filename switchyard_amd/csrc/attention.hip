@@ -90,7 +90,7 @@ template <int D, int STEP, bool WIDE>
 __global__ void __launch_bounds__(ATT_WAVES * WAVE, 2)
 prefill_attention_kernel(const half_t* __restrict__ q, const half_t* __restrict__ kcache, const half_t* __restrict__ vcache,
                          const uint8_t* __restrict__ real, int first, int T, int pairs, int heads, int kv_heads, int capacity,
-                         float scale_log2e, half_t* __restrict__ out) {
+                         float scale_log2e, half_t* __restrict__ out, const int* __restrict__ place) {
   constexpr int NW = ATT_WAVES;
   constexpr int ROW_BYTES = D * 2, CHUNKS = D / 8;        // 16-byte chunks of a row
   constexpr int TILE_BYTES = ATT_KEYS * ROW_BYTES;
@@ -123,8 +123,14 @@ prefill_attention_kernel(const half_t* __restrict__ q, const half_t* __restrict_
   // ---- the wavefront's queries: lane (half, l32) holds 8 halves of query l32 per K step
   const int tw = t0 + wave * ATT_QROWS, t = tw + l32;     // this lane's query
   const int tq = min(t, T - 1);
+  // with `place`, position r of the batch is row place[r], or (negative) one of the rows that exist once, ~place[r], of
+  // which another position writes the output (prompt.hip)
+  int row = b * T + tq;
+  if (place) row = place[row];
+  const bool own = row >= 0;
+  row = own ? row : ~row;
   half8_t qf[QSTEPS];
-  const half_t* qrow = q + ((size_t)b * T + tq) * ((size_t)heads * D) + (size_t)h * D + half * 8;
+  const half_t* qrow = q + (size_t)row * ((size_t)heads * D) + (size_t)h * D + half * 8;
 #pragma unroll
   for (int s = 0; s < QSTEPS; ++s) qf[s] = *reinterpret_cast<const half8_t*>(qrow + 16 * s);
   const int slot = first + tq;
@@ -283,8 +289,8 @@ prefill_attention_kernel(const half_t* __restrict__ q, const half_t* __restrict_
     alone = (i < last ? masks[i] : masks[i] & ((2ull << (slot - last * ATT_KEYS)) - 1)) == 0;
   const float inv = 1.f / l;
   if (!wave_live) return;
-  half_t* orow = out + ((size_t)b * T + tq) * ((size_t)heads * D) + (size_t)h * D;
-  const half_t* own = vcache + cache_at + (size_t)slot * D;
+  half_t* orow = out + (size_t)row * ((size_t)heads * D) + (size_t)h * D;
+  const half_t* own_value = vcache + cache_at + (size_t)slot * D;
 #pragma unroll
   for (int d = 0; d < DBLOCKS; ++d)
 #pragma unroll
@@ -303,8 +309,8 @@ prefill_attention_kernel(const half_t* __restrict__ q, const half_t* __restrict_
       const u4_t w = {x0[0], x1[0], x0[1], x1[1]};
       half8_t v = __builtin_bit_cast(half8_t, w);
       const int col = 32 * d + 8 * (g + half);
-      if (alone) v = *reinterpret_cast<const half8_t*>(own + col);
-      if (t < T) *reinterpret_cast<half8_t*>(orow + col) = v;
+      if (alone) v = *reinterpret_cast<const half8_t*>(own_value + col);
+      if (t < T && own) *reinterpret_cast<half8_t*>(orow + col) = v;
     }
 }
 
@@ -315,14 +321,14 @@ size_t att_lds_bytes(int positions, int D) {
 
 template <int D, int STEP, bool WIDE>
 int launch_prefill_attention(const half_t* q, const half_t* kc, const half_t* vc, const uint8_t* real, int first, int B, int T,
-                             int heads, int kv_heads, int capacity, half_t* out, hipStream_t st) {
+                             int heads, int kv_heads, int capacity, const int* place, half_t* out, hipStream_t st) {
   const int pairs = B * heads, rows = ATT_WAVES * ATT_QROWS, nblocks = (T + rows - 1) / rows;
   const size_t lds = att_lds_bytes(first + T, D);
   const auto kern = prefill_attention_kernel<D, STEP, WIDE>;
   if (lds > 48 * 1024 && hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
     return sy_fail(SY_ERR_LAUNCH, "prefill_attention: cannot reserve %zu bytes of LDS", lds);
   kern<<<(unsigned)(pairs * nblocks), ATT_WAVES * WAVE, lds, st>>>(q, kc, vc, real, first, T, pairs, heads, kv_heads, capacity,
-                                                          1.4426950408889634f / sqrtf((float)D), out);
+                                                          1.4426950408889634f / sqrtf((float)D), out, place);
   return sy_check_launch("prefill_attention");
 }
 
@@ -337,10 +343,10 @@ int launch_prefill_attention(const half_t* q, const half_t* kc, const half_t* vc
 // and 1500 positions, heads of 128; this kernel is not.)
 template <int D>
 int launch_steps(const half_t* q, const half_t* kc, const half_t* vc, const uint8_t* real, int first, int B, int T, int heads,
-                 int kv_heads, int capacity, half_t* out, hipStream_t st) {
+                 int kv_heads, int capacity, const int* place, half_t* out, hipStream_t st) {
   const int positions = first + T;
 #define SY_PREFILL(STEP_, WIDE_) \
-  launch_prefill_attention<D, STEP_, WIDE_>(q, kc, vc, real, first, B, T, heads, kv_heads, capacity, out, st)
+  launch_prefill_attention<D, STEP_, WIDE_>(q, kc, vc, real, first, B, T, heads, kv_heads, capacity, place, out, st)
   if (kv_heads != heads) return SY_PREFILL(64, true);
   if (positions <= 256 || (T <= 64 && positions <= 1024)) return SY_PREFILL(16, false);
   if constexpr (D == 128) {
@@ -359,6 +365,11 @@ extern "C" SY_API int sy_prefill_attention_takes(int positions, int capacity, in
 
 extern "C" SY_API int sy_prefill_attention(const void* q, const void* kcache, const void* vcache, const uint8_t* real, int first,
                                            int B, int T, int heads, int kv_heads, int D, int capacity, void* out, void* stream) {
+  return sy_prefill_attention_rows(q, kcache, vcache, real, first, B, T, heads, kv_heads, D, capacity, nullptr, out, stream);
+}
+
+int sy_prefill_attention_rows(const void* q, const void* kcache, const void* vcache, const uint8_t* real, int first, int B, int T,
+                              int heads, int kv_heads, int D, int capacity, const int32_t* place, void* out, void* stream) {
   SY_REQUIRE(B >= 0 && T >= 1 && heads >= 1 && kv_heads >= 1 && heads % kv_heads == 0,
              "prefill_attention: B = %d, T = %d, heads = %d, kv_heads = %d", B, T, heads, kv_heads);
   SY_REQUIRE(D == 64 || D == 128, "prefill_attention: head_dim must be 64 or 128 (got %d)", D);
@@ -372,6 +383,6 @@ extern "C" SY_API int sy_prefill_attention(const void* q, const void* kcache, co
   const half_t *qh = (const half_t*)q, *kc = (const half_t*)kcache, *vc = (const half_t*)vcache;
   half_t* o = (half_t*)out;
   hipStream_t st = (hipStream_t)stream;
-  return D == 128 ? launch_steps<128>(qh, kc, vc, real, first, B, T, heads, kv_heads, capacity, o, st)
-                  : launch_steps<64>(qh, kc, vc, real, first, B, T, heads, kv_heads, capacity, o, st);
+  return D == 128 ? launch_steps<128>(qh, kc, vc, real, first, B, T, heads, kv_heads, capacity, place, o, st)
+                  : launch_steps<64>(qh, kc, vc, real, first, B, T, heads, kv_heads, capacity, place, o, st);
 }

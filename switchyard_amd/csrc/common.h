@@ -29,7 +29,7 @@ int sy_sort_assign_counted(const int32_t* idx, const void* w, int N, int k, int 
                            int32_t* token, void* wsorted, int32_t* pos_of, void* workspace, void* stream);
 // front.hip: router logits + route in one launch; with `hist` also the sort's per-piece histograms
 int sy_router_route_counting(const void* h, const void* router, int N, int H, int E, int k, int norm, void* logits,
-                             int32_t* idx, void* w, void* hist, const int32_t* twin, void* stream);
+                             int32_t* idx, void* w, void* hist, const int32_t* twin, const int32_t* count, void* stream);
 bool sy_router_route_counts(int N, int k);
 // front.hip: whether that launch takes the shape (H a multiple of 512, at most 128 experts, top-8)
 bool sy_router_route_shape_ok(int N, int H, int E, int k);
@@ -42,8 +42,22 @@ int sy_embed_rmsnorm_step(const int64_t* tokens, const void* embed, int vocab, c
 int sy_add_rmsnorm_route(const void* x, const void* delta, const void* weight, float eps, const void* router, int E, int N,
                          int H, int k, int norm, void* x_out, void* h_out, void* logits, int32_t* idx, void* w, void* stream);
 int sy_combine_add_rmsnorm_twins(const void* y, const int32_t* pos_of, const int32_t* idx, const void* w, int k,
-                                 const int32_t* twin, const void* x, const void* weight, float eps, int N, int H,
-                                 void* x_out, void* h_out, void* stream);
+                                 const int32_t* twin, const int32_t* count, const void* x, const void* weight, float eps, int N,
+                                 int H, void* x_out, void* h_out, void* stream);
+// decode.hip: the row kernels of a packed batch of prompts (prompt.hip), of whose N rows the first *count exist
+int sy_embed_rmsnorm_packed(const int64_t* tokens, const int32_t* map, const int32_t* count, const void* embed, int vocab,
+                            const void* weight, float eps, int N, int H, void* x_out, void* h_out, void* stream);
+int sy_add_rmsnorm_counted(const void* x, const void* delta, const void* weight, float eps, int N, const int32_t* count, int H,
+                           void* x_out, void* h_out, void* stream);
+int sy_qk_norm_rope_prompt(const void* qkv, const void* q_norm, const void* k_norm, float eps, float clip, const void* cos_table,
+                           const void* sin_table, int max_positions, const int64_t* positions, int first, const int32_t* place, int B,
+                           int T, int heads, int kv_heads, int D, int capacity, void* q_out, void* kcache, void* vcache, void* stream);
+// attention.hip: sy_prefill_attention with the rows that exist
+int sy_prefill_attention_rows(const void* q, const void* kcache, const void* vcache, const uint8_t* real, int first, int B, int T,
+                              int heads, int kv_heads, int D, int capacity, const int32_t* place, void* out, void* stream);
+// abi.hip: sy_moe_add_rmsnorm for the first *count rows (all where count is null)
+int sy_moe_add_rmsnorm_rows(const SyMoeLayer* L, const void* h, const int32_t* twin, const int32_t* count, const void* x,
+                            const void* weight, float eps, void* x_out, void* h_out, void* stream);
 // decode.hip: router GEMM + route for a few rows (one workgroup per row)
 int sy_router_route_rows(const void* h, const void* router, int N, int H, int E, int k, int norm, void* logits, int32_t* idx,
                          void* w, void* stream);

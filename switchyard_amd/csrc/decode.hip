@@ -89,8 +89,10 @@ constexpr int ROW_MAX_K = 64;  // choices per token the combining variant ranks 
 // first, and a token's choices are ranked without LDS and their rows of y asked for together (combine_core.h):
 // one row 5.2 -> 4.4 us a launch, 8 rows 5.6 -> 5.0. It takes 26 more registers, and with many rows it is
 // the wavefronts in flight that count: 437 rows 6.7 -> 7.3, 4096 rows 31.9 -> 33.2.
+// COUNTED (and PACKED, which is EMBEDDED for such rows): only the first *count of the launch's rows exist (prompt.hip);
+// PACKED looks up row t by gather[map[t]].
 constexpr int FRONT_ROUTE = 1, FRONT_SORT = 2;
-constexpr int OWN_ROWS = 0, EMBEDDED = 1, TWINNED = 2;
+constexpr int OWN_ROWS = 0, EMBEDDED = 1, TWINNED = 2, COUNTED = 3, PACKED = 4;
 template <bool COMBINE, bool LOGITS, int FRONT = 0, int FROM = OWN_ROWS, bool FEW = false>
 __global__ void __launch_bounds__(LOGITS ? 1024 : ROW_THREADS)
 row_kernel(const half_t* x, const half_t* __restrict__ delta, const half_t* __restrict__ y,
@@ -98,12 +100,14 @@ row_kernel(const half_t* x, const half_t* __restrict__ delta, const half_t* __re
            float eps, const half_t* __restrict__ router, int E, int H, half_t* x_out, half_t* __restrict__ h_out,
            half_t* __restrict__ logits, const int64_t* __restrict__ gather, int src_rows,
            front_core::Outputs front = front_core::Outputs{}, const int* __restrict__ twin = nullptr,
-           unsigned* __restrict__ clear = nullptr, int nclear = 0) {  // x_out may be x
+           unsigned* __restrict__ clear = nullptr, int nclear = 0, const int* __restrict__ count = nullptr,
+           const int* __restrict__ map = nullptr) {  // x_out may be x
   extern __shared__ __attribute__((aligned(16))) half_t hs[];  // LOGITS: the normalised row [H]; FRONT: the tail's LDS behind it
   __shared__ __attribute__((aligned(16))) float part[16];
   __shared__ int rows[ROW_MAX_K];
   __shared__ float wts[ROW_MAX_K];   // COMBINE: the router weight of each row, 1 where y is already scaled
   const int t = blockIdx.x, tid = threadIdx.x, nthreads = blockDim.x;
+  if ((FROM == COUNTED || FROM == PACKED) && t >= *count) return;
   const size_t row = (size_t)t * H;
   const int chunks = H >> 3;
   half8_t v[MAX_CHUNKS], wn[MAX_CHUNKS];
@@ -120,11 +124,11 @@ row_kernel(const half_t* x, const half_t* __restrict__ delta, const half_t* __re
     own = combine_core::ranked(idx, pos_of, delta, (size_t)t * k, k);
   }
   const half_t* xrow = x + row;
-  if (FROM == EMBEDDED) {
-    long g = (long)gather[t];
+  if (FROM == EMBEDDED || FROM == PACKED) {
+    long g = (long)gather[FROM == PACKED ? map[t] : t];
     g = g < 0 ? 0 : g >= src_rows ? src_rows - 1 : g;
     xrow = x + (size_t)g * H;
-    if (t == 0)
+    if (FROM == EMBEDDED && t == 0)
       for (int i = tid; i < nclear; i += nthreads) clear[i] = 0;
   }
   if (COMBINE && !FEW) {
@@ -285,20 +289,29 @@ __device__ __forceinline__ half_t rotary_f16(half_t y, half_t rot, half_t cos_v,
 }
 
 // One workgroup per token. qkv row = [q (heads*D) | k (kv_heads*D) | v (kv_heads*D)].
+// PROMPT: the first token goes to cache position `first`. With `place`, rows of padding that are the same in every layer
+// exist once (prompt.hip): position r is row place[r], or, where it is one of those but not the first of them,
+// row ~place[r], of which only key and value are made again, for its own place in the cache.
+template <bool PROMPT>
 __global__ void __launch_bounds__(ROW_THREADS)
 qk_norm_rope_cache_kernel(const half_t* __restrict__ qkv, const half_t* __restrict__ q_norm,
                           const half_t* __restrict__ k_norm, float eps, float clip, const half_t* __restrict__ cos_t,
                           const half_t* __restrict__ sin_t, int max_positions, const int64_t* __restrict__ positions,
                           const int64_t* __restrict__ slot_ptr, int T, int heads, int kv_heads, int D, int capacity,
-                          half_t* __restrict__ q_out, half_t* __restrict__ kcache, half_t* __restrict__ vcache) {
+                          half_t* __restrict__ q_out, half_t* __restrict__ kcache, half_t* __restrict__ vcache,
+                          const int* __restrict__ place = nullptr, int first = 0) {
   extern __shared__ __attribute__((aligned(16))) half_t normed[];  // [qd + kvd] after norm and clamp
   __shared__ float part[32];
   // row r of qkv is token t = r % T of sequence b = r / T; it goes to cache position slot + t
   const int r = blockIdx.x, b = r / T;
   const int qd = heads * D, kvd = kv_heads * D;
-  const half_t* row = qkv + (size_t)r * (qd + 2 * kvd);
-  const int qchunks = qd >> 3, kchunks = kvd >> 3;
-  const long slot = (long)*slot_ptr + (r - b * T);
+  int at = r;
+  if (PROMPT && place) at = place[r];
+  const bool own = at >= 0;   // the same in the whole workgroup
+  at = own ? at : ~at;
+  const half_t* row = qkv + (size_t)at * (qd + 2 * kvd);
+  const int qchunks = own ? qd >> 3 : 0, kchunks = kvd >> 3;
+  const long slot = (PROMPT ? (long)first : (long)*slot_ptr) + (r - b * T);
   long pos = (long)positions[r];
   pos = pos < 0 ? 0 : pos >= max_positions ? max_positions - 1 : pos;
   const bool slot_ok = slot >= 0 && slot < capacity;
@@ -347,8 +360,7 @@ qk_norm_rope_cache_kernel(const half_t* __restrict__ qkv, const half_t* __restri
   const int half_d = D >> 1;
   const half_t* cs = cos_t + (size_t)pos * D;
   const half_t* sn = sin_t + (size_t)pos * D;
-  const int all = qchunks + kchunks;
-  for (int c = threadIdx.x; c < all; c += ROW_THREADS) {
+  for (int c = (own ? 0 : qd >> 3) + threadIdx.x; c < (qd >> 3) + kchunks; c += ROW_THREADS) {
     const int d0 = (c * 8) % D;  // qd is a multiple of D, so this also holds in the k part
     const half8_t y = *reinterpret_cast<const half8_t*>(normed + c * 8);
     const bool low = d0 < half_d;
@@ -361,9 +373,9 @@ qk_norm_rope_cache_kernel(const half_t* __restrict__ qkv, const half_t* __restri
       o[j] = rotary_f16(y[j], low ? -other[j] : other[j], cc[j], ssn[j]);
     }
     if (c < qchunks) {
-      *reinterpret_cast<half8_t*>(q_out + (size_t)r * qd + c * 8) = o;
+      *reinterpret_cast<half8_t*>(q_out + (size_t)at * qd + c * 8) = o;
     } else if (slot_ok) {
-      const int e = (c - qchunks) * 8, h = e / D;
+      const int e = (c - (qd >> 3)) * 8, h = e / D;
       *reinterpret_cast<half8_t*>(kcache + (((size_t)b * kv_heads + h) * capacity + slot) * D + (e - h * D)) = o;
     }
   }
@@ -836,6 +848,31 @@ extern "C" SY_API int sy_embed_rmsnorm(const int64_t* tokens, const void* embed,
   return sy_embed_rmsnorm_step(tokens, embed, vocab, weight, eps, N, H, x_out, h_out, nullptr, 0, stream);
 }
 
+// The rows of a packed batch of prompts (prompt.hip): the first *count of N, row t from tokens[map[t]].
+int sy_embed_rmsnorm_packed(const int64_t* tokens, const int32_t* map, const int32_t* count, const void* embed, int vocab,
+                            const void* weight, float eps, int N, int H, void* x_out, void* h_out, void* stream) {
+  ROW_LIMITS("embed_rmsnorm");
+  SY_REQUIRE(vocab >= 1, "embed_rmsnorm: vocab = %d", vocab);
+  if (N == 0) return SY_OK;
+  SY_REQUIRE(tokens && map && count && embed && weight && x_out && h_out, "embed_rmsnorm: null pointer");
+  row_kernel<false, false, 0, PACKED><<<N, ROW_THREADS, 0, (hipStream_t)stream>>>(
+      (const half_t*)embed, nullptr, nullptr, nullptr, nullptr, 0, (const half_t*)weight, eps, nullptr, 0, H, (half_t*)x_out,
+      (half_t*)h_out, nullptr, tokens, vocab, front_core::Outputs{}, nullptr, nullptr, 0, count, map);
+  return sy_check_launch("embed_rmsnorm");
+}
+
+int sy_add_rmsnorm_counted(const void* x, const void* delta, const void* weight, float eps, int N, const int32_t* count, int H,
+                           void* x_out, void* h_out, void* stream) {
+  if (!count) return sy_add_rmsnorm(x, delta, weight, eps, N, H, x_out, h_out, stream);
+  ROW_LIMITS("add_rmsnorm");
+  if (N == 0) return SY_OK;
+  SY_REQUIRE(x && weight && h_out, "add_rmsnorm: null pointer");
+  row_kernel<false, false, 0, COUNTED><<<N, ROW_THREADS, 0, (hipStream_t)stream>>>(
+      (const half_t*)x, (const half_t*)delta, nullptr, nullptr, nullptr, 0, (const half_t*)weight, eps, nullptr, 0, H,
+      (half_t*)x_out, (half_t*)h_out, nullptr, nullptr, 0, front_core::Outputs{}, nullptr, nullptr, 0, count, nullptr);
+  return sy_check_launch("add_rmsnorm");
+}
+
 extern "C" SY_API int sy_add_rmsnorm_logits(const void* x, const void* delta, const void* weight, float eps,
                                             const void* router, int E, int N, int H, void* x_out, void* h_out,
                                             void* logits, void* stream) {
@@ -985,24 +1022,26 @@ extern "C" SY_API int sy_add_rmsnorm_route_sort(const void* x, const void* delta
 }
 
 int sy_combine_add_rmsnorm_twins(const void* y, const int32_t* pos_of, const int32_t* idx, const void* w, int k,
-                                 const int32_t* twin, const void* x, const void* weight, float eps, int N, int H,
-                                 void* x_out, void* h_out, void* stream) {
+                                 const int32_t* twin, const int32_t* count, const void* x, const void* weight, float eps, int N,
+                                 int H, void* x_out, void* h_out, void* stream) {
   ROW_LIMITS("combine_add_rmsnorm");
   SY_REQUIRE(k >= 1 && k <= ROW_MAX_K, "combine_add_rmsnorm: 1 <= k <= %d (got %d)", ROW_MAX_K, k);
   if (N == 0) return SY_OK;
   SY_REQUIRE(y && pos_of && idx && x && weight && h_out, "combine_add_rmsnorm: null pointer");
+  SY_REQUIRE(!twin || !count, "combine_add_rmsnorm: rows that exist once have no twins");
   auto kern = twin ? row_kernel<true, false, 0, TWINNED>
+              : count ? row_kernel<true, false, 0, COUNTED>
               : N <= FEW_ROWS && k <= combine_core::AT_ONCE ? row_kernel<true, false, 0, OWN_ROWS, true> : row_kernel<true, false>;
   kern<<<N, ROW_THREADS, 0, (hipStream_t)stream>>>(
       (const half_t*)x, (const half_t*)w, (const half_t*)y, pos_of, idx, k, (const half_t*)weight, eps, nullptr, 0, H,
-      (half_t*)x_out, (half_t*)h_out, nullptr, nullptr, 0, front_core::Outputs{}, twin, nullptr, 0);
+      (half_t*)x_out, (half_t*)h_out, nullptr, nullptr, 0, front_core::Outputs{}, twin, nullptr, 0, count, nullptr);
   return sy_check_launch("combine_add_rmsnorm");
 }
 
 extern "C" SY_API int sy_combine_add_rmsnorm(const void* y, const int32_t* pos_of, const int32_t* idx, const void* w, int k,
                                              const void* x, const void* weight, float eps, int N, int H, void* x_out,
                                              void* h_out, void* stream) {
-  return sy_combine_add_rmsnorm_twins(y, pos_of, idx, w, k, nullptr, x, weight, eps, N, H, x_out, h_out, stream);
+  return sy_combine_add_rmsnorm_twins(y, pos_of, idx, w, k, nullptr, nullptr, x, weight, eps, N, H, x_out, h_out, stream);
 }
 
 // One workgroup per sequence of a batch of prompts. A row in front of its sequence's first real token
@@ -1046,11 +1085,9 @@ extern "C" SY_API int sy_padding_twins(const int64_t* tokens, const uint8_t* rea
   return sy_check_launch("padding_twins");
 }
 
-extern "C" SY_API int sy_qk_norm_rope_cache(const void* qkv, const void* q_norm, const void* k_norm, float eps, float clip,
-                                            const void* cos_table, const void* sin_table, int max_positions,
-                                            const int64_t* positions, const int64_t* slot, int B, int T, int heads,
-                                            int kv_heads, int D, int capacity, void* q_out, void* kcache, void* vcache,
-                                            void* stream) {
+static int qk_norm_check(const void* qkv, const void* q_norm, const void* k_norm, const void* cos_table, const void* sin_table,
+                         int max_positions, const int64_t* positions, int B, int T, int heads, int kv_heads, int D, int capacity,
+                         const void* q_out, const void* kcache, const void* vcache) {
   SY_REQUIRE(B >= 0 && T >= 1 && (long)B * T < (1l << 31) && heads >= 1 && kv_heads >= 1 && heads % kv_heads == 0,
              "qk_norm_rope_cache: B = %d, T = %d, heads = %d, kv_heads = %d", B, T, heads, kv_heads);
   SY_REQUIRE(D >= 16 && D % 16 == 0 && (long)heads * D <= 8 * ROW_THREADS * MAX_CHUNKS,
@@ -1059,14 +1096,43 @@ extern "C" SY_API int sy_qk_norm_rope_cache(const void* qkv, const void* q_norm,
   SY_REQUIRE(capacity >= 1 && max_positions >= 1, "qk_norm_rope_cache: capacity = %d, max_positions = %d", capacity,
              max_positions);
   if (B == 0) return SY_OK;
-  SY_REQUIRE(qkv && q_norm && k_norm && cos_table && sin_table && positions && slot && q_out && kcache && vcache,
+  SY_REQUIRE(qkv && q_norm && k_norm && cos_table && sin_table && positions && q_out && kcache && vcache,
              "qk_norm_rope_cache: null pointer");
+  return SY_OK;
+}
+
+extern "C" SY_API int sy_qk_norm_rope_cache(const void* qkv, const void* q_norm, const void* k_norm, float eps, float clip,
+                                            const void* cos_table, const void* sin_table, int max_positions,
+                                            const int64_t* positions, const int64_t* slot, int B, int T, int heads,
+                                            int kv_heads, int D, int capacity, void* q_out, void* kcache, void* vcache,
+                                            void* stream) {
+  if (int rc = qk_norm_check(qkv, q_norm, k_norm, cos_table, sin_table, max_positions, positions, B, T, heads, kv_heads, D, capacity,
+                             q_out, kcache, vcache))
+    return rc;
+  if (B == 0) return SY_OK;
+  SY_REQUIRE(slot, "qk_norm_rope_cache: null pointer");
   const size_t lds = (size_t)(heads + kv_heads) * D * sizeof(half_t);
-  qk_norm_rope_cache_kernel<<<B * T, ROW_THREADS, lds, (hipStream_t)stream>>>(
+  qk_norm_rope_cache_kernel<false><<<B * T, ROW_THREADS, lds, (hipStream_t)stream>>>(
       (const half_t*)qkv, (const half_t*)q_norm, (const half_t*)k_norm, eps, clip, (const half_t*)cos_table,
       (const half_t*)sin_table, max_positions, positions, slot, T, heads, kv_heads, D, capacity, (half_t*)q_out,
       (half_t*)kcache, (half_t*)vcache);
   return sy_check_launch("qk_norm_rope_cache");
+}
+
+// The same for a prompt whose first token goes to position `first`, with the rows that exist (`place`, or null: all).
+int sy_qk_norm_rope_prompt(const void* qkv, const void* q_norm, const void* k_norm, float eps, float clip, const void* cos_table,
+                           const void* sin_table, int max_positions, const int64_t* positions, int first, const int32_t* place, int B,
+                           int T, int heads, int kv_heads, int D, int capacity, void* q_out, void* kcache, void* vcache, void* stream) {
+  if (int rc = qk_norm_check(qkv, q_norm, k_norm, cos_table, sin_table, max_positions, positions, B, T, heads, kv_heads, D, capacity,
+                             q_out, kcache, vcache))
+    return rc;
+  if (B == 0) return SY_OK;
+  const size_t lds = (size_t)(heads + kv_heads) * D * sizeof(half_t);
+  qk_norm_rope_cache_kernel<true><<<B * T, ROW_THREADS, lds, (hipStream_t)stream>>>(
+      (const half_t*)qkv, (const half_t*)q_norm, (const half_t*)k_norm, eps, clip, (const half_t*)cos_table,
+      (const half_t*)sin_table, max_positions, positions, nullptr, T, heads, kv_heads, D, capacity, (half_t*)q_out,
+      (half_t*)kcache, (half_t*)vcache, place, first);
+  return sy_check_launch("qk_norm_rope_prompt");
 }
 
 // Whether the (sequence, head) pairs are too few to fill the chip with four wavefronts each: they then

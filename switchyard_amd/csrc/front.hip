@@ -82,7 +82,8 @@ front_kernel(const half_t* __restrict__ logits, int N, int E, int k, int norm, i
 // leaves the histogram of its choices where the sort's second launch expects it. `twin` names for
 // every token one that has the same row (itself, as a rule; for the padding of a batch of prompts
 // one row of that padding): a token that is not its own twin gets -1 for its choices, which the sort
-// passes over, so the experts see the row once and the combine reads the twin's results.
+// passes over, so the experts see the row once and the combine reads the twin's results. With `count` only the
+// first *count tokens exist; the others get -1 too, and nothing is computed for them.
 //
 // Fuses F.linear(h, router) + route() of the reference (switchyard/kernels.py:30-32,
 // switchyard/csrc/moe_kernels.cu:23-89) and count_kernel (:91-104).
@@ -94,7 +95,7 @@ template <int PER_LANE, int RR_WAVES>
 __global__ void __launch_bounds__(RR_WAVES * WAVE)
 router_route_kernel(const half_t* __restrict__ h, const half_t* __restrict__ router, int N, int H, int E, int k, int norm,
                     int nbits, int groups, half_t* __restrict__ logits, int* __restrict__ idx, half_t* __restrict__ w,
-                    int* __restrict__ hist_out, const int* __restrict__ twin) {
+                    int* __restrict__ hist_out, const int* __restrict__ twin, const int* __restrict__ count) {
   constexpr int EB = 4 * PER_LANE;             // blocks of 16 experts
   constexpr int RR_THREADS = RR_WAVES * WAVE;
   constexpr int EP = 16 * EB;                  // experts, padded
@@ -106,12 +107,13 @@ router_route_kernel(const half_t* __restrict__ h, const half_t* __restrict__ rou
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int row = lane & 15, kq = (lane >> 4) * 8;   // the operand row of this lane and its 8 halves of a K step
   const int kwave = H / RR_WAVES, steps = kwave / RR_KSTEP;   // a multiple of 4 steps per wavefront
+  const int live = count ? min(*count, N) : N;                // tokens that exist
   const __amdgpu_buffer_rsrc_t hrsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(h), 0, (int)((size_t)N * H * 2), 0x00020000);
   const __amdgpu_buffer_rsrc_t rrsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(router), 0, (int)((size_t)E * H * 2), 0x00020000);
 
   for (int g = 0; g < groups; ++g) {
     const int t0 = (blockIdx.x * groups + g) * RR_TOKENS;
-    if (t0 < N) {
+    if (t0 < live) {
       // ---- this wavefront's share of the dot products. Loads go through buffer descriptors: a
       // token past N or an expert past E is out of range and reads as 0
       const unsigned aoff = ((unsigned)(t0 + row) * (unsigned)H + (unsigned)(wave * kwave + kq)) * 2u;
@@ -152,7 +154,7 @@ router_route_kernel(const half_t* __restrict__ h, const half_t* __restrict__ rou
         for (int r = 0; r < 4; ++r) part[(wave * RR_TOKENS + 4 * (lane >> 4) + r) * EP + 16 * b + row] = acc[b][r];
     }
     __syncthreads();
-    if (t0 < N) {
+    if (t0 < live) {
       for (int o = tid; o < RR_TOKENS * EP; o += RR_THREADS) {
         const int tok = o / EP, e = o - tok * EP;
         float v = part[o];
@@ -160,7 +162,7 @@ router_route_kernel(const half_t* __restrict__ h, const half_t* __restrict__ rou
         for (int q = 1; q < RR_WAVES; ++q) v += part[q * RR_TOKENS * EP + o];
         const half_t hv = (half_t)v;
         lg[o] = hv;
-        if (t0 + tok < N && e < E) logits[(size_t)(t0 + tok) * E + e] = hv;
+        if (t0 + tok < live && e < E) logits[(size_t)(t0 + tok) * E + e] = hv;
       }
     }
     __syncthreads();
@@ -168,7 +170,7 @@ router_route_kernel(const half_t* __restrict__ h, const half_t* __restrict__ rou
     for (int tok = wave; tok < RR_TOKENS; tok += RR_WAVES) {
       const int t = t0 + tok;
       int my_e = -1;
-      if (t < N) {
+      if (t < live) {
         float my_w;
         route_core::route_token<half_t, PER_LANE>(lg + tok * EP, E, k, norm, my_e, my_w);
         if (twin && twin[t] != t) my_e = -1;   // another token's rows are this one's too: the sort passes it over
@@ -176,6 +178,8 @@ router_route_kernel(const half_t* __restrict__ h, const half_t* __restrict__ rou
           idx[(size_t)t * k + lane] = my_e;
           w[(size_t)t * k + lane] = (half_t)my_w;
         }
+      } else if (t < N && lane < k) {
+        idx[(size_t)t * k + lane] = -1;
       }
       if (lane < k) sidx[(g * RR_TOKENS + tok) * k + lane] = my_e;
     }
@@ -240,7 +244,8 @@ __device__ __forceinline__ void buffer_to_lds(int4v_t rsrc, unsigned voffset, un
 __global__ void __launch_bounds__(RS_THREADS)
 router_route_staged_kernel(const half_t* __restrict__ h, const half_t* __restrict__ router, int N, int H, int E, int k,
                            int norm, int nbits, int groups, half_t* __restrict__ logits, int* __restrict__ idx,
-                           half_t* __restrict__ w, int* __restrict__ hist_out, const int* __restrict__ twin) {
+                           half_t* __restrict__ w, int* __restrict__ hist_out, const int* __restrict__ twin,
+                           const int* __restrict__ count) {
   constexpr int EP = 64;
   constexpr unsigned OUT_OF_RANGE = 0x80000000u;
   extern __shared__ __attribute__((aligned(1024))) char lds_raw[];
@@ -249,7 +254,7 @@ router_route_staged_kernel(const half_t* __restrict__ h, const half_t* __restric
   int* sidx = reinterpret_cast<int*>(lg + RR_TOKENS * EP);                // [groups * RR_TOKENS * k]
   int* hist = sidx + groups * RR_TOKENS * k;                             // [E]
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int nk = H / RS_BK;
+  const int nk = H / RS_BK, live = count ? min(*count, N) : N;   // tokens that exist
   const unsigned lds_base = (unsigned)(size_t)(__attribute__((address_space(3))) char*)lds_raw;
   const int4v_t rrsrc = raw_descriptor(router, (unsigned)((size_t)E * H * 2));
   const int4v_t hrsrc = raw_descriptor(h, (unsigned)((size_t)N * H * 2));
@@ -262,7 +267,7 @@ router_route_staged_kernel(const half_t* __restrict__ h, const half_t* __restric
 
   for (int g = 0; g < groups; ++g) {
     const int t0 = (blockIdx.x * groups + g) * RR_TOKENS;
-    if (t0 < N) {
+    if (t0 < live) {
       // the row of the stage that this lane fetches a chunk of (rows 0..63 the router's, 64..79 the tokens')
       const int srow = 8 * wave + (lane >> 3);
       const unsigned chunk = (unsigned)((lane & 7) ^ ((srow >> 1) & 7));
@@ -311,18 +316,18 @@ router_route_staged_kernel(const half_t* __restrict__ h, const half_t* __restric
       }
     }
     __syncthreads();
-    if (t0 < N) {
+    if (t0 < live) {
       const int o = tid, tok = o / EP, e = o - tok * EP;   // RS_THREADS == RR_TOKENS * EP
       const half_t hv = (half_t)(part[o] + part[RR_TOKENS * EP + o]);
       lg[o] = hv;
-      if (t0 + tok < N && e < E) logits[(size_t)(t0 + tok) * E + e] = hv;
+      if (t0 + tok < live && e < E) logits[(size_t)(t0 + tok) * E + e] = hv;
     }
     __syncthreads();
     // ---- route: one wavefront per token
     {
       const int tok = wave, t = t0 + tok;
       int my_e = -1;
-      if (t < N) {
+      if (t < live) {
         float my_w;
         route_core::route_token<half_t, 1>(lg + tok * EP, E, k, norm, my_e, my_w);
         if (twin && twin[t] != t) my_e = -1;   // another token's rows are this one's too: the sort passes it over
@@ -330,6 +335,8 @@ router_route_staged_kernel(const half_t* __restrict__ h, const half_t* __restric
           idx[(size_t)t * k + lane] = my_e;
           w[(size_t)t * k + lane] = (half_t)my_w;
         }
+      } else if (t < N && lane < k) {
+        idx[(size_t)t * k + lane] = -1;
       }
       if (lane < k) sidx[(g * RR_TOKENS + tok) * k + lane] = my_e;
     }
@@ -352,7 +359,7 @@ bool router_route_shape_ok(int N, int H, int E, int k) {
 }
 
 int launch_router_route(const void* h, const void* router, int N, int H, int E, int k, int norm, void* logits,
-                        int32_t* idx, void* w, void* hist, const int32_t* twin, hipStream_t st) {
+                        int32_t* idx, void* w, void* hist, const int32_t* twin, const int32_t* count, hipStream_t st) {
   int nbits = 0;
   while ((1 << nbits) < E) ++nbits;
   const long M = (long)N * k;
@@ -367,7 +374,7 @@ int launch_router_route(const void* h, const void* router, int N, int H, int E, 
     if (hipFuncSetAttribute((const void*)router_route_staged_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
       return sy_fail(SY_ERR_LAUNCH, "router_route: cannot reserve %zu bytes of LDS", lds);
     router_route_staged_kernel<<<grid, RS_THREADS, lds, st>>>((const half_t*)h, (const half_t*)router, N, H, E, k, norm, nbits,
-                                                             groups, (half_t*)logits, idx, (half_t*)w, (int*)hist, twin);
+                                                             groups, (half_t*)logits, idx, (half_t*)w, (int*)hist, twin, count);
     return sy_check_launch("router_route");
   }
   const int EP = E <= 64 ? 64 : 128;
@@ -376,12 +383,12 @@ int launch_router_route(const void* h, const void* router, int N, int H, int E, 
   const size_t lds = sizeof(float) * waves * RR_TOKENS * EP + sizeof(half_t) * RR_TOKENS * EP +
                      sizeof(int) * ((size_t)groups * RR_TOKENS * k + E);
   void (*kern)(const half_t*, const half_t*, int, int, int, int, int, int, int, half_t*, int*, half_t*, int*,
-               const int*) =
+               const int*, const int*) =
       wide ? router_route_kernel<1, 16> : E <= 64 ? router_route_kernel<1, 4> : router_route_kernel<2, 4>;
   if (lds > 48 * 1024 && hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
     return sy_fail(SY_ERR_LAUNCH, "router_route: cannot reserve %zu bytes of LDS", lds);
   kern<<<grid, waves * WAVE, lds, st>>>((const half_t*)h, (const half_t*)router, N, H, E, k, norm, nbits, groups,
-                                        (half_t*)logits, idx, (half_t*)w, (int*)hist, twin);
+                                        (half_t*)logits, idx, (half_t*)w, (int*)hist, twin, count);
   return sy_check_launch("router_route");
 }
 
@@ -421,12 +428,12 @@ bool sy_router_route_counts(int N, int k) {
 }
 
 int sy_router_route_counting(const void* h, const void* router, int N, int H, int E, int k, int norm, void* logits,
-                             int32_t* idx, void* w, void* hist, const int32_t* twin, void* stream) {
+                             int32_t* idx, void* w, void* hist, const int32_t* twin, const int32_t* count, void* stream) {
   SY_REQUIRE(router_route_shape_ok(N, H, E, k),
              "router_route: H a multiple of 512, at most 128 experts and top-8 (got N = %d, H = %d, E = %d, k = %d)", N, H, E, k);
   SY_REQUIRE(h && router && logits && idx && w, "router_route: null pointer");
   SY_REQUIRE(!hist || sy_router_route_counts(N, k), "router_route: no histograms for N = %d, k = %d", N, k);
-  return launch_router_route(h, router, N, H, E, k, norm, logits, idx, w, hist, twin, (hipStream_t)stream);
+  return launch_router_route(h, router, N, H, E, k, norm, logits, idx, w, hist, twin, count, (hipStream_t)stream);
 }
 
 extern "C" SY_API int sy_router_route(const void* h, const void* router, int N, int H, int E, int k, int norm, void* logits,
@@ -434,5 +441,5 @@ extern "C" SY_API int sy_router_route(const void* h, const void* router, int N, 
   if (N == 0) return SY_OK;
   // a decode step: one workgroup per row (the kernels above take 16 rows to a workgroup)
   if (N <= 64) return sy_router_route_rows(h, router, N, H, E, k, norm, logits, idx, w, stream);
-  return sy_router_route_counting(h, router, N, H, E, k, norm, logits, idx, w, nullptr, nullptr, stream);
+  return sy_router_route_counting(h, router, N, H, E, k, norm, logits, idx, w, nullptr, nullptr, nullptr, stream);
 }

@@ -32,6 +32,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "passes.h"
 
 namespace {
 
@@ -420,6 +421,27 @@ __device__ __forceinline__ void scales_of_rows(const half_t* scale, int M, int f
   hi16 = pick(h + 16);
 }
 
+// Row tiles of a DENSE launch: `rows` rows cut into tiles of one height (a multiple of 32 up to 256), so that
+// the tiles, over all column tiles, fill the G workgroups' rounds: a tile costs its blocks of 32 rows and about one
+// and a half more, a launch its rounds times its tiles' cost. 3080 rows by 24 column tiles are 20 tiles of
+// 160 rows in two rounds, where 256 rows each would be two rounds as well, the second one a fifth full.
+__host__ __device__ __forceinline__ int dense_row_tiles(int rows, int ncol_tiles, int G) {
+  if (rows <= 0) return 0;
+  int tiles = (rows + BIG_BM - 1) / BIG_BM;
+  const int least = (int)(((long)tiles * ncol_tiles + G - 1) / G);
+  int best = least * (2 * (((rows + tiles - 1) / tiles + 31) / 32) + 3);
+  for (int r = least; r < least + 3; ++r) {
+    const int most = (int)((long)r * G / ncol_tiles);
+    if (most == 0) continue;
+    const int blocks = ((rows + most - 1) / most + 31) / 32, cost = r * (2 * blocks + 3);
+    if (blocks * 32 <= BIG_BM && cost < best) {
+      best = cost;
+      tiles = (rows + 32 * blocks - 1) / (32 * blocks);
+    }
+  }
+  return tiles;
+}
+
 template <int EPL>
 struct ExpertTable {
   int first[EPL], count[EPL], tiles[EPL], lo[EPL];  // lane x holds experts x, x + 64, ...
@@ -440,7 +462,9 @@ struct StreamTile {
 // is not issued. A compute unit takes one such load every 25 to 40 cycles, empty or not. The layer, us,
 // without and with: 437 tokens 166 -> 162, with uneven routing (Zipf, exponent 1.1) 190 -> 176; 768
 // tokens 181 -> 175 and 205 -> 191; at 1024 tokens the branches cost what the loads did (191, 194).
-template <bool SWIGLU, bool SCALE, int EPL, bool STREAMED, bool LOW = false>
+// DENSE: one matrix, and rows 0 .. count - 1 of A in their own order: count is *offsets, which only the device
+// knows, or M where offsets is null.
+template <bool SWIGLU, bool SCALE, int EPL, bool STREAMED, bool LOW = false, bool DENSE = false>
 __global__ void __launch_bounds__(512, 1)
 gemm_stream_kernel(const half_t* __restrict__ A, const int* __restrict__ a_rows, const half_t* __restrict__ B,
                    const int* __restrict__ offsets, int E, int M, int Nout, int K, const half_t* __restrict__ scale,
@@ -463,10 +487,16 @@ gemm_stream_kernel(const half_t* __restrict__ A, const int* __restrict__ a_rows,
 #pragma unroll
   for (int s = 0; s < EPL; ++s) {
     const int x = s * WAVE + lane;
-    const int f = x < E ? offsets[x] : 0, l = x < E ? offsets[x + 1] : 0;
+    int f = 0, l = 0;
+    if (DENSE) {
+      if (x == 0) l = offsets ? min(*offsets, M) : M;
+    } else if (x < E) {
+      f = offsets[x];
+      l = offsets[x + 1];
+    }
     tb.first[s] = f;
     tb.count[s] = l - f;
-    tb.tiles[s] = (l - f + BM - 1) / BM;
+    tb.tiles[s] = DENSE ? dense_row_tiles(l, ncol_tiles, gridDim.x) : (l - f + BM - 1) / BM;
     cls[s] = tb.tiles[s] ? (((l - f + tb.tiles[s] - 1) / tb.tiles[s] + 31) >> 5) : 0;
     tb.lo[s] = 0;
   }
@@ -936,6 +966,24 @@ int launch_gemm(const half_t* a, const int32_t* a_rows, const half_t* b, const i
 }
 
 }  // namespace
+
+// x f16 [rows, K] @ weight f16 [Nout, K]^T on the 256-row tile's stream; with `count` (device) only the first
+// *count rows.
+extern "C" SY_API int sy_dense_gemm(const void* x, const void* weight, int rows, const int32_t* count, int Nout, int K, void* out,
+                                    void* stream) {
+  SY_REQUIRE(rows >= 0 && Nout >= 1 && K >= 4 * BIG_BK && K % BIG_BK == 0, "dense_gemm: rows = %d, Nout = %d, K = %d (a multiple of %d from %d on)",
+             rows, Nout, K, BIG_BK, 4 * BIG_BK);
+  SY_REQUIRE((long)Nout * K * 2 < (1l << 31) && (long)rows * K * 2 < (1l << 31), "dense_gemm: an operand must stay under 2 GiB");
+  if (rows == 0) return SY_OK;
+  SY_REQUIRE(x && weight && out, "dense_gemm: null pointer");
+  const int ncol_tiles = (Nout + BW - 1) / BW, grid = sy_compute_units() / XCDS * XCDS;
+  const int tiles = dense_row_tiles(rows, ncol_tiles, grid);
+  const bool low = (rows + tiles - 1) / tiles <= 96;   // most of a tile's rows do not exist
+  const auto kern = low ? gemm_stream_kernel<false, false, 1, false, true, true> : gemm_stream_kernel<false, false, 1, false, false, true>;
+  kern<<<grid, 512, 0, (hipStream_t)stream>>>((const half_t*)x, nullptr, (const half_t*)weight, count, 1, rows, Nout, K, nullptr,
+                                              (half_t*)out, ncol_tiles);
+  return sy_check_launch("dense_gemm");
+}
 
 // Rows per tile. Where the 256-row tile takes the shape: 256 above 32 rows per expert, 64 up to that. Its
 // loads run three slices ahead, into the next tile, so it wants K in whole slices and four of them;

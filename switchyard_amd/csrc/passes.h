@@ -59,9 +59,50 @@ SY_API int sy_dense_rows(const void* x, const void* weight, int rows, int Nout, 
 SY_API int sy_dense_tiles(const void* x, const void* weight, int rows, int Nout, int K, void* out, void* stream);
 SY_API int sy_dense_tiles_takes(int rows, int Nout, int K);
 
+/* x f16 [rows, K] @ weight f16 [Nout, K]^T -> out f16 [rows, Nout] on the 256-row MFMA tile, K summed in order. count: int32
+ * on the device or null; only rows 0 .. min(rows, *count) - 1 are read and written. K a multiple of 64 from 256 on;
+ * each operand under 2 GiB. */
+SY_API int sy_dense_gemm(const void* x, const void* weight, int rows, const int32_t* count, int Nout, int K, void* out,
+                         void* stream);
+
 /* Whether decode attention's (sequence, head) pairs are few enough for sy_decode_attention_qkv_split to
  * deal their keys to several workgroups. */
 SY_API int sy_decode_attention_shares(int B, int heads);
+
+/* What a prompt's pass says about its batch, in two launches (one without `pack`): T new tokens of B sequences at cache
+ * positions first .. first + T - 1, real uint8 [B*T] (null: all) -> cache_real [B, capacity] at those positions,
+ * positions int64 [B*T] (index among a sequence's real tokens, behind seen int64 [B]; not below 0), next int64 [B] =
+ * seen + real tokens. pack int32 [2 B T + 3 B + 1] or null: place [B*T], map [B*T], last [B], count [1] and scratch.
+ * Rows of left padding with the token of the batch's first such row (sy_padding_twins says which) exist once:
+ * place[r] is position r's row among those that exist, in order, or ~row of the one that stands for it; map[i] is the
+ * position of row i, last[b] the row of (b, T - 1), *count the number of rows. */
+SY_API int sy_prompt_span(const int64_t* tokens, const uint8_t* real, int B, int T, int first, int capacity, const int64_t* seen,
+                          uint8_t* cache_real, int64_t* positions, int64_t* next, int32_t* pack, void* stream);
+
+/* A prompt's pass layer by layer, around projections that the caller makes: sy_prompt_embed (x = embedding rows, h =
+ * their norm), then per layer sy_prompt_attention (qkv f16 [N, (heads + 2 kv_heads) D] -> out [N, heads D]; q is
+ * scratch of that size) and sy_prompt_moe (o [N, H]: x += o, h = its norm, x += the MoE layer of h, xn = the next
+ * norm). N = B * T rows; where count, map and place (sy_prompt_span) are given only the first *count rows exist, and
+ * the others are neither read nor written. Limits: sy_prefill_attention's and sy_moe_add_rmsnorm's. */
+typedef struct SyPrompt {
+  int B, T, first, capacity, H, heads, kv_heads, D, k, norm, max_positions;
+  float eps, clip;
+  const void *cos, *sin;
+  const int64_t* positions;
+  const uint8_t* real;
+  const int32_t *place, *map, *count;
+  void* scratch; /* sy_moe_layer_scratch_bytes of the largest layer */
+  size_t scratch_bytes;
+} SyPrompt;
+typedef struct SyPromptLayer {
+  int E, I;
+  const void *q_norm, *k_norm, *mlp_norm, *router, *gate_up, *down, *next_norm;
+  void *kcache, *vcache; /* [B, kv_heads, capacity, D] */
+} SyPromptLayer;
+SY_API int sy_prompt_embed(const SyPrompt* p, const int64_t* tokens, const void* embed, int vocab, const void* weight, void* x, void* h,
+                           void* stream);
+SY_API int sy_prompt_attention(const SyPrompt* p, const SyPromptLayer* L, const void* qkv, void* q, void* out, void* stream);
+SY_API int sy_prompt_moe(const SyPrompt* p, const SyPromptLayer* L, const void* o, void* x, void* h, void* xn, void* stream);
 
 /* One decode step of a model of `layers` layers for B <= SY_STEP_MAX_ROWS sequences: tok int64 [B] -> out f16
  * [B, vocab] (logits), the new keys and values written at *slot and real[:, *slot] set; the counters

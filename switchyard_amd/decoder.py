@@ -180,6 +180,9 @@ class KVCache:
         self.capacity = capacity
 
 
+PACKED_GEMM_MIN_ROWS = 2048   # up to here the library's GEMM on every row is faster than own tiles on those that exist
+
+
 class Decoder:
     def __init__(self, shape, weights, moe=None, max_positions=4096, attention="auto"):
         """attention: "kernels" (the library's kernels for the decode step and for prompts), "torch"
@@ -261,8 +264,10 @@ class Decoder:
 
         s, W, E = self.s, self.w, kernels.ext()
         B, T = tokens.shape
-        span = Span(tokens, cache, valid)
         wqkv = self._stacked_qkv()
+        if self._takes_prompt_pass(tokens, cache, valid):
+            return self._prompt_pass(tokens.contiguous(), cache, valid, wqkv)
+        span = Span(tokens, cache, valid)
         slot = torch.tensor([span.first], dtype=torch.long, device=tokens.device)
         flat_positions = span.positions.reshape(-1).contiguous()
         tokens = tokens.contiguous()
@@ -303,6 +308,47 @@ class Decoder:
                 x, xn = E.add_rmsnorm(x, self.moe(i, h).contiguous(), after, s.rms_eps, x_out=x)
         span.commit(cache)
         return kernels.dense(xn.view(B, T, s.hidden)[:, -1].contiguous(), W["lm_head"])
+
+    def _takes_prompt_pass(self, tokens, cache, valid):
+        """Whether prefill_fused goes through `_prompt_pass`: what its kernels take of shapes, and a mask that means what
+        its bytes say."""
+        from . import kernels
+
+        s, E, L = self.s, kernels.ext(), self.w["layers"]
+        (B, T), (n, b, _, capacity, D), i64 = tokens.shape, cache.k.shape, torch.int64
+        experts = max(x["router"].shape[0] for x in L)
+        return (self._own_moe and B * T > kernels.OWN_ROUTER_MAX_TOKENS and tokens.dtype == i64 and (n, b) == (len(L), B)
+                and E.router_route_ok(B * T, s.hidden, experts, s.top_k) and E.prefill_attention_ok(cache.filled + T, capacity, D)
+                and cache.k.is_contiguous() and cache.v.is_contiguous() and cache.real.is_contiguous()
+                and cache.next_position.dtype == i64 and cache.next_position.is_contiguous()
+                and (valid is None or (valid.dtype == torch.bool and valid.shape == tokens.shape and valid.device == tokens.device))
+                and cache.real.device == tokens.device)
+
+    def _prompt_pass(self, tokens, cache, valid, wqkv):
+        """prefill_fused in two host calls a layer beside the projections. The padding of a batch that starts its cache is
+        one row for every launch (csrc/prompt.hip); which rows exist only the device knows, so the projections run on
+        its count where there is enough padding to win (own tiles: 3080 of 4096 rows, q/k/v and output 79 + 37 us, the
+        library's GEMM on all rows 97 + 37; without padding 109 + 38)."""
+        from . import kernels
+
+        s, W, E = self.s, self.w, kernels.ext()
+        B, T = tokens.shape
+        first = cache.filled
+        valid = valid.contiguous() if valid is not None else None
+        pack = B > 1 and valid is not None and first == 0
+        positions, after, rows = E.prompt_span(tokens, valid, first, cache.real, cache.next_position, pack)
+        p = E.prompt_pass(W["layers"], W["final_norm"], tokens, positions, first, cache.real, rows, cache.k, cache.v, self.cos, self.sin,
+                          s.heads, s.kv_heads, s.head_dim, s.top_k, s.norm_topk_prob, s.rms_eps, s.clip_qkv)
+        count = rows[3] if pack and B > 2 and B * T >= PACKED_GEMM_MIN_ROWS else None
+        project = kernels.project if count is None else lambda x, w: E.dense_gemm(x, w, count)
+        xn = p.embed(W["embed"], W["layers"][0]["attn_norm"])
+        for i in range(s.layers):
+            a = p.attention(i, project(xn, wqkv[i]))
+            xn = p.moe(project(a, W["layers"][i]["wo"]))
+        cache.filled = first + T
+        cache.next_position = after
+        last = xn.index_select(0, rows[2]) if pack else xn.view(B, T, s.hidden)[:, -1].contiguous()
+        return kernels.dense(last, W["lm_head"])
 
     def _prefill(self, tokens, cache, valid):
         """Logits of the last prompt position [B, vocab], on the kernels where they apply."""

@@ -640,6 +640,80 @@ def test_moe_layer_with_the_add_and_norm(N, pad, E, H, I, k):
         assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
 
 
+@pytest.mark.parametrize("B,T,other_tokens", [(1, 70, False), (2, 1, False), (5, 300, False), (8, 257, True), (70, 33, True), (3, 256, False)])
+@pytest.mark.parametrize("first,masked", [(0, True), (4, True), (4, False)])
+def test_prompt_span(B, T, other_tokens, first, masked):
+    """Mask, positions and the rows that exist, from their definitions; a row of nothing but padding, padding of several
+    tokens, holes behind the first real token."""
+    g = torch.Generator().manual_seed(B * T)
+    real = torch.arange(T)[None] >= torch.randint(0, T + 1, (B, 1), generator=g)
+    real[0] = False
+    real &= (torch.rand(B, T, generator=g) < 0.9) | (torch.arange(T)[None] < T // 2)
+    tokens = torch.randint(3, 9 if other_tokens else 4, (B, T), generator=g)
+    seen = torch.randint(0, 5, (B,), generator=g)
+    cache_real = torch.rand(B, first + T + 3, generator=g) < 0.5
+    got_real = cache_real.cuda()
+    valid = real if masked else torch.ones_like(real)
+    positions, after, rows = kernels.ext().prompt_span(tokens.cuda(), real.cuda() if masked else None, first, got_real, seen.cuda(), masked)
+    cache_real[:, first:first + T] = valid
+    order = valid.long().cumsum(1)
+    assert torch.equal(got_real.cpu(), cache_real)
+    assert torch.equal(positions.cpu().view(B, T), (seen[:, None] + order - 1).clamp(min=0))
+    assert torch.equal(after.cpu(), seen + order[:, -1])
+    if not masked:
+        assert rows is None
+        return
+    twin = twins_reference(tokens, real) if (~real[:, 0]).any() else torch.arange(B * T)
+    kept = [r for r in range(B * T) if twin[r] == r]
+    row_of = {r: i for i, r in enumerate(kept)}
+    place = torch.tensor([row_of[r] if r in row_of else ~row_of[int(twin[r])] for r in range(B * T)], dtype=torch.int32)
+    n = len(kept)
+    assert rows[3].item() == n and torch.equal(rows[0].cpu(), place) and rows[1][:n].tolist() == kept
+    assert torch.equal(rows[2].cpu(), torch.where(place < 0, ~place, place).view(B, T)[:, -1])
+
+
+@pytest.mark.parametrize("kw", [{}, dict(heads=4, kv_heads=2, head_dim=128, clip_qkv=0.5, experts=100), dict(norm_topk_prob=True, top_k=3)])
+@pytest.mark.parametrize("B,T,pad,own_gemm", [(1, 70, 0, False), (1, 70, 9, False), (4, 90, 40, False), (6, 300, 200, True), (3, 700, 5, True), (5, 64, 64, False)])
+def test_a_prompts_pass_equals_its_launches_one_by_one(kw, B, T, pad, own_gemm, monkeypatch):
+    """With the padding's rows and without them: the same logits, cache and counters, bit for bit, and a second prompt
+    behind the first."""
+    s, w, _ = model(7, 1, **kw)
+    dec = D.Decoder(s, w)
+    g = torch.Generator().manual_seed(B * T + pad)
+    lengths = torch.randint(T - pad, T + 1, (B,), generator=g)
+    lengths[-1] = T - pad
+    valid = (torch.arange(T)[None] >= (T - lengths)[:, None]).cuda()
+    tokens = torch.randint(3, s.vocab, (B, T), generator=g).cuda()
+    tokens = torch.where(valid | (tokens % 50 == 0), tokens, 0)   # some other tokens among the padding
+    outs = []
+    for apart in (False, True):
+        if own_gemm:   # the library's GEMM need not sum in the order of the tiles
+            monkeypatch.setattr(D, "PACKED_GEMM_MIN_ROWS", 0)
+            monkeypatch.setattr(kernels, "project", lambda x, weight: kernels.ext().dense_gemm(x, weight))
+        if apart:
+            monkeypatch.setattr(dec, "_takes_prompt_pass", lambda *a: False)
+        cache = D.KVCache(s, B, T + 75, torch.float16, "cuda")
+        first = dec.prefill_fused(tokens, cache, valid if pad else None)
+        more = dec.prefill_fused(tokens[:, -66:], cache)
+        outs.append((first, more, cache.k, cache.v, cache.real, cache.next_position, torch.tensor(cache.filled)))
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("rows,count,Nout,K", [(1, 1, 8, 256), (31, 31, 300, 256), (700, 0, 256, 256), (700, 1, 256, 256), (3000, 2111, 520, 320),
+                                              (5000, 5000, 1000, 256), (9000, 8999, 264, 512)])
+def test_dense_gemm_of_the_rows_that_exist(rows, count, Nout, K):
+    """Few and many tiles, one round and several, heights from 32 to 256: an in-order fp32 sum (the bound of
+    test_dense_tiles), and rows past the count untouched."""
+    x, w = rnd(rows, K, seed=81), rnd(Nout, K, seed=82, std=0.05)
+    x[count:] = float("nan")
+    n = torch.tensor([count], dtype=torch.int32, device="cuda")
+    got = kernels.ext().dense_gemm(x, w, n)[:count].double()
+    want, size = x[:count].double() @ w.double().T, x[:count].double().abs() @ w.double().abs().T
+    assert ((got - want).abs() <= want.abs() * 2.0 ** -11 + size * K * 2.0 ** -24 + 2.0 ** -24).all()
+    assert torch.equal(got.half(), kernels.ext().dense_gemm(x[:count].contiguous(), w))   # whatever tiles its count makes
+
+
 @pytest.mark.parametrize("rows,Nout,K", [(1, 6144, 2048), (8, 6144, 2048), (8, 2048, 2048), (16, 2048, 2048), (8, 50304, 2048),
                                         (8, 1000, 512), (3, 1001, 512), (17, 2048, 2048), (64, 6144, 2048),
                                         (64, 50304, 2048), (40, 1000, 512)])
