@@ -672,7 +672,8 @@ def test_prompt_span(B, T, other_tokens, first, masked):
     assert torch.equal(rows[2].cpu(), torch.where(place < 0, ~place, place).view(B, T)[:, -1])
 
 
-@pytest.mark.parametrize("kw", [{}, dict(heads=4, kv_heads=2, head_dim=128, clip_qkv=0.5, experts=100), dict(norm_topk_prob=True, top_k=3)])
+@pytest.mark.parametrize("kw", [{}, dict(heads=4, kv_heads=2, head_dim=128, clip_qkv=0.5, experts=100), dict(norm_topk_prob=True, top_k=3),
+                                dict(heads=40, kv_heads=8), dict(heads=3, kv_heads=1)])   # q rows of 2560: more than a chunk to a thread; of 192
 @pytest.mark.parametrize("B,T,pad,own_gemm", [(1, 70, 0, False), (1, 70, 9, False), (4, 90, 40, False), (6, 300, 200, True), (3, 700, 5, True), (5, 64, 64, False)])
 def test_a_prompts_pass_equals_its_launches_one_by_one(kw, B, T, pad, own_gemm, monkeypatch):
     """With the padding's rows and without them: the same logits, cache and counters, bit for bit, and a second prompt
