@@ -114,6 +114,7 @@ SIGNATURES = {
     "sy_moe_add_rmsnorm": (_c_int, [ctypes.POINTER(SyMoeLayer), _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_float,
                                     _c_void_p, _c_void_p, _c_void_p]),
     "sy_dense_gemm": (_c_int, [_c_void_p, _c_void_p, _c_int, _c_void_p, _c_int, _c_int, _c_void_p, _c_void_p]),
+    "sy_dense_gemm_takes": (_c_int, [_c_int, _c_int, _c_int]),
     "sy_prompt_span": (_c_int, [_c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
                                 _c_void_p, _c_void_p]),
     "sy_prompt_embed": (_c_int, [ctypes.POINTER(SyPrompt), _c_void_p, _c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p]),
@@ -893,6 +894,9 @@ class Ext:
         self._call(self.lib.sy_dense_tiles, x.data_ptr(), weight.data_ptr(), x.shape[0], weight.shape[0], x.shape[1],
                    out.data_ptr(), _stream())
         return out
+
+    def dense_gemm_ok(self, rows, Nout, K):
+        return bool(self.lib.sy_dense_gemm_takes(int(rows), int(Nout), int(K)))
 
     def dense_gemm(self, x, weight, count=None):
         """x [rows, K] @ weight [Nout, K]^T on the 256-row MFMA tile (K a multiple of 64 from 256 on); with count, an

@@ -967,13 +967,16 @@ int launch_gemm(const half_t* a, const int32_t* a_rows, const half_t* b, const i
 
 }  // namespace
 
+extern "C" SY_API int sy_dense_gemm_takes(int rows, int Nout, int K) {
+  return rows >= 0 && Nout >= 1 && K >= 4 * BIG_BK && K % BIG_BK == 0 && (long)Nout * K * 2 < (1l << 31) && (long)rows * K * 2 < (1l << 31);
+}
+
 // x f16 [rows, K] @ weight f16 [Nout, K]^T on the 256-row tile's stream; with `count` (device) only the first
 // *count rows.
 extern "C" SY_API int sy_dense_gemm(const void* x, const void* weight, int rows, const int32_t* count, int Nout, int K, void* out,
                                     void* stream) {
-  SY_REQUIRE(rows >= 0 && Nout >= 1 && K >= 4 * BIG_BK && K % BIG_BK == 0, "dense_gemm: rows = %d, Nout = %d, K = %d (a multiple of %d from %d on)",
+  SY_REQUIRE(sy_dense_gemm_takes(rows, Nout, K), "dense_gemm: rows = %d, Nout = %d, K = %d: K a multiple of %d from %d on, operands under 2 GiB",
              rows, Nout, K, BIG_BK, 4 * BIG_BK);
-  SY_REQUIRE((long)Nout * K * 2 < (1l << 31) && (long)rows * K * 2 < (1l << 31), "dense_gemm: an operand must stay under 2 GiB");
   if (rows == 0) return SY_OK;
   SY_REQUIRE(x && weight && out, "dense_gemm: null pointer");
   const int ncol_tiles = (Nout + BW - 1) / BW, grid = sy_compute_units() / XCDS * XCDS;

@@ -61,7 +61,8 @@ SY_API int sy_dense_tiles_takes(int rows, int Nout, int K);
 
 /* x f16 [rows, K] @ weight f16 [Nout, K]^T -> out f16 [rows, Nout] on the 256-row MFMA tile, K summed in order. count: int32
  * on the device or null; only rows 0 .. min(rows, *count) - 1 are read and written. K a multiple of 64 from 256 on;
- * each operand under 2 GiB. */
+ * each operand under 2 GiB (sy_dense_gemm_takes). */
+SY_API int sy_dense_gemm_takes(int rows, int Nout, int K);
 SY_API int sy_dense_gemm(const void* x, const void* weight, int rows, const int32_t* count, int Nout, int K, void* out,
                          void* stream);
 

@@ -339,7 +339,10 @@ class Decoder:
         positions, after, rows = E.prompt_span(tokens, valid, first, cache.real, cache.next_position, pack)
         p = E.prompt_pass(W["layers"], W["final_norm"], tokens, positions, first, cache.real, rows, cache.k, cache.v, self.cos, self.sin,
                           s.heads, s.kv_heads, s.head_dim, s.top_k, s.norm_topk_prob, s.rms_eps, s.clip_qkv)
-        count = rows[3] if pack and B > 2 and B * T >= PACKED_GEMM_MIN_ROWS else None
+        count = None
+        if (pack and B > 2 and B * T >= PACKED_GEMM_MIN_ROWS
+                and all(E.dense_gemm_ok(B * T, *t.shape) for t in (wqkv[0], W["layers"][0]["wo"]))):
+            count = rows[3]
         project = kernels.project if count is None else lambda x, w: E.dense_gemm(x, w, count)
         xn = p.embed(W["embed"], W["layers"][0]["attn_norm"])
         for i in range(s.layers):

@@ -690,7 +690,8 @@ def test_a_prompts_pass_equals_its_launches_one_by_one(kw, B, T, pad, own_gemm, 
     for apart in (False, True):
         if own_gemm:   # the library's GEMM need not sum in the order of the tiles
             monkeypatch.setattr(D, "PACKED_GEMM_MIN_ROWS", 0)
-            monkeypatch.setattr(kernels, "project", lambda x, weight: kernels.ext().dense_gemm(x, weight))
+            monkeypatch.setattr(kernels, "project", lambda x, weight: (
+                kernels.ext().dense_gemm if s.heads * s.head_dim >= 256 else kernels.dense)(x, weight))
         if apart:
             monkeypatch.setattr(dec, "_takes_prompt_pass", lambda *a: False)
         cache = D.KVCache(s, B, T + 75, torch.float16, "cuda")
