@@ -49,7 +49,8 @@ class SyDecodeStep(ctypes.Structure):
 
 class SyPrompt(ctypes.Structure):
     """A prompt's pass (csrc/passes.h)."""
-    _fields_ = ([(n, ctypes.c_int) for n in ("B", "T", "first", "capacity", "H", "heads", "kv_heads", "D", "k", "norm", "max_positions")]
+    _fields_ = ([(n, ctypes.c_int) for n in ("B", "T", "first", "capacity", "H", "heads", "kv_heads", "D", "k", "norm", "max_positions",
+                                             "gemv_max_rows")]
                 + [("eps", ctypes.c_float), ("clip", ctypes.c_float)]
                 + [(n, ctypes.c_void_p) for n in ("cos", "sin", "positions", "real", "place", "map", "count", "scratch")]
                 + [("scratch_bytes", ctypes.c_size_t)])
@@ -942,6 +943,7 @@ class Ext:
     def prompt_pass(self, *args, **kw):
         return PromptPass(self, *args, **kw)
 
+    PROMPT_FEW_ROWS = 64   # SY_PROMPT_FEW_ROWS: prompts of so few rows go through the launches of a decode step
     STEP_MAX_ROWS = 16   # SY_STEP_MAX_ROWS: up to here every projection of a step is a weight stream
 
     def decode_step(self, tok, weights, wqkv, cos, sin, positions, slot, real, kcache, vcache, heads, kv_heads, head_dim, k,
@@ -1010,7 +1012,7 @@ class PromptPass:
     layer's tensors are looked at when it is reached: the GPU is at work on the one before by then."""
 
     def __init__(self, ext, layers, final_norm, tokens, positions, first, real, rows, kcache, vcache, cos, sin, heads, kv_heads,
-                 head_dim, k, norm, eps, clip):
+                 head_dim, k, norm, eps, clip, gemv_max_rows):
         f16 = torch.float16
         B, T = tokens.shape
         n, _, _, capacity, D = kcache.shape
@@ -1030,8 +1032,8 @@ class PromptPass:
         self.q, self.a = (torch.empty((N, qd), dtype=f16, device=self.device) for _ in range(2))
         place, map_, _, count = rows if rows is not None else (None,) * 4
         ptr = lambda t: t.data_ptr() if t is not None else None
-        self.desc = SyPrompt(B, T, int(first), capacity, H, heads, kv_heads, D, int(k), int(bool(norm)), cos.shape[0], float(eps),
-                             float(clip or 0.0), cos.data_ptr(), sin.data_ptr(), positions.data_ptr(), real.data_ptr(), ptr(place),
+        self.desc = SyPrompt(B, T, int(first), capacity, H, heads, kv_heads, D, int(k), int(bool(norm)), cos.shape[0],
+                             int(gemv_max_rows), float(eps), float(clip or 0.0), cos.data_ptr(), sin.data_ptr(), positions.data_ptr(), real.data_ptr(), ptr(place),
                              ptr(map_), ptr(count), self.scratch.data_ptr(), self.scratch.numel())
         self.caches = (kcache.data_ptr(), vcache.data_ptr(), B * kv_heads * capacity * D * 2)
         self.stream = _stream()

@@ -201,6 +201,45 @@ int sy_moe_add_rmsnorm_rows(const SyMoeLayer* L, const void* h, const int32_t* t
                                       h_out, stream);
 }
 
+// Up to 64 choices the front only routes and the gate/up stream sorts for itself, as in sy_moe_layer; the weight stream leaves
+// the router weights to the combine, the MFMA tiles apply them.
+int sy_few_rows_moe(void* x, const void* o, const void* mlp_norm, float eps, const void* router, int N, int H, int I, int E, int k, int norm,
+                    const void* gate_up, const void* down, const void* next_norm, bool stream_experts, const SyFewRows& s, void* xn,
+                    void* stream) {
+  const int M = N * k;
+  int rc;
+  if (stream_experts && sy_gemv_sorts(N, k, E, H)) {
+    rc = sy_add_rmsnorm_route(x, o, mlp_norm, eps, router, E, N, H, k, norm, x, s.h, s.logits, s.idx, s.w, stream);
+    if (!rc)
+      rc = sy_grouped_gemv_sorting(s.h, s.idx, s.w, N, k, gate_up, E, I, H, s.counts, s.offsets, s.token, s.wsorted, s.pos_of, s.act, stream);
+  } else {
+    rc = sy_add_rmsnorm_route_sort(x, o, mlp_norm, eps, router, E, N, H, k, norm, x, s.h, s.logits, s.idx, s.w, s.counts, s.offsets,
+                                   s.token, s.wsorted, s.pos_of, stream);
+    if (!rc)
+      rc = stream_experts ? sy_grouped_gemv(s.h, s.token, gate_up, s.offsets, E, M, N, I, H, 1, nullptr, s.act, stream)
+                          : sy_grouped_gemm(s.h, s.token, gate_up, s.offsets, E, M, I, H, 1, nullptr, s.act, stream);
+  }
+  if (!rc)
+    rc = stream_experts ? sy_grouped_gemv(s.act, nullptr, down, s.offsets, E, M, N, H, I, 0, nullptr, s.y, stream)
+                        : sy_grouped_gemm(s.act, nullptr, down, s.offsets, E, M, H, I, 0, s.wsorted, s.y, stream);
+  if (!rc) rc = sy_combine_add_rmsnorm(s.y, s.pos_of, s.idx, stream_experts ? s.w : nullptr, k, x, next_norm, eps, N, H, x, xn, stream);
+  return rc;
+}
+
+int sy_few_rows_moe_layer(const SyMoeLayer* L, void* x, const void* o, const void* mlp_norm, float eps, const void* next_norm, void* h, void* xn,
+                          void* stream) {
+  SY_REQUIRE(L->N >= 1 && L->E >= 1 && L->k >= 1 && L->H >= 8 && L->I >= 8, "few_rows_moe: N = %d, E = %d, k = %d, H = %d, I = %d", L->N, L->E,
+             L->k, L->H, L->I);
+  const LayerScratch s = layer_scratch(L->N, L->E, L->k, L->H, L->I);
+  SY_REQUIRE(L->scratch && L->scratch_bytes >= s.end && ((uintptr_t)L->scratch & 255) == 0,
+             "few_rows_moe: scratch of %zu bytes, 256-byte aligned, needed (%zu given)", s.end, L->scratch_bytes);
+  char* b = (char*)L->scratch;
+  const SyFewRows few = {h, b + s.logits, b + s.w, b + s.wsorted, b + s.act, b + s.y, (int32_t*)(b + s.idx), (int32_t*)(b + s.counts),
+                         (int32_t*)(b + s.offsets), (int32_t*)(b + s.token), (int32_t*)(b + s.pos_of)};
+  return sy_few_rows_moe(x, o, mlp_norm, eps, L->router, L->N, L->H, L->I, L->E, L->k, L->norm, L->gate_up, L->down, next_norm,
+                         !L->mfma_tiles, few, xn, stream);
+}
+
 // experts() of the reference in one call: sort, the two projections, combine, from the routing.
 extern "C" SY_API int sy_experts_routed(const void* h, int N, int E, int k, const void* gate_up, const void* down, int H, int I,
                                         int mfma_tiles, const int32_t* idx, const void* w, int32_t* counts, int32_t* offsets,

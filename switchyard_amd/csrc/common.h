@@ -55,6 +55,19 @@ int sy_qk_norm_rope_prompt(const void* qkv, const void* q_norm, const void* k_no
 // attention.hip: sy_prefill_attention with the rows that exist
 int sy_prefill_attention_rows(const void* q, const void* kcache, const void* vcache, const uint8_t* real, int first, int B, int T,
                               int heads, int kv_heads, int D, int capacity, const int32_t* place, void* out, void* stream);
+// abi.hip: the MoE layer of a few rows (at most 64, 128 experts, top-8) between its norms: x += o, h = norm, route and sort, the
+// two projections (a weight stream or the MFMA tiles), x += their combination, xn = the next norm. x is updated in
+// place; the other buffers are scratch.
+struct SyFewRows {
+  void *h, *logits, *w, *wsorted, *act, *y;
+  int32_t *idx, *counts, *offsets, *token, *pos_of;
+};
+int sy_few_rows_moe(void* x, const void* o, const void* mlp_norm, float eps, const void* router, int N, int H, int I, int E, int k, int norm,
+                    const void* gate_up, const void* down, const void* next_norm, bool stream_experts, const SyFewRows& s, void* xn,
+                    void* stream);
+// abi.hip: the same in a layer's scratch
+int sy_few_rows_moe_layer(const SyMoeLayer* L, void* x, const void* o, const void* mlp_norm, float eps, const void* next_norm, void* h, void* xn,
+                          void* stream);
 // abi.hip: sy_moe_add_rmsnorm for the first *count rows (all where count is null)
 int sy_moe_add_rmsnorm_rows(const SyMoeLayer* L, const void* h, const int32_t* twin, const int32_t* count, const void* x,
                             const void* weight, float eps, void* x_out, void* h_out, void* stream);

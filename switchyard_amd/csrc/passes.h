@@ -84,9 +84,12 @@ SY_API int sy_prompt_span(const int64_t* tokens, const uint8_t* real, int B, int
  * their norm), then per layer sy_prompt_attention (qkv f16 [N, (heads + 2 kv_heads) D] -> out [N, heads D]; q is
  * scratch of that size) and sy_prompt_moe (o [N, H]: x += o, h = its norm, x += the MoE layer of h, xn = the next
  * norm). N = B * T rows; where count, map and place (sy_prompt_span) are given only the first *count rows exist, and
- * the others are neither read nor written. Limits: sy_prefill_attention's and sy_moe_add_rmsnorm's. */
+ * the others are neither read nor written. Up to SY_PROMPT_FEW_ROWS rows all of them exist, and the experts run on the
+ * weight stream up to gemv_max_rows. Limits: sy_prefill_attention's, and sy_moe_add_rmsnorm's or, for few rows, those of a
+ * decode step. */
+#define SY_PROMPT_FEW_ROWS 64
 typedef struct SyPrompt {
-  int B, T, first, capacity, H, heads, kv_heads, D, k, norm, max_positions;
+  int B, T, first, capacity, H, heads, kv_heads, D, k, norm, max_positions, gemv_max_rows;
   float eps, clip;
   const void *cos, *sin;
   const int64_t* positions;

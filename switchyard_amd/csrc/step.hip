@@ -83,8 +83,8 @@ extern "C" SY_API int sy_decode_step(const SyDecodeStep* step, const SyDecodeLay
   int32_t *token = (int32_t*)(b + at.token), *pos_of = (int32_t*)(b + at.pos_of);
   const bool shares = sy_decode_attention_shares(s.B, s.heads);
   void *parts = shares ? b + at.parts : nullptr, *tickets = shares ? b + at.tickets : nullptr;
-  const int B = s.B, H = s.H, I = s.I, E = s.E, k = s.k, M = B * k, qd = s.heads * s.D, kvd = s.kv_heads * s.D;
-  const bool stream_experts = B <= s.gemv_max_rows, sorts = stream_experts && sy_gemv_sorts(B, k, E, H);
+  const int B = s.B, H = s.H, I = s.I, E = s.E, k = s.k, qd = s.heads * s.D, kvd = s.kv_heads * s.D;
+  const bool stream_experts = B <= s.gemv_max_rows;
 
   int rc = sy_embed_rmsnorm_step(s.tok, s.embed, s.embed_rows, s.first_norm, s.eps, B, H, x, xn, (unsigned*)tickets,
                                  shares ? B * s.heads : 0, stream);
@@ -98,23 +98,9 @@ extern "C" SY_API int sy_decode_step(const SyDecodeStep* step, const SyDecodeLay
                                          tickets, stream);
     if (!rc) rc = sy_dense_rows(a, L.wo, B, H, qd, o, stream);
     if (rc) break;
-    if (sorts) {
-      rc = sy_add_rmsnorm_route(x, o, L.mlp_norm, s.eps, L.router, E, B, H, k, s.norm, x, h, logits, idx, w, stream);
-      if (!rc)
-        rc = sy_grouped_gemv_sorting(h, idx, w, B, k, L.gate_up, E, I, H, counts, offsets, token, wsorted, pos_of, act, stream);
-    } else {
-      rc = sy_add_rmsnorm_route_sort(x, o, L.mlp_norm, s.eps, L.router, E, B, H, k, s.norm, x, h, logits, idx, w, counts, offsets,
-                                     token, wsorted, pos_of, stream);
-      if (!rc)
-        rc = stream_experts ? sy_grouped_gemv(h, token, L.gate_up, offsets, E, M, B, I, H, 1, nullptr, act, stream)
-                            : sy_grouped_gemm(h, token, L.gate_up, offsets, E, M, I, H, 1, nullptr, act, stream);
-    }
-    // the weight stream leaves the router weights to the combine, the MFMA tiles apply them
-    if (!rc)
-      rc = stream_experts ? sy_grouped_gemv(act, nullptr, L.down, offsets, E, M, B, H, I, 0, nullptr, y, stream)
-                          : sy_grouped_gemm(act, nullptr, L.down, offsets, E, M, H, I, 0, wsorted, y, stream);
-    if (!rc)
-      rc = sy_combine_add_rmsnorm(y, pos_of, idx, stream_experts ? w : nullptr, k, x, L.next_norm, s.eps, B, H, x, xn, stream);
+    const SyFewRows few = {h, logits, w, wsorted, act, y, idx, counts, offsets, token, pos_of};
+    rc = sy_few_rows_moe(x, o, L.mlp_norm, s.eps, L.router, B, H, I, E, k, s.norm, L.gate_up, L.down, L.next_norm, stream_experts, few, xn,
+                         stream);
   }
   if (!rc) rc = sy_dense_rows(xn, s.lm_head, B, s.vocab, H, s.out, stream);
   return rc;

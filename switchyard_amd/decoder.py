@@ -316,9 +316,12 @@ class Decoder:
 
         s, E, L = self.s, kernels.ext(), self.w["layers"]
         (B, T), (n, b, _, capacity, D), i64 = tokens.shape, cache.k.shape, torch.int64
-        experts = max(x["router"].shape[0] for x in L)
-        return (self._own_moe and B * T > kernels.OWN_ROUTER_MAX_TOKENS and tokens.dtype == i64 and (n, b) == (len(L), B)
-                and E.router_route_ok(B * T, s.hidden, experts, s.top_k) and E.prefill_attention_ok(cache.filled + T, capacity, D)
+        experts = [x["router"].shape[0] for x in L]
+        if B * T > kernels.OWN_ROUTER_MAX_TOKENS:
+            takes = B * T > E.PROMPT_FEW_ROWS and E.router_route_ok(B * T, s.hidden, max(experts), s.top_k)
+        else:
+            takes = 1 <= B * T <= E.PROMPT_FEW_ROWS and max(experts) <= 128 and s.top_k <= min(8, *experts)
+        return (self._own_moe and takes and tokens.dtype == i64 and (n, b) == (len(L), B) and E.prefill_attention_ok(cache.filled + T, capacity, D)
                 and cache.k.is_contiguous() and cache.v.is_contiguous() and cache.real.is_contiguous()
                 and cache.next_position.dtype == i64 and cache.next_position.is_contiguous()
                 and (valid is None or (valid.dtype == torch.bool and valid.shape == tokens.shape and valid.device == tokens.device))
@@ -335,13 +338,14 @@ class Decoder:
         B, T = tokens.shape
         first = cache.filled
         valid = valid.contiguous() if valid is not None else None
-        pack = B > 1 and valid is not None and first == 0
+        pack = B > 1 and valid is not None and first == 0 and B * T > E.PROMPT_FEW_ROWS
         positions, after, rows = E.prompt_span(tokens, valid, first, cache.real, cache.next_position, pack)
         p = E.prompt_pass(W["layers"], W["final_norm"], tokens, positions, first, cache.real, rows, cache.k, cache.v, self.cos, self.sin,
-                          s.heads, s.kv_heads, s.head_dim, s.top_k, s.norm_topk_prob, s.rms_eps, s.clip_qkv)
+                          s.heads, s.kv_heads, s.head_dim, s.top_k, s.norm_topk_prob, s.rms_eps, s.clip_qkv, kernels.GEMV_MAX_TOKENS)
         count = None
         if (pack and B > 2 and B * T >= PACKED_GEMM_MIN_ROWS
-                and all(E.dense_gemm_ok(B * T, *t.shape) for t in (wqkv[0], W["layers"][0]["wo"]))):
+                and all(E.dense_gemm_ok(B * T, *t.shape) for t in (wqkv[0], W["layers"][0]["wo"]))
+                and all(L["wo"].is_contiguous() for L in W["layers"])):
             count = rows[3]
         project = kernels.project if count is None else lambda x, w: E.dense_gemm(x, w, count)
         xn = p.embed(W["embed"], W["layers"][0]["attn_norm"])

@@ -702,6 +702,27 @@ def test_a_prompts_pass_equals_its_launches_one_by_one(kw, B, T, pad, own_gemm, 
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("kw", [{}, dict(heads=4, kv_heads=2, head_dim=128, experts=100, norm_topk_prob=True, top_k=3)])
+@pytest.mark.parametrize("B,T", [(1, 1), (5, 1), (1, 8), (3, 3), (1, 16), (1, 17), (2, 32)])
+def test_a_short_prompts_pass_equals_its_launches_one_by_one(kw, B, T, monkeypatch):
+    """Up to 64 rows, on either side of where the experts' and the projections' kernels change. The launches one by one
+    take the router's logits from the library's GEMM, so here from the row kernel: then the bits are the same."""
+    s, w, _ = model(7, 1, **kw)
+    dec = D.Decoder(s, w)
+    g = torch.Generator().manual_seed(B * T)
+    valid = (torch.arange(T)[None] >= torch.randint(0, T, (B, 1), generator=g)).cuda()
+    tokens = torch.randint(3, s.vocab, (B, T), generator=g).cuda()
+    outs = []
+    for apart in (False, True):
+        if apart:
+            monkeypatch.setattr(dec, "_takes_prompt_pass", lambda *a: False)
+            monkeypatch.setattr(kernels, "route", lambda h, router, k, norm: kernels.ext().router_route(h, router, k, norm)[:2])
+        cache = D.KVCache(s, B, 2 * T + 3, torch.float16, "cuda")
+        outs.append((dec.prefill_fused(tokens, cache, valid), dec.prefill_fused(tokens, cache), cache.k, cache.v, cache.real, cache.next_position))
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("rows,count,Nout,K", [(1, 1, 8, 256), (31, 31, 300, 256), (700, 0, 256, 256), (700, 1, 256, 256), (3000, 2111, 520, 320),
                                               (5000, 5000, 1000, 256), (9000, 8999, 264, 512)])
 def test_dense_gemm_of_the_rows_that_exist(rows, count, Nout, K):
