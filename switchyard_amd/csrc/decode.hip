@@ -531,11 +531,13 @@ struct HeadChunk {
   }
 };
 
-// A batch of UNROLL key groups of one wavefront: 16 bytes of key and of value per lane each.
+// A batch of UNROLL key groups of one wavefront: 16 bytes of key and of value per lane each, and the key's byte of the
+// mask (0 where there is no key). The byte stays as it is loaded until the batch is used: compared to zero where it
+// is asked for, it is waited for there, and with it every load before, one group after the other.
 template <int UNROLL>
 struct KeyBatch {
   half8_t kk[UNROLL], vv[UNROLL];
-  bool ok[UNROLL];
+  unsigned mask[UNROLL];
 };
 
 // FUSED: the query is taken from the projections' output (norm over the whole q and k rows of
@@ -635,13 +637,13 @@ decode_attention_kernel(const half_t* __restrict__ q, const half_t* kcache, cons
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {
       const int key = (g0 + u * LW) * KPL + sub;
-      kb.ok[u] = key < n;
+      kb.mask[u] = 0;
       kb.kk[u] = zero8;
       kb.vv[u] = zero8;
-      if (kb.ok[u]) {
+      if (key < n) {
         kb.kk[u] = __builtin_nontemporal_load(reinterpret_cast<const half8_t*>(kcache + base + (size_t)key * D));   // the cache is
         kb.vv[u] = __builtin_nontemporal_load(reinterpret_cast<const half8_t*>(vcache + base + (size_t)key * D));   // read once a step
-        kb.ok[u] = rl[key] != 0;
+        kb.mask[u] = rl[key];
       }
     }
   };
@@ -714,7 +716,7 @@ decode_attention_kernel(const half_t* __restrict__ q, const half_t* kcache, cons
 #pragma unroll
       for (int j = 0; j < 8; ++j) d += qf[j] * (float)kb.kk[u][j];
       s[u] = key_sum<LPK>(d);
-      if (kb.ok[u]) mx = fmaxf(mx, s[u]);
+      if (kb.mask[u] != 0) mx = fmaxf(mx, s[u]);
     }
     const float alpha = __builtin_amdgcn_exp2f(m - mx);
     m = mx;
@@ -723,7 +725,7 @@ decode_attention_kernel(const half_t* __restrict__ q, const half_t* kcache, cons
     for (int j = 0; j < 8; ++j) acc[j] *= alpha;
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {
-      const float p = kb.ok[u] ? __builtin_amdgcn_exp2f(s[u] - mx) : 0.f;
+      const float p = kb.mask[u] != 0 ? __builtin_amdgcn_exp2f(s[u] - mx) : 0.f;
       l += p;
 #pragma unroll
       for (int j = 0; j < 8; ++j) acc[j] += p * (float)kb.vv[u][j];
