@@ -288,6 +288,37 @@ __device__ __forceinline__ half_t rotary_f16(half_t y, half_t rot, half_t cos_v,
   return (half_t)((float)t1 + (float)t2);
 }
 
+// The same for eight elements, and the RMS norm's scaling and clamp before it. The product of two f16 numbers is exact
+// in fp32, and their sum is rounded to f16 alike from fp32 or at once (24 bits are twice 11 and two more), so f16
+// arithmetic, two elements to an instruction, has the roundings that fp32 arithmetic followed by a conversion has. The
+// scaling by an fp32 number is the one product that is not exact: elsewhere it is compiled to v_fma_mixlo_f16, which
+// rounds once, and over a vector to a product and a conversion, which round twice; the instruction is named here so
+// that every kernel's keys are the same. These kernels are bound by the instructions in front of their loops: decode
+// attention of 8 sequences 13.7 -> 12.7 us a launch, of 64 45.6 -> 44.0, the prompts' q/k norm of 8 x 512 23.7 -> 19.3.
+__device__ __forceinline__ half8_t norm_f16x8(half8_t x, half8_t w, float rs, float clip) {
+  typedef int i4_t __attribute__((ext_vector_type(4)));
+  i4_t in = __builtin_bit_cast(i4_t, x), out;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    int pair;
+    asm("v_fma_mixlo_f16 %0, %1, %2, 0 op_sel_hi:[1,0,0]" : "=v"(pair) : "v"(in[j]), "v"(rs));
+    asm("v_fma_mixhi_f16 %0, %1, %2, 0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(pair) : "v"(in[j]), "v"(rs));
+    out[j] = pair;
+  }
+  half8_t h = w * __builtin_bit_cast(half8_t, out);
+  if (clip > 0.f) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) h[j] = clamp_f16(h[j], clip);
+  }
+  return h;
+}
+__device__ __forceinline__ half8_t rotary_f16x8(half8_t y, half8_t rot, half8_t cos_v, half8_t sin_v) {
+#pragma clang fp contract(off)
+  const half8_t t1 = y * cos_v;
+  const half8_t t2 = rot * sin_v;
+  return t1 + t2;
+}
+
 // One workgroup per token. qkv row = [q (heads*D) | k (kv_heads*D) | v (kv_heads*D)].
 // PROMPT: the first token goes to cache position `first`. With `place`, rows of padding that are the same in every layer
 // exist once (prompt.hip): position r is row place[r], or, where it is one of those but not the first of them,
@@ -445,17 +476,12 @@ qk_norm_rope_prompt_kernel(const half_t* __restrict__ qkv, const half_t* __restr
   const bool low = d0 < D / 2;
   auto rotate = [&](half8_t x, half8_t w, float rs) {
     typedef int i4_t __attribute__((ext_vector_type(4)));
-    half8_t y;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) y[j] = clamp_f16((half_t)((float)w[j] * (float)(half_t)((float)x[j] * rs)), clip);
+    const half8_t y = norm_f16x8(x, w, rs, clip);
     i4_t words = __builtin_bit_cast(i4_t, y);
 #pragma unroll
     for (int j = 0; j < 4; ++j) words[j] = __shfl_xor(words[j], PARTNER, WAVE);
     const half8_t other = __builtin_bit_cast(half8_t, words);
-    half8_t o;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) o[j] = rotary_f16(y[j], low ? -other[j] : other[j], cc[j], ss[j]);
-    return o;
+    return rotary_f16x8(y, low ? -other : other, cc, ss);
   };
   const half8_t qo = rotate(q, wq, rq), ko = rotate(k, wk, rk);
   if (has_q) *reinterpret_cast<half8_t*>(q_out + (size_t)at * qd + e) = qo;
@@ -519,15 +545,8 @@ struct HeadChunk {
   }
   // RMS norm (scale rs), clamp and rotary embedding, with the roundings of qk_norm_rope_cache
   __device__ __forceinline__ half8_t finish(float rs, float clip, half8_t cc, half8_t ss, int c) const {
-    const bool low = c < LPK / 2;
-    half8_t o;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const half_t a = clamp_f16((half_t)((float)wm[j] * (float)(half_t)((float)mine[j] * rs)), clip);
-      const half_t r = clamp_f16((half_t)((float)wo[j] * (float)(half_t)((float)other[j] * rs)), clip);
-      o[j] = rotary_f16(a, low ? -r : r, cc[j], ss[j]);
-    }
-    return o;
+    const half8_t a = norm_f16x8(mine, wm, rs, clip), r = norm_f16x8(other, wo, rs, clip);
+    return rotary_f16x8(a, c < LPK / 2 ? -r : r, cc, ss);
   }
 };
 
@@ -660,17 +679,18 @@ decode_attention_kernel(const half_t* __restrict__ q, const half_t* kcache, cons
     for (int u = 0; u < SPLITS; ++u) {
       const int v = u * NW + wave;
       float q2 = 0.f, k2 = 0.f;
-      for (int i = v * WAVE + lane; i < (qd >> 3); i += LW * WAVE) {
-        const half8_t e = i < LW * WAVE ? eq[u] : *reinterpret_cast<const half8_t*>(row + i * 8);
+      auto square = [](float& sum, half8_t e) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) q2 += (float)e[j] * (float)e[j];
+        for (int j = 0; j < 8; ++j) sum += (float)e[j] * (float)e[j];
+      };
+      // the chunk that was asked for first (zero where the row has none), then those of longer rows
+      square(q2, eq[u]);
+      for (int i = (LW + v) * WAVE + lane; i < (qd >> 3); i += LW * WAVE) square(q2, *reinterpret_cast<const half8_t*>(row + i * 8));
+      if (owner) {
+        square(k2, ek[u]);
+        for (int i = (LW + v) * WAVE + lane; i < (kvd >> 3); i += LW * WAVE)
+          square(k2, *reinterpret_cast<const half8_t*>(row + qd + i * 8));
       }
-      if (owner)
-        for (int i = v * WAVE + lane; i < (kvd >> 3); i += LW * WAVE) {
-          const half8_t e = i < LW * WAVE ? ek[u] : *reinterpret_cast<const half8_t*>(row + qd + i * 8);
-#pragma unroll
-          for (int j = 0; j < 8; ++j) k2 += (float)e[j] * (float)e[j];
-        }
       q2 = wave_sum(q2);
       k2 = wave_sum(k2);
       if (lane == 0) {
@@ -688,9 +708,11 @@ decode_attention_kernel(const half_t* __restrict__ q, const half_t* kcache, cons
     const half8_t qv = hq.finish(rq, nt.clip, cc, ss, c);
 #pragma unroll
     for (int j = 0; j < 8; ++j) qf[j] = (float)qv[j] * scale_log2e;
-    knew = hk.finish(rk, nt.clip, cc, ss, c);
+    if (vwave == 0) {   // the same in the whole wavefront
+      knew = hk.finish(rk, nt.clip, cc, ss, c);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) vnew[j] = clamp_f16(vnew[j], nt.clip);
+      for (int j = 0; j < 8; ++j) vnew[j] = clamp_f16(vnew[j], nt.clip);
+    }
     if (slot >= 0 && slot < capacity && qh % group == 0 && vwave == 0 && sub == 0) {
       const size_t at = (((size_t)b * kv_heads + kvh) * capacity + slot) * D + c * 8;
       *reinterpret_cast<half8_t*>(nt.kcache_w + at) = knew;
