@@ -41,6 +41,16 @@ extern "C" SY_API int sy_version(void) { return 200; }  // 0.2.0: the decode-ste
 
 extern "C" SY_API const char* sy_last_error(void) { return g_error; }
 
+// What follows the gate/up projection of a decode step of at most 64 choices.
+static int down_of_few(int N, int E, int k, const void* down, int H, int I, const int32_t* idx, const void* w, const int32_t* offsets,
+                       const int32_t* token, const void* wsorted, const int32_t* pos_of, const void* act, void* y, void* out,
+                       void* stream) {
+  // up to 4 tokens the down projection adds a token's rows up itself: no combine launch, no y
+  if (sy_gemv_combines(N, k, E, H, I)) return sy_gemv_down_combine(act, down, offsets, token, wsorted, N, k, E, H, I, out, stream);
+  const int rc = sy_grouped_gemv(act, nullptr, down, offsets, E, N * k, N, H, I, 0, nullptr, y, stream);
+  return rc ? rc : sy_combine_weighted(y, pos_of, idx, w, N, k, H, out, stream);
+}
+
 // The experts of one layer in one call: (the router's logits,) route and sort, the two
 // projections and combine, enqueued back to back. Nothing here that the separate entry points do not do; it exists
 // because a host binding pays several microseconds per call, and in front of the first
@@ -78,8 +88,14 @@ extern "C" SY_API int sy_moe_experts(const void* h, const void* router, void* lo
                  : sy_sort_by_expert(idx, w, 2, N, k, E, counts, offsets, token, wsorted, pos_of, sort_workspace,
                                      sort_workspace_bytes, stream);
   } else if (router && !mfma_tiles && sy_gemv_sorts(N, k, E, H)) {
-    // a decode step of at most 64 choices: logits and route in one launch, and the first
-    // projection sorts for itself
+    // a decode step of at most 64 choices: the first projection sorts for itself, and routes too where it can: the
+    // launch in front of it is then the logits alone, or logits and route
+    if (sy_gemv_routes(N, k, E, H, I)) {
+      rc = sy_logits_spread(h, nullptr, nullptr, 0.f, router, E, N, H, nullptr, nullptr, logits, stream);
+      if (!rc)
+        rc = sy_gemv_routing(h, logits, norm, N, k, gate_up, E, I, H, idx, w, counts, offsets, token, wsorted, pos_of, act, stream);
+      return rc ? rc : down_of_few(N, E, k, down, H, I, idx, w, offsets, token, wsorted, pos_of, act, y, out, stream);
+    }
     rc = sy_router_route_rows(h, router, N, H, E, k, norm, logits, idx, w, stream);
     if (rc) return rc;
     return sy_experts_routed(h, N, E, k, gate_up, down, H, I, 0, idx, w, counts, offsets, token, wsorted, pos_of, act, y, out,
@@ -201,14 +217,21 @@ int sy_moe_add_rmsnorm_rows(const SyMoeLayer* L, const void* h, const int32_t* t
                                       h_out, stream);
 }
 
-// Up to 64 choices the front only routes and the gate/up stream sorts for itself, as in sy_moe_layer; the weight stream leaves
+// Up to 64 choices the gate/up stream sorts for itself, and routes too where it can, as in sy_moe_layer; the weight stream leaves
 // the router weights to the combine, the MFMA tiles apply them.
 int sy_few_rows_moe(void* x, const void* o, const void* mlp_norm, float eps, const void* router, int N, int H, int I, int E, int k, int norm,
                     const void* gate_up, const void* down, const void* next_norm, bool stream_experts, const SyFewRows& s, void* xn,
                     void* stream) {
   const int M = N * k;
   int rc;
-  if (stream_experts && sy_gemv_sorts(N, k, E, H)) {
+  // x after the attention: where the front is spread over many workgroups it goes to another buffer than x
+  const bool spread = stream_experts && sy_gemv_routes(N, k, E, H, I);
+  void* mid = spread ? xn : x;
+  if (spread) {
+    rc = sy_logits_spread(x, o, mlp_norm, eps, router, E, N, H, mid, s.h, s.logits, stream);
+    if (!rc)
+      rc = sy_gemv_routing(s.h, s.logits, norm, N, k, gate_up, E, I, H, s.idx, s.w, s.counts, s.offsets, s.token, s.wsorted, s.pos_of, s.act, stream);
+  } else if (stream_experts && sy_gemv_sorts(N, k, E, H)) {
     rc = sy_add_rmsnorm_route(x, o, mlp_norm, eps, router, E, N, H, k, norm, x, s.h, s.logits, s.idx, s.w, stream);
     if (!rc)
       rc = sy_grouped_gemv_sorting(s.h, s.idx, s.w, N, k, gate_up, E, I, H, s.counts, s.offsets, s.token, s.wsorted, s.pos_of, s.act, stream);
@@ -222,7 +245,7 @@ int sy_few_rows_moe(void* x, const void* o, const void* mlp_norm, float eps, con
   if (!rc)
     rc = stream_experts ? sy_grouped_gemv(s.act, nullptr, down, s.offsets, E, M, N, H, I, 0, nullptr, s.y, stream)
                         : sy_grouped_gemm(s.act, nullptr, down, s.offsets, E, M, H, I, 0, s.wsorted, s.y, stream);
-  if (!rc) rc = sy_combine_add_rmsnorm(s.y, s.pos_of, s.idx, stream_experts ? s.w : nullptr, k, x, next_norm, eps, N, H, x, xn, stream);
+  if (!rc) rc = sy_combine_add_rmsnorm(s.y, s.pos_of, s.idx, stream_experts ? s.w : nullptr, k, mid, next_norm, eps, N, H, x, xn, stream);
   return rc;
 }
 
@@ -252,12 +275,7 @@ extern "C" SY_API int sy_experts_routed(const void* h, int N, int E, int k, cons
   if (!mfma_tiles && sy_gemv_sorts(N, k, E, H)) {
     // at most 64 choices: the gate/up stream sorts them in its own prologue
     rc = sy_grouped_gemv_sorting(h, idx, w, N, k, gate_up, E, I, H, counts, offsets, token, wsorted, pos_of, act, stream);
-    if (rc) return rc;
-    // up to 4 tokens the down projection adds a token's rows up itself: no combine launch, no y
-    if (sy_gemv_combines(N, k, E, H, I)) return sy_gemv_down_combine(act, down, offsets, token, wsorted, N, k, E, H, I, out, stream);
-    rc = sy_grouped_gemv(act, nullptr, down, offsets, E, N * k, N, H, I, 0, nullptr, y, stream);
-    if (rc) return rc;
-    return sy_combine_weighted(y, pos_of, idx, w, N, k, H, out, stream);
+    return rc ? rc : down_of_few(N, E, k, down, H, I, idx, w, offsets, token, wsorted, pos_of, act, y, out, stream);
   }
   rc = sy_sort_by_expert(idx, w, 2, N, k, E, counts, offsets, token, wsorted, pos_of, sort_workspace, sort_workspace_bytes,
                          stream);

@@ -38,6 +38,15 @@ int sy_gemm_rows_per_tile(int rows, int E, int K);
 // decode.hip: sy_embed_rmsnorm at the head of a step, which also sets nclear counters to zero
 int sy_embed_rmsnorm_step(const int64_t* tokens, const void* embed, int vocab, const void* weight, float eps, int N, int H,
                           void* x_out, void* h_out, unsigned* clear, int nclear, void* stream);
+// decode.hip: the router's logits of at most 8 rows of 2048 on many workgroups; with `weight` of the norm of x + delta, which
+// x_out (another buffer than x) and h_out receive
+int sy_logits_spread(const void* x, const void* delta, const void* weight, float eps, const void* router, int E, int N, int H,
+                     void* x_out, void* h_out, void* logits, void* stream);
+// gemv.hip: gate/up of a decode step from those logits
+bool sy_gemv_routes(int N, int k, int E, int H, int I);
+int sy_gemv_routing(const void* h, const void* logits, int norm, int N, int k, const void* gate_up, int E, int I, int H, int32_t* idx,
+                    void* w, int32_t* counts, int32_t* offsets, int32_t* token, void* wsorted, int32_t* pos_of, void* act,
+                    void* stream);
 // decode.hip: sy_add_rmsnorm_route_sort without the sort, for the launch that sorts for itself
 int sy_add_rmsnorm_route(const void* x, const void* delta, const void* weight, float eps, const void* router, int E, int N,
                          int H, int k, int norm, void* x_out, void* h_out, void* logits, int32_t* idx, void* w, void* stream);
@@ -57,7 +66,7 @@ int sy_prefill_attention_rows(const void* q, const void* kcache, const void* vca
                               int heads, int kv_heads, int D, int capacity, const int32_t* place, void* out, void* stream);
 // abi.hip: the MoE layer of a few rows (at most 64, 128 experts, top-8) between its norms: x += o, h = norm, route and sort, the
 // two projections (a weight stream or the MFMA tiles), x += their combination, xn = the next norm. x is updated in
-// place; the other buffers are scratch.
+// place; the other buffers are scratch, and xn is one until it is written.
 struct SyFewRows {
   void *h, *logits, *w, *wsorted, *act, *y;
   int32_t *idx, *counts, *offsets, *token, *pos_of;

@@ -97,11 +97,11 @@ template <bool COMBINE, bool LOGITS, int FRONT = 0, int FROM = OWN_ROWS, bool FE
 __global__ void __launch_bounds__(LOGITS ? 1024 : ROW_THREADS)
 row_kernel(const half_t* x, const half_t* __restrict__ delta, const half_t* __restrict__ y,
            const int* __restrict__ pos_of, const int* __restrict__ idx, int k, const half_t* __restrict__ weight,
-           float eps, const half_t* __restrict__ router, int E, int H, half_t* x_out, half_t* __restrict__ h_out,
+           float eps, const half_t* __restrict__ router, int E, int H, half_t* x_out, half_t* h_out,
            half_t* __restrict__ logits, const int64_t* __restrict__ gather, int src_rows,
            front_core::Outputs front = front_core::Outputs{}, const int* __restrict__ twin = nullptr,
            unsigned* __restrict__ clear = nullptr, int nclear = 0, const int* __restrict__ count = nullptr,
-           const int* __restrict__ map = nullptr) {  // x_out may be x
+           const int* __restrict__ map = nullptr) {  // x_out or h_out may be x
   extern __shared__ __attribute__((aligned(16))) half_t hs[];  // LOGITS: the normalised row [H]; FRONT: the tail's LDS behind it
   __shared__ __attribute__((aligned(16))) float part[16];
   __shared__ int rows[ROW_MAX_K];
@@ -268,6 +268,64 @@ row_kernel(const half_t* x, const half_t* __restrict__ delta, const half_t* __re
       front_core::route_own_sort_last<2>(t, (int)gridDim.x, E, front, tail);
     }
   }
+}
+
+// The router's logits of a few rows for a launch that routes by itself (gemv.hip), with NORM behind the residual add and the
+// norm: every token's experts are dealt to E / 4 workgroups, one to a wavefront. A workgroup that has a token's whole router to
+// read waits for 256 KB at the 60 to 70 bytes a clock that a compute unit pulls from L2, then routes: 6.9 us a launch with one
+// row and 7.6 with 8. Here the router's rows are asked for with the token's, and the norm, which every workgroup of the token
+// computes for itself, runs while they are on their way: 2.8 and 4.8, and the stream behind it takes 1.0 and 2.2 more to
+// route. x_out must not be x: other workgroups may still have x to read.
+constexpr int SPREAD_THREADS = ROW_THREADS, SPREAD_WAVES = SPREAD_THREADS / WAVE, SPREAD_H = SPREAD_THREADS * 8;
+template <bool NORM>
+__global__ void __launch_bounds__(SPREAD_THREADS)
+logits_spread_kernel(const half_t* __restrict__ x, const half_t* __restrict__ delta, const half_t* __restrict__ weight, float eps,
+                     const half_t* __restrict__ router, int E, half_t* __restrict__ x_out, half_t* __restrict__ h_out,
+                     half_t* __restrict__ logits) {
+  constexpr int H = SPREAD_H, PER_LANE = H / (WAVE * 8);
+  __shared__ __attribute__((aligned(16))) half_t hs[NORM ? H : 8];
+  __shared__ __attribute__((aligned(16))) float part[4];
+  const int t = blockIdx.y, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int e = blockIdx.x * SPREAD_WAVES + wave;
+  const size_t row = (size_t)t * H;
+  half8_t v, d, w, hv[PER_LANE], rv[PER_LANE];
+  if (NORM) {
+    v = *reinterpret_cast<const half8_t*>(x + row + tid * 8);
+    d = *reinterpret_cast<const half8_t*>(delta + row + tid * 8);
+    w = *reinterpret_cast<const half8_t*>(weight + tid * 8);
+  } else {
+#pragma unroll
+    for (int i = 0; i < PER_LANE; ++i) hv[i] = *reinterpret_cast<const half8_t*>(x + row + (lane + WAVE * i) * 8);
+  }
+#pragma unroll
+  for (int i = 0; i < PER_LANE; ++i)
+    rv[i] = *reinterpret_cast<const half8_t*>(router + (size_t)min(e, E - 1) * H + (lane + WAVE * i) * 8);
+  if (NORM) {
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = (half_t)((float)v[j] + (float)d[j]);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) ss += (float)v[j] * (float)v[j];
+    const float rs = rsqrtf(block_sum_of_four(ss, part) / (float)H + eps);
+    half8_t h;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) h[j] = (half_t)((float)w[j] * (float)(half_t)((float)v[j] * rs));
+    *reinterpret_cast<half8_t*>(hs + tid * 8) = h;
+    if (blockIdx.x == 0) {
+      *reinterpret_cast<half8_t*>(x_out + row + tid * 8) = v;
+      *reinterpret_cast<half8_t*>(h_out + row + tid * 8) = h;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < PER_LANE; ++i) hv[i] = *reinterpret_cast<const half8_t*>(hs + (lane + WAVE * i) * 8);
+  }
+  float acc = 0.f;
+#pragma unroll
+  for (int i = 0; i < PER_LANE; ++i)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc += (float)hv[i][j] * (float)rv[i][j];
+  acc = wave_sum(acc);
+  if (lane == 0 && e < E) logits[(size_t)t * E + e] = (half_t)acc;
 }
 
 __device__ __forceinline__ half_t clamp_f16(half_t v, float clip) {
@@ -1089,6 +1147,18 @@ int sy_router_route_rows(const void* h, const void* router, int N, int H, int E,
       (const half_t*)h, nullptr, nullptr, nullptr, nullptr, 0, nullptr, 0.f, (const half_t*)router, E, H, nullptr, nullptr,
       (half_t*)logits, nullptr, 0, front);
   return sy_check_launch("router_route");
+}
+
+int sy_logits_spread(const void* x, const void* delta, const void* weight, float eps, const void* router, int E, int N, int H,
+                     void* x_out, void* h_out, void* logits, void* stream) {
+  SY_REQUIRE(N >= 1 && N <= FEW_ROWS && E >= 1 && E <= 128 && H == SPREAD_H, "logits_spread: N = %d, E = %d, H = %d", N, E, H);
+  SY_REQUIRE(x && router && logits && (!weight || (delta && x_out && h_out && x_out != x)), "logits_spread: null pointer, or x_out is x");
+  const dim3 grid((unsigned)((E + SPREAD_WAVES - 1) / SPREAD_WAVES), (unsigned)N);
+  void (*kern)(const half_t*, const half_t*, const half_t*, float, const half_t*, int, half_t*, half_t*, half_t*) =
+      weight ? logits_spread_kernel<true> : logits_spread_kernel<false>;
+  kern<<<grid, SPREAD_THREADS, 0, (hipStream_t)stream>>>((const half_t*)x, (const half_t*)delta, (const half_t*)weight, eps,
+                                                         (const half_t*)router, E, (half_t*)x_out, (half_t*)h_out, (half_t*)logits);
+  return sy_check_launch("logits_spread");
 }
 
 int sy_add_rmsnorm_route(const void* x, const void* delta, const void* weight, float eps, const void* router, int E, int N,

@@ -31,6 +31,7 @@
 // (switchyard/csrc/moe_kernels.cu:301-415); epilogue rounding points as :373-378.
 #include <type_traits>
 
+#include "route_core.h"
 #include "sort_core.h"
 
 namespace {
@@ -232,6 +233,11 @@ struct SortHere {
   int* token;            // [M]
   half_t* wsorted;       // [M]
   int* pos_of;           // [M]
+  // ROUTE: the router's logits in the place of idx and w, which are results then
+  const half_t* logits;  // [N, E]
+  int norm;
+  int* idx_out;          // [N, k]
+  half_t* w_out;         // [N, k]
 };
 constexpr int SORT_HERE_MAX = WAVE;   // choices that one wavefront sorts with one per lane
 __host__ __device__ constexpr size_t sort_here_ints(int E) {
@@ -252,6 +258,10 @@ __host__ __device__ constexpr size_t sort_here_ints(int E) {
 // them, cost the down projection's sixteen wavefronts to a compute unit more than the wait: 9.8 -> 12.0 and
 // 30.3 -> 33.4.)
 //
+// ROUTE (with ALL, up to 64 experts): the launch starts from the router's logits and every workgroup routes the tokens
+// too, a wavefront two of them. The launch in front of it is then only the logits, which no workgroup has to have all
+// of, so that one is spread over the chip (logits_spread_kernel in decode.hip).
+//
 // DENSE: one matrix and `sort.M` rows of A in their own order (the projections around the MoE layer):
 // there is no list of experts to build, so a launch begins with its loads: the rows, then the first weights,
 // and the rows go to LDS behind those.
@@ -260,7 +270,7 @@ constexpr int EARLY_ROWS = 2, EARLY_CHUNKS = 4;   // rows that a wavefront asks 
 constexpr int ALL_ROWS = 8;                       // tokens of an ALL launch, a chunk of 16 bytes of each per thread
 constexpr int DENSE_MAX_WAVES = 8;
 
-template <bool SWIGLU, bool SCALE, bool EXACT, int CH, bool SORT = false, bool DENSE = false, bool ALL = false>
+template <bool SWIGLU, bool SCALE, bool EXACT, int CH, bool SORT = false, bool DENSE = false, bool ALL = false, bool ROUTE = false>
 __global__ void __launch_bounds__(DENSE ? DENSE_MAX_WAVES * WAVE : GEMV_THREADS)
 gemv_kernel(const half_t* __restrict__ A, const int* __restrict__ a_rows, const half_t* __restrict__ B,
             const int* __restrict__ offsets, int E, int Nout, int K, const half_t* __restrict__ scale,
@@ -357,16 +367,47 @@ gemv_kernel(const half_t* __restrict__ A, const int* __restrict__ a_rows, const 
   uint16_t* s_wsorted = reinterpret_cast<uint16_t*>(s_pos + SORT_HERE_MAX);
   int key = -1;
   uint16_t weight = 0;
-  if (SORT && wave == 0 && lane < sort.M) {
+  const int tokens = ALL ? sort.M / sort.k : 0;
+  constexpr int ROUTED = ALL_ROWS / GEMV_WAVES;   // tokens that a wavefront routes
+  half_t lg[ROUTED][1];
+  if (ROUTE) {
+#pragma unroll
+    for (int i = 0; i < ROUTED; ++i) lg[i][0] = sort.logits[min(wave + GEMV_WAVES * i, tokens - 1) * E + min(lane, E - 1)];
+  } else if (SORT && wave == 0 && lane < sort.M) {
     key = sort.idx[lane];
     weight = reinterpret_cast<const uint16_t*>(sort.w)[lane];
   }
-  const int tokens = ALL ? sort.M / sort.k : 0;
   half8_t all[ALL ? ALL_ROWS : 1];
   if (ALL) {
 #pragma unroll
     for (int r = 0; r < ALL_ROWS; ++r)
       if (r < tokens && (int)threadIdx.x * 8 < K) all[r] = *reinterpret_cast<const half8_t*>(A + (size_t)r * K + threadIdx.x * 8);
+  }
+  if (ROUTE) {
+    // the choices meet where the sort, which has them in registers by then, leaves its results
+#pragma unroll
+    for (int i = 0; i < ROUTED; ++i) {
+      const int t = wave + GEMV_WAVES * i;
+      if (t < tokens) {
+        int e;
+        float p;
+        route_core::route_loaded<half_t, 1>(lg[i], E, sort.k, sort.norm, e, p);
+        if (lane < sort.k) {
+          s_pos[t * sort.k + lane] = e;
+          s_wsorted[t * sort.k + lane] = __builtin_bit_cast(uint16_t, (half_t)p);
+        }
+      }
+    }
+    __syncthreads();
+    if (wave == 0 && lane < sort.M) {
+      key = s_pos[lane];
+      weight = s_wsorted[lane];
+      if (blockIdx.x == 0) {
+        sort.idx_out[lane] = key;
+        reinterpret_cast<uint16_t*>(sort.w_out)[lane] = weight;
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
   }
   if (wave == 0) {
     if (SORT) {
@@ -524,7 +565,7 @@ int launch_gemv(const void* A, const int32_t* a_rows, const void* B, const int32
   else if (dense) kern = exact ? gemv_kernel<false, false, true, CH_SHORT, false, true> : gemv_kernel<false, false, false, CH_SHORT, false, true>;
   // (more than 8 tokens have at most 64 choices only where k < 8; one row of LDS per token)
   else if (sort && long_chunks && exact && rows / sort->k <= ALL_ROWS && rows / sort->k <= row_cap && K <= GEMV_THREADS * 8)
-    kern = gemv_kernel<true, false, true, CH_LONG, true, false, true>;
+    kern = sort->logits ? gemv_kernel<true, false, true, CH_LONG, true, false, true, true> : gemv_kernel<true, false, true, CH_LONG, true, false, true>;
   else if (sort && long_chunks && exact) kern = gemv_kernel<true, false, true, CH_LONG, true>;
   else if (sort) kern = exact ? gemv_kernel<true, false, true, CH_SHORT, true> : gemv_kernel<true, false, false, CH_SHORT, true>;
   else if (swiglu && long_chunks && exact) kern = gemv_kernel<true, false, true, CH_LONG>;
@@ -766,6 +807,26 @@ extern "C" SY_API int sy_grouped_gemv_sorting(const void* h, const int32_t* idx,
   int nbits = 0;
   while ((1 << nbits) < E) ++nbits;
   const SortHere sort{idx, (const half_t*)w, N * k, k, nbits, counts, offsets, token, (half_t*)wsorted, pos_of};
+  return launch_gemv(h, nullptr, gate_up, nullptr, E, N * k, N, I, H, 1, nullptr, act, (hipStream_t)stream, &sort);
+}
+
+// Whether sy_gemv_routing takes this shape: top-8, an expert to a lane, and a launch that asks for every token's row at once
+// (launch_gemv: rows of 2048, in long chunks, and nothing to mask).
+bool sy_gemv_routes(int N, int k, int E, int H, int I) {
+  return sy_gemv_sorts(N, k, E, H) && N <= ALL_ROWS && k <= 8 && E <= WAVE && H == GEMV_THREADS * 8 && I >= 1 && I % UNIT_COLS == 0;
+}
+
+// sy_grouped_gemv_sorting from the router's logits f16 [N, E]: route, sort and the gate/up projection in one launch, idx
+// and w among its results.
+int sy_gemv_routing(const void* h, const void* logits, int norm, int N, int k, const void* gate_up, int E, int I, int H, int32_t* idx,
+                    void* w, int32_t* counts, int32_t* offsets, int32_t* token, void* wsorted, int32_t* pos_of, void* act,
+                    void* stream) {
+  SY_REQUIRE(sy_gemv_routes(N, k, E, H, I), "gemv_routing: N = %d, k = %d, E = %d, H = %d, I = %d", N, k, E, H, I);
+  SY_REQUIRE((long)2 * I * H * 2 < (1l << 31), "gemv_routing: an expert's matrix must stay under 2 GiB");
+  SY_REQUIRE(h && logits && idx && w && gate_up && counts && offsets && token && wsorted && pos_of && act, "gemv_routing: null pointer");
+  int nbits = 0;
+  while ((1 << nbits) < E) ++nbits;
+  const SortHere sort{nullptr, nullptr, N * k, k, nbits, counts, offsets, token, (half_t*)wsorted, pos_of, (const half_t*)logits, norm, idx, (half_t*)w};
   return launch_gemv(h, nullptr, gate_up, nullptr, E, N * k, N, I, H, 1, nullptr, act, (hipStream_t)stream, &sort);
 }
 

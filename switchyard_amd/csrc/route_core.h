@@ -46,9 +46,9 @@ __device__ __forceinline__ Cand wave_best(Cand c) {
   return better(better(cand_lane(c, 0), cand_lane(c, 16)), better(cand_lane(c, 32), cand_lane(c, 48)));
 }
 
-// Must be called by all 64 lanes of a wavefront. `row` points at the token's E logits.
+// Must be called by all 64 lanes of a wavefront. own[j] is the token's logit of expert lane + 64 j, if there is one.
 template <typename T, int PER_LANE>
-__device__ __forceinline__ void route_token(const T* row, int E, int k, int norm, int& my_e, float& my_w) {
+__device__ __forceinline__ void route_loaded(const T (&own)[PER_LANE], int E, int k, int norm, int& my_e, float& my_w) {
   const int lane = threadIdx.x & 63;
   float v[PER_LANE], p[PER_LANE];
   bool open[PER_LANE];
@@ -57,7 +57,7 @@ __device__ __forceinline__ void route_token(const T* row, int E, int k, int norm
   for (int j = 0; j < PER_LANE; ++j) {
     const int e = lane + WAVE * j;
     open[j] = e < E;
-    v[j] = open[j] ? (float)row[e] : -INFINITY;
+    v[j] = open[j] ? (float)own[j] : -INFINITY;
     mx = fmaxf(mx, v[j]);
   }
   mx = wave_max(mx);
@@ -126,6 +126,16 @@ __device__ __forceinline__ void route_token(const T* row, int E, int k, int norm
     }
   }
   my_w = norm ? my_p / total : my_p;
+}
+
+// The same with the token's E logits in memory, at `row`.
+template <typename T, int PER_LANE>
+__device__ __forceinline__ void route_token(const T* row, int E, int k, int norm, int& my_e, float& my_w) {
+  const int lane = threadIdx.x & 63;
+  T own[PER_LANE];
+#pragma unroll
+  for (int j = 0; j < PER_LANE; ++j) own[j] = lane + WAVE * j < E ? row[lane + WAVE * j] : T(0);
+  route_loaded<T, PER_LANE>(own, E, k, norm, my_e, my_w);
 }
 
 }  // namespace route_core

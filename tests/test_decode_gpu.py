@@ -527,6 +527,23 @@ def test_a_step_in_one_call_equals_its_launches_one_by_one(B, kw, monkeypatch):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("N,E,k,norm", [(1, 64, 8, False), (8, 64, 8, True), (5, 61, 8, False), (8, 3, 2, True), (2, 1, 1, False),
+                                        (7, 33, 1, False), (3, 65, 8, False), (9, 64, 4, True)])   # the last two: not by the gate/up stream
+def test_a_layer_whose_gate_up_stream_routes(N, E, k, norm):
+    """Against the layer from a routing of its own launch, bit for bit, with equal logits among the choices."""
+    h, router = rnd(N, 2048, seed=71), rnd(E, 2048, seed=72, std=0.02)
+    router[E // 2:] = router[:E - E // 2].clone()
+    gate_up, down = rnd(E, 512, 2048, seed=73, std=0.03), rnd(E, 2048, 256, seed=74, std=0.05)
+    _, idx, w, *_ = kernels.ext().router_route_sort(h, router, k, norm)
+    want = kernels.experts(h, idx, w, gate_up, down, mode="gemv")
+    assert torch.equal(kernels.moe_layer(h, router, gate_up, down, k, norm, mode="gemv"), want)
+
+
+@pytest.mark.parametrize("B,kw", [(1, {}), (8, {}), (6, dict(experts=10, top_k=3, norm_topk_prob=True)), (4, dict(experts=65))])
+def test_a_step_whose_gate_up_stream_routes(B, kw, monkeypatch):
+    test_a_step_in_one_call_equals_its_launches_one_by_one(B, dict(hidden=2048, layers=2, heads=16, kv_heads=16, **kw), monkeypatch)
+
+
 @pytest.mark.parametrize("B", [3, 12])
 def test_layers_of_different_sizes_and_norms_of_any_shape(B, monkeypatch):
     """A model whose layers differ in the number and the width of their experts (pruned ones), with norms that
