@@ -141,8 +141,8 @@ SY_API int sy_combine(const void* y, const int32_t* pos_of, const int32_t* idx, 
 /* Replaces moe_layer() (switchyard/kernels.py:91-93: route() with its router GEMM, :30-32, then
  * experts(), :76-88: sort -> pick -> ffn -> combine) in ONE call: the router's logits
  * (when `router` is given: up to 64 tokens sy_router_route_sort, which is the whole front in one
- * launch, or, with the weight-stream kernels and at most 64 choices, sy_router_route and a
- * gate/up projection that sorts for itself; above that sy_router_route, which routes in the same launch and is also the first pass
+ * launch, or, with the weight-stream kernels and at most 64 choices, the logits, with or without
+ * route, and a gate/up projection that does the rest for itself; above that sy_router_route, which routes in the same launch and is also the first pass
  * of the sort; with router NULL `logits` is an input), route and sort (sy_route_sort when one_launch_front is nonzero, else sy_route and
  * sy_sort_by_expert with the given workspace), the gate/up projection (SwiGLU, rows of h gathered through `token`), the
  * down projection (x router weight) and sy_combine are enqueued back to back, exactly as the

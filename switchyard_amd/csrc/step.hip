@@ -8,8 +8,8 @@
 //
 // What the launches are, per layer: q/k/v projection (a weight stream), attention with the q/k norm, the
 // rotary embedding and the cache write in its prologue, output projection, residual add + norm + router
-// logits + route (+ sort), gate/up, down, and combine + residual add + the next norm. Up to 64 choices
-// (8 tokens of top-8) the front only routes and the gate/up stream sorts for itself, as in sy_moe_layer.
+// logits + route + sort, gate/up, down, and combine + residual add + the next norm. Up to 64 choices
+// (8 tokens of top-8) the gate/up stream sorts for itself, and routes too where it can, as in sy_moe_layer.
 #include "common.h"
 #include "../../include/switchyard_decode.h"
 #include "passes.h"
