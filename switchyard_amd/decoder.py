@@ -180,7 +180,14 @@ class KVCache:
         self.capacity = capacity
 
 
-PACKED_GEMM_MIN_ROWS = 2048   # up to here the library's GEMM on every row is faster than own tiles on those that exist
+# Where a padded batch's projections run on the own tiles, which stop at the rows that exist, instead of the library's GEMM on every
+# row: from 2048 rows on, where at most so many of them are real. us for q/k/v ([6144, 2048]) and output ([2048, 2048]) projection:
+#   of 4096 rows: library 94 + 36; own with all of them real 103 + 38, 90 % 86 + 36, 80 % 76 + 35, 70 % 75 + 31
+#   of 8192 rows: library 152 + 53; own 180 + 61, 164 + 59, 148 + 52, 134 + 47
+# At four fifths the two together are faster on the own tiles at all of 19 sizes measured from 2048 to 32768 rows (1.02 to 1.39
+# times), at nine tenths at 11 of them (0.91 to 1.17), and without padding at 3 (0.84 to 1.11).
+PACKED_GEMM_MIN_ROWS = 2048
+PACKED_GEMM_MAX_REAL = 0.8
 
 
 class Decoder:
@@ -252,21 +259,24 @@ class Decoder:
         return F.linear(_rms(x, W["final_norm"], s.rms_eps), W["lm_head"])
 
     @torch.no_grad()
-    def prefill_fused(self, tokens, cache, valid=None):
+    def prefill_fused(self, tokens, cache, valid=None, real_tokens=None):
         """`forward` for a prompt on the library's kernels, returning the logits of the last
         position only, [B, vocab]: norms, residual adds, the q/k norm with the rotary embedding
         and the cache write are one launch each over all B*T rows (in PyTorch they are some
         seventy element-wise launches per layer, each a pass over the activations), the three
         input projections are one GEMM, and the lm_head runs on B rows instead of B*T.
         Attention is one launch too, with the mask's rule instead of a mask tensor, straight from
-        and into the layouts of its neighbours."""
+        and into the layouts of its neighbours.
+
+        `real_tokens`: how many positions `valid` marks, if the caller knows (the pass reads nothing back from the GPU).
+        It chooses between launches that compute the same, and is no more than that: a wrong one costs time."""
         from . import kernels
 
         s, W, E = self.s, self.w, kernels.ext()
         B, T = tokens.shape
         wqkv = self._stacked_qkv()
         if self._takes_prompt_pass(tokens, cache, valid):
-            return self._prompt_pass(tokens.contiguous(), cache, valid, wqkv)
+            return self._prompt_pass(tokens.contiguous(), cache, valid, wqkv, real_tokens)
         span = Span(tokens, cache, valid)
         slot = torch.tensor([span.first], dtype=torch.long, device=tokens.device)
         flat_positions = span.positions.reshape(-1).contiguous()
@@ -327,23 +337,23 @@ class Decoder:
                 and (valid is None or (valid.dtype == torch.bool and valid.shape == tokens.shape and valid.device == tokens.device))
                 and cache.real.device == tokens.device)
 
-    def _prompt_pass(self, tokens, cache, valid, wqkv):
+    def _prompt_pass(self, tokens, cache, valid, wqkv, real_tokens=None):
         """prefill_fused in two host calls a layer beside the projections. The padding of a batch that starts its cache is
         one row for every launch (csrc/prompt.hip); which rows exist only the device knows, so the projections run on
-        its count where there is enough padding to win (own tiles: 3080 of 4096 rows, q/k/v and output 79 + 37 us, the
-        library's GEMM on all rows 97 + 37; without padding 109 + 38)."""
+        its count where the caller says that there is enough padding to win (PACKED_GEMM_MAX_REAL), and else, as it may
+        be a mask without padding, on every row. A batch known to have none is not packed at all."""
         from . import kernels
 
         s, W, E = self.s, self.w, kernels.ext()
         B, T = tokens.shape
         first = cache.filled
         valid = valid.contiguous() if valid is not None else None
-        pack = B > 1 and valid is not None and first == 0 and B * T > E.PROMPT_FEW_ROWS
+        pack = B > 1 and valid is not None and first == 0 and B * T > E.PROMPT_FEW_ROWS and real_tokens != B * T
         positions, after, rows = E.prompt_span(tokens, valid, first, cache.real, cache.next_position, pack)
         p = E.prompt_pass(W["layers"], W["final_norm"], tokens, positions, first, cache.real, rows, cache.k, cache.v, self.cos, self.sin,
                           s.heads, s.kv_heads, s.head_dim, s.top_k, s.norm_topk_prob, s.rms_eps, s.clip_qkv, kernels.GEMV_MAX_TOKENS)
         count = None
-        if (pack and B > 2 and B * T >= PACKED_GEMM_MIN_ROWS
+        if (pack and real_tokens is not None and B * T >= PACKED_GEMM_MIN_ROWS and real_tokens <= PACKED_GEMM_MAX_REAL * B * T
                 and all(E.dense_gemm_ok(B * T, *t.shape) for t in (wqkv[0], W["layers"][0]["wo"]))
                 and all(L["wo"].is_contiguous() for L in W["layers"])):
             count = rows[3]
@@ -357,10 +367,10 @@ class Decoder:
         last = xn.index_select(0, rows[2]) if pack else xn.view(B, T, s.hidden)[:, -1].contiguous()
         return kernels.dense(last, W["lm_head"])
 
-    def _prefill(self, tokens, cache, valid):
+    def _prefill(self, tokens, cache, valid, real_tokens=None):
         """Logits of the last prompt position [B, vocab], on the kernels where they apply."""
         if self.fused:
-            return self.prefill_fused(tokens, cache, valid)
+            return self.prefill_fused(tokens, cache, valid, real_tokens)
         return self.forward(tokens, cache, valid)[:, -1]
 
     # ---- one decode step with every index on the device, so that it can be captured in a HIP graph
@@ -496,7 +506,7 @@ class Decoder:
         if timings is not None:
             torch.cuda.synchronize()
             t0 = time.perf_counter()
-        first_logits = self._prefill(tokens, cache, valid)
+        first_logits = self._prefill(tokens, cache, valid, sum(len(p) for p in prompts))
         if timings is not None:
             torch.cuda.synchronize()
             timings["prefill_s"] = time.perf_counter() - t0
@@ -557,7 +567,7 @@ class Decoder:
         tokens, valid = left_padded(prompts, dev)
         B, P = tokens.shape
         cache = KVCache(self.s, B, P + max_new_tokens, dtype, dev)
-        logits = self._prefill(tokens, cache, valid)
+        logits = self._prefill(tokens, cache, valid, sum(len(p) for p in prompts))
         first_logits = logits
         out = torch.zeros(B, max_new_tokens, dtype=torch.long, device=dev)
         steps = 0

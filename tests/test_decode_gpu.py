@@ -707,12 +707,13 @@ def test_a_prompts_pass_equals_its_launches_one_by_one(kw, B, T, pad, own_gemm, 
     for apart in (False, True):
         if own_gemm:   # the library's GEMM need not sum in the order of the tiles
             monkeypatch.setattr(D, "PACKED_GEMM_MIN_ROWS", 0)
+            monkeypatch.setattr(D, "PACKED_GEMM_MAX_REAL", 1)
             monkeypatch.setattr(kernels, "project", lambda x, weight: (
                 kernels.ext().dense_gemm if s.heads * s.head_dim >= 256 else kernels.dense)(x, weight))
         if apart:
             monkeypatch.setattr(dec, "_takes_prompt_pass", lambda *a: False)
         cache = D.KVCache(s, B, T + 75, torch.float16, "cuda")
-        first = dec.prefill_fused(tokens, cache, valid if pad else None)
+        first = dec.prefill_fused(tokens, cache, valid if pad else None, int(lengths.sum()) if pad else None)
         more = dec.prefill_fused(tokens[:, -66:], cache)
         outs.append((first, more, cache.k, cache.v, cache.real, cache.next_position, torch.tensor(cache.filled)))
     for a, b in zip(*outs):
@@ -738,6 +739,30 @@ def test_a_short_prompts_pass_equals_its_launches_one_by_one(kw, B, T, monkeypat
         outs.append((dec.prefill_fused(tokens, cache, valid), dec.prefill_fused(tokens, cache), cache.k, cache.v, cache.real, cache.next_position))
     for a, b in zip(*outs):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("lengths,own", [([300] * 8, 0), ([300] * 7 + [299], 0), ([2000, 480], 1), ([300] + [230] * 9, 1), ([300, 230], 0)])
+def test_prompts_projections_stop_at_the_padding_where_there_is_enough(lengths, own, monkeypatch):
+    """Batches without padding, with next to none and with a fifth of it and more, of two prompts and of many, through
+    generate, which knows the lengths: the projections on the rows that exist only where that is the faster way. A
+    mask that comes without a count may have no padding, and a wrong count changes nothing but the way."""
+    s, w, _ = model(7, 1, experts=4, top_k=4)   # no router's tie: every expert is taken
+    dec = D.Decoder(s, w)
+    ext, calls = kernels.ext(), []
+    dense_gemm = ext.dense_gemm
+    monkeypatch.setattr(ext, "dense_gemm", lambda *a: calls.append(0) or dense_gemm(*a), raising=False)
+    g = torch.Generator().manual_seed(len(lengths))
+    prompts = [torch.randint(3, s.vocab, (n,), generator=g).tolist() for n in lengths]
+    _, first = dec.generate(prompts, 1, return_first_logits=True)
+    assert len(calls) == 2 * s.layers * own
+    tokens, valid = D.left_padded(prompts, "cuda")
+    for count in (None, 1, tokens.numel()):
+        calls.clear()
+        cache = D.KVCache(s, len(lengths), tokens.shape[1] + 1, torch.float16, "cuda")
+        logits = dec.prefill_fused(tokens, cache, valid) if count is None else dec.prefill_fused(tokens, cache, valid, real_tokens=count)
+        assert count == 1 or not calls
+        assert (logits.float() - first.float()).abs().max() <= 2e-2
+        assert torch.equal(cache.real[:, :-1], valid) and torch.equal(cache.next_position, valid.sum(1))
 
 
 @pytest.mark.parametrize("rows,count,Nout,K", [(1, 1, 8, 256), (31, 31, 300, 256), (700, 0, 256, 256), (700, 1, 256, 256), (3000, 2111, 520, 320),
