@@ -337,6 +337,15 @@ class Decoder:
                 and (valid is None or (valid.dtype == torch.bool and valid.shape == tokens.shape and valid.device == tokens.device))
                 and cache.real.device == tokens.device)
 
+    def _packed_projections(self, rows, real_tokens):
+        """Whether a packed batch's projections stop at the rows that exist: enough padding, and weights that the tiles take, whose
+        loads are of 16 aligned bytes (a slice of a larger buffer may begin anywhere; the library's GEMM takes any)."""
+        from . import kernels
+
+        weights = self._stacked_qkv() + [L["wo"] for L in self.w["layers"]]
+        return (real_tokens is not None and rows >= PACKED_GEMM_MIN_ROWS and real_tokens <= PACKED_GEMM_MAX_REAL * rows
+                and all(t.is_contiguous() and t.data_ptr() % 16 == 0 and kernels.ext().dense_gemm_ok(rows, *t.shape) for t in weights))
+
     def _prompt_pass(self, tokens, cache, valid, wqkv, real_tokens=None):
         """prefill_fused in two host calls a layer beside the projections. The padding of a batch that starts its cache is
         one row for every launch (csrc/prompt.hip); which rows exist only the device knows, so the projections run on
@@ -352,11 +361,7 @@ class Decoder:
         positions, after, rows = E.prompt_span(tokens, valid, first, cache.real, cache.next_position, pack)
         p = E.prompt_pass(W["layers"], W["final_norm"], tokens, positions, first, cache.real, rows, cache.k, cache.v, self.cos, self.sin,
                           s.heads, s.kv_heads, s.head_dim, s.top_k, s.norm_topk_prob, s.rms_eps, s.clip_qkv, kernels.GEMV_MAX_TOKENS)
-        count = None
-        if (pack and real_tokens is not None and B * T >= PACKED_GEMM_MIN_ROWS and real_tokens <= PACKED_GEMM_MAX_REAL * B * T
-                and all(E.dense_gemm_ok(B * T, *t.shape) for t in (wqkv[0], W["layers"][0]["wo"]))
-                and all(L["wo"].is_contiguous() for L in W["layers"])):
-            count = rows[3]
+        count = rows[3] if pack and self._packed_projections(B * T, real_tokens) else None
         project = kernels.project if count is None else lambda x, w: E.dense_gemm(x, w, count)
         xn = p.embed(W["embed"], W["layers"][0]["attn_norm"])
         for i in range(s.layers):

@@ -202,3 +202,17 @@ def test_the_kernels_are_not_silently_replaced_on_the_cpu():
     assert m.fused is False
     with pytest.raises(RuntimeError):
         m.forward(torch.tensor([[3, 4, 5]]))      # the default hook calls the HIP kernels: CPU tensors are refused
+
+
+def test_packed_projections_take_weights_that_are_aligned_and_contiguous():
+    """The tiles load 16 aligned bytes: an output projection that begins anywhere else goes to the library's GEMM."""
+    s = D.Shape(vocab=64, hidden=256, intermediate=64, layers=2, heads=4, kv_heads=4, head_dim=64, experts=8, top_k=2)
+    dec = D.Decoder(s, D.random_weights(s, device="cpu", seed=0))
+    assert dec._packed_projections(4096, 3000) and dec._packed_projections(2048, 1)
+    assert not any(dec._packed_projections(*a) for a in ((4096, None), (4096, 4096), (4096, 3500), (2047, 1)))
+    wo, buffer = dec.w["layers"][1]["wo"], torch.empty(256 * 512 + 8, dtype=torch.float16)
+    for other in (buffer[1:1 + 256 * 256].view(256, 256), buffer[4:4 + 256 * 256].view(256, 256), wo.t(), buffer[:256 * 512].view(256, 512)[:, ::2]):
+        dec.w["layers"][1]["wo"] = other
+        assert not dec._packed_projections(4096, 3000)
+    dec.w["layers"][1]["wo"] = buffer[8:8 + 256 * 256].view(256, 256)
+    assert dec._packed_projections(4096, 3000)
