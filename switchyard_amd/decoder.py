@@ -329,11 +329,12 @@ class Decoder:
         experts = [x["router"].shape[0] for x in L]
         if B * T > kernels.OWN_ROUTER_MAX_TOKENS:
             takes = B * T > E.PROMPT_FEW_ROWS and E.router_route_ok(B * T, s.hidden, max(experts), s.top_k)
-        else:
-            takes = 1 <= B * T <= E.PROMPT_FEW_ROWS and max(experts) <= 128 and s.top_k <= min(8, *experts)
+        else:   # (the launches one by one leave the router to the library's GEMM, and the experts may be more than it has rows)
+            takes = (1 <= B * T <= E.PROMPT_FEW_ROWS and max(experts) <= 128 and s.top_k <= min(8, *experts)
+                     and all(x["router"].is_contiguous() and len(x["router"]) == len(x["gate_up"]) for x in L))
         return (self._own_moe and takes and tokens.dtype == i64 and (n, b) == (len(L), B) and E.prefill_attention_ok(cache.filled + T, capacity, D)
                 and cache.k.is_contiguous() and cache.v.is_contiguous() and cache.real.is_contiguous()
-                and cache.next_position.dtype == i64 and cache.next_position.is_contiguous()
+                and cache.next_position.dtype == i64 and cache.next_position.shape == (B,) and cache.next_position.is_contiguous()
                 and (valid is None or (valid.dtype == torch.bool and valid.shape == tokens.shape and valid.device == tokens.device))
                 and cache.real.device == tokens.device)
 

@@ -741,6 +741,33 @@ def test_a_short_prompts_pass_equals_its_launches_one_by_one(kw, B, T, monkeypat
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("change", ["router transposed", "router strided", "more experts than the router has rows", "one position for all"])
+@pytest.mark.parametrize("B,T", [(1, 5), (2, 15)])
+def test_a_short_prompt_takes_what_the_launches_one_by_one_take(change, B, T):
+    """Up to 64 rows the router may be any view, the experts more than it has rows, and the position of a cache that starts
+    one number; the results are those of the plain layout."""
+    s, w, _ = model(7, 1, experts=16, top_k=16 // 2)
+    tokens = torch.randint(3, s.vocab, (B, T), generator=torch.Generator().manual_seed(B)).cuda()
+    outs = []
+    for changed in (False, True):
+        cache = D.KVCache(s, B, T + 1, torch.float16, "cuda")
+        if changed:
+            for L in w["layers"]:
+                if change == "router transposed":
+                    L["router"] = L["router"].t().contiguous().t()
+                elif change == "router strided":
+                    L["router"] = torch.cat([L["router"], L["router"]], 1)[:, :s.hidden]
+                elif change.startswith("more"):
+                    L["gate_up"], L["down"] = (torch.cat([L[n], L[n][:3]]) for n in ("gate_up", "down"))
+            if change.startswith("one"):
+                cache.next_position = torch.zeros(1, dtype=torch.long, device="cuda")
+        outs.append((D.Decoder(s, w).prefill_fused(tokens, cache), cache.k, cache.v, cache.next_position))
+    (a, ka, va, pa), (b, kb, vb, pb) = outs
+    assert torch.equal(pa, pb)
+    # the router's logits differ by the order of their sums, so a nearly tied choice may differ
+    assert all(((x.float() - y.float()).abs() > 2e-2).float().mean() <= 0.05 for x, y in ((a, b), (ka, kb), (va, vb)))
+
+
 @pytest.mark.parametrize("lengths,own", [([300] * 8, 0), ([300] * 7 + [299], 0), ([2000, 480], 1), ([300] + [230] * 9, 1), ([300, 230], 0)])
 def test_prompts_projections_stop_at_the_padding_where_there_is_enough(lengths, own, monkeypatch):
     """Batches without padding, with next to none and with a fifth of it and more, of two prompts and of many, through
