@@ -146,10 +146,20 @@ def dense(x, weight):
 def project(x, weight):
     """`dense` inside the decoder's fused passes (f16 on the GPU, no gradients): where there are a few dozen
     rows and the library's own tiles take the shape, they do (64 rows, [2048, 2048]: 6.9 us against 11.0)."""
-    if (x.shape[0] > 16 and weight.is_contiguous() and weight.dtype == torch.float16 and weight.data_ptr() % 16 == 0
-            and ext().dense_tiles_ok(x.shape[0], *weight.shape)):
+    if (x.shape[0] > 16 and _tiles_pay(*weight.shape) and weight.is_contiguous() and weight.dtype == torch.float16
+            and weight.data_ptr() % 16 == 0 and ext().dense_tiles_ok(x.shape[0], *weight.shape)):
         return ext().dense_tiles(x, weight)
     return dense(x, weight)
+
+
+def _tiles_pay(Nout, K):
+    """Whether the own tiles are the faster ones for weights [Nout, K], at any number of rows that they take. A tile sums all of K
+    in one workgroup, and few columns are few tiles; the library's GEMM cuts K into parts. us for 17 to 256 rows in a replayed
+    graph, the library's and the own: K = 2048 with 192 columns 7.9 to 8.1 and 6.5 to 6.7, 64 columns 5.2 to 8.0 and 6.3 to 6.5;
+    K = 2304 with 1024 columns 6.2 to 9.1 and 7.2 to 8.5, 2048 columns 8.2 to 12.9 and 7.6 to 11.9; K = 3584 with 5120 columns 13.6
+    to 19.3 and 12.9 to 17.3 (33 rows: 14.4 and 16.6); K = 4096 with 512 columns 8.1 to 8.9 and 10.5 to 10.8; K = 8192 with 2048
+    columns 13.2 to 26.9 and 19.4 to 32.2. On this side of the line the own tiles won at 623 of 624 sizes from K = 128 up."""
+    return K <= 2048 and Nout >= 192 or K <= 3072 and Nout >= 2048
 
 
 # Up to this many tokens route and sort run as one launch of one workgroup (a decode step is

@@ -856,6 +856,21 @@ def test_dense_tiles_limits():
     assert torch.equal(kernels.project(x, w), F.linear(x, w))   # weights that are not contiguous go to the library
 
 
+@pytest.mark.parametrize("rows,Nout,K,own", [(17, 192, 2048, True), (256, 2048, 2048, True), (64, 6144, 2048, True), (33, 2048, 3072, True),
+                                            (64, 128, 2048, False), (33, 2047, 2176, False), (32, 512, 4096, False), (17, 2048, 8192, False),
+                                            (65, 6144, 2048, False), (16, 2048, 2048, False)])
+def test_projections_run_on_the_tiles_where_those_are_faster(rows, Nout, K, own, monkeypatch):
+    """Long sums and few columns, many tiles and few rows are for the other kernels, with the same result."""
+    ext, calls = kernels.ext(), []
+    tiles = ext.dense_tiles
+    monkeypatch.setattr(ext, "dense_tiles", lambda *a: calls.append(0) or tiles(*a), raising=False)
+    x, w = rnd(rows, K, seed=91), rnd(Nout, K, seed=92, std=0.03)
+    got, want = kernels.project(x, w).double(), x.double() @ w.double().T
+    assert len(calls) == own
+    size = x.double().abs() @ w.double().abs().T   # the bound of test_dense_tiles
+    assert ((got - want).abs() <= want.abs() * 2.0 ** -11 + size * K * 2.0 ** -24 + 2.0 ** -24).all()
+
+
 def model(seed, batch, **kw):
     s = D.Shape(**{**dict(vocab=1000, hidden=512, intermediate=256, layers=3, heads=8, kv_heads=8, head_dim=64, experts=64,
                           top_k=8), **kw})
