@@ -298,8 +298,9 @@ gemv_kernel(const half_t* __restrict__ A, const int* __restrict__ a_rows, const 
     p.r0 = r0;
     p.nr = nr;
     const half8_t zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
-    // DENSE: the rows are asked for first, then the first weights, and the rows go to LDS behind those
-    const bool early = DENSE && nq * QUAD <= EARLY_ROWS * waves && K <= EARLY_CHUNKS * WAVE * 8;
+    // DENSE: the rows are asked for first, then the first weights, and the rows go to LDS behind those (but not 9 to 12
+    // short rows, whose weights are few: K = 256 to 6144 columns 5.9 us so, 5.0 with the rows in LDS first)
+    const bool early = DENSE && nq * QUAD <= EARLY_ROWS * waves && K <= EARLY_CHUNKS * WAVE * 8 && (nq != 3 || K > 1024);
     half8_t x[EARLY_ROWS][EARLY_CHUNKS];
     if (early) {
 #pragma unroll
@@ -494,15 +495,21 @@ gemv_kernel(const half_t* __restrict__ A, const int* __restrict__ a_rows, const 
 
 // Workgroups per compute unit and wavefronts per workgroup of a DENSE launch, for `units` units per compute
 // unit. The wavefronts of a compute unit take its units in rounds and the last round should be full: the
-// number of wavefronts, up to 12 (more only take registers from the loads in flight), with the fewest places
-// left empty, the most wavefronts where that is equal. 6 units (q/k/v of 2048, 6144 columns on 256 compute units) are 6
-// wavefronts in one workgroup, 2 (output projection) are 2, and 49 (50 304 columns) are 10 in two, where 4
+// number of wavefronts with the fewest places left empty, the most wavefronts where that is equal. 6 units (q/k/v of
+// 2048, 6144 columns on 256 compute units) are 6 wavefronts in one workgroup, 2 (output projection) are 2, where 4
 // wavefronts to a workgroup and a unit to a wavefront left 128 compute units with half the work of the others
-// or none: q/k/v and output projection on average 8.1 -> 6.9 us a launch with one row, 8.6 -> 7.5 with 8. A single workgroup gets as many wavefronts as ask for its rows in one go, with or
-// without units of their own.
-void dense_shape(long units, int rows, long fit, long& per_cu, int& waves) {
-  long best = 1, spare = units + 12;
-  for (long n = 1; n <= 12; ++n) {
+// or none: q/k/v and output projection on average 8.1 -> 6.9 us a launch with one row, 8.6 -> 7.5 with 8.
+// Up to 8 wavefronts where a unit is 16 KB or more, whose loads keep the compute unit busy: 50 304 columns (50 units), us with 8
+// and with 10 in two workgroups: K = 2048 36.5 and 37.0 with one row, 37.0 and 38.4 with 8, 41.5 and 43.8 with 16; K = 4096
+// 68.8 and 72.2, 67.3 and 75.0, 72.9 and 77.0. Shorter units wait more than they load, and up to 12 hide more of it: K = 1024 with
+// 8 rows, 10 240 columns, 8.4 in 8 wavefronts and 7.2 in 12 (K = 256: 5.7 and 5.3).
+// A single workgroup gets as many wavefronts as ask for its rows in one go, with or without units of their own: two
+// rows each in registers, or one each where the rows are too long for that (K = 3072 to 3072 columns, 4 rows: 8.1 us with 3
+// wavefronts, 7.3 with more).
+void dense_shape(long units, int rows, int K, long fit, long& per_cu, int& waves) {
+  const int most = K * UNIT_COLS * 2 >= 16384 ? DENSE_MAX_WAVES : 12;
+  long best = 1, spare = units + most;
+  for (long n = 1; n <= most; ++n) {
     const long left = (units + n - 1) / n * n - units;
     if (n > units && n > 1) break;
     // fewer wavefronts than 8 only where they are a round by themselves
@@ -515,7 +522,7 @@ void dense_shape(long units, int rows, long fit, long& per_cu, int& waves) {
   per_cu = (best + DENSE_MAX_WAVES - 1) / DENSE_MAX_WAVES;
   per_cu = per_cu > fit ? (fit > 0 ? fit : 1) : per_cu;
   waves = (int)((best + per_cu - 1) / per_cu);
-  const int ask = (rows + EARLY_ROWS - 1) / EARLY_ROWS;
+  const int ask = K <= EARLY_CHUNKS * WAVE * 8 ? (rows + EARLY_ROWS - 1) / EARLY_ROWS : rows;
   if (per_cu == 1 && waves < ask) waves = ask;
   waves = waves > DENSE_MAX_WAVES ? DENSE_MAX_WAVES : waves;
 }
@@ -552,7 +559,7 @@ int launch_gemv(const void* A, const int32_t* a_rows, const void* B, const int32
   int waves = GEMV_WAVES;
   if (dense) {
     const long cus = sy_compute_units();
-    dense_shape((max_units + cus - 1) / cus, row_cap, fit, per_cu, waves);
+    dense_shape((max_units + cus - 1) / cus, row_cap, K, fit, per_cu, waves);
     grid = cus * per_cu;
     grid = grid > max_units ? max_units : grid;
   }

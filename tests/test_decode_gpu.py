@@ -821,7 +821,7 @@ def test_dense_projection(rows, Nout, K):
 
 @pytest.mark.parametrize("rows", [1, 3, 4, 5, 8, 9, 16, 17, 33])
 @pytest.mark.parametrize("Nout,K", [(6144, 2048), (2048, 1024), (1001, 2048), (7, 512), (130, 520), (36, 4096), (64, 8),
-                                    (4100, 3072)])
+                                    (4100, 3072), (12000, 512)])   # the last in two workgroups to a compute unit
 def test_dense_rows_equal_the_weight_stream_of_one_expert(rows, Nout, K):
     """Rows staged early and late, chunks of both lengths, ragged edges, several passes over 16 rows."""
     x, w = rnd(rows, K, seed=51), rnd(Nout, K, seed=52, std=0.03)
