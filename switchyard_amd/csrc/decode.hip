@@ -66,6 +66,7 @@ __device__ __forceinline__ float block_sum_of_four(float v, float* lds) {
 }
 
 constexpr int FEW_ROWS = 64;   // up to these the row kernels are built for a short chain of waits, not for many wavefronts
+constexpr int FEW_MIN_K = 4;   // ... where a token has at least so many rows to combine: it asks for AT_ONCE rows, used or not
 constexpr int ROW_MAX_K = 64;  // choices per token the combining variant ranks in one wavefront
 
 // One workgroup per token (row). The residual `delta` is either a tensor, or (COMBINE) the
@@ -87,7 +88,8 @@ constexpr int ROW_MAX_K = 64;  // choices per token the combining variant ranks 
 // (with COMBINE) takes the expert outputs of token twin[t] (front.hip).
 // FEW (with COMBINE): a launch of few rows is a chain of waits. The norm's weights and the row are asked for
 // first, and a token's choices are ranked without LDS and their rows of y asked for together (combine_core.h):
-// one row 5.2 -> 4.4 us a launch, 8 rows 5.6 -> 5.0. It takes 26 more registers, and with many rows it is
+// one row 5.2 -> 4.4 us a launch, 8 rows 5.6 -> 5.0. (A replayed graph of such launches, 8 rows of 2048: top-8 4.20 -> 3.73, top-5
+// 3.71 -> 3.58, top-4 3.48 -> 3.53 and rows of 3072 4.31 -> 4.13; top-2 would be 3.11 -> 3.42, top-1 3.01 -> 3.35.) It takes 26 more registers, and with many rows it is
 // the wavefronts in flight that count: 437 rows 6.7 -> 7.3, 4096 rows 31.9 -> 33.2.
 // COUNTED (and PACKED, which is EMBEDDED for such rows): only the first *count of the launch's rows exist (prompt.hip);
 // PACKED looks up row t by gather[map[t]].
@@ -1205,7 +1207,7 @@ int sy_combine_add_rmsnorm_twins(const void* y, const int32_t* pos_of, const int
   SY_REQUIRE(!twin || !count, "combine_add_rmsnorm: rows that exist once have no twins");
   auto kern = twin ? row_kernel<true, false, 0, TWINNED>
               : count ? row_kernel<true, false, 0, COUNTED>
-              : N <= FEW_ROWS && k <= combine_core::AT_ONCE ? row_kernel<true, false, 0, OWN_ROWS, true> : row_kernel<true, false>;
+              : N <= FEW_ROWS && k >= FEW_MIN_K && k <= combine_core::AT_ONCE ? row_kernel<true, false, 0, OWN_ROWS, true> : row_kernel<true, false>;
   kern<<<N, ROW_THREADS, 0, (hipStream_t)stream>>>(
       (const half_t*)x, (const half_t*)w, (const half_t*)y, pos_of, idx, k, (const half_t*)weight, eps, nullptr, 0, H,
       (half_t*)x_out, (half_t*)h_out, nullptr, nullptr, 0, front_core::Outputs{}, twin, nullptr, 0, count, nullptr);

@@ -106,7 +106,7 @@ def test_combine_add_rmsnorm(N, H, E, k):
 
 
 @pytest.mark.parametrize("N", [1, 64, 65])   # 64: the last of the launches for few rows
-@pytest.mark.parametrize("H,k", [(8, 1), (2048, 3), (2056, 8), (8192, 8), (512, 9)])   # 9: more choices than are ranked in registers
+@pytest.mark.parametrize("H,k", [(8, 1), (2048, 3), (64, 4), (4096, 5), (2056, 8), (8192, 8), (512, 9)])   # 4 to 8 are ranked in registers
 def test_combine_add_rmsnorm_of_few_rows(N, H, k):
     """The rows in any order of ids, ids that repeat inside a token among them: the bits of the two launches."""
     E = 16
