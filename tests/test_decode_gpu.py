@@ -793,17 +793,25 @@ def test_prompts_projections_stop_at_the_padding_where_there_is_enough(lengths, 
 
 
 @pytest.mark.parametrize("rows,count,Nout,K", [(1, 1, 8, 256), (31, 31, 300, 256), (700, 0, 256, 256), (700, 1, 256, 256), (3000, 2111, 520, 320),
-                                              (5000, 5000, 1000, 256), (9000, 8999, 264, 512)])
+                                              (5000, 5000, 1000, 256), (9000, 8999, 264, 512),
+                                              # (on 256 compute units) three rounds of 128 rows that become two of 160; three of 192, two
+                                              # of 224; three of 256; the same with next to no rows; two of 256; six of 256
+                                              (4096, 3080, 6144, 256), (6000, 4500, 6144, 320), (8192, 8192, 6144, 256), (8192, 100, 6144, 256),
+                                              (16384, 16384, 2048, 256), (16000, 15999, 6144, 256)])
 def test_dense_gemm_of_the_rows_that_exist(rows, count, Nout, K):
-    """Few and many tiles, one round and several, heights from 32 to 256: an in-order fp32 sum (the bound of
-    test_dense_tiles), and rows past the count untouched."""
+    """Few and many tiles, one round and several, heights from 32 to 256, with the loads of missing rows and without: an
+    in-order fp32 sum (the bound of test_dense_tiles), and rows past the count untouched."""
+    ext = kernels.ext()
     x, w = rnd(rows, K, seed=81), rnd(Nout, K, seed=82, std=0.05)
     x[count:] = float("nan")
-    n = torch.tensor([count], dtype=torch.int32, device="cuda")
-    got = kernels.ext().dense_gemm(x, w, n)[:count].double()
+    n, out = torch.tensor([count], dtype=torch.int32, device="cuda"), torch.full((rows, Nout), 7.0, dtype=torch.float16, device="cuda")
+    ext._call(ext.lib.sy_dense_gemm, x.data_ptr(), w.data_ptr(), rows, n.data_ptr(), Nout, K, out.data_ptr(),
+              torch.cuda.current_stream().cuda_stream)
+    assert (out[count:] == 7).all()
+    got = out[:count].double()
     want, size = x[:count].double() @ w.double().T, x[:count].double().abs() @ w.double().abs().T
     assert ((got - want).abs() <= want.abs() * 2.0 ** -11 + size * K * 2.0 ** -24 + 2.0 ** -24).all()
-    assert torch.equal(got.half(), kernels.ext().dense_gemm(x[:count].contiguous(), w))   # whatever tiles its count makes
+    assert torch.equal(got.half(), ext.dense_gemm(x[:count].contiguous(), w))   # whatever tiles its count makes
 
 
 @pytest.mark.parametrize("rows,Nout,K", [(1, 6144, 2048), (8, 6144, 2048), (8, 2048, 2048), (16, 2048, 2048), (8, 50304, 2048),
@@ -834,8 +842,8 @@ def test_dense_rows_equal_the_weight_stream_of_one_expert(rows, Nout, K):
                                         (33, 2048, 2048), (64, 2048, 2048), (65, 2048, 2048), (128, 2048, 2048), (129, 2048, 2048),
                                         (256, 2048, 2048), (48, 2041, 128), (50, 3001, 384), (31, 100, 4096), (64, 6145, 640)])
 def test_dense_tiles(rows, Nout, K):
-    """Every tile, at the last and first rows of each, ragged columns, a ring longer than K: an in-order sum of
-    fp32 products, one rounding. fp32 sums in another order differ by K rounding errors of 2^-24 at most, which
+    """Every tile, at the last and first rows of each, ragged columns, a ring longer than K: a sum of fp32 products in some
+    order, one rounding. fp32 sums in another order differ by K rounding errors of 2^-24 at most, which
     is far below half an fp16 ulp of a result of the size of the terms' sum."""
     ext = kernels.ext()
     assert ext.dense_tiles_ok(rows, Nout, K)
@@ -844,6 +852,40 @@ def test_dense_tiles(rows, Nout, K):
     want = x.double() @ w.double().T
     size = x.double().abs() @ w.double().abs().T
     assert ((got - want).abs() <= want.abs() * 2.0 ** -11 + size * K * 2.0 ** -24 + 2.0 ** -24).all()
+
+
+@pytest.mark.parametrize("rows,Nout,K", [(17, 2048, 2048), (64, 2048, 2048), (31, 100, 4096), (1, 16, 256)])
+def test_the_smallest_dense_tiles_four_accumulators(rows, Nout, K):
+    """Where there are no more tiles of 32 x 16 than compute units, every fourth step of 32 of K has an accumulator of its own, and
+    the four are added up in order. One product in every step, whole numbers up to 2^28 that cancel inside each accumulator
+    over another step's: what is left is the roundings of fp32, a small whole number that shows the order and that f16 holds.
+    Each accumulator alone comes from the grouped kernel, in order, with the other steps zero."""
+    ext, g, steps = kernels.ext(), torch.Generator().manual_seed(rows), K // 32
+    assert -(-rows // 32) * -(-Nout // 16) <= torch.cuda.get_device_properties(0).multi_processor_count
+    whole = lambda n: torch.randint(-2047, 2048, (n, steps // 2), generator=g) * 2.0 ** torch.randint(0, 4, (n, steps // 2), generator=g)
+    mine = torch.cat([u + 4 * torch.randperm(steps // 4, generator=g) for u in range(4)]).view(-1, 2)   # pairs of steps of one accumulator
+    place = 32 * mine + torch.randint(32, mine.shape, generator=g)
+    x, w, a, b = torch.zeros(rows, K), torch.zeros(Nout, K), whole(rows), whole(Nout)
+    x[:, place[:, 0]], x[:, place[:, 1]] = a, -a
+    w[:, place[:, 0]] = w[:, place[:, 1]] = b
+    x, w = x.half().cuda(), w.half().cuda()
+    offsets = torch.tensor([0, rows], dtype=torch.int32, device="cuda")
+    in_order = lambda y: ext.grouped_gemm(y.contiguous(), None, w[None], offsets, None, 0, rows, False, None).float()
+    step = torch.arange(K, device="cuda") // 32
+    parts = [in_order(torch.where(step % 4 == u, x, 0)) for u in range(4)]
+    want = ((parts[0] + parts[1]) + parts[2]) + parts[3]
+    assert max(p.abs().max() for p in parts) <= 2048 and (K < 2048 or (want != in_order(x)).float().mean() > 0.25)
+    assert torch.equal(ext.dense_tiles(x, w).float(), want)
+
+
+@pytest.mark.parametrize("rows,Nout,K", [(32, 6144, 2048), (65, 2048, 2048), (128, 2041, 384), (17, 5000, 640),      # 32 x 32
+                                        (33, 6144, 2048), (129, 2048, 2048), (256, 2048, 640)])              # 64 x 32
+def test_larger_dense_tiles_sum_in_order(rows, Nout, K):
+    """The bits of the grouped kernel with one expert."""
+    x, w = rnd(rows, K, seed=71), rnd(Nout, K, seed=72, std=0.03)
+    offsets = torch.tensor([0, rows], dtype=torch.int32, device="cuda")
+    want = kernels.ext().grouped_gemm(x, None, w[None], offsets, None, 0, rows, False, None)
+    assert torch.equal(kernels.ext().dense_tiles(x, w), want)
 
 
 def test_dense_tiles_limits():
@@ -882,8 +924,8 @@ def model(seed, batch, **kw):
 
 @pytest.mark.parametrize("batch,kw", [(6, {}), (6, {"kv_heads": 2}), (6, {"head_dim": 128, "heads": 4, "kv_heads": 4}),
                                       (6, {"clip_qkv": 0.5}), (6, {"norm_topk_prob": True}),
-                                      # 64 sequences: route and sort as two launches, MFMA tiles for the experts, library
-                                      # GEMMs for the projections, four wavefronts per (sequence, head) in attention
+                                      # 64 sequences: MFMA tiles for the experts and the projections (the lm_head on the library's
+                                      # GEMM), four wavefronts per (sequence, head) in attention
                                       (64, {}), (17, {"kv_heads": 4})])
 def test_a_step_on_the_decode_kernels_gives_the_logits_of_the_torch_step(batch, kw):
     """Same weights, same prefilled cache, one new token per sequence of a left-padded batch:
