@@ -274,11 +274,11 @@ row_kernel(const half_t* x, const half_t* __restrict__ delta, const half_t* __re
 
 // The router's logits of a few rows for a launch that routes by itself (gemv.hip), with NORM behind the residual add and the
 // norm: every token's experts are dealt to E / 4 workgroups, one to a wavefront. A workgroup that has a token's whole router to
-// read waits for 256 KB at the 60 to 70 bytes a clock that a compute unit pulls from L2, then routes: 6.9 us a launch with one
+// read waits for 256 KB at the 55 to 57 bytes a clock that a compute unit pulls from L2, then routes: 6.9 us a launch with one
 // row and 7.6 with 8. Here the router's rows are asked for with the token's, and the norm, which every workgroup of the token
 // computes for itself, runs while they are on their way: 2.8 and 4.8, and the stream behind it takes 1.0 and 2.2 more to
 // route. x_out must not be x: other workgroups may still have x to read.
-constexpr int SPREAD_THREADS = ROW_THREADS, SPREAD_WAVES = SPREAD_THREADS / WAVE, SPREAD_H = SPREAD_THREADS * 8;
+constexpr int SPREAD_THREADS = ROW_THREADS, SPREAD_WAVES = SPREAD_THREADS / WAVE, SPREAD_H = SPREAD_THREADS * 8, SPREAD_ROWS = 8;
 template <bool NORM>
 __global__ void __launch_bounds__(SPREAD_THREADS)
 logits_spread_kernel(const half_t* __restrict__ x, const half_t* __restrict__ delta, const half_t* __restrict__ weight, float eps,
@@ -1153,7 +1153,7 @@ int sy_router_route_rows(const void* h, const void* router, int N, int H, int E,
 
 int sy_logits_spread(const void* x, const void* delta, const void* weight, float eps, const void* router, int E, int N, int H,
                      void* x_out, void* h_out, void* logits, void* stream) {
-  SY_REQUIRE(N >= 1 && N <= FEW_ROWS && E >= 1 && E <= 128 && H == SPREAD_H, "logits_spread: N = %d, E = %d, H = %d", N, E, H);
+  SY_REQUIRE(N >= 1 && N <= SPREAD_ROWS && E >= 1 && E <= 128 && H == SPREAD_H, "logits_spread: N = %d, E = %d, H = %d", N, E, H);
   SY_REQUIRE(x && router && logits && (!weight || (delta && x_out && h_out && x_out != x)), "logits_spread: null pointer, or x_out is x");
   const dim3 grid((unsigned)((E + SPREAD_WAVES - 1) / SPREAD_WAVES), (unsigned)N);
   void (*kern)(const half_t*, const half_t*, const half_t*, float, const half_t*, int, half_t*, half_t*, half_t*) =

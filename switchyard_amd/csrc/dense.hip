@@ -1,9 +1,9 @@
 // dense_tiles: x [rows, K] @ weight [Nout, K]^T for a few dozen rows: the projections around the MoE layer where a
 // step has more sequences than the weight stream (gemv.hip) is for, and of short prompts.
 //
-// What bounds such a product is a compute unit's pull of operands (about 20 bytes a clock by loads that write LDS
-// directly), the latency of a launch's first loads and the barriers of its K loop; the MFMAs need a fraction of
-// the time. So the tile is chosen to put one tile on each compute unit with as few rows and columns together as
+// What bounds such a product is the latency of a launch's first loads, weights out of HBM among them, and the barriers of its
+// K loop: the tiles get 20 to 25 bytes a clock and compute unit of the 55 to 57 that loads straight to LDS bring from L2 in a
+// loop of nothing else. The MFMAs need a fraction of the time. So the tile is chosen to put one tile on each compute unit with as few rows and columns together as
 // possible (pick_tile below), and the whole of LDS is a ring of K slices: rows and weight rows in slices of 64
 // (128 bytes: whole lines), up to fourteen deep, by buffer loads that write LDS directly, XOR-swizzled by row so that
 // the operand reads spread over the banks, two slices to a barrier. The waits for the loads are counted by hand: the

@@ -8,8 +8,9 @@
 //   map[i]    the position of row i
 //   count     how many rows there are
 // and every launch of the pass works on `count` rows, which only the device knows: its grid is for all B T, and the
-// workgroups without rows leave at once. 8 prompts of 256 to 512 tokens: about 3200 rows for 4096, and a layer's projections
-// 138 -> 128 us, combine + norm 32.0 -> 29.1, add + norm 13.2 -> 11.2; 3 of 1000 to 2000: 181 -> 167, 44.1 -> 40.6, 18.3 -> 15.7.
+// workgroups without rows leave at once. 8 prompts of 256 to 512 tokens: about 3200 rows for 4096, and a layer's combine + norm
+// 32.0 -> 29.1 us, add + norm 13.2 -> 11.2; 3 of 1000 to 2000: 44.1 -> 40.6, 18.3 -> 15.7. The projections follow the count only where
+// the caller knows that there is enough padding (PACKED_GEMM_MAX_REAL in decoder.py).
 //
 // The host: mask, positions and counters were fourteen launches of PyTorch's (65 us) in front of the first layer, now two,
 // and a layer five calls beside its projections, now two: 128 tokens in 2489 us, now 2369.

@@ -277,6 +277,8 @@ class Decoder:
         wqkv = self._stacked_qkv()
         if self._takes_prompt_pass(tokens, cache, valid):
             return self._prompt_pass(tokens.contiguous(), cache, valid, wqkv, real_tokens)
+        # The launches one by one, for what the pass above does not take: a mask that is not bool or not [B, T], a cache that is
+        # not contiguous or longer than the own attention's masks, tokens that are not int64, a hook for the experts
         span = Span(tokens, cache, valid)
         slot = torch.tensor([span.first], dtype=torch.long, device=tokens.device)
         flat_positions = span.positions.reshape(-1).contiguous()
