@@ -269,7 +269,8 @@ class Decoder:
         and into the layouts of its neighbours.
 
         `real_tokens`: how many positions `valid` marks, if the caller knows (the pass reads nothing back from the GPU).
-        It chooses between launches that compute the same, and is no more than that: a wrong one costs time."""
+        It chooses between launches of the same products (whose order of sums may differ from the library's at some widths), and
+        is no more than that: a wrong one costs time."""
         from . import kernels
 
         s, W, E = self.s, self.w, kernels.ext()
