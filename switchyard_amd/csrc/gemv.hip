@@ -260,7 +260,8 @@ __host__ __device__ constexpr size_t sort_here_ints(int E) {
 //
 // ROUTE (with ALL, up to 64 experts): the launch starts from the router's logits and every workgroup routes the tokens
 // too, a wavefront two of them. The launch in front of it is then only the logits, which no workgroup has to have all
-// of, so that one is spread over the chip (logits_spread_kernel in decode.hip).
+// of, so that one is spread over the chip (logits_spread_kernel in decode.hip). Normalised weights have an instance of their
+// own: with both in one the prologue's instructions cost a layer of one token 0.1 us.
 //
 // DENSE: one matrix and `sort.M` rows of A in their own order (the projections around the MoE layer):
 // there is no list of experts to build, so a launch begins with its loads: the rows, then the first weights,
@@ -269,8 +270,9 @@ __host__ __device__ constexpr size_t sort_here_ints(int E) {
 constexpr int EARLY_ROWS = 2, EARLY_CHUNKS = 4;   // rows that a wavefront asks for ahead, in chunks of 64 x 16 bytes
 constexpr int ALL_ROWS = 8;                       // tokens of an ALL launch, a chunk of 16 bytes of each per thread
 constexpr int DENSE_MAX_WAVES = 8;
+constexpr int NO_ROUTE = 0, ROUTE_PLAIN = 1, ROUTE_NORMED = 2;
 
-template <bool SWIGLU, bool SCALE, bool EXACT, int CH, bool SORT = false, bool DENSE = false, bool ALL = false, bool ROUTE = false>
+template <bool SWIGLU, bool SCALE, bool EXACT, int CH, bool SORT = false, bool DENSE = false, bool ALL = false, int ROUTE = NO_ROUTE>
 __global__ void __launch_bounds__(DENSE ? DENSE_MAX_WAVES * WAVE : GEMV_THREADS)
 gemv_kernel(const half_t* __restrict__ A, const int* __restrict__ a_rows, const half_t* __restrict__ B,
             const int* __restrict__ offsets, int E, int Nout, int K, const half_t* __restrict__ scale,
@@ -392,7 +394,7 @@ gemv_kernel(const half_t* __restrict__ A, const int* __restrict__ a_rows, const 
       if (t < tokens) {
         int e;
         float p;
-        route_core::route_loaded<half_t, 1>(lg[i], E, sort.k, sort.norm, e, p);
+        route_core::route_picks<ROUTE == ROUTE_NORMED>(lg[i], E, sort.k, e, p);
         if (lane < sort.k) {
           s_pos[t * sort.k + lane] = e;
           s_wsorted[t * sort.k + lane] = __builtin_bit_cast(uint16_t, (half_t)p);
@@ -572,7 +574,9 @@ int launch_gemv(const void* A, const int32_t* a_rows, const void* B, const int32
   else if (dense) kern = exact ? gemv_kernel<false, false, true, CH_SHORT, false, true> : gemv_kernel<false, false, false, CH_SHORT, false, true>;
   // (more than 8 tokens have at most 64 choices only where k < 8; one row of LDS per token)
   else if (sort && long_chunks && exact && rows / sort->k <= ALL_ROWS && rows / sort->k <= row_cap && K <= GEMV_THREADS * 8)
-    kern = sort->logits ? gemv_kernel<true, false, true, CH_LONG, true, false, true, true> : gemv_kernel<true, false, true, CH_LONG, true, false, true>;
+    kern = !sort->logits ? gemv_kernel<true, false, true, CH_LONG, true, false, true>
+           : sort->norm  ? gemv_kernel<true, false, true, CH_LONG, true, false, true, ROUTE_NORMED>
+                         : gemv_kernel<true, false, true, CH_LONG, true, false, true, ROUTE_PLAIN>;
   else if (sort && long_chunks && exact) kern = gemv_kernel<true, false, true, CH_LONG, true>;
   else if (sort) kern = exact ? gemv_kernel<true, false, true, CH_SHORT, true> : gemv_kernel<true, false, false, CH_SHORT, true>;
   else if (swiglu && long_chunks && exact) kern = gemv_kernel<true, false, true, CH_LONG>;
